@@ -113,8 +113,8 @@ def _scale(types):
     return 0.25 if types in ("e4m3e4m3f16", "e5m2e5m2f16") else 1.0
 
 
-def prepare(case, seed):
-    tin, tout, dt_in, dt_out = TYPES[case["types"]]
+def _inputs(case, seed):
+    _, _, dt_in, dt_out = TYPES[case["types"]]
     m, n, k = case["m"], case["n"], case["k"]
     dev = torch.device("cuda", torch.cuda.current_device())
     gen = torch.Generator(device=dev).manual_seed(seed)
@@ -124,16 +124,37 @@ def prepare(case, seed):
             return torch.randint(-128, 128, (count,), generator=gen, device=dev, dtype=dtype)
         return (torch.randn(count, generator=gen, device=dev) * scale).to(dtype)
 
+    a, b = values(m * k, dt_in, 1.0), values(k * n, dt_in, case["scale_b"])
+    return a, b, values(m * n, dt_out, 1.0) if case["beta"] else None
+
+
+def prepare(case, seed):
+    tin, tout, _, dt_out = TYPES[case["types"]]
+    m, n, k = case["m"], case["n"], case["k"]
+    a, b, c = _inputs(case, seed)
     la, lb = LAYOUTS[case["a"]], LAYOUTS[case["b"]]
     kernel = functors.functor("auto_gemm", tin, tout, layout_a=la, layout_b=lb)(m, n, k, functors.DeviceProps.current())
-    return {"kernel": kernel, "a": values(m * k, dt_in, 1.0), "b": values(k * n, dt_in, case["scale_b"]),
-            "c": values(m * n, dt_out, 1.0) if case["beta"] else None,
-            "d": torch.empty(m, n, dtype=dt_out, device=dev), "beta": case["beta"], "stream": torch.cuda.current_stream()}
+    return {"kernel": kernel, "a": a, "b": b, "c": c, "d": torch.empty(m, n, dtype=dt_out, device=a.device),
+            "beta": case["beta"], "stream": torch.cuda.current_stream()}
 
 
 def run(state):
     state["kernel"](state["a"], state["b"], state["c"], state["d"], 1, state["beta"], state["stream"])
     return state["d"]
+
+
+def exact(case, seed):
+    """D in 64 bits: products and sums of the 8-bit and 16-bit types are exact there or nearly so."""
+    m, n, k = case["m"], case["n"], case["k"]
+    a, b, c = _inputs(case, seed)
+    # (8-bit floats widen through fp32: every value of theirs is one of fp32)
+    a, b = (x.float().double() for x in (a, b))
+    a = a.view(m, k) if case["a"] == "row" else a.view(k, m).t()
+    b = b.view(k, n) if case["b"] == "row" else b.view(n, k).t()
+    d = torch.matmul(a, b)
+    if c is not None:
+        d += c.double().view(m, n)
+    return d.round().long() if TYPES[case["types"]][3] == torch.int32 else d
 
 
 def work(case):
