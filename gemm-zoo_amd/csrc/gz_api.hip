@@ -157,6 +157,13 @@ static int resolve_rung(int types, int64_t M, int64_t N, int64_t K, int layoutA,
   return GZ_RUNG_MFMA;
 }
 
+static int check_named_skinny(int types, int M, int N, int K, int layoutA, int layoutB) {
+  if (skinny_supported(types, M, N, K, layoutA, layoutB)) return GZ_OK;
+  set_error("skinny rung needs a 16-bit float type with fp32 accumulation, row-major A, column-major B, 1 <= M <= %d and "
+            "K %% %d == 0 (M=%d K=%d)", SKINNY_MAX_M, SKINNY_K_STEP, M, K);
+  return GZ_ERR_UNSUPPORTED;
+}
+
 // Leading dimensions: 0 stands for the packed value; otherwise at least the line's extent and below 2^31.
 static int resolve_ld(const char* name, int64_t given, int64_t extent, int64_t* out) {
   if (given == 0) given = extent > 0 ? extent : 1;
@@ -208,8 +215,10 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
   int resolved = resolve_rung(TYPES, M, N, K, layoutA, layoutB, rung);
   // the streaming kernel needs 16-byte aligned operands and lines; AUTO falls back to the tiled kernel otherwise
   if (rung == GZ_RUNG_AUTO && resolved == GZ_RUNG_SKINNY &&
-      (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15u) || !skinny_lines_ok(lda, ldb)))
+      (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15u) || !skinny_lines_ok((int)sizeof(typename T::in_t), lda, ldb)))
     resolved = GZ_RUNG_MFMA;
+  // a caller that names the streaming rung gets it for what the rung is offered for, not for all that its kernels run
+  if (rung == GZ_RUNG_SKINNY && (st = check_named_skinny(TYPES, g.M, g.N, g.K, layoutA, layoutB)) != GZ_OK) return st;
   switch (resolved) {
     case GZ_RUNG_NAIVE: return launch_naive<TYPES>(g, variant, s);
     case GZ_RUNG_COALESCED: return launch_coalesced<TYPES>(g, variant, s);
@@ -362,7 +371,7 @@ int gz_variant_count(int types, int rung) {
   switch (rung) {
     case GZ_RUNG_NAIVE: case GZ_RUNG_COALESCED: case GZ_RUNG_LDS_TILED: case GZ_RUNG_DOUBLE_BUFFERED: return 1;
     case GZ_RUNG_MFMA: return is_acc16(types) ? 1 : kNumMfmaCfgs;
-    case GZ_RUNG_SKINNY: return (types == GZ_S8S8S32 || types == GZ_F32F32F32 || is_fp8(types) || is_acc16(types)) ? 0 : 1;
+    case GZ_RUNG_SKINNY: return skinny_rung_types(types) ? 1 : 0;
     default: return 0;
   }
 }
@@ -538,16 +547,14 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
       return GZ_OK;
     }
     case GZ_RUNG_SKINNY: {
-      if (!skinny_supported(types, m, n, k, layoutA, layoutB)) {
-        set_error("skinny rung needs a 16-bit float type, row-major A, column-major B, M <= %d and K %% %d == 0",
-                  SKINNY_MAX_M, SKINNY_K_STEP);
-        return GZ_ERR_UNSUPPORTED;
-      }
+      if (rung == GZ_RUNG_SKINNY && (st = check_named_skinny(types, m, n, k, layoutA, layoutB)) != GZ_OK) return st;
       if (variant > 1) { set_error("skinny rung has a single variant"); return GZ_ERR_UNSUPPORTED; }
-      SkinnyCfg c = skinny_resolve(m, n, k, num_cus, (unsigned long long)ws_limit);
+      SkinnyCfg c = skinny_resolve(types, m, n, k, num_cus, (unsigned long long)ws_limit);
       plan->variant = 1;
       plan->tile_m = c.mb; plan->tile_n = c.cols_per_wg;
-      plan->tile_k = c.kind == SKINNY_KIND_TILE ? STREAM_TILE_K_STEP : c.kind == SKINNY_KIND_DTL ? SKINNY_DTL_K_STEP : SKINNY_K_STEP;
+      // bytes of K per stage: 256 of the direct-to-LDS kernel (128 where the last one is half a stage), 128 of the others
+      plan->tile_k = (c.kind == SKINNY_KIND_DTL && (int64_t)k * es % SKINNY_DTL_CHUNK_BYTES != STREAM_TILE_ROW_BYTES
+                          ? SKINNY_DTL_CHUNK_BYTES : STREAM_TILE_ROW_BYTES) / es;
       plan->wave_m = c.kind == SKINNY_KIND_TILE ? 32 : c.mb; plan->wave_n = c.cols_per_wave;
       plan->threads = c.threads; plan->split_k = c.split_k; plan->lds_bytes = c.lds_bytes;
       plan->grid = (int64_t)c.grid_n * c.split_k;

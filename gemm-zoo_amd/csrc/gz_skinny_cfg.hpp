@@ -7,17 +7,23 @@
 namespace gz {
 
 constexpr int SKINNY_MAX_M = 128;      // most rows of activations the streaming kernels take
-constexpr int SKINNY_REG_MAX_M = 16;   // above: activations are shared through LDS (stream_tile_kernel)
-constexpr int SKINNY_COLS_PER_WAVE = 16;
-constexpr int SKINNY_K_STEP = 64;      // elements of K consumed per super-step (128 bytes per weight row)
-// direct-to-LDS kernel: 128-element K chunks, 32 rows x 256 bytes per stage, waves per work-group, stages per wave
-constexpr int SKINNY_DTL_K_STEP = 128;
-constexpr int SKINNY_DTL_STAGE_BYTES = 8192;
-constexpr int SKINNY_DTL_WAVES = 4;
-constexpr int SKINNY_DTL_STAGES = 2;
-// producer / consumer tile kernel: 64 K elements (128-byte rows) per stage, at most 64 columns per work-group,
+constexpr int SKINNY_REG_MAX_M = 16;   // activations in registers; above they are shared through LDS (stream_tile_kernel)
+constexpr int SKINNY_K_STEP = 64;      // an explicitly named rung takes whole multiples of this K (of 16-bit elements)
+// direct-to-LDS kernel: 256-byte K chunks of 4 NCP columns per stage.  A compute unit streams at its full rate with
+// about 128 KiB in flight, and a narrow share of columns has few bytes per stage: more waves and more stages there.
+constexpr int SKINNY_DTL_CHUNK_BYTES = 256;
+struct SkinnyDtlShape { int waves, stages; };
+constexpr SkinnyDtlShape skinny_dtl_shape(int ncp) {
+  return ncp == 8 ? SkinnyDtlShape{4, 2} : ncp == 4 ? SkinnyDtlShape{8, 4} : SkinnyDtlShape{8, 6};
+}
+inline int skinny_dtl_copies(int cols) { return cols <= 4 ? 1 : cols <= 8 ? 2 : cols <= 16 ? 4 : 8; }
+// (fragments are read for whole blocks of 16 columns: the ring of the last wave is followed by what a block is longer
+// than its stage)
+inline int skinny_dtl_lds_bytes(int ncp) {
+  return skinny_dtl_shape(ncp).waves * skinny_dtl_shape(ncp).stages * ncp * 1024 + (ncp < 4 ? (4 - ncp) * 1024 : 0);
+}
+// producer / consumer tile kernel: 128 bytes of K per row and stage, at most 64 columns per work-group,
 // four consumer and four producer waves, ring depth by number of 32-row blocks of A
-constexpr int STREAM_TILE_K_STEP = 64;
 constexpr int STREAM_TILE_ROW_BYTES = 128;
 constexpr int STREAM_TILE_COLS = 64;
 constexpr int STREAM_TILE_THREADS = 512;
@@ -25,17 +31,18 @@ constexpr int STREAM_TILE_STAGES_1 = 8, STREAM_TILE_STAGES_2 = 4, STREAM_TILE_ST
 
 // the same with wide column blocks and a split K (65 ... 128 rows, long K): 64 CB columns per work-group, CB = 2 ... 4,
 // ring depth by CB; a work-group's partial sums are 4 waves x 2 row blocks x CB column blocks x 4 KiB
+constexpr int STREAM_WIDE_K_STEP = 64;   // elements (16-bit) per stage
 constexpr int STREAM_WIDE_MIN_K = 8192;
 constexpr int STREAM_WIDE_MAX_CB = 4;
 constexpr int STREAM_WIDE_STAGES_2 = 4, STREAM_WIDE_STAGES_3 = 3, STREAM_WIDE_STAGES_4 = 3;
 inline int stream_wide_stages(int cb) { return cb == 2 ? STREAM_WIDE_STAGES_2 : cb == 3 ? STREAM_WIDE_STAGES_3 : STREAM_WIDE_STAGES_4; }
 inline long long stream_wide_slot_bytes(int cb) { return 4LL * 2 * cb * 4 * 1024; }
 
-enum { SKINNY_KIND_REG = 0, SKINNY_KIND_DTL = 1, SKINNY_KIND_TILE = 2, SKINNY_KIND_TILE_WIDE = 3 };
+enum { SKINNY_KIND_DTL = 1, SKINNY_KIND_TILE = 2, SKINNY_KIND_TILE_WIDE = 3 };
 
 struct SkinnyCfg {
   int mb;             // rows of A the kernel instance covers: 16, 32, 64 or 128
-  int cols_per_wave;  // 16
+  int cols_per_wave;  // columns that one wave works on
   int waves;          // wavefronts per work-group
   int cols_per_wg;
   int threads;
@@ -48,26 +55,39 @@ struct SkinnyCfg {
   long long workspace_bytes;   // partial sums of a split K (0: none)
 };
 
-// Decode-shaped problems only: 16-bit float inputs, activations row-major (K
-// contiguous), weights column-major (K contiguous), whole K super-steps.
-inline bool skinny_supported(int types, int M, int N, int K, int layoutA, int layoutB) {
-  if (types != GZ_BF16BF16F32 && types != GZ_BF16BF16BF16 && types != GZ_F16F16F16) return false;
+// Element types of the kernels, and those for which the rung can be named by the caller (the 8-bit ones come here through
+// the launcher's own choice only).
+constexpr bool skinny_rung_types(int types) { return types == GZ_BF16BF16F32 || types == GZ_BF16BF16BF16 || types == GZ_F16F16F16; }
+constexpr bool skinny_stream_types(int types) {
+  return skinny_rung_types(types) || types == GZ_S8S8S32 || types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16;
+}
+
+// What the kernels can run: activations row-major (K contiguous), weights column-major (K contiguous), K in whole
+// 16-byte pieces.
+inline bool skinny_stream_supported(int types, int M, int N, int K, int layoutA, int layoutB) {
+  if (!skinny_stream_types(types)) return false;
   if (layoutA != GZ_ROW_MAJOR || layoutB != GZ_COL_MAJOR) return false;
-  if (M < 1 || M > SKINNY_MAX_M || N < 1 || K < SKINNY_K_STEP) return false;
-  if ((long long)K * 2 * SKINNY_MAX_M >= (1LL << 32)) return false;  // rows are addressed with 32-bit byte offsets
-  return K % SKINNY_K_STEP == 0;
+  const int es = skinny_rung_types(types) ? 2 : 1;
+  if (M < 1 || M > SKINNY_MAX_M || N < 1 || K < 1) return false;
+  if ((long long)K * es * SKINNY_MAX_M >= (1LL << 32)) return false;  // rows are addressed with 32-bit byte offsets
+  return (long long)K * es % 16 == 0;
+}
+// What a caller that names the rung may ask for: 16-bit float inputs and whole 64-element super-steps of K.
+inline bool skinny_supported(int types, int M, int N, int K, int layoutA, int layoutB) {
+  return skinny_rung_types(types) && K >= SKINNY_K_STEP && K % SKINNY_K_STEP == 0 &&
+         skinny_stream_supported(types, M, N, K, layoutA, layoutB);
 }
 
 // The streaming kernels copy 16-byte pieces of the rows of A and the columns of B and address them with 32-bit byte
-// offsets from the first row (column of the work-group): leading dimensions of whole pieces, below 2^32 / (2 * 128).
-inline bool skinny_lines_ok(long long lda, long long ldb) {
-  return lda % 8 == 0 && ldb % 8 == 0 && lda * 2 * SKINNY_MAX_M < (1LL << 32) && ldb * 2 * SKINNY_MAX_M < (1LL << 32);
+// offsets from the first row (column of the work-group): leading dimensions of whole pieces, below 2^32 / (es * 128).
+inline bool skinny_lines_ok(int es, long long lda, long long ldb) {
+  return lda * es % 16 == 0 && ldb * es % 16 == 0 && lda * es * SKINNY_MAX_M < (1LL << 32) && ldb * es * SKINNY_MAX_M < (1LL << 32);
 }
 
 // What the launcher's own choice sends here: always the register-resident cases; the LDS-shared tile kernel only
 // while the tiled MFMA rung could not give every compute unit a 128 x 128 tile of its own.
 inline bool skinny_preferred(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
-  if (!skinny_supported(types, M, N, K, layoutA, layoutB)) return false;
+  if (!skinny_stream_supported(types, M, N, K, layoutA, layoutB)) return false;
   if (num_cus <= 0) num_cus = 256;
   return M <= 32 || (long long)((N + 127) / 128) <= num_cus;
 }
@@ -94,13 +114,13 @@ inline int skinny_balanced_cols(int N, int num_cus, int max_cols) {
 // blocks come out at 65 ... 256 columns and the workspace fits.  The first launch then runs at the rate of the B
 // stream (M = 128, N = 14336: 43 us at K = 8192, 75 at 14336); the second costs 8 us: 60.1 -> 53.9 us and
 // 108.5 -> 83.1.
-inline bool skinny_resolve_wide(int M, int N, int K, int num_cus, unsigned long long ws_limit, int* split, int* cols) {
+inline bool skinny_resolve_wide(int types, int M, int N, int K, int num_cus, unsigned long long ws_limit, int* split, int* cols) {
   if (num_cus <= 0) num_cus = 256;
-  if (M <= 64 || M > SKINNY_MAX_M || K < STREAM_WIDE_MIN_K) return false;
+  if (!skinny_rung_types(types) || M <= 64 || M > SKINNY_MAX_M || K < STREAM_WIDE_MIN_K || K % STREAM_WIDE_K_STEP) return false;
   // four parts where the column blocks allow it, else two (M = 128, N = 14336, us, two / four parts: K = 8192
   // 56.0 / 56.3, K = 14336 93.9 / 84.5, before the second launch wrote whole rows; at K = 4096 the split loses to the one-launch kernel, 34.2 against 31.6)
   for (int ks = 4; ks >= 2; ks >>= 1) {
-    if (num_cus % ks || (K / STREAM_TILE_K_STEP) < 8 * ks) continue;
+    if (num_cus % ks || (K / STREAM_WIDE_K_STEP) < 8 * ks) continue;
     const int groups = num_cus / ks;
     int per = (N + groups - 1) / groups;
     per = (per + 3) / 4 * 4;
@@ -115,14 +135,14 @@ inline bool skinny_resolve_wide(int M, int N, int K, int num_cus, unsigned long 
   return false;
 }
 
-inline SkinnyCfg skinny_resolve(int M, int N, int K, int num_cus, unsigned long long ws_limit = ~0ULL) {
+inline SkinnyCfg skinny_resolve(int types, int M, int N, int K, int num_cus, unsigned long long ws_limit = ~0ULL) {
   SkinnyCfg c;
   c.split_k = 1;
   c.k_per_split = K;
   c.cb = 1;
   c.workspace_bytes = 0;
   int wide_split = 1, wide_cols = 0;
-  if (skinny_resolve_wide(M, N, K, num_cus, ws_limit, &wide_split, &wide_cols)) {
+  if (skinny_resolve_wide(types, M, N, K, num_cus, ws_limit, &wide_split, &wide_cols)) {
     c.kind = SKINNY_KIND_TILE_WIDE;
     c.mb = 128;
     c.cols_per_wg = wide_cols;
@@ -145,20 +165,14 @@ inline SkinnyCfg skinny_resolve(int M, int N, int K, int num_cus, unsigned long 
     c.cols_per_wave = 32;
     c.waves = STREAM_TILE_THREADS / 64;
     c.lds_bytes = stages * (c.mb + STREAM_TILE_COLS) * STREAM_TILE_ROW_BYTES;
-  } else if (K % SKINNY_DTL_K_STEP == 0) {
+  } else {
     c.kind = SKINNY_KIND_DTL;
     c.mb = 16;
     c.cols_per_wg = skinny_balanced_cols(N, num_cus, 32);
     c.cols_per_wave = c.cols_per_wg;  // every wave of the work-group works on all of its columns (K is split)
-    c.waves = SKINNY_DTL_WAVES;
-    c.lds_bytes = SKINNY_DTL_WAVES * SKINNY_DTL_STAGES * SKINNY_DTL_STAGE_BYTES;
-  } else {
-    c.kind = SKINNY_KIND_REG;
-    c.mb = 16;
-    c.cols_per_wave = SKINNY_COLS_PER_WAVE;
-    c.waves = 2;
-    c.cols_per_wg = c.cols_per_wave * c.waves;
-    c.lds_bytes = 0;
+    const int ncp = skinny_dtl_copies(c.cols_per_wg);
+    c.waves = skinny_dtl_shape(ncp).waves;
+    c.lds_bytes = skinny_dtl_lds_bytes(ncp);
   }
   c.threads = c.waves * 64;
   c.grid_n = (N + c.cols_per_wg - 1) / c.cols_per_wg;

@@ -10,16 +10,19 @@
 //     same L2 / memory channel at the same moment: every work-group starts at a different K chunk (rot);
 //   * each byte is used once: the copies carry the non-temporal hint.
 //
-// skinny_dtl_kernel (M <= 16, K % 128 == 0): a work-group of KS waves owns up to 32 columns; its waves take the
-// 128-element K chunks round-robin.  A wave moves its chunk of the 32 rows (8 KiB) from global memory straight
+// Element types: the 16-bit floats, int8 and the 8-bit floats.  The kernels work on bytes of K - a fragment is 16 bytes
+// per lane whatever the type - and take any K that is whole 16-byte pieces: the last chunk or stage of a row moves the
+// pieces that exist, and the rest counts as zeros on both operands.
+//
+// skinny_dtl_kernel (M <= 16): a work-group of KS waves owns up to 32 columns; its waves take the 256-byte
+// K chunks round-robin.  A wave moves its chunk of the 4 NCP rows from global memory straight
 // into a private LDS ring with global_load_lds_dwordx4 -- every instruction moves four 256-byte row pieces --
 // and reads the MFMA fragments back with ds_read_b128; the 16-byte pieces of a row are XOR-swizzled with the
 // row number on the way in, so the reads are bank-conflict free.  There is no barrier in the main loop and
 // S stages are in flight per wave; the waits are hand-counted (the compiler does not see LDS-DMA).  The K
 // partial sums of the KS waves meet in LDS at the end.  Activations (at most 16 rows) come from L2 into
-// registers with the same depth.
-//
-// skinny_reg_kernel (M <= 16, K % 64 == 0 only): the earlier design, B straight into MFMA operand registers.
+// registers with the same depth.  A narrow share of columns moves little per stage, so it gets more waves and more
+// stages (skinny_dtl_shape): what a compute unit has in flight stays near 128 KiB.
 //
 // stream_wide_kernel + stream_wide_reduce_kernel (64 < M <= 128, K >= 8192): stream_tile_kernel with column blocks of
 // up to 256 columns and K split in two or four parts, so that a compute unit pulls a part of A instead of all of it;
@@ -49,113 +52,57 @@ typedef float sk_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t sk_u32x4_t __attribute__((ext_vector_type(4)));
 typedef float sk_f32x16_t __attribute__((ext_vector_type(16)));
 
-template <int TYPES>
-__device__ inline sk_f32x4_t mfma16(sk_u32x4_t first, sk_u32x4_t second, sk_f32x4_t acc) {
-  if constexpr (TYPES == GZ_F16F16F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(sk_f16x8_t, first),
-                                                  __builtin_bit_cast(sk_f16x8_t, second), acc, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8_t, first),
-                                                   __builtin_bit_cast(sk_bf16x8_t, second), acc, 0, 0, 0);
-}
+typedef int sk_i32x4_t __attribute__((ext_vector_type(4)));
+typedef int sk_i32x8_t __attribute__((ext_vector_type(8)));
+typedef int sk_i32x16_t __attribute__((ext_vector_type(16)));
 
-template <int TYPES>
-__device__ inline sk_f32x16_t mfma32x16(sk_u32x4_t first, sk_u32x4_t second, sk_f32x16_t acc) {
-  if constexpr (TYPES == GZ_F16F16F16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(sk_f16x8_t, first),
-                                                  __builtin_bit_cast(sk_f16x8_t, second), acc, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(sk_bf16x8_t, first),
-                                                   __builtin_bit_cast(sk_bf16x8_t, second), acc, 0, 0, 0);
-}
+template <int TYPES> struct SkAcc { using v4 = sk_f32x4_t; using v16 = sk_f32x16_t; };
+template <> struct SkAcc<GZ_S8S8S32> { using v4 = sk_i32x4_t; using v16 = sk_i32x16_t; };
 
-template <int TYPES, int MBLK, int WAVES, int PF>
-__global__ void __launch_bounds__(WAVES * 64) skinny_reg_kernel(GemmArgs<TYPES> g) {
-  using T = Traits<TYPES>;
-  using in_t = typename T::in_t;
-  using out_t = typename T::out_t;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n_base = (blockIdx.x * WAVES + wave) * SKINNY_COLS_PER_WAVE;
-  if (n_base >= g.N) return;  // no barriers in this kernel: a whole wave may leave
-  const int r16 = lane & 15, grp = lane >> 4;
-  const int K = g.K;
-
-  // Rows past the end are clamped, not zeroed: an output element depends on one
-  // row of A and one column of B only, and the clamped ones are never stored.
-  const int n_ld = min(n_base + r16, g.N - 1);
-  const in_t* __restrict__ bp = g.B + (size_t)n_ld * (size_t)g.ldb + grp * 16;
-  const in_t* __restrict__ ap[MBLK];
+// `n` consecutive 16-byte K fragments of the weights (first operand) and of the activations.  A lane's 16 bytes are 8 or
+// 16 elements of K, and which k they stand for is the same on both operands, which is all a dot product needs: so the
+// 8-bit floats put two fragments side by side for v_mfma_f32_*_f8f6f4, which takes 32 bytes per lane.
+template <int TYPES, int NF>
+__device__ __forceinline__ void mfma16_run(const sk_u32x4_t (&first)[NF], const sk_u32x4_t (&second)[NF], typename SkAcc<TYPES>::v4& acc) {
+  if constexpr (is_fp8(TYPES)) {
+    constexpr int FMT = TYPES == GZ_E5M2E5M2F16 ? 1 : 0;
+    static_assert(NF % 2 == 0, "fragments in pairs");
 #pragma unroll
-  for (int i = 0; i < MBLK; i++) ap[i] = g.A + (size_t)min(16 * i + r16, g.M - 1) * (size_t)g.lda + grp * 16;
-
-  sk_f32x4_t acc[MBLK];
-#pragma unroll
-  for (int i = 0; i < MBLK; i++) acc[i] = sk_f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  sk_u32x4_t bq[PF][2], aq[PF][MBLK][2];
-  const int steps = K / SKINNY_K_STEP;
-
-  auto issue = [&](int slot, int s) {
-    const size_t off = (size_t)s * SKINNY_K_STEP;
-    bq[slot][0] = __builtin_nontemporal_load(reinterpret_cast<const sk_u32x4_t*>(bp + off));
-    bq[slot][1] = __builtin_nontemporal_load(reinterpret_cast<const sk_u32x4_t*>(bp + off + 8));
-#pragma unroll
-    for (int i = 0; i < MBLK; i++) {
-      aq[slot][i][0] = *reinterpret_cast<const sk_u32x4_t*>(ap[i] + off);
-      aq[slot][i][1] = *reinterpret_cast<const sk_u32x4_t*>(ap[i] + off + 8);
+    for (int t = 0; t < NF; t += 2) {
+      const sk_i32x8_t f = __builtin_shufflevector(__builtin_bit_cast(sk_i32x4_t, first[t]), __builtin_bit_cast(sk_i32x4_t, first[t + 1]), 0, 1, 2, 3, 4, 5, 6, 7);
+      const sk_i32x8_t s = __builtin_shufflevector(__builtin_bit_cast(sk_i32x4_t, second[t]), __builtin_bit_cast(sk_i32x4_t, second[t + 1]), 0, 1, 2, 3, 4, 5, 6, 7);
+      acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f, s, acc, FMT, FMT, 0, 0, 0, 0);
     }
-  };
-
+  } else {
 #pragma unroll
-  for (int u = 0; u < PF; u++)
-    if (u < steps) issue(u, u);
-
-  for (int s0 = 0; s0 < steps; s0 += PF) {
-#pragma unroll
-    for (int u = 0; u < PF; u++) {
-      const int s = s0 + u;
-      if (s < steps) {
-        sk_u32x4_t cb[2], ca[MBLK][2];
-        cb[0] = bq[u][0];
-        cb[1] = bq[u][1];
-#pragma unroll
-        for (int i = 0; i < MBLK; i++) {
-          ca[i][0] = aq[u][i][0];
-          ca[i][1] = aq[u][i][1];
-        }
-        if (s + PF < steps) issue(u, s + PF);
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-          for (int i = 0; i < MBLK; i++) acc[i] = mfma16<TYPES>(cb[t], ca[i][t], acc[i]);
-      }
-    }
-  }
-
-  // acc[i][v] = D(16 i + r16, n_base + 4 grp + v)
-  const int N = g.N;
-  const int n = n_base + 4 * grp;
-  const bool vec_ok = (g.ldd % 4 == 0) && (g.beta == 0 || g.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(g.D) & 15u) == 0) &&
-                      (g.beta == 0 || (reinterpret_cast<uintptr_t>(g.C) & 15u) == 0);
-#pragma unroll
-  for (int i = 0; i < MBLK; i++) {
-    const int m = 16 * i + r16;
-    if (m >= g.M) continue;
-    const size_t o = (size_t)m * (size_t)g.ldd + n, oc = (size_t)m * (size_t)g.ldc + n;
-    if (vec_ok && n + 3 < N) {
-      out_t cv[4] = {0, 0, 0, 0}, dv[4];
-      if (g.beta != 0) __builtin_memcpy(cv, g.C + oc, sizeof(cv));
-#pragma unroll
-      for (int e = 0; e < 4; e++) dv[e] = epilogue<TYPES>(acc[i][e], g.alpha, g.beta, &cv[e]);
-      __builtin_memcpy(g.D + o, dv, sizeof(dv));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        if (n + e < N) g.D[o + e] = epilogue<TYPES>(acc[i][e], g.alpha, g.beta, g.C + oc + e);
+    for (int t = 0; t < NF; t++) {
+      if constexpr (TYPES == GZ_S8S8S32)
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(sk_i32x4_t, first[t]), __builtin_bit_cast(sk_i32x4_t, second[t]), acc, 0, 0, 0);
+      else if constexpr (TYPES == GZ_F16F16F16)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(sk_f16x8_t, first[t]), __builtin_bit_cast(sk_f16x8_t, second[t]), acc, 0, 0, 0);
+      else
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sk_bf16x8_t, first[t]), __builtin_bit_cast(sk_bf16x8_t, second[t]), acc, 0, 0, 0);
     }
   }
 }
 
+// one fragment pair of 32 rows each (not the 8-bit floats)
+template <int TYPES>
+__device__ inline typename SkAcc<TYPES>::v16 mfma32x16(sk_u32x4_t first, sk_u32x4_t second, typename SkAcc<TYPES>::v16 acc) {
+  if constexpr (TYPES == GZ_S8S8S32)
+    return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(sk_i32x4_t, first), __builtin_bit_cast(sk_i32x4_t, second), acc, 0, 0, 0);
+  else if constexpr (TYPES == GZ_F16F16F16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(sk_f16x8_t, first), __builtin_bit_cast(sk_f16x8_t, second), acc, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(sk_bf16x8_t, first), __builtin_bit_cast(sk_bf16x8_t, second), acc, 0, 0, 0);
+}
+template <int TYPES>
+__device__ inline sk_f32x16_t mfma32x64_f8(sk_u32x4_t f0, sk_u32x4_t f1, sk_u32x4_t s0, sk_u32x4_t s1, sk_f32x16_t acc) {
+  constexpr int FMT = TYPES == GZ_E5M2E5M2F16 ? 1 : 0;
+  const sk_i32x8_t f = __builtin_shufflevector(__builtin_bit_cast(sk_i32x4_t, f0), __builtin_bit_cast(sk_i32x4_t, f1), 0, 1, 2, 3, 4, 5, 6, 7);
+  const sk_i32x8_t s = __builtin_shufflevector(__builtin_bit_cast(sk_i32x4_t, s0), __builtin_bit_cast(sk_i32x4_t, s1), 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f, s, acc, FMT, FMT, 0, 0, 0, 0);
+}
 
 // ---------------------------------------------------------------------------------------------------------
 // Direct-to-LDS streaming kernel
@@ -168,6 +115,10 @@ template <int N, class F> __device__ __forceinline__ void sk_for(F&& f) {
 }
 template <int OFF> __device__ __forceinline__ void sk_ds_read16(sk_u32x4_t& dst, uint32_t addr) {
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "i"(OFF));
+}
+template <int OFF> __device__ __forceinline__ void sk_ds_zero16(uint32_t addr) {
+  const sk_u32x4_t z = {0, 0, 0, 0};
+  asm volatile("ds_write_b128 %0, %1 offset:%2" : : "v"(addr), "v"(z), "i"(OFF) : "memory");
 }
 __device__ __forceinline__ void sk_set_m0(uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_addr) : "memory");
@@ -190,6 +141,11 @@ __device__ __forceinline__ void sk_copy16_keep(uint32_t voff, const void* sbase_
                : "v"(voff), "s"(sbase_minus_off), "i"(OFF), "s"(mask)
                : "memory");
 }
+// every lane
+template <int OFF> __device__ __forceinline__ void sk_copy16_all(uint32_t voff, const void* sbase) {
+  static_assert(OFF >= -4096 && OFF <= 4095, "13-bit signed immediate");
+  asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "i"(OFF) : "memory");
+}
 template <int OFF> __device__ __forceinline__ void sk_load16(sk_u32x4_t& dst, uint32_t voff, const void* sbase) {
   asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=&v"(dst) : "v"(voff), "s"(sbase), "i"(OFF) : "memory");
 }
@@ -202,14 +158,16 @@ template <int N> __device__ __forceinline__ void sk_wait_lgkm() {
 // orders later uses of a register after the asm statements that precede this one
 __device__ __forceinline__ void sk_touch(sk_u32x4_t& v) { asm volatile("" : "+v"(v)); }
 
-template <int TYPES, int MBLK, int KS, int S>
+template <int TYPES, int NCP, int KS, int S>
 __global__ void __launch_bounds__(KS * 64) skinny_dtl_kernel(GemmArgs<TYPES> g, int cols_per_wg) {
   using T = Traits<TYPES>;
   using out_t = typename T::out_t;
+  using acc_t = typename T::acc_t;
   extern __shared__ __attribute__((aligned(1024))) char sk_lds[];
-  constexpr int CB = 2;                          // 16-column MFMA blocks per work-group
-  constexpr int NCP = CB * 4;                    // 1 KiB copies per stage (4 rows x 256 bytes each)
-  constexpr int STAGE = SKINNY_DTL_STAGE_BYTES;  // 32 rows x 256 bytes
+  constexpr int ES = sizeof(typename T::in_t);
+  constexpr int MBLK = 1;
+  constexpr int CB = NCP > 4 ? 2 : 1;            // 16-column MFMA blocks per work-group
+  constexpr int STAGE = NCP * 1024;              // 4 NCP rows x 256 bytes, NCP copies of 4 rows each
   constexpr int PER = NCP + 4 * MBLK;            // vector-memory instructions per stage
   constexpr int NA = MBLK * CB;
   static_assert((S - 1) * PER < 64, "vmcnt is a 6-bit counter");
@@ -217,9 +175,10 @@ __global__ void __launch_bounds__(KS * 64) skinny_dtl_kernel(GemmArgs<TYPES> g, 
   const int lane = threadIdx.x & 63;
   const int ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n_base = blockIdx.x * cols_per_wg;
-  const int K = g.K, N = g.N, M = g.M;
+  const int N = g.N, M = g.M;
+  const uint32_t Kb = (uint32_t)g.K * ES;        // a multiple of 16 (the launcher checks)
   const uint32_t ring = lds_base + ks * (S * STAGE);
-  const size_t rowb = (size_t)g.ldb * 2, rowb_a = (size_t)g.lda * 2;   // bytes between the columns of B and the rows of A
+  const size_t rowb = (size_t)g.ldb * ES, rowb_a = (size_t)g.lda * ES;   // bytes between the columns of B and the rows of A
 
   // copy j moves rows 4j .. 4j+3 of the group: 16 lanes per row; the lane that fills position p of the LDS row
   // fetches piece p ^ (row & 15) of the 256-byte chunk.  The offsets stay below 2^32: a work-group's columns times
@@ -233,53 +192,59 @@ __global__ void __launch_bounds__(KS * 64) skinny_dtl_kernel(GemmArgs<TYPES> g, 
   }
   const char* sb = reinterpret_cast<const char*>(g.B) + (size_t)n_base * rowb;
   const int r16 = lane & 15, grp = lane >> 4;
-  uint32_t a_voff[MBLK];
+  uint32_t a_row[MBLK];
 #pragma unroll
-  for (int mb = 0; mb < MBLK; mb++) a_voff[mb] = (uint32_t)((size_t)min(mb * 16 + r16, M - 1) * rowb_a) + grp * 16;
+  for (int mb = 0; mb < MBLK; mb++) a_row[mb] = (uint32_t)((size_t)min(mb * 16 + r16, M - 1) * rowb_a);
   const char* sa = reinterpret_cast<const char*>(g.A);
-  // fragment of MFMA step t: row r16 of a column block, K piece 4t + grp
+  // fragment of MFMA step t: row r16 of a column block, K piece 4t + grp.  (Fewer than 16 columns: the rows past the
+  // stage are whatever lies behind it in LDS; they only reach columns that are not stored.)
   uint32_t b_addr[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) b_addr[t] = ring + r16 * 256 + (((t * 4 + grp) ^ r16) * 16);
 
-  sk_f32x4_t acc[MBLK][CB];
+  typename SkAcc<TYPES>::v4 acc[MBLK][CB];
 #pragma unroll
   for (int mb = 0; mb < MBLK; mb++)
 #pragma unroll
-    for (int cb = 0; cb < CB; cb++) acc[mb][cb] = sk_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[mb][cb][e] = 0;
   sk_u32x4_t aq[S][MBLK][4];
 
-  const int chunks = K / SKINNY_DTL_K_STEP;
+  const int chunks = (int)((Kb + 255) / 256);
   const int mine = (chunks - ks + KS - 1) / KS;          // this wave's chunks: ks, ks + KS, ... (before rotation)
   const int rot = (int)(blockIdx.x % (unsigned)chunks);
 
   auto chunk_byte = [&](int i) {
     int c = i * KS + ks + rot;
     if (c >= chunks) c -= chunks;
-    return (size_t)c * 256;
+    return (uint32_t)c * 256;
   };
   auto issue_copies = [&](auto slot_c, int i) {
     constexpr int SL = decltype(slot_c)::value;
-    const size_t kbyte = chunk_byte(i);
-    sk_for<CB>([&](auto q_c) {
+    const uint32_t kbyte = chunk_byte(i), left = Kb - kbyte;
+    sk_for<(NCP + 3) / 4>([&](auto q_c) {
       constexpr int Q = decltype(q_c)::value;  // four copies share one M0
       sk_set_m0(ring + SL * STAGE + Q * 4096 + 2048);
-      sk_for<4>([&](auto j_c) {
+      sk_for<(NCP < 4 ? NCP : 4)>([&](auto j_c) {
         constexpr int J = decltype(j_c)::value;
-        // cols_per_wg is a multiple of 4: a copy moves four whole rows or nothing (mask as a scalar register pair)
+        // cols_per_wg is a multiple of 4: a copy moves four whole rows or nothing; of a last, shorter chunk only the
+        // pieces that exist
         const uint32_t on = (uint32_t)__builtin_amdgcn_readfirstlane(4 * (Q * 4 + J) < cols_per_wg ? -1 : 0);
-        sk_copy16<(J - 2) * 1024>(voff[Q * 4 + J], sb + kbyte - (J - 2) * 1024, ((uint64_t)on << 32) | on);
+        const uint64_t pieces = __builtin_amdgcn_ballot_w64((uint32_t)(((lane & 15) ^ ((4 * J + (lane >> 4)) & 15)) * 16) < left);
+        sk_copy16<(J - 2) * 1024>(voff[Q * 4 + J], sb + kbyte - (J - 2) * 1024, (((uint64_t)on << 32) | on) & pieces);
       });
     });
   };
   auto issue_a = [&](auto slot_c, int i) {
     constexpr int SL = decltype(slot_c)::value;
-    const size_t kbyte = chunk_byte(i);
+    const uint32_t kbyte = chunk_byte(i);
     sk_for<MBLK>([&](auto mb_c) {
       constexpr int MB = decltype(mb_c)::value;
       sk_for<4>([&](auto t_c) {
         constexpr int TT = decltype(t_c)::value;
-        sk_load16<TT * 64>(aq[SL][MB][TT], a_voff[MB], sa + kbyte);
+        const uint32_t k = kbyte + TT * 64 + grp * 16;     // (a piece past the end: the row's first, zeroed below)
+        sk_load16<0>(aq[SL][MB][TT], a_row[MB] + (k < Kb ? k : 0u), sa);
       });
     });
   };
@@ -318,19 +283,32 @@ __global__ void __launch_bounds__(KS * 64) skinny_dtl_kernel(GemmArgs<TYPES> g, 
           for (int t = 0; t < 4; t++) sk_touch(aq[SL][mb][t]);
         const bool more = i + S < mine;
         if (more) issue_copies(sl, i + S);  // the fragments are in registers: the stage buffer is free
+        const uint32_t left = Kb - chunk_byte(i);
+        if (left < 256) {
+          // pieces past the end of K count as zeros on both sides (what is left in LDS may be NaN or infinite)
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+          for (int t = 0; t < 4; t++) {
+            const bool exists = (uint32_t)((t * 4 + grp) * 16) < left;
 #pragma unroll
-          for (int mb = 0; mb < MBLK; mb++)
+            for (int e = 0; e < 4; e++) {
 #pragma unroll
-            for (int cb = 0; cb < CB; cb++) acc[mb][cb] = mfma16<TYPES>(bf[cb][t], aq[SL][mb][t], acc[mb][cb]);
+              for (int mb = 0; mb < MBLK; mb++) aq[SL][mb][t][e] = exists ? aq[SL][mb][t][e] : 0u;
+#pragma unroll
+              for (int cb = 0; cb < CB; cb++) bf[cb][t][e] = exists ? bf[cb][t][e] : 0u;
+            }
+          }
+        }
+#pragma unroll
+        for (int mb = 0; mb < MBLK; mb++)
+#pragma unroll
+          for (int cb = 0; cb < CB; cb++) mfma16_run<TYPES, 4>(bf[cb], aq[SL][mb], acc[mb][cb]);
         if (more) issue_a(sl, i + S);
       }
     });
   }
 
   // every wave has waited for all of its copies (the last stages wait with vmcnt(0)): the rings can be reused
-  float* red = reinterpret_cast<float*>(sk_lds);
+  acc_t* red = reinterpret_cast<acc_t*>(sk_lds);
   if constexpr (KS > 1) {
     __syncthreads();
 #pragma unroll
@@ -391,6 +369,8 @@ __global__ void __launch_bounds__(STREAM_TILE_THREADS) stream_tile_kernel(GemmAr
   constexpr int NCW = 4;  // consumer waves; the four producer waves follow
   using T = Traits<TYPES>;
   using out_t = typename T::out_t;
+  using acc_t = typename T::acc_t;
+  constexpr int ES = sizeof(typename T::in_t);
   extern __shared__ __attribute__((aligned(1024))) char sk_lds[];
   constexpr int RB = STREAM_TILE_ROW_BYTES, B_BYTES = STREAM_TILE_COLS * RB, A_ROWS = MB32 * 32, A_BYTES = A_ROWS * RB, STAGE = A_BYTES + B_BYTES;
   constexpr int NA = MB32, NB = 2, NCP = NA + NB;      // copies per producer wave and stage
@@ -402,60 +382,98 @@ __global__ void __launch_bounds__(STREAM_TILE_THREADS) stream_tile_kernel(GemmAr
   const uint32_t lds_base = (uint32_t)(uintptr_t)sk_lds;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int K = g.K, N = g.N, M = g.M;
+  const int N = g.N, M = g.M;
   const int n_base = blockIdx.x * cols_per_wg;
   const int n_end = min(n_base + cols_per_wg, N);
-  const size_t rowb = (size_t)g.ldb * 2, rowb_a = (size_t)g.lda * 2;   // bytes between the columns of B and the rows of A
-  const int nst = K / STREAM_TILE_K_STEP;
+  const size_t rowb = (size_t)g.ldb * ES, rowb_a = (size_t)g.lda * ES;   // bytes between the columns of B and the rows of A
+  const uint32_t Kb = (uint32_t)g.K * ES;                       // a multiple of 16 (the launcher checks)
+  const int nst = (int)((Kb + RB - 1) / RB);
+  const uint32_t last = Kb - (uint32_t)(nst - 1) * RB;           // bytes per row of the last stage
   const int rot = (int)(blockIdx.x % (unsigned)nst);
 
   if (wave >= NCW) {
-    // ---------------- producers: wave p moves A rows [8 NA p, 8 NA (p+1)) and B rows [16 p, 16 p + 16) of every stage ----------------
+    // ---------------- producers: wave p moves A rows [8 NA p, 8 NA (p+1)) and B rows [16 (3 - p), 16 (3 - p) + 16) of every stage,
+    // eight rows per copy.  Copies of rows that do not exist - past M, past the work-group's columns - are not issued
+    // at all: a copy occupies its wave and the compute unit's address path whether or not its lanes move anything.
     const int p = wave - NCW;
-    uint32_t voffA[NA], voffB[NB];
-    uint64_t maskB[NB];
     const int row_in = lane >> 3, pos = lane & 7;
+    const int a_row0 = p * NA * 8, b_row0 = (NCW - 1 - p) * NB * 8;
+    // per-lane offsets with the copy's own share of the immediate taken off and a bias, taken off the base, that keeps
+    // them non-negative: the copies of an operand in a stage share one scalar base
+    constexpr uint32_t BIAS = 4096;
+    uint32_t voffA[NA], voffB[NB];
+    uint64_t maskB[NB], lastA[NA], lastB[NB];   // lanes that move something: of any stage, and of the last one (shorter rows)
 #pragma unroll
     for (int j = 0; j < NA; j++) {
-      const int row = (p * NA + j) * 8 + row_in;
-      voffA[j] = (uint32_t)((size_t)min(row, M - 1) * rowb_a) + (pos ^ ((row >> 1) & 7)) * 16;
+      const int row = a_row0 + j * 8 + row_in;
+      const uint32_t piece = (uint32_t)((pos ^ ((row >> 1) & 7)) * 16);
+      voffA[j] = (uint32_t)((size_t)min(row, M - 1) * rowb_a) + piece + BIAS - (j - 2) * 1024;
+      lastA[j] = __builtin_amdgcn_ballot_w64(piece < last);
     }
 #pragma unroll
     for (int j = 0; j < NB; j++) {
-      const int row = (p * NB + j) * 8 + row_in;
+      const int row = b_row0 + j * 8 + row_in;
       const int n = min(n_base + row, N - 1);
-      voffB[j] = (uint32_t)((size_t)(n - n_base) * rowb) + (pos ^ ((row >> 1) & 7)) * 16;
+      const uint32_t piece = (uint32_t)((pos ^ ((row >> 1) & 7)) * 16);
+      voffB[j] = (uint32_t)((size_t)(n - n_base) * rowb) + piece + BIAS - (j - 2) * 1024;
       maskB[j] = __builtin_amdgcn_ballot_w64(n_base + row < n_end);
+      lastB[j] = maskB[j] & __builtin_amdgcn_ballot_w64(piece < last);
     }
-    const char* sA = reinterpret_cast<const char*>(g.A);
-    const char* sB = reinterpret_cast<const char*>(g.B) + (size_t)n_base * rowb;
-    int slot = 0;
-    auto issue = [&](int s) {   // a stage past the end: every copy masked off but still counted
-      const bool exists = s < nst;
-      int c = s + rot;
-      if (c >= nst) c -= nst;
-      if (!exists) c = 0;
-      const uint32_t dst = lds_base + (uint32_t)slot * STAGE;
-      slot = slot + 1 == S ? 0 : slot + 1;
-      sk_set_m0(dst + p * (NA * 1024) + 2048);
-      sk_for<NA>([&](auto j_c) {
-        constexpr int J = decltype(j_c)::value;
-        sk_copy16_keep<(J - 2) * 1024>(voffA[J], sA + (size_t)c * RB - (J - 2) * 1024, __builtin_amdgcn_ballot_w64(exists));
-      });
-      sk_set_m0(dst + A_BYTES + p * (NB * 1024) + 2048);
-      sk_for<NB>([&](auto j_c) {
-        constexpr int J = decltype(j_c)::value;
-        const uint64_t m = maskB[J] & __builtin_amdgcn_ballot_w64(exists);
-        sk_copy16<(J - 2) * 1024>(voffB[J], sB + (size_t)c * RB - (J - 2) * 1024, m);
-      });
+    const char* sA = reinterpret_cast<const char*>(g.A) - BIAS;
+    const char* sB = reinterpret_cast<const char*>(g.B) + (size_t)n_base * rowb - BIAS;
+    const uint32_t dstA = lds_base + a_row0 * RB + 2048, dstB = lds_base + A_BYTES + b_row0 * RB + 2048;
+    const int na = __builtin_amdgcn_readfirstlane(max(0, min(NA, (M - a_row0 + 7) / 8)));
+    const int nb = __builtin_amdgcn_readfirstlane(max(0, min(NB, (n_end - n_base - b_row0 + 7) / 8)));
+    auto produce = [&](auto na_c, auto nb_c) {
+      constexpr int CA = decltype(na_c)::value, CB = decltype(nb_c)::value;   // copies of this wave per stage
+      uint32_t so = 0;
+      int s = 0, c = rot;
+      auto issue = [&]() {
+        const char *pa = sA + (size_t)c * RB, *pb = sB + (size_t)c * RB;
+        if (s < nst && (c < nst - 1 || last == RB)) {
+          if constexpr (CA > 0) sk_set_m0(dstA + so);
+          sk_for<CA>([&](auto j_c) {
+            constexpr int J = decltype(j_c)::value;
+            sk_copy16_all<(J - 2) * 1024>(voffA[J], pa);
+          });
+          if constexpr (CB > 0) sk_set_m0(dstB + so);
+          sk_for<CB>([&](auto j_c) {
+            constexpr int J = decltype(j_c)::value;
+            sk_copy16<(J - 2) * 1024>(voffB[J], pb, maskB[J]);
+          });
+        } else {   // the shorter last chunk of the rows, or a stage past the end: every copy masked off but still counted
+          const uint64_t any = __builtin_amdgcn_ballot_w64(s < nst);
+          if constexpr (CA > 0) sk_set_m0(dstA + so);
+          sk_for<CA>([&](auto j_c) {
+            constexpr int J = decltype(j_c)::value;
+            sk_copy16_keep<(J - 2) * 1024>(voffA[J], pa, any & lastA[J]);
+          });
+          if constexpr (CB > 0) sk_set_m0(dstB + so);
+          sk_for<CB>([&](auto j_c) {
+            constexpr int J = decltype(j_c)::value;
+            sk_copy16<(J - 2) * 1024>(voffB[J], pb, any & lastB[J]);
+          });
+        }
+        so = so + STAGE == S * STAGE ? 0 : so + STAGE;
+        s++;
+        c = c + 1 == nst ? 0 : c + 1;
+      };
+      for (int i = 0; i < S - 1; i++) issue();
+      for (int i = 0; i < nst; i++) {
+        sk_wait_vm<(S - 2) * (CA + CB)>();           // stage i has landed
+        asm volatile("s_barrier" ::: "memory");     // consumers are done with stage i - 1
+        issue();
+      }
+      sk_wait_vm<0>();
     };
-    for (int s = 0; s < S - 1; s++) issue(s);
-    for (int i = 0; i < nst; i++) {
-      sk_wait_vm<(S - 2) * NCP>();                 // stage i has landed
-      asm volatile("s_barrier" ::: "memory");     // consumers are done with stage i - 1
-      issue(i + S - 1);
-    }
-    sk_wait_vm<0>();
+    auto with_a = [&](auto na_c) {
+      if (nb == 0) produce(na_c, std::integral_constant<int, 0>{});
+      else if (nb == 1) produce(na_c, std::integral_constant<int, 1>{});
+      else produce(na_c, std::integral_constant<int, 2>{});
+    };
+    sk_for<NA + 1>([&](auto na_c) {
+      if (na == decltype(na_c)::value) with_a(na_c);
+    });
     if constexpr (KSPLIT > 1) { __syncthreads(); __syncthreads(); }
     return;
   }
@@ -471,15 +489,32 @@ __global__ void __launch_bounds__(STREAM_TILE_THREADS) stream_tile_kernel(GemmAr
     a_addr[t] = lds_base + (rb0 * 32 + r32) * RB + pp;
     b_addr[t] = lds_base + A_BYTES + (cbw * 32 + r32) * RB + pp;
   }
-  sk_f32x16_t acc[NRB];
+  typename SkAcc<TYPES>::v16 acc[NRB];
 #pragma unroll
   for (int r = 0; r < NRB; r++)
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[r][e] = 0.f;
+    for (int e = 0; e < 16; e++) acc[r][e] = 0;
 
+  const bool has_cols = n_base + cbw * 32 < n_end;   // a wave whose column block is empty only keeps the barriers company
   uint32_t so = 0;
-  for (int i = 0; i < nst; i++) {
+  for (int i = 0, c = rot; i < nst; i++, c = c + 1 == nst ? 0 : c + 1) {
     asm volatile("s_barrier" ::: "memory");
+    if (!has_cols) continue;
+    if (c == nst - 1 && last < (uint32_t)RB) {
+      // Pieces past the end of K count as zeros on both sides (what is left in LDS may be NaN or infinite): the wave
+      // clears the ones that it is about to read.  (Its LDS accesses execute in order.  Clearing the fragments in
+      // registers instead cost every stage of the loop: bf16 M = 128, N = 14336, K = 4096 33.1 us against 31.)
+      sk_for<NT>([&](auto t_c) {
+        constexpr int TT = decltype(t_c)::value;
+        if ((uint32_t)((2 * (TT + t0) + g2) * 16) >= last) {
+          sk_ds_zero16<0>(b_addr[TT] + so);
+          sk_for<NRB>([&](auto r_c) {
+            constexpr int R = decltype(r_c)::value;
+            sk_ds_zero16<R * 32 * RB>(a_addr[TT] + so);
+          });
+        }
+      });
+    }
     // All fragment reads of the stage are requested at once, k-step by k-step, and the MFMAs of a k-step start as
     // soon as its own fragments are there (LDS reads return in order), instead of one wait for all of them.
     sk_u32x4_t bf[NT], af[NRB][NT];
@@ -499,11 +534,14 @@ __global__ void __launch_bounds__(STREAM_TILE_THREADS) stream_tile_kernel(GemmAr
 #pragma unroll
       for (int r = 0; r < NRB; r++) sk_touch(af[r][TT]);
 #pragma unroll
-      for (int r = 0; r < NRB; r++) acc[r] = mfma32x16<TYPES>(bf[TT], af[r][TT], acc[r]);
+      for (int r = 0; r < NRB; r++) {
+        if constexpr (!is_fp8(TYPES)) acc[r] = mfma32x16<TYPES>(bf[TT], af[r][TT], acc[r]);
+        else if constexpr (TT % 2 == 1) acc[r] = mfma32x64_f8<TYPES>(bf[TT - 1], bf[TT], af[r][TT - 1], af[r][TT], acc[r]);
+      }
     });
   }
   if constexpr (KSPLIT > 1) {
-    float* red = reinterpret_cast<float*>(sk_lds);
+    acc_t* red = reinterpret_cast<acc_t*>(sk_lds);
     __syncthreads();   // every copy has landed and every fragment has been read: the rings are free
     const int tile = wave % (2 * NRG);
     if (kq > 0) {
@@ -581,7 +619,7 @@ __global__ void __launch_bounds__(STREAM_TILE_THREADS) stream_wide_kernel(GemmAr
   const int n_base = cg * cols_per_wg;
   const int n_end = min(n_base + cols_per_wg, N);
   const size_t rowb = (size_t)g.ldb * 2, rowb_a = (size_t)g.lda * 2;
-  const int nst_all = g.K / STREAM_TILE_K_STEP;
+  const int nst_all = g.K / STREAM_WIDE_K_STEP;
   const int st_q = nst_all / KS, st_r = nst_all % KS;
   const int st0 = ks * st_q + min(ks, st_r), nst = st_q + (ks < st_r ? 1 : 0);
   const int rot = (int)((unsigned)cg % (unsigned)nst);
@@ -750,28 +788,48 @@ __global__ void __launch_bounds__(256) stream_wide_reduce_kernel(GemmArgs<TYPES>
 }
 
 template <int TYPES> int launch_skinny(const GemmArgs<TYPES>& g, int variant, hipStream_t s) {
-  if constexpr (TYPES == GZ_S8S8S32 || TYPES == GZ_F32F32F32 || is_fp8(TYPES) || is_acc16(TYPES)) {
+  if constexpr (!skinny_stream_types(TYPES)) {
     (void)g; (void)variant; (void)s;
-    set_error("skinny rung is built for the 16-bit float types with fp32 accumulation only");
+    set_error("skinny rung is built for 8- and 16-bit elements with 32-bit accumulation only");
     return GZ_ERR_UNSUPPORTED;
   } else {
     if (variant > 1) {
       set_error("skinny rung has a single variant (got %d)", variant);
       return GZ_ERR_UNSUPPORTED;
     }
-    if (!skinny_supported(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB)) {
-      set_error("skinny rung needs row-major A, column-major B, 1 <= M <= %d and K %% %d == 0 (M=%d K=%d)",
-                SKINNY_MAX_M, SKINNY_K_STEP, g.M, g.K);
+    if (!skinny_stream_supported(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB)) {
+      set_error("skinny rung needs row-major A, column-major B, 1 <= M <= %d and whole 16-byte pieces of K (M=%d K=%d)",
+                SKINNY_MAX_M, g.M, g.K);
       return GZ_ERR_UNSUPPORTED;
     }
-    if (((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15u) || !skinny_lines_ok(g.lda, g.ldb)) {
-      set_error("skinny rung needs 16-byte aligned A and B and leading dimensions that are multiples of 8 elements "
+    constexpr int ES = sizeof(typename Traits<TYPES>::in_t);
+    if (((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15u) || !skinny_lines_ok(ES, g.lda, g.ldb)) {
+      set_error("skinny rung needs 16-byte aligned A and B and leading dimensions that are whole 16-byte pieces "
                 "(lda=%lld ldb=%lld)", (long long)g.lda, (long long)g.ldb);
       return GZ_ERR_UNSUPPORTED;
     }
-    const SkinnyCfg c = skinny_resolve(g.M, g.N, g.K, device_compute_units(), (unsigned long long)workspace_limit());
+    const SkinnyCfg c = skinny_resolve(TYPES, g.M, g.N, g.K, device_compute_units(), (unsigned long long)workspace_limit());
     const dim3 grid((unsigned)c.grid_n), block((unsigned)c.threads);
-    if (c.kind == SKINNY_KIND_TILE_WIDE) {
+    // (more than 64 KiB of dynamic LDS needs the opt-in; harmless below)
+    auto one = [&](auto kern) {
+      GZ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     c.lds_bytes));
+      hipLaunchKernelGGL(kern, grid, block, c.lds_bytes, s, g, c.cols_per_wg);
+      GZ_HIP_TRY(hipGetLastError());
+      return (int)GZ_OK;
+    };
+    if (c.kind == SKINNY_KIND_TILE) {
+      if (c.mb == 32) return one(stream_tile_kernel<TYPES, 1, STREAM_TILE_STAGES_1>);
+      if (c.mb == 64) return one(stream_tile_kernel<TYPES, 2, STREAM_TILE_STAGES_2>);
+      return one(stream_tile_kernel<TYPES, 4, STREAM_TILE_STAGES_4>);
+    }
+    if (c.kind == SKINNY_KIND_DTL) {
+      if (c.cols_per_wg <= 4) return one(skinny_dtl_kernel<TYPES, 1, skinny_dtl_shape(1).waves, skinny_dtl_shape(1).stages>);
+      if (c.cols_per_wg <= 8) return one(skinny_dtl_kernel<TYPES, 2, skinny_dtl_shape(2).waves, skinny_dtl_shape(2).stages>);
+      if (c.cols_per_wg <= 16) return one(skinny_dtl_kernel<TYPES, 4, skinny_dtl_shape(4).waves, skinny_dtl_shape(4).stages>);
+      return one(skinny_dtl_kernel<TYPES, 8, skinny_dtl_shape(8).waves, skinny_dtl_shape(8).stages>);
+    }
+    if constexpr (skinny_rung_types(TYPES)) {   // wide column blocks, split K (skinny_resolve_wide)
       void* ws = nullptr;
       const int st = workspace_acquire((size_t)c.workspace_bytes, s, &ws);
       if (st != GZ_OK) return st;
@@ -787,26 +845,11 @@ template <int TYPES> int launch_skinny(const GemmArgs<TYPES>& g, int variant, hi
       GZ_HIP_TRY(hipGetLastError());
       hipLaunchKernelGGL((stream_wide_reduce_kernel<TYPES>), dim3((unsigned)(c.grid_n * 4 * 2 * c.cb)), dim3(256), 0, s, g,
                          c.cols_per_wg, c.grid_n, c.split_k, c.cb, static_cast<const float*>(ws));
-    } else if (c.kind == SKINNY_KIND_TILE) {
-      auto k1 = stream_tile_kernel<TYPES, 1, STREAM_TILE_STAGES_1>;
-      auto k2 = stream_tile_kernel<TYPES, 2, STREAM_TILE_STAGES_2>;
-      auto k4 = stream_tile_kernel<TYPES, 4, STREAM_TILE_STAGES_4>;
-      auto kern = c.mb == 32 ? k1 : c.mb == 64 ? k2 : k4;
-      GZ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     c.lds_bytes));
-      hipLaunchKernelGGL(kern, grid, block, c.lds_bytes, s, g, c.cols_per_wg);
-    } else if (c.kind == SKINNY_KIND_DTL) {
-      constexpr int KS = SKINNY_DTL_WAVES, S = SKINNY_DTL_STAGES;
-      auto kern = skinny_dtl_kernel<TYPES, 1, KS, S>;
-      // more than 64 KiB of dynamic LDS needs the opt-in; harmless below
-      GZ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     c.lds_bytes));
-      hipLaunchKernelGGL(kern, grid, block, c.lds_bytes, s, g, c.cols_per_wg);
-    } else {
-      hipLaunchKernelGGL((skinny_reg_kernel<TYPES, 1, 2, 4>), grid, block, 0, s, g);
+      GZ_HIP_TRY(hipGetLastError());
+      return GZ_OK;
     }
-    GZ_HIP_TRY(hipGetLastError());
-    return GZ_OK;
+    set_error("skinny rung: no kernel for this plan");
+    return GZ_ERR_UNSUPPORTED;
   }
 }
 

@@ -277,6 +277,37 @@ def test_skinny_rung_long_k_wide_column_blocks(G, types):
     G.assert_within(types, got, truth, f"skinny long K {types}")
 
 
+STREAM_TYPES = (O.S8S8S32, O.BF16BF16F32, O.BF16BF16BF16, O.F16F16F16, O.E4M3E4M3F16, O.E5M2E5M2F16)
+
+
+@pytest.mark.parametrize("types", STREAM_TYPES)
+def test_launcher_streams_decode_shapes_of_every_narrow_type(G, types):
+    """The launcher's own choice for M <= 128 with K-contiguous operands and K in whole 16-byte pieces: shares of 4, 8,
+    16 and 32 columns, rows on both sides of each kernel's limit, K that ends in a piece, in half a chunk and in whole
+    chunks, K shorter than one chunk.  Integer-valued data (int8: its whole range): every partial sum is exact."""
+    es = 1 if types in (O.S8S8S32, O.E4M3E4M3F16, O.E5M2E5M2F16) else 2
+    kind = O.FILL_INT8_UNIFORM if types == O.S8S8S32 else O.FILL_SMALL_INT
+    for (m, n, kb), (al, be) in itertools.product(
+            [(1, 1024, 4096), (16, 37, 16), (16, 2044, 2048 + 16), (7, 4096, 1024 + 128), (3, 7170, 512 + 240),
+             (16, 9001, 3072), (17, 1029, 4096 + 112), (32, 4100, 1024 + 16), (33, 515, 640), (64, 3000, 2048 + 96),
+             (65, 1500, 48), (100, 7000, 1024 + 64), (128, 2100, 2048)], [(1, 0), (2, 3)]):
+        k = kb // es
+        assert G.capi.plan(types, m, n, k, O.ROW, O.COL).rung == SKINNY
+        a, b, c = O.make_inputs(types, m, n, k, kind=kind, seed=m + n)
+        print("case", types, m, n, k, al, be, flush=True)
+        got = G.run_gemm(types, a, b, c, m, n, k, O.ROW, O.COL, al, be, -1)
+        ref = O.gemm(types, a, b, c, m, n, k, O.ROW, O.COL, al, be)
+        assert np.array_equal(got, ref), (types, m, n, k, al, be)
+    # sub-matrix views whose padding is NaN: the pieces past the end of K count as zeros, not as what lies there
+    for m, n, kb in [(9, 700, 1024 + 48), (40, 700, 1024 + 48)]:
+        k = kb // es
+        a, b, c = O.make_inputs(types, m, n, k, kind=kind, seed=m)
+        ref = O.gemm(types, a, b, c, m, n, k, O.ROW, O.COL, 1, 1)
+        for pads in [(16, 32, 4, 8), (32, 16, 1, 3), (3, 16, 0, 0)]:
+            got = G.run_gemm_ld(types, a, b, c, m, n, k, O.ROW, O.COL, 1, 1, -1, 0, pads)
+            assert np.array_equal(got, ref), (types, m, n, k, pads)
+
+
 def test_skinny_rung_refuses_what_it_cannot_do(G):
     a = torch.zeros(129 * 64, dtype=torch.int16, device="cuda")
     for kw in (dict(m=129), dict(lb=O.ROW), dict(k=96), dict(types=O.S8S8S32), dict(types=O.F32F32F32),
