@@ -56,14 +56,35 @@ static int scratch_address(void** out) {
 }
 
 namespace {
-struct PoolBuffer { void* ptr = nullptr; size_t bytes = 0; };
+struct PoolBuffer {
+  std::mutex in_use;   // held by the call whose launches are being enqueued
+  void* ptr = nullptr;
+  size_t bytes = 0;
+};
 std::mutex g_pool_mutex;
-std::map<std::pair<int, hipStream_t>, PoolBuffer> g_pool;   // never freed before the process ends
+std::map<std::pair<int, hipStream_t>, PoolBuffer> g_pool;   // entries stay where they are; never freed before the process ends
 }  // namespace
 
 size_t workspace_limit() { return t_static_scratch ? (size_t)GZ_STATIC_SCRATCH_BYTES : ~(size_t)0; }
 
-int workspace_acquire(size_t bytes, hipStream_t s, void** out) {
+size_t splitk_workspace_limit(hipStream_t s) {
+  if (t_static_scratch) return (size_t)GZ_STATIC_SCRATCH_BYTES;
+  if (s != nullptr) {   // (the null stream is never captured)
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+      (void)hipGetLastError();   // a handle that cannot be asked: the launch itself will say what is wrong with it
+      return 0;
+    }
+    if (st != hipStreamCaptureStatusNone) return 0;
+  }
+  return ~(size_t)0;
+}
+
+WorkspaceLease::~WorkspaceLease() {
+  if (held_) static_cast<PoolBuffer*>(held_)->in_use.unlock();
+}
+
+int WorkspaceLease::acquire(size_t bytes, hipStream_t s) {
   if (t_static_scratch) {   // no allocation on this path
     if (bytes > (size_t)GZ_STATIC_SCRATCH_BYTES) {
       set_error("this launch needs %zu bytes of scratch memory, the static buffer holds %lld: use gz_gemm, which "
@@ -71,10 +92,16 @@ int workspace_acquire(size_t bytes, hipStream_t s, void** out) {
                 (long long)GZ_STATIC_SCRATCH_BYTES);
       return GZ_ERR_UNSUPPORTED;
     }
-    return scratch_address(out);
+    return scratch_address(&ptr);
   }
-  std::lock_guard<std::mutex> lock(g_pool_mutex);
-  PoolBuffer& b = g_pool[{current_device_index(), s}];
+  PoolBuffer* entry = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    entry = &g_pool[{current_device_index(), s}];
+  }
+  entry->in_use.lock();
+  held_ = entry;
+  PoolBuffer& b = *entry;
   if (b.bytes < bytes) {
     if (b.ptr) {
       // work queued on this stream may still use the old buffer
@@ -83,11 +110,13 @@ int workspace_acquire(size_t bytes, hipStream_t s, void** out) {
       b.ptr = nullptr;
       b.bytes = 0;
     }
-    const size_t want = (bytes + (size_t)(1 << 20) - 1) & ~((size_t)(1 << 20) - 1);
+    // (at least 16 MiB: most requests of a program then fit the first one)
+    size_t want = (bytes + (size_t)(1 << 20) - 1) & ~((size_t)(1 << 20) - 1);
+    if (want < (size_t)(16 << 20)) want = (size_t)(16 << 20);
     GZ_HIP_TRY(hipMalloc(&b.ptr, want));
     b.bytes = want;
   }
-  *out = b.ptr;
+  ptr = b.ptr;
   return GZ_OK;
 }
 
@@ -110,6 +139,91 @@ int device_compute_units() {
     cus = v;
   }
   return cus;
+}
+
+// ---------------------------------------------------------------------------
+// When K is split on 64 x 64 tiles
+// ---------------------------------------------------------------------------
+// us per 128-byte slab of a 64 x 64 tile whose work-group has a compute unit to itself, measured over 20 ... 880 tiles
+// and 7 ... 194 slabs: what a layout costs is its transposing stores (row-major B, column-major A), and 8-bit rows that
+// are not whole 16-byte pieces are loaded from unaligned addresses.
+static double splitk_slab_us(int types, int M, int N, int K, int layoutA, int layoutB) {
+  if (types == GZ_F32F32F32) return 0.56;
+  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR;
+  if (mfma_in_size(types) == 1) {
+    const bool aligned = (a_kc ? K : M) % 16 == 0 && (b_kc ? K : N) % 16 == 0;
+    if (a_kc && b_kc) return aligned ? 0.40 : 0.50;
+    if (a_kc != b_kc) return aligned ? 0.56 : 0.70;
+    return 0.74;
+  }
+  return a_kc && b_kc ? 0.42 : a_kc ? 0.48 : b_kc ? 0.40 : 0.60;
+}
+// How much longer a slab takes with w work-groups per compute unit.  fp32 is bound by its matrix rate: the compute unit
+// with the most work-groups decides.  The other types wait for memory, so a second work-group is nearly free (bf16,
+// 80 tiles x 194 slabs in 4, 6, 8, 12 parts, w = 1.25, 1.9, 2.5, 3.75: 1.2, 1.35, 1.9, 2.8).
+static double splitk_share(int types, double w) {
+  if (w <= 1.0) return 1.0;
+  if (types == GZ_F32F32F32) return std::ceil(w);
+  const double a = 1.0 + 0.4 * (w - 1.0), b = 0.77 * w;
+  return a > b ? a : b;
+}
+
+bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, SplitKPlan* out) {
+  if (is_acc16(types) || M <= 0 || N <= 0 || K <= 0) return false;
+  if (num_cus <= 0) num_cus = 256;
+  const long long slabs = ((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
+  const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  if (slabs < 4 || tiles > 4LL * num_cus) return false;
+  const double slab_us = splitk_slab_us(types, M, N, K, layoutA, layoutB);
+  // (a large operand that is read once: bf16 50 x 9600 x 8192 in 3 parts 39 us, of which 8 are the two launches)
+  const double stream_us = ((double)M + (double)N) * (double)K * mfma_in_size(types) / 5.5e6;
+  double best = 0;
+  int parts = 0;
+  for (int p = 2; p <= 32 && p <= slabs; p++) {
+    const long long bytes = p * tiles * 64 * 64 * 4;
+    if (bytes > MFMA_SPLITK_MAX_BYTES || tiles * p > 8LL * num_cus) break;
+    // two launches, the sums written and read back, the slabs of the longest part (us, measured / this line: bf16
+    // 24 x 1280 x 11001 in 12 parts 14.4 / 13.7, 100 x 2560 x 12416 in 6 27.6 / 26.7, fp32 512^3 in 4 10.1 / 9.6)
+    const double walk = (double)((slabs + p - 1) / p) * slab_us * splitk_share(types, (double)(tiles * p) / num_cus);
+    const double t = 6.5 + 0.22 * (double)bytes / (1 << 20) + (walk > stream_us ? walk : stream_us);
+    if (parts == 0 || t < best) {
+      best = t;
+      parts = p;
+    }
+  }
+  if (parts == 0) return false;
+  out->parts = parts;
+  out->q = (int)(slabs / parts);
+  out->rem = (int)(slabs % parts);
+  out->workspace_bytes = parts * tiles * 64 * 64 * 4;
+  out->estimate_us = best;
+  return true;
+}
+
+bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, SplitKPlan* out) {
+  if (!mfma_best_splitk(types, M, N, K, layoutA, layoutB, num_cus, out)) return false;
+  if (num_cus <= 0) num_cus = 256;
+  const double slabs = std::ceil((double)K * mfma_in_size(types) / MFMA_SLAB_BYTES);
+  const double round_us = 16.0 + 1.45 * slabs;   // the unit of mfma_choose
+  StreamKPlan skp;
+  // (stream-K, where it applies, already cuts K so that every compute unit has a share, on a tile with four times the
+  // products per byte: bf16 145 x 6656 x 7040 row/row 58.7 us, in three parts on 64 x 64 tiles 52.8; 1024^2 x 16384 54 / 61)
+  if (mfma_plan_streamk(types, M, N, K, layoutA, layoutB, num_cus, false, nullptr, &skp)) return false;
+  MfmaCfg c;
+  if (layoutA == GZ_COL_MAJOR && layoutB == GZ_COL_MAJOR && mfma_transposed_ring(types, M, N, K, layoutA, layoutB, 0, num_cus, &c, nullptr))
+    return out->estimate_us < 0.85 * round_us * mfma_choose(types, N, M, K, GZ_ROW_MAJOR, GZ_ROW_MAJOR, num_cus, &c);
+  MfmaSplit rows;
+  MfmaColSplit cols;
+  double est = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &c) * round_us;
+  if (c.bm == 64) {   // the same tile unsplit, by the same measure
+    const double w = (double)((M + 63) / 64) * ((N + 63) / 64) / num_cus;
+    est = 2.6 + slabs * splitk_slab_us(types, M, N, K, layoutA, layoutB) * splitk_share(types, w);
+    return out->estimate_us < 0.90 * est;
+  }
+  double cut = 0;
+  if (mfma_resolve_split(types, M, N, K, layoutA, layoutB, num_cus, &rows, &cut) && cut * round_us < est) est = cut * round_us;
+  if (mfma_resolve_colsplit(types, M, N, K, layoutA, layoutB, num_cus, &cols, &cut) && cut * round_us < est) est = cut * round_us;
+  return out->estimate_us < 0.85 * est;
 }
 
 static const char* kRungNames[GZ_NUM_RUNGS] = {"naive", "coalesced", "lds_tiled", "double_buffered", "mfma", "skinny"};
@@ -219,6 +333,14 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
     resolved = GZ_RUNG_MFMA;
   // a caller that names the streaming rung gets it for what the rung is offered for, not for all that its kernels run
   if (rung == GZ_RUNG_SKINNY && (st = check_named_skinny(TYPES, g.M, g.N, g.K, layoutA, layoutB)) != GZ_OK) return st;
+  if constexpr (skinny_stream_types(TYPES)) {
+    // (only where the launcher chose the streaming rung: a caller that names it gets its kernels)
+    SplitKPlan kp;
+    const int how = rung == GZ_RUNG_AUTO && resolved == GZ_RUNG_SKINNY && variant == 0
+                        ? skinny_choose(TYPES, g.M, g.N, g.K, device_compute_units(), splitk_workspace_limit(s), &kp) : SKINNY_STREAM;
+    if (how == SKINNY_TILES_SPLITK) return launch_splitk<TYPES>(g, kp, s);
+    if (how == SKINNY_TILES_64) return launch_mfma<TYPES>(g, kMfmaCfgs[MFMA_CFG_64].id, s);
+  }
   switch (resolved) {
     case GZ_RUNG_NAIVE: return launch_naive<TYPES>(g, variant, s);
     case GZ_RUNG_COALESCED: return launch_coalesced<TYPES>(g, variant, s);
@@ -376,6 +498,19 @@ int gz_variant_count(int types, int rung) {
   }
 }
 
+static void plan_splitk(const SplitKPlan& kp, int types, int m, int n, gz_plan_t* plan) {
+  const int es = in_size(types);
+  const MfmaCfg& c = es == 1 ? kMfmaCfg64Int8 : kMfmaCfgs[MFMA_CFG_64];
+  plan->variant = c.id;
+  plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
+  plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
+  plan->threads = c.waves_m * c.waves_n * 64;
+  plan->lds_bytes = mfma_lds_bytes(c);
+  plan->split_k = kp.parts;
+  plan->grid = (int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * kp.parts;
+  plan->workspace_bytes = kp.workspace_bytes;
+}
+
 // ws_limit: the most device memory beyond the matrices that the launch may use (what workspace_limit() will say
 // inside the entry point the plan is asked for)
 static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung, int variant,
@@ -429,6 +564,15 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
         plan->tile_m = 128; plan->tile_n = 128; plan->tile_k = 32; plan->wave_m = 64; plan->wave_n = 64;
         plan->threads = 256; plan->lds_bytes = 256 * (64 + 16);
         plan->grid = (int64_t)ceil_div(m, 128) * ceil_div(n, 128);
+        return GZ_OK;
+      }
+      if (SplitKPlan kp; variant == 0 && mfma_plan_splitk(types, m, n, k, layoutA, layoutB, num_cus, &kp) &&
+                         (unsigned long long)kp.workspace_bytes <= (unsigned long long)ws_limit) {
+        plan_splitk(kp, types, m, n, plan);
+        if (plan->lds_bytes > lds_per_cu) {
+          set_error("mfma variant %d needs %d bytes of LDS, device has %d", plan->variant, plan->lds_bytes, lds_per_cu);
+          return GZ_ERR_UNSUPPORTED;
+        }
         return GZ_OK;
       }
       MfmaSplit tsp;
@@ -549,6 +693,18 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
     case GZ_RUNG_SKINNY: {
       if (rung == GZ_RUNG_SKINNY && (st = check_named_skinny(types, m, n, k, layoutA, layoutB)) != GZ_OK) return st;
       if (variant > 1) { set_error("skinny rung has a single variant"); return GZ_ERR_UNSUPPORTED; }
+      SplitKPlan kp;
+      const int how = rung == GZ_RUNG_AUTO && variant == 0 ? skinny_choose(types, m, n, k, num_cus, ws_limit, &kp) : SKINNY_STREAM;
+      if (how != SKINNY_STREAM) {   // the MFMA rung's 64 x 64 tiles, split along K or not
+        if (how == SKINNY_TILES_SPLITK) {
+          plan_splitk(kp, types, m, n, plan);
+        } else {
+          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, kMfmaCfgs[MFMA_CFG_64].id, num_cus, lds_per_cu, ws_limit, plan);
+          if (st != GZ_OK) return st;
+        }
+        plan->rung = GZ_RUNG_SKINNY;
+        return GZ_OK;
+      }
       SkinnyCfg c = skinny_resolve(types, m, n, k, num_cus, (unsigned long long)ws_limit);
       plan->variant = 1;
       plan->tile_m = c.mb; plan->tile_n = c.cols_per_wg;

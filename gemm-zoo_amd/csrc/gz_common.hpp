@@ -293,14 +293,27 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 int device_compute_units();
 int current_device_index();
 
-// Device memory beyond the caller's matrices for a launch on stream `s` (partial sums of the stream-K launches): at
-// least `bytes`, 256-byte aligned, valid until the next call for the same stream.  From the library's own pool
-// (one buffer per device and stream, grown with hipMalloc when a call needs more), or - inside the entry point that
-// allocates nothing - the static buffer, which refuses what it cannot hold.  Returns a gz_status.
-int workspace_acquire(size_t bytes, hipStream_t s, void** out);
-// The most workspace_acquire can give on the calling thread right now: unbounded from the pool, the size of the static
+// Device memory beyond the caller's matrices for the launches of one call on stream `s` (partial sums): at least
+// `bytes`, 256-byte aligned.  From the library's own pool (one buffer per device and stream, grown with hipMalloc when
+// a call needs more), or - inside the entry point that allocates nothing - the static buffer, which refuses what it
+// cannot hold.  The lease lasts while the call enqueues its launches: another thread that uses the same stream waits,
+// so that its launches come behind all of this call's and not between them.
+struct WorkspaceLease {
+  void* ptr = nullptr;
+  int acquire(size_t bytes, hipStream_t s);   // a gz_status
+  WorkspaceLease() = default;
+  ~WorkspaceLease();
+  WorkspaceLease(const WorkspaceLease&) = delete;
+  WorkspaceLease& operator=(const WorkspaceLease&) = delete;
+ private:
+  void* held_ = nullptr;
+};
+// The most a lease can give on the calling thread right now: unbounded from the pool, the size of the static
 // buffer inside the entry point that allocates nothing.  The launcher's own choice stays within it.
 size_t workspace_limit();
+// The same for a split K, which competes with plans that need no memory: nothing while `s` is being captured (a graph
+// would keep the address of a buffer that a later call may replace, and the pool cannot grow there).
+size_t splitk_workspace_limit(hipStream_t s);
 
 // Raises a kernel's dynamic LDS limit once per device instead of on every launch.
 #define GZ_SET_LDS_LIMIT(kern, bytes)                                                                        \
@@ -322,5 +335,7 @@ template <int TYPES> int launch_lds_tiled(const GemmArgs<TYPES>& g, int variant,
 template <int TYPES> int launch_double_buffered(const GemmArgs<TYPES>& g, int variant, hipStream_t s);
 template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& g, int variant, hipStream_t s);
 template <int TYPES> int launch_skinny(const GemmArgs<TYPES>& g, int variant, hipStream_t s);
+struct SplitKPlan;
+template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPlan& p, hipStream_t s);   // in the MFMA rung's units
 
 }  // namespace gz

@@ -584,6 +584,20 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   return out->estimate_us < 0.99 * best * round_us;
 }
 
+// Split K on 64 x 64 tiles: a grid that leaves most of the device empty, or waiting for a single long column of slabs per
+// compute unit, is cut along K as well; the parts' 32-bit sums meet in a workspace and a second launch adds them in
+// their order.  Any shape, layout and alignment (the register-staged kernel).
+struct SplitKPlan {
+  int parts, q, rem;           // K parts; slabs per part, the first rem parts one more
+  long long workspace_bytes;   // parts x tiles x 16 KiB of 32-bit sums
+  double estimate_us;
+};
+constexpr long long MFMA_SPLITK_MAX_BYTES = 64ll << 20;
+// the parts that the estimate likes best, whatever the alternatives cost; false: nothing to split (gz_api.hip)
+bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, SplitKPlan* out);
+// the launcher's own choice on the MFMA rung: against what it would run otherwise (gz_api.hip)
+bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, SplitKPlan* out);
+
 // Work-groups of a launch of whole tiles on the ring kernel: past one round of the compute units the kernel is
 // persistent, one work-group per compute unit walking tiles b, b + grid, ... (the order in which the hardware deals
 // work-groups out anyway) and asking for its next tile's first slab before it stores the current one.  (Variants 9

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "../../include/gemm_zoo.h"
+#include "gz_mfma_cfg.hpp"
 
 namespace gz {
 
@@ -177,6 +178,36 @@ inline SkinnyCfg skinny_resolve(int types, int M, int N, int K, int num_cus, uns
   c.threads = c.waves * 64;
   c.grid_n = (N + c.cols_per_wg - 1) / c.cols_per_wg;
   return c;
+}
+
+// The launcher's choice between the tile kernel above and the MFMA rung's 64 x 64 tiles for 17 ... 128 rows.  Every
+// work-group of the tile kernel walks all of K and takes in all of A beside its share of the columns: with few columns
+// per work-group and a long K it takes in mostly A, and the 64 x 64 tiles with a split K are faster; with many rows and a
+// short K its fill and its one pass of stores are not paid back, and the same tiles unsplit are.  Measured, us, tile
+// kernel / split K: bf16 20 x 2560 x 8192 18.2 / 14.6, 50 x 1024 x 8192 27.1 / 12.5, 100 x 2560 x 4096 20.3 / 14.0,
+// 128 x 5120 x 4096 23.6 / 20.9, 20 x 5120 x 8192 19.6 / 22.3, 100 x 9600 x 4096 26.1 / 36; e4m3 50 x 2560 x 8192
+// 16.3 / 12.3, 100 x 9600 x 8192 25.4 / 32.9.  Tile kernel / unsplit, K = 1280 bf16: 128 rows on 1024, 5120, 9600 and
+// 14336 columns 9.4 / 9.3, 11.6 / 9.7, 14.3 / 11.8, 16.2 / 12.1; 50 rows 6.5 / 8.4, 7.7 / 9.7, 9.1 / 10, 10.3 / 10.3;
+// at K = 4096 128 x 14336 32.9 / 44.
+inline double skinny_tile_estimate_us(int stages, int mb, int cols) {
+  if (mb == 32) return 3.4 + stages * (cols < 26 ? 0.118 : 0.0046 * cols);   // (many columns: the rate of the B stream)
+  if (mb == 64) return 3.2 + 0.015 * cols + stages * (0.185 + 0.0019 * cols);
+  return 4.2 + 0.075 * cols + stages * (0.225 + 0.0026 * cols);
+}
+enum { SKINNY_STREAM = 0, SKINNY_TILES_SPLITK = 1, SKINNY_TILES_64 = 2 };
+inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned long long ws_limit, SplitKPlan* split) {
+  if (M <= SKINNY_REG_MAX_M) return SKINNY_STREAM;
+  const SkinnyCfg c = skinny_resolve(types, M, N, K, num_cus, ws_limit);
+  if (c.kind != SKINNY_KIND_TILE) return SKINNY_STREAM;
+  const int es = skinny_rung_types(types) ? 2 : 1;
+  const int stages = (int)(((long long)K * es + STREAM_TILE_ROW_BYTES - 1) / STREAM_TILE_ROW_BYTES);
+  // (the two lines cross at 21, 25 and 31 stages for 20, 40 and 56 columns per work-group)
+  if (M > 64 && c.cols_per_wg >= 16 && stages <= 16 + c.cols_per_wg / 4) return SKINNY_TILES_64;
+  if (mfma_best_splitk(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus, split) &&
+      (unsigned long long)split->workspace_bytes <= ws_limit &&
+      split->estimate_us < 0.9 * skinny_tile_estimate_us(stages, c.mb, c.cols_per_wg))
+    return SKINNY_TILES_SPLITK;
+  return SKINNY_STREAM;
 }
 
 }  // namespace gz

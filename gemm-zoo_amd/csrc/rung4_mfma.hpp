@@ -584,9 +584,13 @@ __device__ inline void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm,
   tile_of_lid(lid_of_block(bid, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
 }
 
-template <int TYPES, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool EDGE>
+// K cut in `parts` (SPLIT instances of mfma_gemm_kernel): part p takes q slabs, the first rem parts one more, and leaves
+// its sums as accumulated in ws (32-bit, see splitk_reduce_kernel, which adds the parts in their order).
+struct SplitK { int parts = 1, q = 0, rem = 0; void* ws = nullptr; };
+
+template <int TYPES, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool EDGE, bool SPLIT = false>
 __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
-    mfma_gemm_kernel(GemmArgs<TYPES> g, int tiles_m, int tiles_n) {
+    mfma_gemm_kernel(GemmArgs<TYPES> g, int tiles_m, int tiles_n, SplitK sk) {
   using T = Traits<TYPES>;
   using in_t = typename T::in_t;
   using acc_v = typename AccVec<TYPES>::type;
@@ -607,8 +611,23 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave % WAVES_M, wn = wave / WAVES_M;
-  int tm, tn;
-  tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  int tm, tn, slot = 0;
+  // k lines from this work-group's first to the end of the matrix: a K range is a sub-matrix with the same pitch
+  int k_avail = g.K;
+  if constexpr (SPLIT) {
+    // (the tiles of one K part side by side: the work-groups of an XCD share their operands)
+    const int tiles = tiles_m * tiles_n, lid = lid_of_block(blockIdx.x, tiles * sk.parts);
+    const int part = lid / tiles;
+    tile_of_lid(lid - part * tiles, tiles_m, tiles_n, tm, tn);
+    const int first = part * sk.q + min(part, sk.rem), k0 = first * BK;
+    g.A += A_KC ? (size_t)k0 : (size_t)k0 * (size_t)g.lda;
+    g.B += B_KC ? (size_t)k0 : (size_t)k0 * (size_t)g.ldb;
+    k_avail = g.K - k0;
+    g.K = min(k_avail, (sk.q + (part < sk.rem ? 1 : 0)) * BK);
+    slot = part * tiles + tm * tiles_n + tn;
+  } else {
+    tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  }
   const int m0 = tm * BM, n0 = tn * BN;
 
   StagerA sa;
@@ -685,7 +704,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
   const bool ragged_lines = (!A_KC && m0 + BM > g.M) || (!B_KC && n0 + BN > g.N);
   // (lines shorter than a 16-byte piece: a piece could reach further than the next k line, so no such slabs)
   const bool short_lines = (!A_KC && g.lda < 16) || (!B_KC && g.ldb < 16);
-  const int full_slabs = ragged_lines ? (short_lines ? 0 : (g.K - 1) / BK) : g.K / BK;
+  const int full_slabs = ragged_lines ? (short_lines ? 0 : min((k_avail - 1) / BK, g.K / BK)) : g.K / BK;
   // how a slab is loaded: predicated, unconditionally (inside), or not at all (the last two iterations of the edge
   // kernels have no slab left to ask for; the registers keep what they hold and what is stored from them is never read)
   using LoadPredicated = std::integral_constant<int, 0>;
@@ -826,9 +845,77 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
     if constexpr (PEEL) run_iters(slab_iter, LoadNothing{}, kt, ktiles);
   }
 
+  if constexpr (SPLIT) {
+    // 32 x 32 blocks of a tile in row order, a block's 4 KiB as the lanes hold them: whole 1 KiB stores
+    typedef typename T::acc_t raw4_t __attribute__((ext_vector_type(4)));
+    raw4_t* out = reinterpret_cast<raw4_t*>(sk.ws) + (size_t)slot * (BM * BN / 4) + lane;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        const int bi = wm * FM + i, bj = wn * FN + j;
+        if (m0 + 32 * bi >= g.M || n0 + 32 * bj >= g.N) continue;   // (the same for all lanes)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+          out[(bi * (BN / 32) + bj) * 256 + q * 64] =
+              raw4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+      }
+    return;
+  }
   static_assert(NT / 64 * epilogue_region_bytes<FN>() <= 2 * STAGE_BYTES, "the epilogue reuses the operand buffers");
   __syncthreads();   // every wave has its last fragments: the operand buffers are free
   store_accumulators_lds<TYPES, FM, FN, EDGE>(g, acc, m0 + wm * WM, n0 + wn * WN, lane, lds + wave * epilogue_region_bytes<FN>());
+}
+
+// Second launch of a split K: a work-group per 32 x 32 block of the output.  Its 256 lanes read the block's sums in the
+// order the first launch stored them (whole lines), add the parts in their order - a fixed one: the result does not
+// depend on which work-group finished first - turn the block through LDS and write it row by row with alpha, beta and
+// the rounding.  Bound by the reads of the parts, which are still in the last-level cache.
+template <int TYPES, int BM, int BN>
+__global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmArgs<TYPES> g, int tiles_n, int tiles, SplitK sk) {
+  using T = Traits<TYPES>;
+  using out_t = typename T::out_t;
+  using acc_t = typename T::acc_t;
+  typedef acc_t raw4_t __attribute__((ext_vector_type(4)));
+  constexpr int NBN = BN / 32, NB = (BM / 32) * NBN;
+  __shared__ acc_t turn[32][36];
+  const int tile = (int)blockIdx.x / NB, blk = (int)blockIdx.x % NB;
+  const int m0 = tile / tiles_n * BM + blk / NBN * 32, n0 = tile % tiles_n * BN + blk % NBN * 32;
+  if (m0 >= g.M || n0 >= g.N) return;
+  const int tid = threadIdx.x, lane = tid % 64, q = tid / 64;
+  const raw4_t* in = reinterpret_cast<const raw4_t*>(sk.ws) + (size_t)tile * (BM * BN / 4) + blk * 256 + tid;
+  const size_t part = (size_t)tiles * (BM * BN / 4);
+  const int row = tid / 8, n = n0 + 4 * (tid % 8), m = m0 + row;
+  raw4_t sum = in[0];
+  int p = 1;
+  for (; p + 3 < sk.parts; p += 4) {   // four parts in flight
+    const raw4_t v0 = in[p * part], v1 = in[(p + 1) * part], v2 = in[(p + 2) * part], v3 = in[(p + 3) * part];
+#pragma unroll
+    for (int e = 0; e < 4; e++) sum[e] = ((sum[e] + v0[e]) + v1[e]) + v2[e] + v3[e];
+  }
+  for (; p < sk.parts; p++) {
+    const raw4_t v = in[p * part];
+#pragma unroll
+    for (int e = 0; e < 4; e++) sum[e] += v[e];
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) turn[lane & 31][q * 8 + (lane >> 5) * 4 + e] = sum[e];
+  __syncthreads();
+  if (m >= g.M || n >= g.N) return;
+  const size_t o = (size_t)m * (size_t)g.ldd + n, oc = (size_t)m * (size_t)g.ldc + n;
+  const bool vec_ok = (g.ldd % 4 == 0) && (g.beta == 0 || g.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(g.D) & 15u) == 0) &&
+                      (g.beta == 0 || (reinterpret_cast<uintptr_t>(g.C) & 15u) == 0);
+  if (vec_ok && n + 3 < g.N) {
+    out_t cv[4] = {0, 0, 0, 0}, dv[4];
+    if (g.beta != 0) __builtin_memcpy(cv, g.C + oc, sizeof(cv));
+#pragma unroll
+    for (int e = 0; e < 4; e++) dv[e] = epilogue<TYPES>(turn[row][4 * (tid % 8) + e], g.alpha, g.beta, &cv[e]);
+    __builtin_memcpy(g.D + o, dv, sizeof(dv));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (n + e < g.N) g.D[o + e] = epilogue<TYPES>(turn[row][4 * (tid % 8) + e], g.alpha, g.beta, g.C + oc + e);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1098,7 +1185,7 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   do {                                                                                              \
     auto kern = mfma_gemm_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, AKC, BKC, EDGE>;                   \
     GZ_SET_LDS_LIMIT(kern, lds);                                                                    \
-    hipLaunchKernelGGL(kern, grid, block, lds, s, g, tiles_m, tiles_n);                             \
+    hipLaunchKernelGGL(kern, grid, block, lds, s, g, tiles_m, tiles_n, SplitK{});                   \
   } while (0)
 
   const bool edge = shape_class != MFMA_SHAPE_WHOLE;
@@ -1457,6 +1544,39 @@ template <int TYPES> static int launch_one(const GemmArgs<TYPES>& g, const MfmaC
   return GZ_ERR_UNSUPPORTED;
 }
 
+// A split K on 64 x 64 tiles (mfma_plan_splitk): the parts' sums in one launch, then the launch that adds them.
+template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPlan& p, hipStream_t s) {
+  if constexpr (is_acc16(TYPES)) {
+    set_error("mfma rung: no split K for this type bundle");
+    return GZ_ERR_UNSUPPORTED;
+  } else {
+    WorkspaceLease lease;
+    const int st = lease.acquire((size_t)p.workspace_bytes, s);
+    if (st != GZ_OK) return st;
+    constexpr int WAVES_M = sizeof(typename Traits<TYPES>::in_t) >= 2 ? 2 : 1, WAVES_N = 2;   // as the unsplit tile
+    const int tiles_m = ceil_div(g.M, 64), tiles_n = ceil_div(g.N, 64), tiles = tiles_m * tiles_n;
+    const SplitK sk{p.parts, p.q, p.rem, lease.ptr};
+    const dim3 grid((unsigned)(tiles * p.parts)), block(WAVES_M * WAVES_N * 64);
+    const size_t lds = 2u * (size_t)(64 + 64) * PITCH;
+#define GZ_LAUNCH_SPLIT(AKC, BKC)                                                                \
+  do {                                                                                           \
+    auto kern = mfma_gemm_kernel<TYPES, 64, 64, WAVES_M, WAVES_N, AKC, BKC, true, true>;          \
+    GZ_SET_LDS_LIMIT(kern, lds);                                                                 \
+    hipLaunchKernelGGL(kern, grid, block, lds, s, g, tiles_m, tiles_n, sk);                      \
+  } while (0)
+    const bool akc = g.layoutA == GZ_ROW_MAJOR, bkc = g.layoutB == GZ_COL_MAJOR;
+    if (akc && bkc) GZ_LAUNCH_SPLIT(true, true);
+    else if (akc) GZ_LAUNCH_SPLIT(true, false);
+    else if (bkc) GZ_LAUNCH_SPLIT(false, true);
+    else GZ_LAUNCH_SPLIT(false, false);
+#undef GZ_LAUNCH_SPLIT
+    GZ_HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL((splitk_reduce_kernel<TYPES, 64, 64>), dim3((unsigned)tiles * 4), dim3(256), 0, s, g, tiles_n, tiles, sk);
+    GZ_HIP_TRY(hipGetLastError());
+    return GZ_OK;
+  }
+}
+
 // Stream-K: the whole tiles and the runs of the remaining tiles' slabs in one launch, then the launch that adds the
 // pieces (see struct StreamK).  The workspace comes from workspace_acquire: the library's own pool, or the static
 // buffer of the entry point that allocates nothing.
@@ -1466,10 +1586,10 @@ static int launch_streamk(const GemmArgs<TYPES>& g, const StreamKPlan& p, bool r
     set_error("mfma rung: no stream-K kernel for this type bundle");
     return GZ_ERR_UNSUPPORTED;
   } else {
-    void* ws = nullptr;
-    const int st = workspace_acquire((size_t)p.slots * MFMA_STREAMK_SLOT_BYTES, s, &ws);
+    WorkspaceLease lease;
+    const int st = lease.acquire((size_t)p.slots * MFMA_STREAMK_SLOT_BYTES, s);
     if (st != GZ_OK) return st;
-    StreamK sk{p.dp_tiles, p.sk_tiles, p.blocks, p.q, p.rem, ws};
+    StreamK sk{p.dp_tiles, p.sk_tiles, p.blocks, p.q, p.rem, lease.ptr};
     const int tiles_m = ceil_div(g.M, 256), tiles_n = ceil_div(g.N, 256);
     const dim3 grid((unsigned)(p.dp_tiles + p.blocks)), block(2 * WAVES_N * 64);
     const size_t rlds = 5u * (size_t)(256 + 256) * 64;
@@ -1496,6 +1616,12 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
   GemmArgs<TYPES> g = args;
   const int num_cus = device_compute_units();
   g.store_hint = mfma_store_hint(TYPES, g.M, g.N, g.K, (int)sizeof(typename Traits<TYPES>::out_t), num_cus);
+  if (variant == 0) {
+    SplitKPlan skp;
+    if (mfma_plan_splitk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, &skp) &&
+        (unsigned long long)skp.workspace_bytes <= (unsigned long long)splitk_workspace_limit(s))
+      return launch_splitk<TYPES>(g, skp, s);
+  }
   // Column-major A and B: the transposed problem on the ring kernel - one launch, or where the launcher would cut
   // the rows of the transposed problem (a mostly empty last round) two, over column ranges of the real C and D.
   // Returns -1 where that kernel does not take the problem.

@@ -3,4 +3,5 @@
 
 namespace gz {
 template int launch_mfma<GZ_BF16BF16BF16>(const GemmArgs<GZ_BF16BF16BF16>&, int, hipStream_t);
+template int launch_splitk<GZ_BF16BF16BF16>(const GemmArgs<GZ_BF16BF16BF16>&, const SplitKPlan&, hipStream_t);
 }  // namespace gz

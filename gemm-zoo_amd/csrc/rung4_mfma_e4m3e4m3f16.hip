@@ -3,4 +3,5 @@
 
 namespace gz {
 template int launch_mfma<GZ_E4M3E4M3F16>(const GemmArgs<GZ_E4M3E4M3F16>&, int, hipStream_t);
+template int launch_splitk<GZ_E4M3E4M3F16>(const GemmArgs<GZ_E4M3E4M3F16>&, const SplitKPlan&, hipStream_t);
 }  // namespace gz

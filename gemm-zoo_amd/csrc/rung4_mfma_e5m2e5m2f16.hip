@@ -3,4 +3,5 @@
 
 namespace gz {
 template int launch_mfma<GZ_E5M2E5M2F16>(const GemmArgs<GZ_E5M2E5M2F16>&, int, hipStream_t);
+template int launch_splitk<GZ_E5M2E5M2F16>(const GemmArgs<GZ_E5M2E5M2F16>&, const SplitKPlan&, hipStream_t);
 }  // namespace gz

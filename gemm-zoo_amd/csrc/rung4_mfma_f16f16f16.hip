@@ -3,4 +3,5 @@
 
 namespace gz {
 template int launch_mfma<GZ_F16F16F16>(const GemmArgs<GZ_F16F16F16>&, int, hipStream_t);
+template int launch_splitk<GZ_F16F16F16>(const GemmArgs<GZ_F16F16F16>&, const SplitKPlan&, hipStream_t);
 }  // namespace gz

@@ -3,4 +3,5 @@
 
 namespace gz {
 template int launch_mfma<GZ_S8S8S32>(const GemmArgs<GZ_S8S8S32>&, int, hipStream_t);
+template int launch_splitk<GZ_S8S8S32>(const GemmArgs<GZ_S8S8S32>&, const SplitKPlan&, hipStream_t);
 }  // namespace gz

@@ -830,9 +830,10 @@ template <int TYPES> int launch_skinny(const GemmArgs<TYPES>& g, int variant, hi
       return one(skinny_dtl_kernel<TYPES, 8, skinny_dtl_shape(8).waves, skinny_dtl_shape(8).stages>);
     }
     if constexpr (skinny_rung_types(TYPES)) {   // wide column blocks, split K (skinny_resolve_wide)
-      void* ws = nullptr;
-      const int st = workspace_acquire((size_t)c.workspace_bytes, s, &ws);
+      WorkspaceLease lease;
+      const int st = lease.acquire((size_t)c.workspace_bytes, s);
       if (st != GZ_OK) return st;
+      void* ws = lease.ptr;
       const int per_round = 8 / c.split_k;   // column groups per round of the eight XCDs
       const dim3 wgrid((unsigned)((c.grid_n + per_round - 1) / per_round * 8));
       auto k2 = stream_wide_kernel<TYPES, 2, STREAM_WIDE_STAGES_2>;
