@@ -103,6 +103,12 @@ int WorkspaceLease::acquire(size_t bytes, hipStream_t s) {
   held_ = entry;
   PoolBuffer& b = *entry;
   if (b.bytes < bytes) {
+    // another thread may be capturing: growing this pool is none of that graph's business
+    struct RelaxedCapture {
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+      ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    } relaxed;
     if (b.ptr) {
       // work queued on this stream may still use the old buffer
       GZ_HIP_TRY(hipStreamSynchronize(s));
@@ -164,8 +170,10 @@ static double splitk_slab_us(int types, int M, int N, int K, int layoutA, int la
 static double splitk_share(int types, double w) {
   if (w <= 1.0) return 1.0;
   if (types == GZ_F32F32F32) return std::ceil(w);
-  const double a = 1.0 + 0.4 * (w - 1.0), b = 0.77 * w;
-  return a > b ? a : b;
+  auto line = [](double x) { return 1.0 + 0.4 * (x - 1.0) > 0.77 * x ? 1.0 + 0.4 * (x - 1.0) : 0.77 * x; };
+  // (half of the weight on the compute units with the most work-groups: 280 tiles x 128 slabs, w = 1.09, cost 0.6 us a
+  // slab and not 0.5)
+  return 0.5 * (line(w) + line(std::ceil(w)));
 }
 
 bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, SplitKPlan* out) {
@@ -338,7 +346,9 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
     SplitKPlan kp;
     const int how = rung == GZ_RUNG_AUTO && resolved == GZ_RUNG_SKINNY && variant == 0
                         ? skinny_choose(TYPES, g.M, g.N, g.K, device_compute_units(), splitk_workspace_limit(s), &kp) : SKINNY_STREAM;
-    if (how == SKINNY_TILES_SPLITK) return launch_splitk<TYPES>(g, kp, s);
+    if (how == SKINNY_TILES_SPLITK) {   // (-1: no memory for the parts)
+      if ((st = launch_splitk<TYPES>(g, kp, s)) >= 0) return st;
+    }
     if (how == SKINNY_TILES_64) return launch_mfma<TYPES>(g, kMfmaCfgs[MFMA_CFG_64].id, s);
   }
   switch (resolved) {

@@ -1544,15 +1544,18 @@ template <int TYPES> static int launch_one(const GemmArgs<TYPES>& g, const MfmaC
   return GZ_ERR_UNSUPPORTED;
 }
 
-// A split K on 64 x 64 tiles (mfma_plan_splitk): the parts' sums in one launch, then the launch that adds them.
+// A split K on 64 x 64 tiles (mfma_plan_splitk): the parts' sums in one launch, then the launch that adds them.  -1: the
+// workspace cannot be had, nothing was launched.
 template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPlan& p, hipStream_t s) {
   if constexpr (is_acc16(TYPES)) {
     set_error("mfma rung: no split K for this type bundle");
     return GZ_ERR_UNSUPPORTED;
   } else {
     WorkspaceLease lease;
-    const int st = lease.acquire((size_t)p.workspace_bytes, s);
-    if (st != GZ_OK) return st;
+    if (lease.acquire((size_t)p.workspace_bytes, s) != GZ_OK) {   // no memory: the caller runs a plan that needs none
+      (void)hipGetLastError();
+      return -1;
+    }
     constexpr int WAVES_M = sizeof(typename Traits<TYPES>::in_t) >= 2 ? 2 : 1, WAVES_N = 2;   // as the unsplit tile
     const int tiles_m = ceil_div(g.M, 64), tiles_n = ceil_div(g.N, 64), tiles = tiles_m * tiles_n;
     const SplitK sk{p.parts, p.q, p.rem, lease.ptr};
@@ -1620,7 +1623,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     SplitKPlan skp;
     if (mfma_plan_splitk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, &skp) &&
         (unsigned long long)skp.workspace_bytes <= (unsigned long long)splitk_workspace_limit(s))
-      return launch_splitk<TYPES>(g, skp, s);
+      if (const int st = launch_splitk<TYPES>(g, skp, s); st >= 0) return st;
   }
   // Column-major A and B: the transposed problem on the ring kernel - one launch, or where the launcher would cut
   // the rows of the transposed problem (a mostly empty last round) two, over column ranges of the real C and D.
