@@ -153,6 +153,15 @@ __device__ __forceinline__ void store_accumulators(const GemmArgs<TYPES>& g, Acc
 // entered the compiler waits for ALL memory operations there (loads and stores return in no fixed order with respect to
 // each other), i.e. for the previous store, 64 times per wave on the four-wave 256 x 256 tile (7 us per launch).
 // Without loads of C nothing is waited for; with them, they are waited for once per block, before its first store.
+// a loaded value is in its register from here on
+template <class T> __device__ __forceinline__ void arrived(T& v) {
+  uint32_t w;
+  if constexpr (sizeof(T) == 4) w = __builtin_bit_cast(uint32_t, v);
+  else w = (uint32_t)v;
+  asm volatile("" : "+v"(w));
+  if constexpr (sizeof(T) == 4) v = __builtin_bit_cast(T, w);
+  else v = (T)w;
+}
 template <int UC, int TYPES, int FM, int FN, bool RAGGED, int BLK, bool TRANSPOSED, bool BY4, class Acc, int AM, int AN>
 __device__ __forceinline__ void store_accumulators_lds_impl(const GemmArgs<TYPES>& g, Acc (&acc)[AM][AN], int row0, int col0,
                                                             int lane, char* region) {
@@ -291,30 +300,38 @@ __device__ __forceinline__ void store_accumulators_lds_impl(const GemmArgs<TYPES
         }
       });
     } else if constexpr (RAGGED) {
-      // eight rows at a time: their LDS reads first, then the stores, so that a row does not wait for the one before
-      // (a sub-tile 32 columns wide: the upper half of the lanes has no column)
-      constexpr int RG = 8, NC = (COLS + 63) / 64;
-      const bool has_col = COLS % 64 == 0 || lane < COLS % 64;   // in the last group of 64 columns
-      for (int r0 = 0; r0 < 32; r0 += RG) {
+      // eight stores at a time: their LDS reads (and loads of C, from clamped addresses) first, so that a store does not
+      // wait for the one before.  A sub-tile 32 columns wide: two rows per store.
+      constexpr int RPS = COLS < 64 ? 64 / COLS : 1, RG = 8, NC = (COLS + 63) / 64;
+      static_assert(COLS % 64 == 0 || COLS == 32, "columns of a wave's sub-tile");
+      const int lr = RPS == 1 ? 0 : lane / COLS, lc = RPS == 1 ? lane : lane % COLS;
+      for (int r0 = 0; r0 < 32; r0 += RG * RPS) {
         const int mg = row0 + 32 * I + r0;
         if (mg >= M) break;
         acc_t v[RG][NC];
+        out_t ce[RG][NC];
         static_for<RG>([&](auto r_c) {
           constexpr int R = decltype(r_c)::value;
           static_for<NC>([&](auto c_c) {
             constexpr int C = decltype(c_c)::value;
-            v[R][C] = 0;
-            if (C < NC - 1 || has_col) __builtin_memcpy(&v[R][C], region + (r0 + R) * PITCH_E + (C * 64 + lane) * 4, 4);
+            __builtin_memcpy(&v[R][C], region + (r0 + R * RPS + lr) * PITCH_E + (C * 64 + lc) * 4, 4);
+            ce[R][C] = 0;
+            if constexpr (UC == 1)
+              ce[R][C] = g.C[(size_t)min(mg + R * RPS + lr, M - 1) * LDC + min(col0 + C * 64 + lc, N - 1)];
           });
         });
+        if constexpr (UC == 1) {   // they have arrived before the first region of a store is entered
+          static_for<RG>([&](auto r_c) {
+            static_for<NC>([&](auto c_c) { arrived(ce[decltype(r_c)::value][decltype(c_c)::value]); });
+          });
+        }
         static_for<RG>([&](auto r_c) {
           constexpr int R = decltype(r_c)::value;
-          const int m = mg + R;
+          const int m = mg + R * RPS + lr;
           static_for<NC>([&](auto c_c) {
             constexpr int C = decltype(c_c)::value;
-            const int nn = col0 + C * 64 + lane;
-            if (m < M && nn < N && (C < NC - 1 || has_col))
-              g.D[(size_t)m * LDD + nn] = epilogue<TYPES>(v[R][C], g.alpha, beta_e, g.C + (size_t)m * LDC + nn);
+            const int nn = col0 + C * 64 + lc;
+            if (m < M && nn < N) g.D[(size_t)m * LDD + nn] = epilogue<TYPES>(v[R][C], g.alpha, beta_e, &ce[R][C]);
           });
         });
       }
@@ -414,6 +431,18 @@ template <int N_ST, int N_LD, int N_MFMA> __device__ inline void mix2_into_mfmas
   }
 }
 
+// The 16 bytes of v moved down by `bytes` (0 and more), zeros from above.
+__device__ inline u32x4_t shift_down(u32x4_t v, int bytes) {
+  uint64_t lo = v.x | (uint64_t)v.y << 32, hi = v.z | (uint64_t)v.w << 32;
+  lo = bytes >= 8 ? hi : lo;
+  hi = bytes >= 8 ? 0 : hi;
+  lo = bytes >= 16 ? 0 : lo;
+  const int s = (bytes & 7) * 8;
+  lo = (lo >> s) | ((hi << 1) << (63 - s));
+  hi >>= s;
+  return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
 // ---------------------------------------------------------------------------
 // Slab staging: global -> registers -> LDS.
 // KC == true : operand lines are K-contiguous (row-major A, column-major B).
@@ -485,6 +514,50 @@ template <typename in_t, int ROWS, int NT, bool KC, bool EDGE> struct Stager {
 #pragma unroll
         for (int t = 0; t < TR; t++)
           __builtin_memcpy(&r[u * TR + t], base + (size_t)(k0 + ku * TR + t) * pitch + min(row0 + mc * EPV, rows_total - 1), 16);
+      }
+    }
+  }
+  // The same for a slab that the end of K or of the lines cuts: every load is again unconditional, from an address
+  // clamped into the matrix, and fix() puts right what the clamping moved, when the slab goes to LDS.  (Element by
+  // element under each lane's own condition, which load() does, a slab of 8-bit elements was 2000 branches and as many
+  // loads, fetched for the first time by every launch: e4m3 270^3, three slabs, took 13.6 us of which 8 were this.)
+  // The lines hold at least one 16-byte piece (K of a K-contiguous operand, M or N of the other kind).
+  __device__ inline void load_clamped(const in_t* __restrict__ base, int rows_total, int K, int row0, int k0, int tid, size_t pitch) {
+    if constexpr (KC) {
+#pragma unroll
+      for (int it = 0; it < VECS; it++) {
+        const int id = it * NT + tid;
+        const int row = min(row0 + (id >> 3), rows_total - 1), k = min(k0 + (id & 7) * EPV, K - EPV);
+        __builtin_memcpy(&r[it], base + (ptrdiff_t)((size_t)row * pitch) + k, 16);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < UNITS; u++) {
+        int mc, ku;
+        unit_of(u * NT + tid, mc, ku);
+#pragma unroll
+        for (int t = 0; t < TR; t++)
+          __builtin_memcpy(&r[u * TR + t], base + (size_t)min(k0 + ku * TR + t, K - 1) * pitch + min(row0 + mc * EPV, rows_total - EPV), 16);
+      }
+    }
+  }
+  // What load_clamped fetched becomes what the slab holds: elements moved down by as many as the address was moved,
+  // zeros for those past the end of K.
+  __device__ inline void fix(int rows_total, int K, int row0, int k0, int tid) {
+    if constexpr (KC) {
+#pragma unroll
+      for (int it = 0; it < VECS; it++) {
+        const int id = it * NT + tid, k = k0 + (id & 7) * EPV;
+        r[it] = shift_down(r[it], (k - min(k, K - EPV)) * ES);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < UNITS; u++) {
+        int mc, ku;
+        unit_of(u * NT + tid, mc, ku);
+        const int n = row0 + mc * EPV, moved = (n - min(n, rows_total - EPV)) * ES;
+#pragma unroll
+        for (int t = 0; t < TR; t++) r[u * TR + t] = shift_down(r[u * TR + t], k0 + ku * TR + t < K ? moved : 16);
       }
     }
   }
@@ -614,6 +687,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
   int tm, tn, slot = 0;
   // k lines from this work-group's first to the end of the matrix: a K range is a sub-matrix with the same pitch
   int k_avail = g.K;
+  // (lines shorter than one 16-byte piece are loaded element by element)
+  const bool tiny_lines = (A_KC ? g.K : g.M) < 16 / ES || (B_KC ? g.K : g.N) < 16 / ES;
   if constexpr (SPLIT) {
     // (the tiles of one K part side by side: the work-groups of an XCD share their operands)
     const int tiles = tiles_m * tiles_n, lid = lid_of_block(blockIdx.x, tiles * sk.parts);
@@ -710,14 +785,34 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
   using LoadPredicated = std::integral_constant<int, 0>;
   using LoadInside = std::integral_constant<int, 1>;
   using LoadNothing = std::integral_constant<int, 2>;
+  // Cut slabs by clamped loads (see Stager::load_clamped).  Not on the larger tiles, whose registers are all taken: the
+  // moves are a few per cent of a launch there, and spills cost more (e4m3 4000 x 4001 x 4001, K-contiguous operands,
+  // 98.7 / 105.9 us; f16 1677 x 3976 x 5351 on 128 x 128 tiles 134.8 / 140.3).
+  constexpr bool CLAMPED = EDGE && (BM * BN <= 64 * 64 || (BM * BN <= 128 * 128 && !(ES == 2 && A_KC && B_KC)));
   auto load_slab = [&](auto mode_c, int k0, StagerA& xa, StagerB& xb) __attribute__((always_inline)) {
     constexpr int MODE = decltype(mode_c)::value;
     if constexpr (MODE == 1) {
       xa.load_inside(g.A, g.M, g.K, m0, k0, tid, (size_t)g.lda);
       xb.load_inside(g.B, g.N, g.K, n0, k0, tid, (size_t)g.ldb);
     } else if constexpr (MODE == 0) {
+      if constexpr (CLAMPED) {
+        if (!tiny_lines) {
+          xa.load_clamped(g.A, g.M, g.K, m0, k0, tid, (size_t)g.lda);
+          xb.load_clamped(g.B, g.N, g.K, n0, k0, tid, (size_t)g.ldb);
+          return;
+        }
+      }
       xa.load(g.A, g.M, g.K, m0, k0, tid, (size_t)g.lda);
       xb.load(g.B, g.N, g.K, n0, k0, tid, (size_t)g.ldb);
+    }
+  };
+  // before slab `slab` goes from its registers to LDS
+  auto fix_slab = [&](int slab, StagerA& xa, StagerB& xb) __attribute__((always_inline)) {
+    if constexpr (CLAMPED) {
+      if (!tiny_lines && slab >= full_slabs && slab < ktiles) {
+        xa.fix(g.M, g.K, m0, slab * BK, tid);
+        xb.fix(g.N, g.K, n0, slab * BK, tid);
+      }
     }
   };
   auto load_slab_checked = [&](int slab, StagerA& xa, StagerB& xb) __attribute__((always_inline)) {
@@ -732,6 +827,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
   // Prologue: slab 0 into LDS, slab 1 parked in registers (DEEP: and slab 2 in the second set), fragments of
   // (slab 0, step 0) requested.
   load_slab_checked(0, sa, sb);
+  fix_slab(0, sa, sb);
   sa.store(lds, tid);
   sb.store(lds + A_BYTES, tid);
   if (ktiles > 1) load_slab_checked(1, sa, sb);
@@ -794,6 +890,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
       StagerB& xb = [&]() -> StagerB& { if constexpr (decltype(set_c)::value) return sb2; else return sb; }();
       read_frags(2, cur, 2);
       read_frags(3, cur, 3);
+      if constexpr (decltype(mode_c)::value != 1) fix_slab(kt + 1, xa, xb);
       xa.store(nxt, tid);
       xb.store(nxt + A_BYTES, tid);
       load_slab(mode_c, (EDGE || kt + LEAD < ktiles ? kt + LEAD : ktiles - 1) * BK, xa, xb);
@@ -819,6 +916,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64)
       StagerB& xb = [&]() -> StagerB& { if constexpr (decltype(set_c)::value) return sb2; else return sb; }();
 
       read_frags(1, cur, 1);
+      if constexpr (decltype(mode_c)::value != 1) fix_slab(kt + 1, xa, xb);
       xa.store(nxt, tid);
       xb.store(nxt + A_BYTES, tid);
       load_slab(mode_c, (EDGE || kt + LEAD < ktiles ? kt + LEAD : ktiles - 1) * BK, xa, xb);

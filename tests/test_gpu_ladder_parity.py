@@ -320,6 +320,27 @@ def test_skinny_rung_refuses_what_it_cannot_do(G):
 
 
 @pytest.mark.parametrize("types", ALL_TYPES)
+def test_last_slab_and_line_ends_of_the_register_staged_kernel(G, types):
+    """Slabs that the end of K or of the operands' lines cuts: K one element short of, equal to and one past a 16-byte
+    piece, a slab, two and three slabs; M and N around a piece and around the tiles; lines shorter than a piece.  The
+    padding of every operand is NaN (or large), so that a value read from it would show; stores element by element."""
+    bk = 128 // np.dtype(O.IN_DTYPE[types]).itemsize
+    epv = bk // 8
+    ks = [epv - 1, epv, epv + 1, bk - 1, bk + 1, 2 * bk + epv - 1, 3 * bk - 1, 4 * bk + 3]
+    mns = [(65, 33), (epv + 1, 70), (130, epv - 1), (64, 129)]
+    for variant, (la, lb) in itertools.product((12, 3, 2), itertools.product((O.ROW, O.COL), (O.ROW, O.COL))):
+        for i, k in enumerate(ks):
+            m, n = mns[(i + variant) % len(mns)]
+            a, b, c = O.make_inputs(types, m, n, k, kind=exact_kind(types), seed=k + variant)
+            al, be = ((1, 0), (2, 1))[i % 2]
+            print("case", types, variant, la, lb, m, n, k, flush=True)
+            ref = O.gemm(types, a, b, c, m, n, k, la, lb, al, be)
+            for pads, mis in (((1, 3, 1, 1), 0), ((0, 0, 0, 0), 1)):
+                got = G.run_gemm_ld(types, a, b, c, m, n, k, la, lb, al, be, MFMA, variant, pads, misalign=mis)
+                assert np.array_equal(got, ref), (types, variant, la, lb, m, n, k, pads)
+
+
+@pytest.mark.parametrize("types", ALL_TYPES)
 @pytest.mark.parametrize("rung", VALU_RUNGS + (MFMA,))
 def test_degenerate_and_unaligned(G, types, rung):
     # K = 0: D = beta * C
