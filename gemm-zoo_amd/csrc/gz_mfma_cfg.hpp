@@ -433,6 +433,10 @@ inline bool mfma_resolve_colsplit(int types, int M, int N, int K, int layoutA, i
   const int cols_main = N - r;
   MfmaCfg main_cfg, tail_cfg;
   double cost_main = mfma_choose(types, M, cols_main, K, layoutA, layoutB, num_cus, &main_cfg);
+  // (64 x 64 tiles for the first launch: the columns past a multiple of 256 are half a tile there, not a column of large
+  // ones, and a second launch of a few tiles through all of K takes as long as the first: e4m3 562 x 3616 x 2509 row/row
+  // 42.4 us in two launches, 23.1 in one; int8 500 x 3090 x 3000 row/col 25.1 / 18.9)
+  if (main_cfg.bm == 64) return false;
   // (column-major A and B: what the ring kernel on the transposed problem costs, where it takes the whole problem
   // and where it takes the first launch)
   if (MfmaCfg t; mfma_transposed_ring(types, M, N, K, layoutA, layoutB, 0, num_cus, &t, nullptr))
