@@ -92,8 +92,9 @@ typedef enum gz_types {
   GZ_NUM_TYPES = 9
 } gz_types;
 
-/* The ladder.  GZ_RUNG_AUTO lets the launcher pick (MFMA, or the weight-streaming
- * kernel for skinny M).                                                            */
+/* The ladder.  GZ_RUNG_AUTO lets the launcher pick: MFMA, or for skinny M what the plan
+ * reports as GZ_RUNG_SKINNY - the weight-streaming kernels, there for the 8-bit types as
+ * well, or the MFMA rung's 64x64 tiles (then plan.variant is theirs) where those are faster. */
 typedef enum gz_rung {
   GZ_RUNG_AUTO = -1,
   GZ_RUNG_NAIVE = 0,           /* one thread per output, scalar loads              */
@@ -101,7 +102,7 @@ typedef enum gz_rung {
   GZ_RUNG_LDS_TILED = 2,       /* LDS tiles with bank-conflict-free padding        */
   GZ_RUNG_DOUBLE_BUFFERED = 3, /* global->LDS prefetch overlapped with compute     */
   GZ_RUNG_MFMA = 4,            /* wavefront-level matrix-core kernel               */
-  GZ_RUNG_SKINNY = 5,          /* weight-streaming kernels for M <= 128            */
+  GZ_RUNG_SKINNY = 5,          /* weight-streaming kernels for M <= 128; by name for 16-bit types, K % 64 == 0 */
   GZ_NUM_RUNGS = 6
 } gz_rung;
 
@@ -116,7 +117,9 @@ typedef struct gz_plan_t {
   int32_t threads;             /* work-group size                              */
   int32_t lds_bytes;           /* static + dynamic LDS per work-group          */
   int64_t grid;                /* number of work-groups                        */
-  int32_t split_k;             /* >1: partial sums reduced in a second pass    */
+  int32_t split_k;             /* >1: K in that many parts, whose 32-bit sums (workspace_bytes in all) a second
+                                * launch adds in their order.  A call on a stream that is being captured runs
+                                * the plan without it (64x64 tiles only; not gz_gemm_static_scratch).         */
   int32_t vector_bytes_a, vector_bytes_b; /* widest aligned global access used */
   /* MFMA rung, launcher's choice only: when the tiles would leave a mostly empty last round of the compute
    * units, the last tail_rows rows of the problem run in a second launch with their own tile (0: one launch).
@@ -208,7 +211,7 @@ int gz_gemm_ld(int types, const void* A, int64_t lda, const void* B, int64_t ldb
 
 /* gz_gemm for callers that cannot allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments and the same results,
- * bit for bit, as gz_gemm.  The one difference is where a stream-K launch (see gz_plan_t) keeps its partial sums:
+ * bit for bit, as gz_gemm.  The one difference is where a launch that cuts K (see gz_plan_t) keeps its partial sums:
  * not in the library's pool, which hipMalloc grows on demand, but in a buffer of GZ_STATIC_SCRATCH_BYTES (384
  * slots of 256 x 256 accumulators) that is part of the library's device image, so that every GPU the library runs
  * on holds its own copy until the process ends.  This entry point never allocates or frees.  A launch that would
