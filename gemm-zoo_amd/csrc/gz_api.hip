@@ -65,9 +65,7 @@ std::mutex g_pool_mutex;
 std::map<std::pair<int, hipStream_t>, PoolBuffer> g_pool;   // entries stay where they are; never freed before the process ends
 }  // namespace
 
-size_t workspace_limit() { return t_static_scratch ? (size_t)GZ_STATIC_SCRATCH_BYTES : ~(size_t)0; }
-
-size_t splitk_workspace_limit(hipStream_t s) {
+size_t workspace_limit(hipStream_t s) {
   if (t_static_scratch) return (size_t)GZ_STATIC_SCRATCH_BYTES;
   if (s != nullptr) {   // (the null stream is never captured)
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -93,6 +91,10 @@ int WorkspaceLease::acquire(size_t bytes, hipStream_t s) {
       return GZ_ERR_UNSUPPORTED;
     }
     return scratch_address(&ptr);
+  }
+  if (bytes > workspace_limit(s)) {   // (the launchers ask before they plan; this is for the one that forgets)
+    set_error("a launch with a workspace on a stream that may use none");
+    return GZ_ERR_UNSUPPORTED;
   }
   PoolBuffer* entry = nullptr;
   {
@@ -345,7 +347,7 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
     // (only where the launcher chose the streaming rung: a caller that names it gets its kernels)
     SplitKPlan kp;
     const int how = rung == GZ_RUNG_AUTO && resolved == GZ_RUNG_SKINNY && variant == 0
-                        ? skinny_choose(TYPES, g.M, g.N, g.K, device_compute_units(), splitk_workspace_limit(s), &kp) : SKINNY_STREAM;
+                        ? skinny_choose(TYPES, g.M, g.N, g.K, device_compute_units(), workspace_limit(s), &kp) : SKINNY_STREAM;
     if (how == SKINNY_TILES_SPLITK) {   // (-1: no memory for the parts)
       if ((st = launch_splitk<TYPES>(g, kp, s)) >= 0) return st;
     }
@@ -491,7 +493,7 @@ int gz_device_props(int32_t* num_cus, int32_t* lds_per_cu) {
 int gz_gemm_static_scratch(int types, const void* A, const void* B, const void* C, void* D, int64_t M, int64_t N,
                            int64_t K, int layoutA, int layoutB, double alpha, double beta, int rung, int variant,
                            gz_stream stream) {
-  struct Scope {   // the launchers below ask workspace_acquire, which looks at this flag
+  struct Scope {   // workspace_limit and the leases of the launchers below look at this flag
     Scope() { t_static_scratch = true; }
     ~Scope() { t_static_scratch = false; }
   } scope;
@@ -521,8 +523,8 @@ static void plan_splitk(const SplitKPlan& kp, int types, int m, int n, gz_plan_t
   plan->workspace_bytes = kp.workspace_bytes;
 }
 
-// ws_limit: the most device memory beyond the matrices that the launch may use (what workspace_limit() will say
-// inside the entry point the plan is asked for)
+// ws_limit: the most device memory beyond the matrices that the launch may use (what workspace_limit(s) will say
+// inside the entry point the plan is asked for, on a stream that may use the pool)
 static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung, int variant,
                      int num_cus, int lds_per_cu, size_t ws_limit, gz_plan_t* plan) {
   if (!plan) { set_error("plan is NULL"); return GZ_ERR_BAD_ARG; }

@@ -308,12 +308,11 @@ struct WorkspaceLease {
  private:
   void* held_ = nullptr;
 };
-// The most a lease can give on the calling thread right now: unbounded from the pool, the size of the static
-// buffer inside the entry point that allocates nothing.  The launcher's own choice stays within it.
-size_t workspace_limit();
-// The same for a split K, which competes with plans that need no memory: nothing while `s` is being captured (a graph
-// would keep the address of a buffer that a later call may replace, and the pool cannot grow there).
-size_t splitk_workspace_limit(hipStream_t s);
+// The most a lease can give on the calling thread for stream `s` right now: unbounded from the pool, the size of the
+// static buffer inside the entry point that allocates nothing, and nothing from the pool while `s` is being captured: a
+// graph would keep the address of a buffer that a later call may replace, and that calls beside a replay use.  Every
+// launcher plans within it; an explicit stream-K variant is the plain variant where it is zero.
+size_t workspace_limit(hipStream_t s);
 
 // Raises a kernel's dynamic LDS limit once per device instead of on every launch.
 #define GZ_SET_LDS_LIMIT(kern, bytes)                                                                        \

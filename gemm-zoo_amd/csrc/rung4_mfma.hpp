@@ -1679,7 +1679,7 @@ template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPla
 }
 
 // Stream-K: the whole tiles and the runs of the remaining tiles' slabs in one launch, then the launch that adds the
-// pieces (see struct StreamK).  The workspace comes from workspace_acquire: the library's own pool, or the static
+// pieces (see struct StreamK).  The workspace is leased: from the library's own pool, or the static
 // buffer of the entry point that allocates nothing.
 template <int TYPES, int WAVES_N>
 static int launch_streamk(const GemmArgs<TYPES>& g, const StreamKPlan& p, bool ragged, hipStream_t s) {
@@ -1720,7 +1720,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
   if (variant == 0) {
     SplitKPlan skp;
     if (mfma_plan_splitk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, &skp) &&
-        (unsigned long long)skp.workspace_bytes <= (unsigned long long)splitk_workspace_limit(s))
+        (unsigned long long)skp.workspace_bytes <= (unsigned long long)workspace_limit(s))
       if (const int st = launch_splitk<TYPES>(g, skp, s); st >= 0) return st;
   }
   // Column-major A and B: the transposed problem on the ring kernel - one launch, or where the launcher would cut
@@ -1781,10 +1781,11 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
   if ((variant == 0 || variant == MFMA_VARIANT_STREAMK_W4 || variant == MFMA_VARIANT_STREAMK_W8) && g.K > 0) {
     StreamKPlan skp;
     const MfmaCfg* forced = variant == 0 ? nullptr : &kMfmaCfgs[variant - 1];
-    // the launcher's own choice stays within the workspace this entry point may use (the entry point that
-    // allocates nothing has a fixed one); an explicit stream-K variant is refused by workspace_acquire instead
+    // the launcher's own choice stays within the workspace this call may use (the entry point that allocates nothing has a
+    // fixed one); an explicit stream-K variant that needs more is refused by the lease instead, and where there is none
+    // at all (a captured stream) it runs the plain launch below, as on unaligned operands
     if (mfma_plan_streamk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, forced != nullptr, forced, &skp) &&
-        (forced || (size_t)skp.slots * MFMA_STREAMK_SLOT_BYTES <= workspace_limit())) {
+        (forced ? 1 : (size_t)skp.slots * MFMA_STREAMK_SLOT_BYTES) <= workspace_limit(s)) {
       const int cls = mfma_launch_class(skp.cfg, (int)sizeof(typename Traits<TYPES>::in_t),
                                         (int)sizeof(typename Traits<TYPES>::out_t), g.M, g.N, g.K, g.layoutA, g.layoutB,
                                         g.A, g.B, g.C, g.D, g.lda, g.ldb, g.ldc, g.ldd);

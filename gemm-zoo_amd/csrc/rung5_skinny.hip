@@ -816,7 +816,7 @@ template <int TYPES> int launch_skinny(const GemmArgs<TYPES>& g, int variant, hi
                 "(lda=%lld ldb=%lld)", (long long)g.lda, (long long)g.ldb);
       return GZ_ERR_UNSUPPORTED;
     }
-    const SkinnyCfg c = skinny_resolve(TYPES, g.M, g.N, g.K, device_compute_units(), (unsigned long long)workspace_limit());
+    const SkinnyCfg c = skinny_resolve(TYPES, g.M, g.N, g.K, device_compute_units(), (unsigned long long)workspace_limit(s));
     const dim3 grid((unsigned)c.grid_n), block((unsigned)c.threads);
     // (more than 64 KiB of dynamic LDS needs the opt-in; harmless below)
     auto one = [&](auto kern) {

@@ -118,8 +118,7 @@ typedef struct gz_plan_t {
   int32_t lds_bytes;           /* static + dynamic LDS per work-group          */
   int64_t grid;                /* number of work-groups                        */
   int32_t split_k;             /* >1: K in that many parts, whose 32-bit sums (workspace_bytes in all) a second
-                                * launch adds in their order.  A call on a stream that is being captured runs
-                                * the plan without it (64x64 tiles only; not gz_gemm_static_scratch).         */
+                                * launch adds in their order.                                                 */
   int32_t vector_bytes_a, vector_bytes_b; /* widest aligned global access used */
   /* MFMA rung, launcher's choice only: when the tiles would leave a mostly empty last round of the compute
    * units, the last tail_rows rows of the problem run in a second launch with their own tile (0: one launch).
@@ -137,6 +136,9 @@ typedef struct gz_plan_t {
    * run leaves partial sums in a workspace of workspace_bytes that the caller never sees, and a second launch
    * adds a tile's pieces in a fixed order (results do not depend on timing).  0: no such decomposition.       */
   int32_t streamk_tiles, streamk_blocks;
+  /* Memory beyond the matrices, from a pool of the library's own (one buffer per device and stream).  A call on a
+   * stream that is being captured takes none of it - a graph keeps addresses, the pool replaces its buffers - and
+   * runs the best plan with workspace_bytes == 0 instead (gz_gemm_static_scratch: its own buffer, and this plan).  */
   int64_t workspace_bytes;
 } gz_plan_t;
 
@@ -211,7 +213,7 @@ int gz_gemm_ld(int types, const void* A, int64_t lda, const void* B, int64_t ldb
 
 /* gz_gemm for callers that cannot allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments and the same results,
- * bit for bit, as gz_gemm.  The one difference is where a launch that cuts K (see gz_plan_t) keeps its partial sums:
+ * bit for bit, as gz_gemm outside a capture (where gz_gemm runs plans without a workspace).  The one difference is where a launch that cuts K (see gz_plan_t) keeps its partial sums:
  * not in the library's pool, which hipMalloc grows on demand, but in a buffer of GZ_STATIC_SCRATCH_BYTES (384
  * slots of 256 x 256 accumulators) that is part of the library's device image, so that every GPU the library runs
  * on holds its own copy until the process ends.  This entry point never allocates or frees.  A launch that would

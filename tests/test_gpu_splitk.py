@@ -126,3 +126,49 @@ def test_under_capture(G):
         G.capi.gemm(O.S8S8S32, other[0], other[1], None, e, mo, no, ko, O.ROW, O.COL, 1, 0, -1, 0, stream.cuda_stream)
         torch.cuda.synchronize()
         assert torch.equal(e, other[2])
+
+
+def _bf16_problem(m, n, k):
+    """Small whole numbers: every sum is exact."""
+    gen = torch.Generator(device="cuda").manual_seed(m + n)
+    a, b = (torch.randint(-1, 2, (rows, k), generator=gen, device="cuda").bfloat16() for rows in (m, n))
+    return a.reshape(-1), b.reshape(-1), a.float() @ b.float().t().contiguous(), (m, n, k)
+
+
+# what cuts K outside a capture: split K on 64 x 64 tiles, stream-K by the launcher's choice and by name, the wide column
+# blocks of the streaming rung by choice and by name
+CAPTURED = {"split": (O.S8S8S32, (192, 128, 5120), -1, 0), "stream-K": (O.BF16BF16F32, (1024, 1024, 8192), -1, 0),
+            "stream-K, named": (O.BF16BF16F32, (1024, 1024, 8192), 4, 7), "wide": (O.BF16BF16F32, (128, 14336, 8192), -1, 0),
+            "wide, named": (O.BF16BF16F32, (128, 14336, 8192), 5, 0)}
+
+
+@pytest.mark.parametrize("what", CAPTURED)
+@pytest.mark.parametrize("entry", ("gemm", "gemm_static_scratch"))
+def test_every_plan_that_cuts_k_under_capture(G, what, entry):
+    """A captured call takes a plan without the pool (the entry point with the static buffer keeps its plan): every replay
+    gives the right result, whatever eager calls on the same stream, with more memory than the captured problem would
+    take, have done to the pool in between."""
+    types, shape, rung, variant = CAPTURED[what]
+    a, b, ref, (m, n, k) = _problem(G, 7, *shape) if types == O.S8S8S32 else _bf16_problem(*shape)
+    p = G.capi.plan(types, m, n, k, O.ROW, O.COL, rung, variant)
+    assert p.workspace_bytes > 0
+    d = torch.empty(m, n, dtype=ref.dtype, device="cuda")
+    other = _problem(G, 8, 1024, 1536, 16384)
+    mo, no, ko = other[3]
+    po = G.capi.plan(O.S8S8S32, mo, no, ko, O.ROW, O.COL, 4, 7)
+    assert po.workspace_bytes > p.workspace_bytes
+    e = torch.empty(mo, no, dtype=torch.int32, device="cuda")
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        getattr(G.capi, entry)(types, a, b, None, d, m, n, k, O.ROW, O.COL, 1, 0, rung, variant, stream.cuda_stream)
+    for _ in range(4):
+        d.fill_(-1)
+        e.fill_(-1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(d, ref)
+        G.capi.gemm(O.S8S8S32, other[0], other[1], None, e, mo, no, ko, O.ROW, O.COL, 1, 0, 4, 7, stream.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(e, other[2])

@@ -1,0 +1,62 @@
+"""The library's workspace pool on a stand-in for the HIP runtime (hip_stub.c), without a GPU: which calls take memory, from
+whom it is kept, and what a call does that cannot have any.  Nothing runs; what is checked is what the runtime is asked
+for, call by call."""
+import json
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+S8, BF16F32, BF16 = 0, 1, 2
+MFMA, SKINNY = 4, 5
+STREAM = 0x1000
+# problems whose plans cut K: split K on 64 x 64 tiles, stream-K, the wide column blocks of the streaming rung
+SPLITK = dict(types=S8, m=192, n=128, k=5120)
+STREAMK = dict(types=BF16F32, m=1024, n=1024, k=16384)
+WIDE = dict(types=BF16, m=128, n=14336, k=8192)
+CUT_K = ("splitk_reduce", "streamk_fixup", "stream_wide_reduce")
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory, capi):
+    stub = tmp_path_factory.mktemp("stub") / "libhipstub.so"
+    subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", str(HERE / "hip_stub.c"), "-o", str(stub), "-ldl", "-lpthread"], check=True)
+
+    def steps(*what):
+        p = subprocess.run([sys.executable, str(HERE / "hip_stub_run.py"), str(stub), str(capi.LIB_PATH), json.dumps(what)],
+                           capture_output=True, text=True, timeout=120)
+        assert p.returncode == 0, p.stderr
+        return json.loads(p.stdout)
+    return steps
+
+
+def events(step, kind):
+    return [e for e in step["events"] if e[0] == kind]
+
+
+def cuts_k(step):
+    return [e for e in events(step, "launch") if any(name in e[3] for name in CUT_K)]
+
+
+@pytest.mark.parametrize("problem", (SPLITK, STREAMK, WIDE, dict(STREAMK, rung=MFMA, variant=7), dict(STREAMK, rung=MFMA, variant=8),
+                                     dict(WIDE, rung=SKINNY)))
+@pytest.mark.parametrize("warm", (False, True))
+def test_a_captured_call_takes_no_pool_memory(run, problem, warm):
+    """A graph keeps the addresses of what it captured, and the pool's buffers are replaced when a call needs more: a call
+    on a stream that is being captured runs a plan without a workspace, whether or not the stream has a buffer by then."""
+    call = dict(problem, stream=STREAM)
+    plain, cap, captured, off, after = run(*((["gemm", call],) if warm else (["stub_capture", 0],)), ["stub_capture", STREAM],
+                                           ["gemm", call], ["stub_capture", 0], ["gemm", call])
+    assert captured["result"][0] == 0, captured
+    assert not events(captured, "malloc") and not events(captured, "refused") and not events(captured, "free"), captured
+    assert events(captured, "launch") and not cuts_k(captured), captured
+    assert after["result"][0] == 0 and cuts_k(after), "outside the capture the same call cuts K"
+
+
+def test_static_scratch_cuts_k_under_capture(run):
+    """The entry point that allocates nothing has its buffer in the device image: captured calls keep their plan."""
+    for problem in (SPLITK, STREAMK, WIDE):
+        _, step = run(["stub_capture", STREAM], ["gemm", dict(problem, stream=STREAM, entry="gz_gemm_static_scratch")])
+        assert step["result"][0] == 0 and cuts_k(step) and not events(step, "malloc"), step
