@@ -67,6 +67,7 @@ std::map<std::pair<int, hipStream_t>, PoolBuffer> g_pool;   // entries stay wher
 
 size_t workspace_limit(hipStream_t s) {
   if (t_static_scratch) return (size_t)GZ_STATIC_SCRATCH_BYTES;
+  if (s == hipStreamPerThread) return 0;   // one handle, another stream in every thread: no key for a buffer
   if (s != nullptr) {   // (the null stream is never captured)
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess) {

@@ -310,8 +310,9 @@ struct WorkspaceLease {
 };
 // The most a lease can give on the calling thread for stream `s` right now: unbounded from the pool, the size of the
 // static buffer inside the entry point that allocates nothing, and nothing from the pool while `s` is being captured: a
-// graph would keep the address of a buffer that a later call may replace, and that calls beside a replay use.  Every
-// launcher plans within it; an explicit stream-K variant is the plain variant where it is zero.
+// graph would keep the address of a buffer that a later call may replace, and that calls beside a replay use.  Nothing
+// either on hipStreamPerThread, whose handle says nothing about which stream it is.  Every launcher plans within it; an
+// explicit stream-K variant is the plain variant where it is zero.
 size_t workspace_limit(hipStream_t s);
 
 // Raises a kernel's dynamic LDS limit once per device instead of on every launch.

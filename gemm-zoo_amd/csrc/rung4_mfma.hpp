@@ -1783,7 +1783,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     const MfmaCfg* forced = variant == 0 ? nullptr : &kMfmaCfgs[variant - 1];
     // the launcher's own choice stays within the workspace this call may use (the entry point that allocates nothing has a
     // fixed one); an explicit stream-K variant that needs more is refused by the lease instead, and where there is none
-    // at all (a captured stream) it runs the plain launch below, as on unaligned operands
+    // at all (workspace_limit) it runs the plain launch below, as on unaligned operands
     if (mfma_plan_streamk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, forced != nullptr, forced, &skp) &&
         (forced ? 1 : (size_t)skp.slots * MFMA_STREAMK_SLOT_BYTES) <= workspace_limit(s)) {
       const int cls = mfma_launch_class(skp.cfg, (int)sizeof(typename Traits<TYPES>::in_t),

@@ -138,7 +138,8 @@ typedef struct gz_plan_t {
   int32_t streamk_tiles, streamk_blocks;
   /* Memory beyond the matrices, from a pool of the library's own (one buffer per device and stream).  A call on a
    * stream that is being captured takes none of it - a graph keeps addresses, the pool replaces its buffers - and
-   * runs the best plan with workspace_bytes == 0 instead (gz_gemm_static_scratch: its own buffer, and this plan).  */
+   * neither does one on hipStreamPerThread, whose handle is the same in threads that run side by side: they run
+   * the best plan with workspace_bytes == 0 instead (gz_gemm_static_scratch: its own buffer, and this plan).     */
   int64_t workspace_bytes;
 } gz_plan_t;
 
@@ -213,7 +214,7 @@ int gz_gemm_ld(int types, const void* A, int64_t lda, const void* B, int64_t ldb
 
 /* gz_gemm for callers that cannot allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments and the same results,
- * bit for bit, as gz_gemm outside a capture (where gz_gemm runs plans without a workspace).  The one difference is where a launch that cuts K (see gz_plan_t) keeps its partial sums:
+ * bit for bit, as gz_gemm where that has its pool (not under capture, not on hipStreamPerThread).  The one difference is where a launch that cuts K (see gz_plan_t) keeps its partial sums:
  * not in the library's pool, which hipMalloc grows on demand, but in a buffer of GZ_STATIC_SCRATCH_BYTES (384
  * slots of 256 x 256 accumulators) that is part of the library's device image, so that every GPU the library runs
  * on holds its own copy until the process ends.  This entry point never allocates or frees.  A launch that would

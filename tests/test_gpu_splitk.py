@@ -128,6 +128,34 @@ def test_under_capture(G):
         assert torch.equal(e, other[2])
 
 
+def test_threads_on_the_per_thread_stream(G):
+    """hipStreamPerThread is one handle and another stream in every thread: calls that run side by side on it share no
+    partial sums."""
+    problems = [_problem(G, 20 + s) for s in range(4)]
+    outs = [[torch.empty(192, 128, dtype=torch.int32, device="cuda") for _ in range(25)] for _ in problems]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            a, b, _, (m, n, k) = problems[i]
+            for d in outs[i]:
+                G.capi.gemm(O.S8S8S32, a, b, None, d, m, n, k, O.ROW, O.COL, 1, 0, -1, 0, 2)
+        except Exception as e:   # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(problems))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for (_, _, ref, _), ds in zip(problems, outs):
+        for d in ds:
+            assert torch.equal(d, ref)
+
+
 def _bf16_problem(m, n, k):
     """Small whole numbers: every sum is exact."""
     gen = torch.Generator(device="cuda").manual_seed(m + n)

@@ -60,3 +60,16 @@ def test_static_scratch_cuts_k_under_capture(run):
     for problem in (SPLITK, STREAMK, WIDE):
         _, step = run(["stub_capture", STREAM], ["gemm", dict(problem, stream=STREAM, entry="gz_gemm_static_scratch")])
         assert step["result"][0] == 0 and cuts_k(step) and not events(step, "malloc"), step
+
+
+PER_THREAD = 2   # hipStreamPerThread: one handle, another stream in every thread
+
+
+@pytest.mark.parametrize("problem", (SPLITK, STREAMK, WIDE, dict(STREAMK, rung=MFMA, variant=7), dict(WIDE, rung=SKINNY)))
+def test_the_per_thread_stream_takes_no_pool_memory(run, problem):
+    """The pool keeps one buffer per stream handle; the per-thread stream's handle is the same in threads whose streams
+    run side by side, so calls on it run plans without a workspace."""
+    call = dict(problem, stream=PER_THREAD)
+    for step in run(["gemm", call], ["other_thread", call]):
+        assert step["result"][0] == 0 and events(step, "launch"), step
+        assert not events(step, "malloc") and not cuts_k(step), step
