@@ -276,8 +276,11 @@ static int check_problem(int types, int64_t M, int64_t N, int64_t K, int layoutA
   return GZ_OK;
 }
 
-static int resolve_rung(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung) {
+static int resolve_rung(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung, int variant) {
   if (rung != GZ_RUNG_AUTO) return rung;
+  // a pinned variant means a tile configuration of the MFMA rung, but for the problems that the streaming rung is offered
+  // for by name
+  if (variant != 0 && !skinny_supported(types, (int)M, (int)N, (int)K, layoutA, layoutB)) return GZ_RUNG_MFMA;
   if (skinny_preferred(types, (int)M, (int)N, (int)K, layoutA, layoutB, 0)) return GZ_RUNG_SKINNY;
   return GZ_RUNG_MFMA;
 }
@@ -337,7 +340,7 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
   g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ldd = ldd;
   hipStream_t s = static_cast<hipStream_t>(stream);
 
-  int resolved = resolve_rung(TYPES, M, N, K, layoutA, layoutB, rung);
+  int resolved = resolve_rung(TYPES, M, N, K, layoutA, layoutB, rung, variant);
   // the streaming kernel needs 16-byte aligned operands and lines; AUTO falls back to the tiled kernel otherwise
   if (rung == GZ_RUNG_AUTO && resolved == GZ_RUNG_SKINNY &&
       (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15u) || !skinny_lines_ok((int)sizeof(typename T::in_t), lda, ldb)))
@@ -535,7 +538,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
   if (num_cus <= 0) num_cus = 256;
   if (lds_per_cu <= 0) lds_per_cu = 160 * 1024;
   memset(plan, 0, sizeof(*plan));
-  const int r = resolve_rung(types, M, N, K, layoutA, layoutB, rung);
+  const int r = resolve_rung(types, M, N, K, layoutA, layoutB, rung, variant);
   plan->rung = r;
   plan->split_k = 1;
   const int es = in_size(types);

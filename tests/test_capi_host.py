@@ -276,3 +276,20 @@ def test_plan_skinny_split_k(capi):
     # the entry point that allocates nothing: the split only while its partial sums fit the static buffer
     p = capi.plan_static_scratch(capi.BF16BF16F32, 128, 14336, 8192, capi.ROW_MAJOR, capi.COL_MAJOR, capi.RUNG_SKINNY, 0, 256, 160 * 1024)
     assert p.split_k == 4 and p.workspace_bytes <= capi.STATIC_SCRATCH_BYTES
+
+
+def test_a_pinned_variant_means_the_mfma_rung_outside_what_the_streaming_rung_is_offered_for(capi):
+    """The launcher streams decode problems of the 8-bit types and of a K that is no multiple of 64; a caller who leaves
+    the rung to it and names a tile configuration gets that configuration there."""
+    MF, SK = capi.RUNG_MFMA, capi.RUNG_SKINNY
+    for types, m, n, k in [(capi.S8S8S32, 64, 4096, 4096), (capi.S8S8S32, 1, 4096, 4096), (capi.E4M3E4M3F16, 128, 14336, 4096),
+                           (capi.E5M2E5M2F16, 16, 37, 16), (capi.BF16BF16F32, 8, 4096, 1000), (capi.F16F16F16, 65, 1500, 48)]:
+        assert capi.plan(types, m, n, k, 0, 1).rung == SK
+        for variant in range(1, capi.variant_count(types, MF) + 1):
+            p = capi.plan(types, m, n, k, 0, 1, -1, variant)
+            assert p.as_dict() == capi.plan(types, m, n, k, 0, 1, MF, variant).as_dict(), (types, m, n, k, variant)
+    # where the rung can be named it has one variant, with or without the name
+    assert capi.plan(capi.BF16BF16F32, 8, 4096, 1024, 0, 1, -1, 1).rung == SK
+    with pytest.raises(capi.GzError) as e:
+        capi.plan(capi.BF16BF16F32, 8, 4096, 1024, 0, 1, -1, 3)
+    assert e.value.status == capi.ERR_UNSUPPORTED

@@ -73,3 +73,12 @@ def test_the_per_thread_stream_takes_no_pool_memory(run, problem):
     for step in run(["gemm", call], ["other_thread", call]):
         assert step["result"][0] == 0 and events(step, "launch"), step
         assert not events(step, "malloc") and not cuts_k(step), step
+
+
+def test_a_pinned_variant_launches_its_kernel(run):
+    """What the plan says of a pinned variant is what is launched (the streaming rung's kernels take no variants)."""
+    shapes = [dict(types=S8, m=64, n=4096, k=4096), dict(types=BF16, m=8, n=4096, k=1000), dict(types=5, m=1, n=4096, k=4096)]
+    for variant in (1, 3, 5, 12):
+        for problem, step in zip(shapes, run(*(["gemm", dict(s, variant=variant)] for s in shapes))):
+            assert step["result"][0] == 0, (problem, variant, step)
+            assert all("mfma" in e[3] for e in events(step, "launch")), (problem, variant, step)
