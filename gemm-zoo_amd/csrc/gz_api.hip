@@ -122,7 +122,12 @@ int WorkspaceLease::acquire(size_t bytes, hipStream_t s) {
     // (at least 16 MiB: most requests of a program then fit the first one)
     size_t want = (bytes + (size_t)(1 << 20) - 1) & ~((size_t)(1 << 20) - 1);
     if (want < (size_t)(16 << 20)) want = (size_t)(16 << 20);
-    GZ_HIP_TRY(hipMalloc(&b.ptr, want));
+    if (const hipError_t e = hipMalloc(&b.ptr, want); e != hipSuccess) {
+      b.ptr = nullptr;
+      (void)hipGetLastError();
+      out_of_memory = e == hipErrorOutOfMemory;
+      return hip_fail(e, "hipMalloc of a workspace");
+    }
     b.bytes = want;
   }
   ptr = b.ptr;

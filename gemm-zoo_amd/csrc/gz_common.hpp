@@ -300,6 +300,7 @@ int current_device_index();
 // so that its launches come behind all of this call's and not between them.
 struct WorkspaceLease {
   void* ptr = nullptr;
+  bool out_of_memory = false;                 // why acquire failed; any other failure is the caller's to know
   int acquire(size_t bytes, hipStream_t s);   // a gz_status
   WorkspaceLease() = default;
   ~WorkspaceLease();

@@ -1642,18 +1642,15 @@ template <int TYPES> static int launch_one(const GemmArgs<TYPES>& g, const MfmaC
   return GZ_ERR_UNSUPPORTED;
 }
 
-// A split K on 64 x 64 tiles (mfma_plan_splitk): the parts' sums in one launch, then the launch that adds them.  -1: the
-// workspace cannot be had, nothing was launched.
+// A split K on 64 x 64 tiles (mfma_plan_splitk): the parts' sums in one launch, then the launch that adds them.  -1: there
+// is no memory for the workspace, nothing was launched, and the caller runs a plan that needs none.
 template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPlan& p, hipStream_t s) {
   if constexpr (is_acc16(TYPES)) {
     set_error("mfma rung: no split K for this type bundle");
     return GZ_ERR_UNSUPPORTED;
   } else {
     WorkspaceLease lease;
-    if (lease.acquire((size_t)p.workspace_bytes, s) != GZ_OK) {   // no memory: the caller runs a plan that needs none
-      (void)hipGetLastError();
-      return -1;
-    }
+    if (const int st = lease.acquire((size_t)p.workspace_bytes, s); st != GZ_OK) return lease.out_of_memory ? -1 : st;
     constexpr int WAVES_M = sizeof(typename Traits<TYPES>::in_t) >= 2 ? 2 : 1, WAVES_N = 2;   // as the unsplit tile
     const int tiles_m = ceil_div(g.M, 64), tiles_n = ceil_div(g.N, 64), tiles = tiles_m * tiles_n;
     const SplitK sk{p.parts, p.q, p.rem, lease.ptr};

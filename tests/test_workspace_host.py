@@ -82,3 +82,22 @@ def test_a_pinned_variant_launches_its_kernel(run):
         for problem, step in zip(shapes, run(*(["gemm", dict(s, variant=variant)] for s in shapes))):
             assert step["result"][0] == 0, (problem, variant, step)
             assert all("mfma" in e[3] for e in events(step, "launch")), (problem, variant, step)
+
+
+LARGER = dict(types=BF16F32, m=408, n=2560, k=8164, lb=0)   # a split K with 17.5 MiB of partial sums
+
+
+def test_without_memory_a_split_k_runs_unsplit(run):
+    """A problem that needs no workspace but is faster with one must not fail for want of it."""
+    _, small, large = run(["stub_memory", 1], ["gemm", dict(SPLITK, stream=STREAM)], ["gemm", dict(LARGER, stream=STREAM)])
+    assert cuts_k(small) and large["result"][0] == 0
+    assert events(large, "nomemory") and events(large, "launch") and not cuts_k(large)
+
+
+def test_an_earlier_failure_is_reported(run):
+    """Growing the pool waits for the stream, which may report what went wrong in work that was queued before: that is no
+    lack of memory, and the caller has to hear of it."""
+    _, _, step, _, again = run(["gemm", dict(SPLITK, stream=STREAM)], ["stub_sync_status", 719], ["gemm", dict(LARGER, stream=STREAM)],
+                               ["stub_sync_status", 0], ["gemm", dict(LARGER, stream=STREAM)])
+    assert step["result"][0] == 3 and "hipStreamSynchronize" in step["result"][1] and not events(step, "launch"), step
+    assert again["result"][0] == 0 and cuts_k(again)
