@@ -35,7 +35,7 @@ int hip_fail(hipError_t e, const char* what) {
 }
 
 // ---------------------------------------------------------------------------
-// Workspace of the stream-K launches
+// Workspace of the launches that cut K
 // ---------------------------------------------------------------------------
 static thread_local bool t_static_scratch = false;   // set for the duration of a gz_gemm_static_scratch call
 
@@ -57,12 +57,36 @@ static int scratch_address(void** out) {
 
 namespace {
 struct PoolBuffer {
-  std::mutex in_use;   // held by the call whose launches are being enqueued
+  std::mutex in_use;      // held by the call whose launches are being enqueued, which alone changes ptr
+  int users = 0;          // calls that hold in_use or wait for it; this and the rest under g_pool_mutex
+  uint64_t last_use = 0;
   void* ptr = nullptr;
   size_t bytes = 0;
 };
 std::mutex g_pool_mutex;
-std::map<std::pair<int, hipStream_t>, PoolBuffer> g_pool;   // entries stay where they are; never freed before the process ends
+std::map<std::pair<int, hipStream_t>, PoolBuffer> g_pool;   // an entry stays where it is while it has users
+uint64_t g_pool_calls = 0;
+// A device that had no memory left is not asked again for as much by the next calls that can do without.
+struct NoMemory { size_t bytes = ~(size_t)0; uint64_t until = 0; };
+std::map<int, NoMemory> g_no_memory;
+constexpr uint64_t POOL_RETRY_CALLS = 256;
+// The buffers of one device together, unless single calls on streams of their own need more at the same time: sixteen
+// streams with the largest split K.  Programs make and drop streams, and a handle does not say that its stream is gone.
+constexpr size_t POOL_BYTES = (size_t)1 << 30;
+
+// The idle buffer that has gone longest without a call leaves the pool (g_pool_mutex is held); null: none is idle.
+// Whoever frees it waits for the work that may still use it: hipFree synchronizes with the device.
+void* pool_take_idle(int dev) {
+  for (;;) {
+    auto oldest = g_pool.end();
+    for (auto it = g_pool.begin(); it != g_pool.end(); ++it)
+      if (it->first.first == dev && it->second.users == 0 && (oldest == g_pool.end() || it->second.last_use < oldest->second.last_use)) oldest = it;
+    if (oldest == g_pool.end()) return nullptr;
+    void* p = oldest->second.ptr;
+    g_pool.erase(oldest);
+    if (p) return p;   // (an entry that never got its memory just goes)
+  }
+}
 }  // namespace
 
 size_t workspace_limit(hipStream_t s) {
@@ -80,10 +104,81 @@ size_t workspace_limit(hipStream_t s) {
 }
 
 WorkspaceLease::~WorkspaceLease() {
-  if (held_) static_cast<PoolBuffer*>(held_)->in_use.unlock();
+  if (!held_) return;
+  PoolBuffer* b = static_cast<PoolBuffer*>(held_);
+  b->in_use.unlock();
+  std::lock_guard<std::mutex> lock(g_pool_mutex);
+  b->users--;
 }
 
-int WorkspaceLease::acquire(size_t bytes, hipStream_t s) {
+// Gives `b`, which the calling thread holds, a buffer of at least `bytes`.
+static int pool_grow(PoolBuffer& b, int dev, uint64_t call, size_t bytes, hipStream_t s, bool optional, bool* out_of_memory) {
+  // (whole powers of two up to 64 MiB, so that a program's growing problems replace a buffer a few times and not each time)
+  size_t want = (bytes + (size_t)(1 << 20) - 1) & ~((size_t)(1 << 20) - 1);
+  for (size_t p = (size_t)1 << 20; p <= ((size_t)64 << 20); p <<= 1)
+    if (p >= want) { want = p; break; }
+  {
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    const NoMemory& n = g_no_memory[dev];
+    if (optional && call < n.until && want >= n.bytes) {
+      *out_of_memory = true;
+      return hip_fail(hipErrorOutOfMemory, "hipMalloc of a workspace (an earlier call's)");
+    }
+  }
+  // another thread may be capturing: growing this pool is none of that graph's business
+  struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  } relaxed;
+  if (b.ptr) {
+    // work queued on this stream may still use the old buffer
+    GZ_HIP_TRY(hipStreamSynchronize(s));
+    GZ_HIP_TRY(hipFree(b.ptr));
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    b.ptr = nullptr;
+    b.bytes = 0;
+  }
+  auto held = [&] {   // by the device's buffers (g_pool_mutex is held)
+    size_t sum = 0;
+    for (const auto& e : g_pool) sum += e.first.first == dev ? e.second.bytes : 0;
+    return sum;
+  };
+  for (;;) {
+    void* p = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(g_pool_mutex);
+      if (held() + want > POOL_BYTES) p = pool_take_idle(dev);
+    }
+    if (!p) break;
+    GZ_HIP_TRY(hipFree(p));
+  }
+  for (;;) {
+    void* fresh = nullptr;
+    const hipError_t e = hipMalloc(&fresh, want);
+    if (e == hipSuccess) {
+      std::lock_guard<std::mutex> lock(g_pool_mutex);
+      b.ptr = fresh;
+      b.bytes = want;
+      return GZ_OK;
+    }
+    (void)hipGetLastError();
+    if (e != hipErrorOutOfMemory) return hip_fail(e, "hipMalloc of a workspace");
+    void* p = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(g_pool_mutex);
+      p = pool_take_idle(dev);
+      if (!p) g_no_memory[dev] = NoMemory{want, call + POOL_RETRY_CALLS};
+    }
+    if (!p) {
+      *out_of_memory = true;
+      return hip_fail(e, "hipMalloc of a workspace");
+    }
+    GZ_HIP_TRY(hipFree(p));   // what idle streams hold may be enough
+  }
+}
+
+int WorkspaceLease::acquire(size_t bytes, hipStream_t s, bool optional) {
   if (t_static_scratch) {   // no allocation on this path
     if (bytes > (size_t)GZ_STATIC_SCRATCH_BYTES) {
       set_error("this launch needs %zu bytes of scratch memory, the static buffer holds %lld: use gz_gemm, which "
@@ -97,40 +192,20 @@ int WorkspaceLease::acquire(size_t bytes, hipStream_t s) {
     set_error("a launch with a workspace on a stream that may use none");
     return GZ_ERR_UNSUPPORTED;
   }
-  PoolBuffer* entry = nullptr;
+  const int dev = current_device_index();
+  PoolBuffer* b = nullptr;
+  uint64_t call = 0;
   {
     std::lock_guard<std::mutex> lock(g_pool_mutex);
-    entry = &g_pool[{current_device_index(), s}];
+    b = &g_pool[{dev, s}];
+    b->users++;
+    call = b->last_use = ++g_pool_calls;
   }
-  entry->in_use.lock();
-  held_ = entry;
-  PoolBuffer& b = *entry;
-  if (b.bytes < bytes) {
-    // another thread may be capturing: growing this pool is none of that graph's business
-    struct RelaxedCapture {
-      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-      RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-      ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-    } relaxed;
-    if (b.ptr) {
-      // work queued on this stream may still use the old buffer
-      GZ_HIP_TRY(hipStreamSynchronize(s));
-      GZ_HIP_TRY(hipFree(b.ptr));
-      b.ptr = nullptr;
-      b.bytes = 0;
-    }
-    // (at least 16 MiB: most requests of a program then fit the first one)
-    size_t want = (bytes + (size_t)(1 << 20) - 1) & ~((size_t)(1 << 20) - 1);
-    if (want < (size_t)(16 << 20)) want = (size_t)(16 << 20);
-    if (const hipError_t e = hipMalloc(&b.ptr, want); e != hipSuccess) {
-      b.ptr = nullptr;
-      (void)hipGetLastError();
-      out_of_memory = e == hipErrorOutOfMemory;
-      return hip_fail(e, "hipMalloc of a workspace");
-    }
-    b.bytes = want;
-  }
-  ptr = b.ptr;
+  b->in_use.lock();
+  held_ = b;
+  if (b->bytes < bytes)
+    if (const int st = pool_grow(*b, dev, call, bytes, s, optional, &out_of_memory); st != GZ_OK) return st;
+  ptr = b->ptr;
   return GZ_OK;
 }
 

@@ -295,13 +295,14 @@ int current_device_index();
 
 // Device memory beyond the caller's matrices for the launches of one call on stream `s` (partial sums): at least
 // `bytes`, 256-byte aligned.  From the library's own pool (one buffer per device and stream, grown with hipMalloc when
-// a call needs more), or - inside the entry point that allocates nothing - the static buffer, which refuses what it
+// a call needs more; past 1 GiB a device, or where memory runs out, the buffers that have been idle longest are freed), or - inside the entry point that allocates nothing - the static buffer, which refuses what it
 // cannot hold.  The lease lasts while the call enqueues its launches: another thread that uses the same stream waits,
 // so that its launches come behind all of this call's and not between them.
 struct WorkspaceLease {
   void* ptr = nullptr;
   bool out_of_memory = false;                 // why acquire failed; any other failure is the caller's to know
-  int acquire(size_t bytes, hipStream_t s);   // a gz_status
+  // a gz_status; optional: the caller has a plan without a workspace, and a full device is not asked on every call
+  int acquire(size_t bytes, hipStream_t s, bool optional = false);
   WorkspaceLease() = default;
   ~WorkspaceLease();
   WorkspaceLease(const WorkspaceLease&) = delete;

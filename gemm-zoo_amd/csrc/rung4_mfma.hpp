@@ -1650,7 +1650,7 @@ template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPla
     return GZ_ERR_UNSUPPORTED;
   } else {
     WorkspaceLease lease;
-    if (const int st = lease.acquire((size_t)p.workspace_bytes, s); st != GZ_OK) return lease.out_of_memory ? -1 : st;
+    if (const int st = lease.acquire((size_t)p.workspace_bytes, s, true); st != GZ_OK) return lease.out_of_memory ? -1 : st;
     constexpr int WAVES_M = sizeof(typename Traits<TYPES>::in_t) >= 2 ? 2 : 1, WAVES_N = 2;   // as the unsplit tile
     const int tiles_m = ceil_div(g.M, 64), tiles_n = ceil_div(g.N, 64), tiles = tiles_m * tiles_n;
     const SplitK sk{p.parts, p.q, p.rem, lease.ptr};

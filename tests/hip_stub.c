@@ -15,7 +15,7 @@ static pthread_mutex_t mutex = PTHREAD_MUTEX_INITIALIZER;
 static char text[1 << 20];
 static size_t used;
 static uintptr_t capturing;              /* the stream that is being captured, 0: none */
-static int sync_status, memory = 1 << 30;
+static int sync_status, room, memory = 1 << 30;
 static uintptr_t next_address = 0x7f0000000000;
 static __thread int mode = MODE_GLOBAL;
 
@@ -30,6 +30,7 @@ static void note(const char* what, uintptr_t a, uintptr_t b, const char* name) {
 void stub_capture(uintptr_t stream) { capturing = stream; }
 void stub_sync_status(int status) { sync_status = status; }
 void stub_memory(int allocations) { memory = allocations; }   /* how many more allocations succeed */
+void stub_room(int on) { room = on, memory = on ? 0 : memory; }   /* every free makes room for one allocation */
 const char* stub_take(void) {
   static char out[sizeof(text)];
   memcpy(out, text, used);
@@ -50,7 +51,7 @@ int hipMalloc(void** p, size_t bytes) {
   note("malloc", bytes, (uintptr_t)*p, "-");
   return OK;
 }
-int hipFree(void* p) { return note("free", (uintptr_t)p, 0, "-"), OK; }
+int hipFree(void* p) { return memory += room, note("free", (uintptr_t)p, 0, "-"), OK; }
 int hipStreamSynchronize(void* s) { return note("sync", (uintptr_t)s, 0, "-"), sync_status; }
 int hipStreamIsCapturing(void* s, int* status) { return *status = (uintptr_t)s == capturing && capturing != 0, OK; }
 int hipThreadExchangeStreamCaptureMode(int* m) {

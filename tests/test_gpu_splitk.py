@@ -156,6 +156,26 @@ def test_threads_on_the_per_thread_stream(G):
             assert torch.equal(d, ref)
 
 
+def test_the_pool_gives_idle_buffers_back(G):
+    """More streams than the pool holds buffers for (68 MiB each, 1 GiB in all): those that have gone longest without a
+    call lose theirs, get new ones when they call again, and every result is right."""
+    a, b, ref, (m, n, k) = _bf16_problem(1024, 1024, 16384)
+    assert 17 * G.capi.plan(O.BF16BF16F32, m, n, k, O.ROW, O.COL).workspace_bytes > 1 << 30
+    streams = [torch.cuda.Stream() for _ in range(20)]
+    torch.cuda.synchronize()
+    free = []
+    for part in (streams[:10], streams[10:], streams[:10]):
+        outs = [torch.full((m, n), -1.0, device="cuda") for _ in part]
+        torch.cuda.synchronize()
+        for d, s in zip(outs, part):
+            G.capi.gemm(O.BF16BF16F32, a, b, None, d, m, n, k, O.ROW, O.COL, 1, 0, -1, 0, s.cuda_stream)
+        torch.cuda.synchronize()
+        assert all(torch.equal(d, ref) for d in outs)
+        del outs
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[2] >= free[1] - (128 << 20), "the third part took the place of the second's buffers"
+
+
 def _bf16_problem(m, n, k):
     """Small whole numbers: every sum is exact."""
     gen = torch.Generator(device="cuda").manual_seed(m + n)

@@ -101,3 +101,48 @@ def test_an_earlier_failure_is_reported(run):
                                ["stub_sync_status", 0], ["gemm", dict(LARGER, stream=STREAM)])
     assert step["result"][0] == 3 and "hipStreamSynchronize" in step["result"][1] and not events(step, "launch"), step
     assert again["result"][0] == 0 and cuts_k(again)
+
+
+def live(steps):
+    """Bytes held after each step."""
+    sizes, out = {}, []
+    for step in steps:
+        for e in step["events"]:
+            if e[0] == "malloc":
+                sizes[e[2]] = e[1]
+            elif e[0] == "free":
+                assert sizes.pop(e[1], None) is not None, "freed twice"
+        out.append(sum(sizes.values()))
+    return out
+
+
+def test_a_small_problem_takes_little(run):
+    step, = run(["gemm", dict(SPLITK, stream=STREAM)])
+    assert live([step])[0] <= 4 << 20, "1.9 MiB of partial sums"
+
+
+def test_streams_that_come_and_go_do_not_pile_up(run, capi):
+    """A handle is all the pool knows of a stream; the buffers that have gone longest without a call are given back."""
+    need = capi.plan(BF16F32, 1024, 1024, 16384, 0, 1).workspace_bytes
+    steps = run(*(["gemm", dict(STREAMK, stream=0x1000 + 16 * i)] for i in range(60)), ["gemm", dict(STREAMK, stream=0x1000 + 16 * 59)],
+                ["gemm", dict(STREAMK, stream=0x1000)])
+    held = live(steps)
+    assert max(held) <= 1 << 30 and held[3] >= 4 * need and all(s["result"][0] == 0 and cuts_k(s) for s in steps)
+    assert not steps[60]["events"][0][0] == "malloc", "the last stream's buffer is still there"
+    assert events(steps[61], "malloc"), "the first stream's is not, and the stream gets another"
+
+
+def test_a_full_device_is_not_asked_on_every_call(run):
+    call = ["gemm", dict(SPLITK, stream=STREAM)]
+    _, *calls = run(["stub_memory", 0], *([call] * 300))
+    assert all(s["result"][0] == 0 and events(s, "launch") and not cuts_k(s) for s in calls)
+    assert 1 <= sum(bool(events(s, "nomemory")) for s in calls) <= 3
+    _, _, _, *later = run(["stub_memory", 0], call, ["stub_memory", 9], *([call] * 300))
+    assert cuts_k(later[-1]), "memory that comes back is found"
+    assert run(["stub_memory", 0], call, ["stub_memory", 9], ["gemm", dict(STREAMK, stream=STREAM)])[3]["result"][0] == 0
+
+
+def test_idle_buffers_make_room(run):
+    """What another stream's idle buffer holds is given back before a call is told that there is no memory."""
+    first, _, second = run(["gemm", dict(SPLITK, stream=STREAM)], ["stub_room", 1], ["gemm", dict(SPLITK, stream=STREAM + 16)])
+    assert events(second, "nomemory") and events(second, "free") and cuts_k(second), second
