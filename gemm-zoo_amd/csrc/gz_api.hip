@@ -361,8 +361,10 @@ static int resolve_rung(int types, int64_t M, int64_t N, int64_t K, int layoutA,
   // a pinned variant means a tile configuration of the MFMA rung, but for the problems that the streaming rung is offered
   // for by name
   if (variant != 0 && !skinny_supported(types, (int)M, (int)N, (int)K, layoutA, layoutB)) return GZ_RUNG_MFMA;
-  if (skinny_preferred(types, (int)M, (int)N, (int)K, layoutA, layoutB, 0)) return GZ_RUNG_SKINNY;
-  return GZ_RUNG_MFMA;
+  if (!skinny_preferred(types, (int)M, (int)N, (int)K, layoutA, layoutB, 0)) return GZ_RUNG_MFMA;
+  // (the 16-bit types with whole K super-steps, which the rung has always had, stay with it)
+  if (!skinny_supported(types, (int)M, (int)N, (int)K, layoutA, layoutB) && skinny_wide_to_mfma(types, (int)M, (int)N, (int)K, 0)) return GZ_RUNG_MFMA;
+  return GZ_RUNG_SKINNY;
 }
 
 static int check_named_skinny(int types, int M, int N, int K, int layoutA, int layoutB) {
@@ -436,6 +438,7 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
       if ((st = launch_splitk<TYPES>(g, kp, s)) >= 0) return st;
     }
     if (how == SKINNY_TILES_64) return launch_mfma<TYPES>(g, kMfmaCfgs[MFMA_CFG_64].id, s);
+    if (how == SKINNY_TILES) return launch_mfma<TYPES>(g, 0, s);
   }
   switch (resolved) {
     case GZ_RUNG_NAIVE: return launch_naive<TYPES>(g, variant, s);
@@ -795,7 +798,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
         if (how == SKINNY_TILES_SPLITK) {
           plan_splitk(kp, types, m, n, plan);
         } else {
-          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, kMfmaCfgs[MFMA_CFG_64].id, num_cus, lds_per_cu, ws_limit, plan);
+          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, how == SKINNY_TILES_64 ? kMfmaCfgs[MFMA_CFG_64].id : 0, num_cus, lds_per_cu, ws_limit, plan);
           if (st != GZ_OK) return st;
         }
         plan->rung = GZ_RUNG_SKINNY;

@@ -93,6 +93,25 @@ inline bool skinny_preferred(int types, int M, int N, int K, int layoutA, int la
   return M <= 32 || (long long)((N + 127) / 128) <= num_cus;
 }
 
+// More columns than one work-group of the tile kernel per compute unit holds (64 each).  A second round of work-groups
+// pays its fill and its stores again with nothing beside them, where the MFMA rung's tiles run several to a compute unit,
+// and from 65 rows on each work-group takes in all of A as well.  Against that the streaming kernels read memory faster
+// than the tiles do.  Whether the tiles win on the whole (geometric mean of both states of the cache); us, streaming / MFMA
+// rung, operands just used; after 512 MiB of other data - they do: int8 16 x 28672 x 1024 8.7 / 7.0; 10.6 / 10.9,
+// 32 x 16640 x 1024 8.6 / 6.7; 9.4 / 9.8, 128 x 20480 x 4096 31.7 / 20.8; 32.4 / 34.3; they do not: 16 x 32768 x 4096
+// 21.4 / 21.3; 23.8 / 41.1, 32 x 20480 x 4096 17.6 / 16.6; 19.1 / 27.9, 64 x 28672 x 3072 21.8 / 16.6; 23.4 / 27.2,
+// 65 x 24576 x 14336 83.1 / 83.5; 83.4 / 98.1.
+inline bool skinny_wide_to_mfma(int types, int M, int N, int K, int num_cus) {
+  if (num_cus <= 0) num_cus = 256;
+  const double rounds = (double)N / (64.0 * num_cus);
+  if (rounds <= 1.0) return false;
+  const long long kb = (long long)K * (skinny_rung_types(types) ? 2 : 1);
+  if (M <= 32) return kb <= 2048 && kb <= (M <= SKINNY_REG_MAX_M ? 640 : 1024) * rounds;
+  // (a few columns past one round and a short K: 64 x 64 tiles, skinny_choose; e4m3 128 x 24576 x 512 streaming / MFMA rung /
+  // 64 x 64 10.6 / 7.3 / 6.5; 11.8 / 10.0 / 9.6)
+  return M > 64 && kb <= 8192 && (kb > 3072 || rounds > (kb <= 512 ? 1.5 : 1.125));
+}
+
 // equal column groups, one or more per compute unit, at most max_cols columns and a multiple of 4 each
 inline int skinny_balanced_cols(int N, int num_cus, int max_cols) {
   if (num_cus <= 0) num_cus = 256;
@@ -183,26 +202,41 @@ inline SkinnyCfg skinny_resolve(int types, int M, int N, int K, int num_cus, uns
 // The launcher's choice between the tile kernel above and the MFMA rung's 64 x 64 tiles for 17 ... 128 rows.  Every
 // work-group of the tile kernel walks all of K and takes in all of A beside its share of the columns: with few columns
 // per work-group and a long K it takes in mostly A, and the 64 x 64 tiles with a split K are faster; with many rows and a
-// short K its fill and its one pass of stores are not paid back, and the same tiles unsplit are.  Measured, us, tile
+// short K its fill and its one pass of stores are not paid back, and the same tiles unsplit are (below).  Measured, us, tile
 // kernel / split K: bf16 20 x 2560 x 8192 18.2 / 14.6, 50 x 1024 x 8192 27.1 / 12.5, 100 x 2560 x 4096 20.3 / 14.0,
 // 128 x 5120 x 4096 23.6 / 20.9, 20 x 5120 x 8192 19.6 / 22.3, 100 x 9600 x 4096 26.1 / 36; e4m3 50 x 2560 x 8192
-// 16.3 / 12.3, 100 x 9600 x 8192 25.4 / 32.9.  Tile kernel / unsplit, K = 1280 bf16: 128 rows on 1024, 5120, 9600 and
-// 14336 columns 9.4 / 9.3, 11.6 / 9.7, 14.3 / 11.8, 16.2 / 12.1; 50 rows 6.5 / 8.4, 7.7 / 9.7, 9.1 / 10, 10.3 / 10.3;
-// at K = 4096 128 x 14336 32.9 / 44.
+// 16.3 / 12.3, 100 x 9600 x 8192 25.4 / 32.9.
 inline double skinny_tile_estimate_us(int stages, int mb, int cols) {
   if (mb == 32) return 3.4 + stages * (cols < 26 ? 0.118 : 0.0046 * cols);   // (many columns: the rate of the B stream)
   if (mb == 64) return 3.2 + 0.015 * cols + stages * (0.185 + 0.0019 * cols);
   return 4.2 + 0.075 * cols + stages * (0.225 + 0.0026 * cols);
 }
-enum { SKINNY_STREAM = 0, SKINNY_TILES_SPLITK = 1, SKINNY_TILES_64 = 2 };
+// 65 rows and more: up to how many 128-byte stages of K the unsplit 64 x 64 tiles are taken.  They win while the operands
+// come from the cache and lose from memory, where the tile kernel's producers keep more in flight, so the line lies where
+// the one outweighs the other (geometric mean), about alike for 8-bit and 16-bit elements.  us, tile kernel / 64 x 64
+// tiles, operands just used; after 512 MiB of other data:
+// up to 32 columns per work-group, 8 stages bf16 96 x 2560 6.1 / 4.9; 6.3 / 7.2, int8 128 x 2560 6.4 / 5.5; 7.0 / 7.5, 16 stages
+// int8 128 x 2560 8.5 / 7.5; 9.1 / 11.4, bf16 128 x 5120 8.5 / 6.8; 9.5 / 11.9, 65 x 7168 8.5 / 6.9; 8.8 / 11.8;
+// more, 4 stages bf16 128 x 9600 5.8 / 5.0; 6.5 / 6.6, e4m3 65 x 14336 5.6 / 5.6; 6.2 / 7.5, 8 stages int8 65 x 9600 6.9 / 7.3; 7.3 / 9.3,
+// bf16 128 x 16384 7.5 / 6.5; 8.3 / 10.0, 16 stages int8 128 x 14336 11.2 / 10.8; 12.4 / 15.2, 24 stages bf16 128 x 16384
+// 15.5 / 13.6; 17.2 / 21.0.
+// Past one round of work-groups (skinny_wide_to_mfma) the tiles win up to a longer K, 64 x 64 ones while there are up to
+// three to a compute unit: bf16 128 x 24576 x 1024 20.6 / 13.6; 21.6 / 20.9, 96 x 20480 x 1536 23.8 / 17.3; 25.0 / 26.4; beyond,
+// those that the MFMA rung chooses: bf16 128 x 32768 x 1024, tile kernel / 64 x 64 / chosen 20.9 / 17.5 / 15.4; 21.9 / 28.6 / 22.2.
+inline int skinny_tiles_max_stages(int cols, bool one_round) {
+  if (!one_round) return 16 + cols / 4;
+  return cols <= 32 ? 8 : 4;
+}
+enum { SKINNY_STREAM = 0, SKINNY_TILES_SPLITK = 1, SKINNY_TILES_64 = 2, SKINNY_TILES = 3 };   // (TILES: the MFMA rung's own choice)
 inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned long long ws_limit, SplitKPlan* split) {
   if (M <= SKINNY_REG_MAX_M) return SKINNY_STREAM;
   const SkinnyCfg c = skinny_resolve(types, M, N, K, num_cus, ws_limit);
   if (c.kind != SKINNY_KIND_TILE) return SKINNY_STREAM;
   const int es = skinny_rung_types(types) ? 2 : 1;
   const int stages = (int)(((long long)K * es + STREAM_TILE_ROW_BYTES - 1) / STREAM_TILE_ROW_BYTES);
-  // (the two lines cross at 21, 25 and 31 stages for 20, 40 and 56 columns per work-group)
-  if (M > 64 && c.cols_per_wg >= 16 && stages <= 16 + c.cols_per_wg / 4) return SKINNY_TILES_64;
+  if (num_cus <= 0) num_cus = 256;
+  if (M > 64 && stages <= skinny_tiles_max_stages(c.cols_per_wg, c.grid_n <= num_cus))
+    return 2LL * ((N + 63) / 64) <= 3LL * num_cus ? SKINNY_TILES_64 : SKINNY_TILES;
   if (mfma_best_splitk(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus, split) &&
       (unsigned long long)split->workspace_bytes <= ws_limit &&
       split->estimate_us < 0.9 * skinny_tile_estimate_us(stages, c.mb, c.cols_per_wg))

@@ -111,7 +111,7 @@ def test_plan_headline_configs(capi):
     assert capi.plan(capi.BF16BF16BF16, 128, 65536, 4096, 0, 1).rung == capi.RUNG_MFMA
     assert capi.plan(capi.BF16BF16BF16, 32, 65536, 4096, 0, 1).rung == capi.RUNG_SKINNY
     assert capi.plan(capi.BF16BF16BF16, 129, 14336, 4096, 0, 1).rung == capi.RUNG_MFMA
-    # K that is a multiple of 64 but not of 128 takes the register-streaming kernel for M <= 16
+    # (bytes of K per stage: 256 for M <= 16, reported as 128 where the last stage is half a one; 128 above)
     assert capi.plan(capi.BF16BF16BF16, 8, 4096, 192, 0, 1).tile_k == 64
     assert capi.plan(capi.BF16BF16BF16, 8, 4096, 256, 0, 1).tile_k == 128
     assert capi.plan(capi.BF16BF16BF16, 24, 4096, 192, 0, 1).tile_k == 64
@@ -293,3 +293,30 @@ def test_a_pinned_variant_means_the_mfma_rung_outside_what_the_streaming_rung_is
     with pytest.raises(capi.GzError) as e:
         capi.plan(capi.BF16BF16F32, 8, 4096, 1024, 0, 1, -1, 3)
     assert e.value.status == capi.ERR_UNSUPPORTED
+
+
+def test_decode_problems_where_the_mfma_rung_is_the_faster_one(capi):
+    """The line between the streaming kernels and the MFMA rung's tiles for M <= 128 with K-contiguous weights (both sides
+    timed, gz_skinny_cfg.hpp: skinny_wide_to_mfma, skinny_tiles_max_stages)."""
+    S8, E4, BF = capi.S8S8S32, capi.E4M3E4M3F16, capi.BF16BF16BF16
+    kernel = lambda *a: capi.plan(*a, 0, 1)
+    # more columns than one round of work-groups: the 8-bit types, and a K that is no multiple of 64
+    for types in (S8, E4):
+        for m, n, k in [(1, 20480, 512), (16, 65536, 2048), (32, 16640, 1024), (128, 20480, 4096), (128, 32768, 4096), (65, 16640, 8192)]:
+            assert kernel(types, m, n, k).as_dict() == capi.plan(types, m, n, k, 0, 1, capi.RUNG_MFMA).as_dict(), (m, n, k)
+        for m, n, k in [(1, 32768, 4096), (32, 20480, 4096), (64, 28672, 2048), (8, 128256, 4096), (128, 32768, 14336), (128, 14336, 4096),
+                        (65, 9600, 1024), (128, 4096, 2048)]:
+            p = kernel(types, m, n, k)
+            assert p.rung == capi.RUNG_SKINNY and p.variant == 1, (m, n, k)
+    assert kernel(BF, 8, 32768, 504).rung == capi.RUNG_MFMA
+    # the 16-bit types with a whole K stay on the rung they had; 65 rows and more with a short K on the MFMA rung's tiles
+    assert kernel(BF, 32, 65536, 512).rung == capi.RUNG_SKINNY
+    for m, n, k in [(65, 16384, 512), (128, 14336, 1536), (128, 16384, 2048), (128, 9600, 512), (96, 5120, 1024), (128, 28672, 4096)]:
+        p = kernel(BF, m, n, k)
+        assert (p.variant, p.threads, p.tile_m) == (1, 512, 128), (m, n, k)
+    p, q = kernel(BF, 128, 32768, 1024), capi.plan(BF, 128, 32768, 1024, 0, 1, capi.RUNG_MFMA)
+    assert (p.variant, p.tile_m, p.tile_n, p.grid) == (q.variant, q.tile_m, q.tile_n, q.grid) and p.tile_n > 64
+    for args in [(BF, 96, 2560, 512), (BF, 128, 8192, 512), (BF, 128, 14336, 256), (S8, 128, 2560, 1024), (S8, 65, 16640, 2048),
+                 (E4, 128, 24576, 512), (BF, 128, 24576, 1024), (BF, 96, 20480, 1536)]:
+        p = kernel(*args)
+        assert (p.rung, p.tile_m, p.tile_n, p.split_k) == (capi.RUNG_SKINNY, 64, 64, 1) and p.grid == 2 * -(-args[2] // 64), args

@@ -230,7 +230,7 @@ def test_a_few_columns_past_a_tile_multiple(G, types):
 
 @pytest.mark.parametrize("types", SKINNY_TYPES)
 def test_skinny_rung(G, types):
-    # three kernels: M <= 16 with K % 128 == 0 (direct-to-LDS), M <= 16 otherwise (registers), 16 < M <= 128 (tile)
+    # two kernels: M <= 16 (direct-to-LDS, an instance each for a K of whole and of cut chunks), 16 < M <= 128 (tile)
     for (m, n, k), (al, be) in itertools.product([(1, 16, 64), (1, 1000, 256), (8, 14336, 512), (16, 250, 128),
                                                   (13, 37, 384), (17, 33, 192), (32, 512, 4096), (33, 100, 64),
                                                   (64, 3000, 1024), (100, 9, 128), (128, 7170, 576)],
@@ -306,6 +306,45 @@ def test_launcher_streams_decode_shapes_of_every_narrow_type(G, types):
         for pads in [(16, 32, 4, 8), (32, 16, 1, 3), (3, 16, 0, 0)]:
             got = G.run_gemm_ld(types, a, b, c, m, n, k, O.ROW, O.COL, 1, 1, -1, 0, pads)
             assert np.array_equal(got, ref), (types, m, n, k, pads)
+
+
+@pytest.mark.parametrize("types", STREAM_TYPES)
+def test_tile_kernel_of_65_to_128_rows_with_a_cut_last_stage(G, types):
+    """The streaming tile kernel for 65 ... 128 rows with several stages of K, the last one shorter: its masked copies, the
+    pieces past the end of K that the consumer waves clear in LDS, shared rows of A, and a rotation that puts the short
+    stage in the middle of a work-group's walk; few and many columns per work-group.  The plan says that this kernel
+    runs.  Integer-valued data: bit-exact."""
+    es = 1 if types in (O.S8S8S32, O.E4M3E4M3F16, O.E5M2E5M2F16) else 2
+    kind = O.FILL_INT8_UNIFORM if types == O.S8S8S32 else O.FILL_SMALL_INT
+    for i, (m, n, kb) in enumerate([(128, 9001, 1024 + 48), (65, 14340, 1152 + 112), (100, 12004, 2048 + 16), (128, 2100, 2304 + 48),
+                                    (96, 4100, 2304 + 16), (70, 1029, 2176 + 96)]):
+        k = kb // es
+        p = G.capi.plan(types, m, n, k, O.ROW, O.COL)
+        assert (p.rung, p.variant, p.tile_m, p.threads, p.split_k) == (SKINNY, 1, 128, 512, 1), (types, m, n, kb)
+        a, b, c = O.make_inputs(types, m, n, k, kind=kind, seed=m + n)
+        al, be = ((1, 0), (2, 3))[i % 2]
+        print("case", types, m, n, k, al, be, flush=True)
+        ref = O.gemm(types, a, b, c, m, n, k, O.ROW, O.COL, al, be)
+        assert np.array_equal(G.run_gemm(types, a, b, c, m, n, k, O.ROW, O.COL, al, be, -1), ref), (types, m, n, k, al, be)
+        if n < 5000:   # views whose padding is NaN (or large)
+            got = G.run_gemm_ld(types, a, b, c, m, n, k, O.ROW, O.COL, al, be, -1, 0, (32, 16, 1, 3))
+            assert np.array_equal(got, ref), (types, m, n, k)
+
+
+@pytest.mark.parametrize("types", STREAM_TYPES)
+def test_decode_problems_of_more_columns_than_one_round(G, types):
+    """Past 64 columns per compute unit, on both sides of the lines between the streaming rung and the MFMA rung's tiles."""
+    es = 1 if types in (O.S8S8S32, O.E4M3E4M3F16, O.E5M2E5M2F16) else 2
+    kind = O.FILL_INT8_UNIFORM if types == O.S8S8S32 else O.FILL_SMALL_INT
+    for i, (m, n, kb) in enumerate([(16, 16400, 512), (16, 16400, 656), (1, 65540, 144), (32, 16640, 1024), (32, 16640, 1056),
+                                    (48, 16644, 512), (64, 28676, 400), (65, 16640, 640), (128, 18440, 384), (128, 20484, 272),
+                                    (100, 28680, 256), (128, 16640, 3200)]):
+        k = kb // es
+        a, b, c = O.make_inputs(types, m, n, k, kind=kind, seed=m + n)
+        al, be = ((1, 0), (2, 3))[i % 2]
+        print("case", types, m, n, k, al, be, flush=True)
+        got = G.run_gemm(types, a, b, c, m, n, k, O.ROW, O.COL, al, be, -1)
+        assert np.array_equal(got, O.gemm(types, a, b, c, m, n, k, O.ROW, O.COL, al, be)), (types, m, n, k, al, be)
 
 
 def test_skinny_rung_refuses_what_it_cannot_do(G):
