@@ -132,6 +132,16 @@ __device__ __forceinline__ void store_accumulators(const GemmArgs<TYPES>& g, Acc
   });
 }
 
+// a loaded value is in its register from here on
+template <class T> __device__ __forceinline__ void arrived(T& v) {
+  uint32_t w;
+  if constexpr (sizeof(T) == 4) w = __builtin_bit_cast(uint32_t, v);
+  else w = (uint32_t)v;
+  asm volatile("" : "+v"(w));
+  if constexpr (sizeof(T) == 4) v = __builtin_bit_cast(T, w);
+  else v = (T)w;
+}
+
 // The same through LDS, so that a store instruction writes whole cache lines.  Straight from the
 // accumulators a wave's store covers 32 rows x 32 bytes, and the output - 64 MiB for fp32 4096^2, 256 MiB for int32
 // 8192^2, written by all compute units at the same moment - left the device at about 3 TB/s (a launch with K = 64:
@@ -153,15 +163,6 @@ __device__ __forceinline__ void store_accumulators(const GemmArgs<TYPES>& g, Acc
 // entered the compiler waits for ALL memory operations there (loads and stores return in no fixed order with respect to
 // each other), i.e. for the previous store, 64 times per wave on the four-wave 256 x 256 tile (7 us per launch).
 // Without loads of C nothing is waited for; with them, they are waited for once per block, before its first store.
-// a loaded value is in its register from here on
-template <class T> __device__ __forceinline__ void arrived(T& v) {
-  uint32_t w;
-  if constexpr (sizeof(T) == 4) w = __builtin_bit_cast(uint32_t, v);
-  else w = (uint32_t)v;
-  asm volatile("" : "+v"(w));
-  if constexpr (sizeof(T) == 4) v = __builtin_bit_cast(T, w);
-  else v = (T)w;
-}
 template <int UC, int TYPES, int FM, int FN, bool RAGGED, int BLK, bool TRANSPOSED, bool BY4, class Acc, int AM, int AN>
 __device__ __forceinline__ void store_accumulators_lds_impl(const GemmArgs<TYPES>& g, Acc (&acc)[AM][AN], int row0, int col0,
                                                             int lane, char* region) {

@@ -24,20 +24,20 @@
 // registers with the same depth.  A narrow share of columns moves little per stage, so it gets more waves and more
 // stages (skinny_dtl_shape): what a compute unit has in flight stays near 128 KiB.
 //
-// stream_wide_kernel + stream_wide_reduce_kernel (64 < M <= 128, K >= 8192): stream_tile_kernel with column blocks of
+// stream_wide_kernel + stream_wide_reduce_kernel (16-bit types, 64 < M <= 128, K >= 8192, K % 64 == 0): stream_tile_kernel with column blocks of
 // up to 256 columns and K split in two or four parts, so that a compute unit pulls a part of A instead of all of it;
 // the parts meet in a workspace and a second launch adds them in a fixed order (gz_skinny_cfg.hpp says when).
 //
-// stream_tile_kernel (16 < M <= 128, K % 64 == 0): here the activations no longer fit a wave's registers and every
+// stream_tile_kernel (16 < M <= 128): here the activations no longer fit a wave's registers and every
 // compute unit needs all of them, so they are shared through LDS.  One work-group per compute unit owns up to 64
-// columns.  Four producer waves move stage after stage (64 K elements: A rows and B rows, 128 bytes each, swizzled)
-// into a ring with direct-to-LDS copies; four consumer waves read the fragments and run v_mfma_f32_32x32x16.
+// columns.  Four producer waves move stage after stage (128 bytes of K: A rows and B rows, swizzled)
+// into a ring with direct-to-LDS copies; four consumer waves read the fragments and run the 32x32 instructions.
 // Splitting the roles matters: a copy instruction occupies its wave for about 55 cycles however many lanes it
 // moves, and with one wave per SIMD doing both jobs the copy issue, the LDS reads and the MFMAs of a stage ran
 // back to back.  One barrier per stage says both "stage i has landed" and "stage i - 1 may be overwritten".
 //
-// v_mfma_f32_16x16x32_{bf16,f16}: the weight fragment is the first operand, so a lane ends with 4 consecutive
-// columns of one output row (64-bit stores).
+// (both kernels: the weight fragment is the first operand, so a lane ends with 4 consecutive
+// columns of one output row.)
 #include "gz_common.hpp"
 #include <type_traits>
 #include <utility>

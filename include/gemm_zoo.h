@@ -94,7 +94,7 @@ typedef enum gz_types {
 
 /* The ladder.  GZ_RUNG_AUTO lets the launcher pick: MFMA, or for skinny M what the plan
  * reports as GZ_RUNG_SKINNY - the weight-streaming kernels, there for the 8-bit types as
- * well, or the MFMA rung's 64x64 tiles (then plan.variant is theirs) where those are faster. */
+ * well, or tiles of the MFMA rung (then plan.variant is theirs) where those are faster.       */
 typedef enum gz_rung {
   GZ_RUNG_AUTO = -1,
   GZ_RUNG_NAIVE = 0,           /* one thread per output, scalar loads              */
