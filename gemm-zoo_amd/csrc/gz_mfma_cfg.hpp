@@ -52,20 +52,22 @@ inline int mfma_lds_bytes(const MfmaCfg& c) {
 
 // How a problem sits on a tile configuration (16-byte alignment of the pointers is the caller's to check):
 //   WHOLE      whole tiles and whole K slabs
-//   RAGGED_MN  whole K slabs, row-major A, rows of A and B a whole number of 16-byte pieces, but M or N not a
-//              multiple of the tile: the 256x256 direct-to-LDS kernels handle it by clamping rows
+//   RAGGED     lines of A and B a whole number of 16-byte pieces and K at least one slab, but M or N not a multiple of the
+//              tile or K not whole slabs: the ring kernel clamps rows and lets the first two slabs overlap
 //   GENERAL    everything else: the predicated kernel
-enum { MFMA_SHAPE_WHOLE = 0, MFMA_SHAPE_RAGGED_MN = 1, MFMA_SHAPE_GENERAL = 2 };
+enum { MFMA_SHAPE_WHOLE = 0, MFMA_SHAPE_RAGGED = 1, MFMA_SHAPE_GENERAL = 2 };
 inline int mfma_shape_class(const MfmaCfg& c, int in_size, int M, int N, int K, int layoutA, int layoutB) {
   const int bk = MFMA_SLAB_BYTES / in_size, epv = 16 / in_size;
-  if (K <= 0 || K % bk) return MFMA_SHAPE_GENERAL;
+  if (K < bk) return MFMA_SHAPE_GENERAL;
+  // (a K-contiguous operand's slabs begin at whole pieces of its rows)
+  if ((layoutA == GZ_ROW_MAJOR || layoutB == GZ_COL_MAJOR) && K % epv) return MFMA_SHAPE_GENERAL;
   // the direct-to-LDS kernels address a tile's rows with 32-bit byte offsets from the tile's first row
   if ((long long)K * in_size * 256 >= (1LL << 32) || (long long)N * in_size * 256 >= (1LL << 32)) return MFMA_SHAPE_GENERAL;
-  if (M % c.bm == 0 && N % c.bn == 0) return MFMA_SHAPE_WHOLE;
+  if (M % c.bm == 0 && N % c.bn == 0 && K % bk == 0) return MFMA_SHAPE_WHOLE;
   // ragged M / N: lines that are not K-contiguous are clamped by whole 16-byte pieces
   if (layoutA != GZ_ROW_MAJOR && (layoutB != GZ_ROW_MAJOR || M % epv)) return MFMA_SHAPE_GENERAL;
   if (layoutB == GZ_ROW_MAJOR && N % epv) return MFMA_SHAPE_GENERAL;
-  return MFMA_SHAPE_RAGGED_MN;
+  return MFMA_SHAPE_RAGGED;
 }
 inline bool mfma_whole_tiles(const MfmaCfg& c, int in_size, int M, int N, int K) {
   return mfma_shape_class(c, in_size, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR) == MFMA_SHAPE_WHOLE;
@@ -159,10 +161,10 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       continue;
     }
     const long long rounds = (tiles + num_cus - 1) / num_cus;
-    // whole tiles: every candidate has a direct-to-LDS kernel; ragged M or N: the 256x256 ones only
+    // whole tiles: every candidate has a direct-to-LDS kernel; ragged M, N or K: the ring kernel
     const int cls = mfma_shape_class(c, in_size, M, N, K, layoutA, layoutB);
     const bool direct = (types == GZ_F32F32F32 ? a_rows && (i == 0 || i == 2) : a_direct) &&
-                        (cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED_MN && i == 0));
+                        (cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED && (i == 0 || (i == 2 && ring128_ok))));
     // (128 x 128 beyond four rounds: each further round costs a little more, 6144^2 x 6144 = 9 rounds measured
     // 478 us against 457 for three rounds of 256 x 256)
     // (256 x 128 up to one round where every tile has to run on the register-staged kernel - a ragged K, unaligned
@@ -202,6 +204,12 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
     if (i == 2 && direct && ring128_ok && types != GZ_F32F32F32) {
       const long long full2 = tiles / (2LL * num_cus), rem2 = tiles % (2LL * num_cus);
       shape_cost = 0.66 * full2 + (rem2 ? 0.36 + 0.15 * (double)rem2 / num_cus : 0.0);
+      // A short K past one round of 256 x 256 tiles: what a launch takes is the writing of D, which on these tiles goes
+      // on beside the other work-group's products (7040 x 2816, column-major A, us, 256 x 256 / 128 x 128: bf16 -> f32 K =
+      // 137 32.7 / 26.5, 300 36.9 / 34.2, 450 44.4 / 42.2; fp16 24.8 / 22.1, 30.4 / 26.9, 37.0 / 34.1; int8 30.7 / 24.7,
+      // 32.1 / 26.2, 34.4 / 30.2; 4096 x 4096, one whole round, level or worse).
+      const long long big = (long long)((M + 255) / 256) * ((N + 255) / 256), nslab = ((long long)K * in_size + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
+      if (big > num_cus && big % num_cus && nslab < 10) shape_cost *= 0.70 + 0.03 * (double)nslab;
     }
     // 128 x 128 tiles on the register-staged kernel (ragged M / N, K-contiguous B), up to three rounds: measured in
     // rounds of 256 x 256, bf16 K = 4096 - 324 tiles 0.70, 504 0.81, 512 0.80, 576 1.09, 640 1.11, 768 1.19 (the line
@@ -276,6 +284,7 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
     // Waves per 256 x 256 tile on the ring kernel.
     const long long tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
     const bool f8 = types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16;
+    const bool k_tail = K % (MFMA_SLAB_BYTES / in_size) != 0;
     bool eight = false;
     if (types == GZ_F32F32F32) {
       eight = false;   // one instance: four waves
@@ -284,7 +293,9 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // four beyond.  e4m3, us, four / eight waves, row/row: 4096^3 56.2 / 53.3, 5120^3 122.8 / 115.7, 6144^3
       // 221.5 / 213.0, 4096^2 x 8192 99.6 / 99.0, 8192^3 404.9 / 419.4; row/col 4096^3 53.8 / 50.9, 8192^3
       // 386.5 / 401.4.  (A row-major B: eight waves at every size, see below.)
-      eight = !(tiles >= 4LL * num_cus && b_cols);
+      // (K that is not whole slabs: four, whose instance has the registers for the clamped offsets - e4m3 4096 x 4096 x
+      // 4000 57.6 / 58.0, 2048 x 7824 x 1088 25.7 / 28.9, 5008^3 124 / 138, row/row 4096^2 x 1040 27.2 / 26.6)
+      eight = !(tiles >= 4LL * num_cus && b_cols) && !k_tail;
     } else {
       // int8 and the 16-bit types: an estimate of the launch on four and on eight waves, in us per round of tiles,
       // a fixed part (first copies, epilogue) and a part per K slab.  Eight waves (two per SIMD, 128 x 64 per wave)
@@ -323,8 +334,14 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // row-major B stays on eight: 2000 x 4000 x 4096 75.2 / 71.0): us, four / eight waves,
       // bf16 -> f32 row/col 3000^2 x 4096 70.8 / 76.4, 4000 x 3000 x 2048 48.1 / 53.9, 8000 x 1000 x 4096 76.3 / 79.3,
       // int8 3000 x 4096 x 2048 28.6 / 31.1; a 16-bit output stays on eight, bf16 -> bf16 3000 x 4096 x 2048 47.4 / 45.3.)
-      const bool ragged = M % 256 != 0 || N % 256 != 0;
-      eight = !a_rows || (under_a_round && (!ragged || out16 || !b_cols)) || fixed8 + slope8 * nslab < fixed4 + slope4 * nslab;
+      // (K that is not whole slabs follows the estimate as ragged shapes do: bf16 -> f32 four / eight waves, row/col
+      // 4096^2 x 4000 108.5 / 119.4, 4096^2 x 2000 56.3 / 59.9, row/row 4096^2 x 4000 101.4 / 111.0; bf16 -> bf16 4096^2 x
+      // 1000 36.6 / 34.9.  Where N and K are both ragged and a row is an odd number of 16-byte pieces the plan has been
+      // eight waves since these ran on the register-staged kernel, and stays so: 3000^2 x 1000 31.0 / 34.8, 6000^2 x 3000
+      // row/row 214.9 / 226.9, bf16 -> bf16 33.5 / 31.1 and 219.9 / 218.8; on the register-staged kernel 35.8 and 261.)
+      const bool ragged = M % 256 != 0 || N % 256 != 0 || k_tail;
+      const bool n_k_ragged = k_tail && N % 128 != 0 && (long long)K * in_size % 32 != 0;
+      eight = !a_rows || n_k_ragged || (under_a_round && (!ragged || out16 || !b_cols)) || fixed8 + slope8 * nslab < fixed4 + slope4 * nslab;
     }
     if (eight) *out = kMfmaCfgs[MFMA_CFG_RING_W8];
   }
@@ -396,6 +413,8 @@ inline bool mfma_resolve_split(int types, int M, int N, int K, int layoutA, int 
   if (main_cfg.bm != 256 || main_cfg.bn != 256) return false;
   // only where the first launch runs a direct-to-LDS kernel, whose speed the estimate knows well
   if (mfma_shape_class(main_cfg, mfma_in_size(types), rows_main, N, K, layoutA, layoutB) == MFMA_SHAPE_GENERAL) return false;
+  // (fp32 with a K that is not whole slabs: 128 x 128 tiles of the ring kernel spread it as evenly in one launch)
+  if (types == GZ_F32F32F32 && K % (MFMA_SLAB_BYTES / 4)) return false;
   const double cost_tail = mfma_choose(types, M - rows_main, N, K, layoutA, layoutB, num_cus, &tail_cfg);
   if (cost_main + cost_tail > 0.97 * cost_single) return false;
   if (estimate) *estimate = cost_main + cost_tail;
@@ -449,8 +468,8 @@ inline bool mfma_resolve_colsplit(int types, int M, int N, int K, int layoutA, i
   const bool f8_types = types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16;
   const bool layouts_ok = layoutA == GZ_ROW_MAJOR || (layoutB == GZ_ROW_MAJOR && !f8_types);
   const bool direct_before = layouts_ok && types != GZ_F32F32F32 &&
-                             (cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED_MN && main_cfg.bm == 256 && main_cfg.bn == 256));
-  const bool direct_after = direct_before && main_cfg.bm == 256 && main_cfg.bn == 256 &&
+                             (cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED && main_cfg.ring != 0));
+  const bool direct_after = direct_before && main_cfg.ring != 0 &&
                             (layoutB == GZ_COL_MAJOR || ((long long)N * mfma_in_size(types)) % 16 == 0);
   if (direct_before && !direct_after) cost_main *= types == GZ_F32F32F32 ? 2.2 : mfma_in_size(types) == 2 ? 1.2 : 1.5;
   // on the register-staged kernel eight waves carry a 256 x 256 tile of 16-bit elements better than four
@@ -523,6 +542,7 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   // 113.8 / 124.2).
   if (!forced && (long long)((M + 255) / 256) * ((N + 255) / 256) < num_cus) cfg = kMfmaCfgs[MFMA_CFG_RING_W4];
   if (mfma_shape_class(cfg, in_size, M, N, K, layoutA, layoutB) == MFMA_SHAPE_GENERAL) return false;
+  if (K % (MFMA_SLAB_BYTES / in_size)) return false;   // runs of whole slabs
   const int nslab = K / (MFMA_SLAB_BYTES / in_size);
   const long long tiles = (long long)((M + 255) / 256) * ((N + 255) / 256);
   const int R = (int)(tiles % num_cus);
@@ -620,7 +640,7 @@ inline long long mfma_persistent_grid(long long tiles, int num_cus) {
 // MFMA operands in the other order and writes the real, row-major D), and does so 10-15 % faster than the
 // register-staged kernel runs the problem as given.  Taken where ONE launch of the ring kernel covers the transposed
 // problem - the launcher's own choice for it is that kernel and neither a cut nor stream-K, or the caller names a
-// variant of the ring kernel - and its tiles are whole (or ragged in M / N on the 256 x 256 tile).  Fills `out` with
+// variant of the ring kernel - and its operands' lines are aligned.  Fills `out` with
 // the configuration in terms of the transposed problem (bm along N, bn along M).
 // `split`, if given: a row cut of the transposed problem (columns of the real one) where the launcher would make one and
 // both parts run the ring kernel; rows_main = 0 otherwise.
@@ -654,7 +674,7 @@ inline bool mfma_transposed_ring(int types, int M, int N, int K, int layoutA, in
   if ((f8 || types == GZ_F32F32F32) && out->waves_m * out->waves_n == 8) *out = kMfmaCfgs[out->id - 2];
   if (types == GZ_F32F32F32 && out->bm != 256 && out->id != kMfmaCfgs[MFMA_CFG_RING_128].id) return false;
   const int cls = mfma_shape_class(*out, mfma_in_size(types), N, M, K, GZ_ROW_MAJOR, GZ_ROW_MAJOR);
-  return cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED_MN && out->bm == 256);
+  return cls != MFMA_SHAPE_GENERAL;
 }
 
 inline int mfma_launch_class(const MfmaCfg& c, int in_size, int out_size, int M, int N, int K, int layoutA, int layoutB,
@@ -668,7 +688,7 @@ inline int mfma_launch_class(const MfmaCfg& c, int in_size, int out_size, int M,
   if (cls == MFMA_SHAPE_WHOLE && ((ldd * out_size) % 16 || (C && (ldc * out_size) % 16))) {
     const int epv = 16 / in_size;
     const bool a_ok = layoutA == GZ_ROW_MAJOR || (layoutB == GZ_ROW_MAJOR && M % epv == 0);
-    cls = (a_ok && (layoutB == GZ_COL_MAJOR || N % epv == 0)) ? MFMA_SHAPE_RAGGED_MN : MFMA_SHAPE_GENERAL;
+    cls = (a_ok && (layoutB == GZ_COL_MAJOR || N % epv == 0)) ? MFMA_SHAPE_RAGGED : MFMA_SHAPE_GENERAL;
   }
   return cls;
 }

@@ -1300,8 +1300,8 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
 #define GZ_LAUNCH_DIRECT(KERN, LDS_BYTES, ...) GZ_LAUNCH_DIRECT_ON(grid, GZ_KERN(KERN), LDS_BYTES, ##__VA_ARGS__)
 #define GZ_KERN(...) __VA_ARGS__   // a template-id with commas as one macro argument
 
-  // The direct-to-LDS kernels: row-major A, whole K slabs, 16-byte aligned rows (the shape class says so), whole
-  // tiles or, on the hand-scheduled 256 x 256 kernel, any M and N (rows clamped).  ring: 0 the compiler-scheduled
+  // The direct-to-LDS kernels: 16-byte aligned lines (the shape class says so), whole tiles and K slabs or, on the
+  // hand-scheduled ring kernel, any M and N and any K of at least a slab.  ring: 0 the compiler-scheduled
   // kernels, 1 the hand-scheduled ring kernel with one work-group per compute unit walking the tiles of a grid of
   // more than one round (ragged M and N included), 2 the same kernel with one work-group per tile.
   constexpr bool TILE_256 = BM == 256 && BN == 256 && WAVES_M == 2 && (WAVES_N == 2 || WAVES_N == 4);
@@ -1313,14 +1313,14 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   // two column-major operands as the transposed problem (v_mfma_f32_16x16x4_f32, four per block and K step)
   if constexpr (TYPES == GZ_F32F32F32 && TILE_256 && WAVES_N == 2) {
     if (transposed) {
-      if (ring && shape_class == MFMA_SHAPE_RAGGED_MN)
+      if (ring && shape_class == MFMA_SHAPE_RAGGED)
         GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, true, false, false, true>), ring_lds, StreamK{});
       if (ring && !edge)
         GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, false, false, false, true>), ring_lds, StreamK{});
       set_error("mfma rung: no kernel for the transposed problem on this tile");
       return GZ_ERR_UNSUPPORTED;
     }
-    if (ring && akc && shape_class == MFMA_SHAPE_RAGGED_MN) {
+    if (ring && akc && shape_class == MFMA_SHAPE_RAGGED) {
       if (bkc) GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true>), ring_lds, StreamK{});
       else GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false>), ring_lds, StreamK{});
     }
@@ -1329,13 +1329,19 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
       else GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false>), ring_lds, StreamK{});
     }
   }
-  // (and the 128 x 128 tile of the same kernel on whole tiles, two work-groups per compute unit)
+  // (and the 128 x 128 tile of the same kernel, two work-groups per compute unit)
   if constexpr (TYPES == GZ_F32F32F32 && BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2) {
     if (transposed) {
+      if (ring && shape_class == MFMA_SHAPE_RAGGED)
+        GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, true, false, false, true>), ring_lds, StreamK{});
       if (ring && !edge)
         GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, false, false, false, true>), ring_lds, StreamK{});
       set_error("mfma rung: no kernel for the transposed problem on this tile");
       return GZ_ERR_UNSUPPORTED;
+    }
+    if (ring && akc && shape_class == MFMA_SHAPE_RAGGED) {
+      if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true>), ring_lds, StreamK{});
+      else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false>), ring_lds, StreamK{});
     }
     if (ring && akc && !edge) {
       if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N>), ring_lds, StreamK{});
@@ -1348,12 +1354,14 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
     // (the waves of a tile laid out the other way round as well: the wave count along the real M stays what it is)
     if (transposed) {
       if constexpr (TILE_256 && !(is_fp8(TYPES) && WAVES_M * WAVES_N == 8)) {
-        if (ring && shape_class == MFMA_SHAPE_RAGGED_MN)
+        if (ring && shape_class == MFMA_SHAPE_RAGGED)
           GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, true, false, false, true>), ring_lds, StreamK{});
         if (ring && !edge)
           GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, false, false, false, true>), ring_lds, StreamK{});
       }
       if constexpr (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2 && !is_fp8(TYPES)) {
+        if (ring && shape_class == MFMA_SHAPE_RAGGED)
+          GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, true, false, false, true>), ring_lds, StreamK{});
         if (ring && !edge)
           GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, false, false, false, true>), ring_lds, StreamK{});
       }
@@ -1363,18 +1371,20 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
     // a column-major A with a row-major B (int8 and the 16-bit types): both operands through the transposing reads
     if constexpr (!is_fp8(TYPES)) {
       if constexpr (TILE_256) {
-        if (ring && !akc && !bkc && shape_class == MFMA_SHAPE_RAGGED_MN)
+        if (ring && !akc && !bkc && shape_class == MFMA_SHAPE_RAGGED)
           GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false, false, false>), ring_lds, StreamK{});
         if (ring && !akc && !bkc && !edge)
           GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false, false, false>), ring_lds, StreamK{});
       }
       if constexpr (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2) {
+        if (ring && !akc && !bkc && shape_class == MFMA_SHAPE_RAGGED)
+          GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false, false, false>), ring_lds, StreamK{});
         if (ring && !akc && !bkc && !edge)
           GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false, false, false>), ring_lds, StreamK{});
       }
     }
     if constexpr (TILE_256) {
-      if (ring && akc && shape_class == MFMA_SHAPE_RAGGED_MN) {
+      if (ring && akc && shape_class == MFMA_SHAPE_RAGGED) {
         if (bkc) GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true>), ring_lds, StreamK{});
         else GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false>), ring_lds, StreamK{});
       }
@@ -1383,8 +1393,12 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
         else GZ_LAUNCH_DIRECT_ON(pgrid, GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false>), ring_lds, StreamK{});
       }
     }
-    // the same kernel on whole 128 x 128 tiles (int8 and the 16-bit types), one work-group per tile, two per compute unit
+    // the same kernel on 128 x 128 tiles (int8 and the 16-bit types), one work-group per tile, two per compute unit
     if constexpr (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2 && !is_fp8(TYPES)) {
+      if (ring && akc && shape_class == MFMA_SHAPE_RAGGED) {
+        if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true>), ring_lds, StreamK{});
+        else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false>), ring_lds, StreamK{});
+      }
       if (ring && akc && !edge) {
         if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N>), ring_lds, StreamK{});
         else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false>), ring_lds, StreamK{});
@@ -1756,7 +1770,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     }
     const int cls = cls_of(t, ct);
     // (unaligned operands, or rows of D that are not: the kernels of the problem as given, below)
-    if (cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED_MN && ct.bm == 256)) return launch_one<TYPES>(t, ct, s, false, true);
+    if (cls != MFMA_SHAPE_GENERAL) return launch_one<TYPES>(t, ct, s, false, true);
     return -1;
   };
   // (a few columns past a multiple of 256 are cut off first, as for the other layouts: the transposed problem would
@@ -1789,8 +1803,8 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
                                         g.A, g.B, g.C, g.D, g.lda, g.ldb, g.ldc, g.ldd);
       if (cls != MFMA_SHAPE_GENERAL) {   // (unaligned operands: the plain launch below, on the register-staged kernel)
         g.store_hint = 0;   // one round at most ends in each launch: plain stores
-        return skp.cfg.waves_n == 4 ? launch_streamk<TYPES, 4>(g, skp, cls == MFMA_SHAPE_RAGGED_MN, s)
-                                    : launch_streamk<TYPES, 2>(g, skp, cls == MFMA_SHAPE_RAGGED_MN, s);
+        return skp.cfg.waves_n == 4 ? launch_streamk<TYPES, 4>(g, skp, cls == MFMA_SHAPE_RAGGED, s)
+                                    : launch_streamk<TYPES, 2>(g, skp, cls == MFMA_SHAPE_RAGGED, s);
       }
     }
   }

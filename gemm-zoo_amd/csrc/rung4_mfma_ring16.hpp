@@ -37,8 +37,8 @@
 // instruction's first operand: a lane ends up with four consecutive columns of one row of D,
 //     acc[i][j][e] = D(row0 + 16 i + l % 16, col0 + 16 j + 4 (l / 16) + e).
 //
-// K a multiple of the slab (128 bytes); either layout of A and of B (template parameters below); whole tiles, or
-// (RAGGED) any M and N with 16-byte aligned lines.
+// Either layout of A and of B (template parameters below); whole tiles and whole slabs of K (128 bytes), or (RAGGED) any M,
+// N and K of at least one slab with 16-byte aligned lines (stream-K: whole slabs).
 #pragma once
 
 namespace gz {
@@ -198,7 +198,12 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WAVES_M, wn = wave / WAVES_M;
   const int K = g.K;
-  const int nslab_all = K / SK;
+  // K tail (RAGGED): where K is not whole slabs, slab 1 begins inside slab 0, so that every copy stays inside the operands
+  // and the last slab ends with K; what the two share is set to zero in slab 0 when it has landed (keep_head below).  The
+  // main loop knows nothing of it: the same cut at the last slab put a branch into it, across which the register
+  // allocator moved accumulators that matrix instructions still had to write.  K is at least one slab.
+  const int nslab_all = RAGGED && !STREAMK ? (K + SK - 1) / SK : K / SK;
+  const int tail_back = RAGGED && !STREAMK ? nslab_all * SK - K : 0;   // elements of K that slabs 0 and 1 share
   // the run of slabs of this work-group: [it, it_end) of the stream-K sequence (STREAMK, past the whole tiles)
   int it = 0, it_end = 0, sk_block = 0;
   if constexpr (STREAMK) {
@@ -328,6 +333,9 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     if constexpr (B_KC) return b_tile + (size_t)(c >> 1) * LINE;
     else return b_tile + (size_t)c * b_group_step;
   };
+  // the same in bytes: how far the bases of slabs 1, 2, ... lie back
+  const size_t a_back = A_KC ? (size_t)tail_back * ES : (size_t)tail_back * LDA;
+  const size_t b_back = B_KC ? (size_t)tail_back * ES : (size_t)tail_back * LDB;
   const uint32_t m0_a = lds_base + (wave * A_PW) * 1024 + (A_PW / 2) * 1024;
   const uint32_t m0_b = lds_base + A_BYTES + (wave * B_PW) * 1024 + (B_PW / 2) * 1024;
   auto copy_a_begin = [&](int st) { asm_set_m0(m0_a + st * STAGE_BYTES); };
@@ -621,6 +629,29 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     });
   };
 
+  // K tail: the pieces of slab 0 that slab 1 holds as well become zeros - each wave those of its own copies, which it has
+  // waited for.  On both operands: an infinity of the one times a zero of the other would be no zero.
+  auto keep_head = [&]() __attribute__((always_inline)) {
+    const u32x4_t z = {0, 0, 0, 0};
+    const int head = SK - tail_back;
+#pragma unroll
+    for (int par = 0; par < 2; par++) {
+      char* const st = lds + par * STAGE_BYTES;
+#pragma unroll
+      for (int t = 0; t < A_PW; t++) {
+        const bool twice = A_KC ? ((cs ^ ci ^ par) * 16) >= head * ES
+                                : par * HK + (wave * A_PW + t) * KRC_A + lane / LPR_A >= head;
+        if (twice) *reinterpret_cast<u32x4_t*>(st + (wave * A_PW + t) * 1024 + lane * 16) = z;
+      }
+#pragma unroll
+      for (int t = 0; t < B_PW; t++) {
+        const bool twice = B_KC ? ((cs ^ ci ^ par) * 16) >= head * ES
+                                : par * HK + (wave * B_PW + t) * KRC + lane / LPR >= head;
+        if (twice) *reinterpret_cast<u32x4_t*>(st + A_BYTES + (wave * B_PW + t) * 1024 + lane * 16) = z;
+      }
+    }
+  };
+
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
   // ---- prologue: groups 0 .. 3 (slabs 0 and 1; a run of one slab has groups 0 and 1 only) ----
@@ -643,12 +674,19 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
   // epilogue's stores are counted between the two pairs of groups.  Loads return in order, so with no more than two
   // groups' worth of operations outstanding none of them can be a load of groups 0 and 1.)
   if (nc > 2) {
-    issue_group(std::integral_constant<int, 2>{}, a_tile, b_tile);
-    issue_group(std::integral_constant<int, 3>{}, a_tile, b_tile);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "i"(2 * NCP) : "memory");
+    issue_group(std::integral_constant<int, 2>{}, a_tile - a_back, b_tile - b_back);
+    issue_group(std::integral_constant<int, 3>{}, a_tile - a_back, b_tile - b_back);
+    asm volatile("s_waitcnt vmcnt(%0)" : : "i"(2 * NCP) : "memory");
   } else {
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
+  if constexpr (RAGGED && !STREAMK) {
+    if (tail_back != 0) {
+      keep_head();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  }
+  asm volatile("s_barrier" ::: "memory");
   if constexpr (F8) {   // lower rows of A and all but the last column of B of slab 0
     static_for<FM>([&](auto r_c) {
       constexpr int R = decltype(r_c)::value;
@@ -663,8 +701,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
   // or, where the run has no such slab, its last slab again ----
   const int nslab = nc / 2;
   const int first_fetch = min(2, nslab - 1);
-  const char* a_cp = a_group(a_tile, 2 * first_fetch);
-  const char* b_cp = b_group(b_tile, 2 * first_fetch);
+  const char* a_cp = a_group(a_tile, 2 * first_fetch) - a_back;
+  const char* b_cp = b_group(b_tile, 2 * first_fetch) - b_back;
   auto slab = [&](auto jr_c, int j) {
     constexpr int JR = decltype(jr_c)::value;
     using NEXT = std::integral_constant<int, (JR + 1) % NST>;

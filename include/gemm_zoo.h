@@ -146,7 +146,7 @@ typedef struct gz_plan_t {
 /* variant: 0 = launcher's choice; other values select a tile configuration of the rung (1 .. gz_variant_count).
  * MFMA rung: 1 256x256 on four waves, 2 on eight, 3 128x128, 4 256x128 (register-staged or compiler-scheduled
  * direct-to-LDS kernels, any shape and layout); 5 / 6 the hand-scheduled 256x256 ring kernel on four / eight waves
- * wherever the problem allows it (row-major A, whole K slabs, 16-byte aligned rows; otherwise the kernel of 1 / 2);
+ * wherever the problem allows it (row-major A, K of at least one slab, 16-byte aligned rows; otherwise the kernel of 1 / 2);
  * 7 / 8 the same with the stream-K decomposition; 9 / 10 as 5 / 6 with one work-group per tile instead of one per
  * compute unit; 11 the ring kernel on 128x128 tiles, two work-groups per compute unit (int8, the 16-bit types and
  * fp32; otherwise the kernel of 3); 12 the register-staged kernel on 64x64 tiles (four waves; two for 8-bit
