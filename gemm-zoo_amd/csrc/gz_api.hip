@@ -233,39 +233,14 @@ int device_compute_units() {
 // ---------------------------------------------------------------------------
 // When K is split on 64 x 64 tiles
 // ---------------------------------------------------------------------------
-// us per 128-byte slab of a 64 x 64 tile whose work-group has a compute unit to itself, measured over 20 ... 880 tiles
-// and 7 ... 194 slabs: what a layout costs is its transposing stores (row-major B, column-major A), and 8-bit rows that
-// are not whole 16-byte pieces are loaded from unaligned addresses.
-static double splitk_slab_us(int types, int M, int N, int K, int layoutA, int layoutB) {
-  if (types == GZ_F32F32F32) return 0.56;
-  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR;
-  if (mfma_in_size(types) == 1) {
-    const bool aligned = (a_kc ? K : M) % 16 == 0 && (b_kc ? K : N) % 16 == 0;
-    if (a_kc && b_kc) return aligned ? 0.40 : 0.50;
-    if (a_kc != b_kc) return aligned ? 0.56 : 0.70;
-    return 0.74;
-  }
-  return a_kc && b_kc ? 0.42 : a_kc ? 0.48 : b_kc ? 0.40 : 0.60;
-}
-// How much longer a slab takes with w work-groups per compute unit.  fp32 is bound by its matrix rate: the compute unit
-// with the most work-groups decides.  The other types wait for memory, so a second work-group is nearly free (bf16,
-// 80 tiles x 194 slabs in 4, 6, 8, 12 parts, w = 1.25, 1.9, 2.5, 3.75: 1.2, 1.35, 1.9, 2.8).
-static double splitk_share(int types, double w) {
-  if (w <= 1.0) return 1.0;
-  if (types == GZ_F32F32F32) return std::ceil(w);
-  auto line = [](double x) { return 1.0 + 0.4 * (x - 1.0) > 0.77 * x ? 1.0 + 0.4 * (x - 1.0) : 0.77 * x; };
-  // (half of the weight on the compute units with the most work-groups: 280 tiles x 128 slabs, w = 1.09, cost 0.6 us a
-  // slab and not 0.5)
-  return 0.5 * (line(w) + line(std::ceil(w)));
-}
-
 bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, SplitKPlan* out) {
   if (is_acc16(types) || M <= 0 || N <= 0 || K <= 0) return false;
   if (num_cus <= 0) num_cus = 256;
   const long long slabs = ((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
   const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
   if (slabs < 4 || tiles > 4LL * num_cus) return false;
-  const double slab_us = splitk_slab_us(types, M, N, K, layoutA, layoutB);
+  const double slab_us = mfma_64_slab_us(types, M, N, K, layoutA, layoutB);
+  const bool own_slabs = mfma_64_own_slabs(types, M, N, K, layoutA, layoutB);
   // (a large operand that is read once: bf16 50 x 9600 x 8192 in 3 parts 39 us, of which 8 are the two launches)
   const double stream_us = ((double)M + (double)N) * (double)K * mfma_in_size(types) / 5.5e6;
   double best = 0;
@@ -275,7 +250,7 @@ bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
     if (bytes > MFMA_SPLITK_MAX_BYTES || tiles * p > 8LL * num_cus) break;
     // two launches, the sums written and read back, the slabs of the longest part (us, measured / this line: bf16
     // 24 x 1280 x 11001 in 12 parts 14.4 / 13.7, 100 x 2560 x 12416 in 6 27.6 / 26.7, fp32 512^3 in 4 10.1 / 9.6)
-    const double walk = (double)((slabs + p - 1) / p) * slab_us * splitk_share(types, (double)(tiles * p) / num_cus);
+    const double walk = (double)((slabs + p - 1) / p) * slab_us * mfma_64_share(types, own_slabs, (double)(tiles * p) / num_cus);
     const double t = 6.5 + 0.22 * (double)bytes / (1 << 20) + (walk > stream_us ? walk : stream_us);
     if (parts == 0 || t < best) {
       best = t;
@@ -306,9 +281,13 @@ bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
   MfmaSplit rows;
   MfmaColSplit cols;
   double est = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &c) * round_us;
-  if (c.bm == 64) {   // the same tile unsplit, by the same measure
-    const double w = (double)((M + 63) / 64) * ((N + 63) / 64) / num_cus;
-    est = 2.6 + slabs * splitk_slab_us(types, M, N, K, layoutA, layoutB) * splitk_share(types, w);
+  if (c.bm <= 64) {   // the same tile unsplit, or the smaller one, by the same measure
+    // (32 x 32 tiles on less than a sixth of the compute units and forty slabs or more: either may win by a quarter, and the
+    // parts are kept up to that - int8 192 x 128 x 5120 row/col parts / 32 x 32 8.8 / 6.5, row/row 8.8 / 10.0, 64 x 128 x
+    // 16384 9.9 / 11.7, bf16 192 x 128 x 2560 row/row 8.7 / 7.8)
+    if (c.bm == 32 && (long long)((M + 31) / 32) * ((N + 31) / 32) * 6 <= num_cus && slabs >= 40)
+      return out->estimate_us < 1.3 * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
+    est = c.bm == 64 ? mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) : mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
     return out->estimate_us < 0.90 * est;
   }
   double cut = 0;
@@ -438,6 +417,7 @@ static int run(const void* A, const void* B, const void* C, void* D, int64_t M, 
       if ((st = launch_splitk<TYPES>(g, kp, s)) >= 0) return st;
     }
     if (how == SKINNY_TILES_64) return launch_mfma<TYPES>(g, kMfmaCfgs[MFMA_CFG_64].id, s);
+    if (how == SKINNY_TILES_32) return launch_mfma<TYPES>(g, kMfmaCfgs[MFMA_CFG_32].id, s);
     if (how == SKINNY_TILES) return launch_mfma<TYPES>(g, 0, s);
   }
   switch (resolved) {
@@ -597,13 +577,13 @@ int gz_variant_count(int types, int rung) {
   }
 }
 
-static void plan_splitk(const SplitKPlan& kp, int types, int m, int n, gz_plan_t* plan) {
+static void plan_splitk(const SplitKPlan& kp, int types, int m, int n, int k, int layoutA, int layoutB, gz_plan_t* plan) {
   const int es = in_size(types);
-  const MfmaCfg& c = es == 1 ? kMfmaCfg64Int8 : kMfmaCfgs[MFMA_CFG_64];
+  const MfmaCfg c = mfma_64_cfg(types, m, n, k, layoutA, layoutB);
   plan->variant = c.id;
   plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
   plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
-  plan->threads = c.waves_m * c.waves_n * 64;
+  plan->threads = mfma_threads(c);
   plan->lds_bytes = mfma_lds_bytes(c);
   plan->split_k = kp.parts;
   plan->grid = (int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * kp.parts;
@@ -667,7 +647,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
       }
       if (SplitKPlan kp; variant == 0 && mfma_plan_splitk(types, m, n, k, layoutA, layoutB, num_cus, &kp) &&
                          (unsigned long long)kp.workspace_bytes <= (unsigned long long)ws_limit) {
-        plan_splitk(kp, types, m, n, plan);
+        plan_splitk(kp, types, m, n, k, layoutA, layoutB, plan);
         if (plan->lds_bytes > lds_per_cu) {
           set_error("mfma variant %d needs %d bytes of LDS, device has %d", plan->variant, plan->lds_bytes, lds_per_cu);
           return GZ_ERR_UNSUPPORTED;
@@ -687,7 +667,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
         plan->variant = ct.id;
         plan->tile_m = ct.bn; plan->tile_n = ct.bm; plan->tile_k = MFMA_SLAB_BYTES / es;
         plan->wave_m = ct.bn / ct.waves_m; plan->wave_n = ct.bm / ct.waves_n;
-        plan->threads = ct.waves_m * ct.waves_n * 64;
+        plan->threads = mfma_threads(ct);
         plan->lds_bytes = mfma_lds_bytes(ct);
         const int n_first = tsp.rows_main > 0 ? tsp.rows_main : n_ring;   // columns of the first launch
         plan->grid = (int64_t)ceil_div(n_first, ct.bm) * ceil_div(m, ct.bn);
@@ -721,7 +701,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
           plan->variant = c.waves_n == 4 ? MFMA_VARIANT_STREAMK_W8 : MFMA_VARIANT_STREAMK_W4;
           plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
           plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
-          plan->threads = c.waves_m * c.waves_n * 64;
+          plan->threads = mfma_threads(c);
           plan->lds_bytes = mfma_lds_bytes(c);
           plan->grid = (int64_t)skp.dp_tiles + skp.blocks;
           plan->streamk_tiles = skp.sk_tiles;
@@ -772,7 +752,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
       plan->variant = c.id;
       plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
       plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
-      plan->threads = c.waves_m * c.waves_n * 64;
+      plan->threads = mfma_threads(c);
       plan->lds_bytes = mfma_lds_bytes(c);
       plan->grid = (int64_t)ceil_div(m_first, c.bm) * ceil_div(n_first, c.bn);
       // the ring kernel with the 16x16 instructions (whole tiles, or ragged M and N on its 256 x 256 tile): one
@@ -796,9 +776,9 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
       const int how = rung == GZ_RUNG_AUTO && variant == 0 ? skinny_choose(types, m, n, k, num_cus, ws_limit, &kp) : SKINNY_STREAM;
       if (how != SKINNY_STREAM) {   // the MFMA rung's 64 x 64 tiles, split along K or not
         if (how == SKINNY_TILES_SPLITK) {
-          plan_splitk(kp, types, m, n, plan);
+          plan_splitk(kp, types, m, n, k, layoutA, layoutB, plan);
         } else {
-          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, how == SKINNY_TILES_64 ? kMfmaCfgs[MFMA_CFG_64].id : 0, num_cus, lds_per_cu, ws_limit, plan);
+          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, how == SKINNY_TILES_64 ? kMfmaCfgs[MFMA_CFG_64].id : how == SKINNY_TILES_32 ? kMfmaCfgs[MFMA_CFG_32].id : 0, num_cus, lds_per_cu, ws_limit, plan);
           if (st != GZ_OK) return st;
         }
         plan->rung = GZ_RUNG_SKINNY;

@@ -338,6 +338,8 @@ template <int TYPES> int launch_double_buffered(const GemmArgs<TYPES>& g, int va
 template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& g, int variant, hipStream_t s);
 template <int TYPES> int launch_skinny(const GemmArgs<TYPES>& g, int variant, hipStream_t s);
 struct SplitKPlan;
+struct SplitK;
+template <int TYPES> int launch_wavek(const GemmArgs<TYPES>& g, int tile, const SplitK& sk, hipStream_t s);   // tile: 64 (where wavek_64 says so) or 32
 template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPlan& p, hipStream_t s);   // in the MFMA rung's units
 
 }  // namespace gz

@@ -16,7 +16,9 @@ struct MfmaCfg {
                 // 1: the hand-scheduled ring kernel wherever the problem allows it, persistent past one round of
                 //    the compute units; 2: the same kernel with one work-group per tile
   bool stream_k;  // the tiles past the last whole round of the compute units are cut along K (see mfma_plan_streamk)
+  int k_waves = 1;  // waves that multiply the same sub-tile, each over slabs of its own (rung4_mfma_wavek.hpp)
 };
+inline int mfma_threads(const MfmaCfg& c) { return c.waves_m * c.waves_n * c.k_waves * 64; }
 
 // K slab per tile row is 128 bytes whatever the element type.
 constexpr int MFMA_SLAB_BYTES = 128;
@@ -34,19 +36,23 @@ static const MfmaCfg kMfmaCfgs[] = {
     {9, 256, 256, 2, 2, 2, false},   // variant 5 with one work-group per tile (for comparisons with the persistent launch)
     {10, 256, 256, 2, 4, 2, false},  // variant 6, the same
     {11, 128, 128, 2, 2, 2, false},  // tile of variant 3 on the ring kernel, two work-groups per compute unit
-    {12, 64, 64, 2, 2, 0, false},    // four waves of 32x32: grids that 128x128 tiles leave mostly empty
+    {12, 64, 64, 1, 1, 0, false, 4},   // grids that 128x128 tiles leave mostly empty: four waves, each the whole tile over its own slabs
+                                       // (unaligned lines and fp32: kMfmaCfg64Staged)
+    {13, 32, 32, 1, 1, 0, false, 8},   // grids that 64x64 tiles leave mostly empty: eight waves, the same
 };
 constexpr int kNumMfmaCfgs = (int)(sizeof(kMfmaCfgs) / sizeof(kMfmaCfgs[0]));
-// variant 12 for 8-bit elements: the same tile on two waves of 64x32 (the transposing stores of 8-bit elements need four 16-byte
-// pieces per lane and operand, which 128 lanes have on this tile and 256 do not)
-static const MfmaCfg kMfmaCfg64Int8 = {12, 64, 64, 1, 2, 0, false};
+// variant 12 on the register-staged kernel: four waves of 32x32, 8-bit elements two of 64x32 (their transposing stores need
+// four 16-byte pieces per lane and operand, which 128 lanes have on this tile and 256 do not)
+static const MfmaCfg kMfmaCfg64Staged = {12, 64, 64, 2, 2, 0, false}, kMfmaCfg64StagedInt8 = {12, 64, 64, 1, 2, 0, false};
 // positions in the table
 enum { MFMA_CFG_256_W4 = 0, MFMA_CFG_256_W8 = 1, MFMA_CFG_128 = 2, MFMA_CFG_256x128 = 3, MFMA_CFG_RING_W4 = 4,
-       MFMA_CFG_RING_W8 = 5, MFMA_CFG_RING_128 = 10, MFMA_CFG_64 = 11 };
+       MFMA_CFG_RING_W8 = 5, MFMA_CFG_RING_128 = 10, MFMA_CFG_64 = 11, MFMA_CFG_32 = 12 };
 enum { MFMA_VARIANT_RING_W4 = 5, MFMA_VARIANT_RING_W8 = 6, MFMA_VARIANT_STREAMK_W4 = 7, MFMA_VARIANT_STREAMK_W8 = 8 };
 
-// the most any kernel of the configuration asks for: the ring kernel keeps five buffers of half a slab each
+// the most any kernel of the configuration asks for: the ring kernel keeps five buffers of half a slab each, a wave that has
+// K slabs to itself two slabs of a 64 x 64 tile or one (padded) of a 32 x 32 tile
 inline int mfma_lds_bytes(const MfmaCfg& c) {
+  if (c.k_waves > 1) return c.k_waves * (c.bm == 64 ? 2 * (c.bm + c.bn) * MFMA_SLAB_BYTES : (c.bm + c.bn) * 160);
   return c.ring ? 5 * (c.bm + c.bn) * 64 : 2 * (c.bm + c.bn) * MFMA_LDS_PITCH;
 }
 
@@ -68,6 +74,11 @@ inline int mfma_shape_class(const MfmaCfg& c, int in_size, int M, int N, int K, 
   if (layoutA != GZ_ROW_MAJOR && (layoutB != GZ_ROW_MAJOR || M % epv)) return MFMA_SHAPE_GENERAL;
   if (layoutB == GZ_ROW_MAJOR && N % epv) return MFMA_SHAPE_GENERAL;
   return MFMA_SHAPE_RAGGED;
+}
+// lines that are whole 16-byte pieces of either operand (packed: their leading dimensions as well)
+inline bool mfma_whole_pieces(int in_size, int M, int N, int K, int layoutA, int layoutB) {
+  const int epv = 16 / in_size;
+  return (layoutA == GZ_ROW_MAJOR ? K : M) % epv == 0 && (layoutB == GZ_COL_MAJOR ? K : N) % epv == 0;
 }
 inline bool mfma_whole_tiles(const MfmaCfg& c, int in_size, int M, int N, int K) {
   return mfma_shape_class(c, in_size, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR) == MFMA_SHAPE_WHOLE;
@@ -114,8 +125,72 @@ inline int mfma_store_hint(int types, long long M, long long N, long long K, int
   return out_bytes <= (64ll << 20) ? 1 : 0;
 }
 
+// ---- the small tiles ----
+// whether a 64 x 64 tile runs on the kernel whose waves have slabs of their own (mfma_wavek_kernel) or on the register-staged one
+inline bool mfma_64_own_slabs(int types, int M, int N, int K, int layoutA, int layoutB) {
+  return types != GZ_F32F32F32 && mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
+}
+inline MfmaCfg mfma_64_cfg(int types, int M, int N, int K, int layoutA, int layoutB) {
+  if (mfma_64_own_slabs(types, M, N, K, layoutA, layoutB)) return kMfmaCfgs[MFMA_CFG_64];
+  return mfma_in_size(types) == 1 ? kMfmaCfg64StagedInt8 : kMfmaCfg64Staged;
+}
+// us per 128-byte slab of a 64 x 64 tile whose work-group has a compute unit to itself.  Register-staged (measured over
+// 20 ... 880 tiles and 7 ... 194 slabs): what a layout costs is its transposing stores (row-major B, column-major A), and
+// 8-bit rows that are not whole 16-byte pieces are loaded from unaligned addresses.  Slabs of the waves' own (64 ... 256
+// tiles, 16 ... 64 slabs): what comes in through the L2, lines of 64 bytes where 8-bit elements lie along M or N.
+inline double mfma_64_slab_us(int types, int M, int N, int K, int layoutA, int layoutB) {
+  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR;
+  if (types == GZ_F32F32F32) return 0.54;
+  const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
+  if (pieces) return mfma_in_size(types) == 2 ? 0.235 : a_kc && b_kc ? 0.22 : a_kc != b_kc ? 0.27 : 0.31;
+  if (mfma_in_size(types) == 1) return a_kc && b_kc ? 0.50 : a_kc != b_kc ? 0.70 : 0.74;
+  return a_kc && b_kc ? 0.42 : a_kc ? 0.48 : b_kc ? 0.40 : 0.60;
+}
+// How much longer a slab takes with w work-groups per compute unit.  fp32 is bound by its matrix rate: the compute unit
+// with the most work-groups decides.  Slabs of the waves' own keep the L2's path to a compute unit busy: in between
+// w and the next whole number (bf16 row/row, 289, 400, 576 tiles: 1.13, 1.7, 2.6).  The register-staged kernel waits for
+// memory, so a second work-group is nearly free (bf16, 80 tiles x 194 slabs in 4, 6, 8, 12 parts, w = 1.25, 1.9, 2.5, 3.75:
+// 1.2, 1.35, 1.9, 2.8).
+inline double mfma_64_share(int types, bool own_slabs, double w) {
+  if (w <= 1.0) return 1.0;
+  const double whole = (double)(long long)w < w ? (double)(long long)w + 1.0 : w;
+  if (types == GZ_F32F32F32) return whole;
+  if (own_slabs) return 0.5 * (w + whole);
+  auto line = [](double x) { return 1.0 + 0.4 * (x - 1.0) > 0.77 * x ? 1.0 + 0.4 * (x - 1.0) : 0.77 * x; };
+  // (half of the weight on the compute units with the most work-groups: 280 tiles x 128 slabs, w = 1.09, cost 0.6 us a
+  // slab and not 0.5)
+  return 0.5 * (line(w) + line(whole));
+}
+// us of an unsplit launch of 64 x 64 tiles (bf16 row/row cubes 256, 512, 1024, 1280: 4.6, 5.9, 8.7, 12.9)
+inline double mfma_64_us(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
+  const double slabs = (double)(((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES);
+  const bool own_slabs = mfma_64_own_slabs(types, M, N, K, layoutA, layoutB);
+  const double w = (double)((M + 63) / 64) * (double)((N + 63) / 64) / num_cus;
+  const double fixed = own_slabs ? (slabs < 8 ? 3.3 + 0.2 * slabs : 4.9) : types == GZ_F32F32F32 ? 3.0 : 2.6;
+  return fixed + slabs * mfma_64_slab_us(types, M, N, K, layoutA, layoutB) * mfma_64_share(types, own_slabs, w);
+}
+// ... and of 32 x 32 tiles.  8- and 16-bit types: a slab of every tile of a compute unit in turn, 0.095 us through copies
+// (lines of 64 and of 32 bytes, elements along M or N: more), 0.28 (0.36 for 8 bits) through registers, and the operands
+// from memory once (us, this line / measured: bf16 row/row 512^3 3.6 / 3.7, 512^2 x 8192 19.2 / 19.3, row/col 512^2 x 2048
+// 5.6 / 5.9, 256 x 1024 x 4096 8.7 / 8.6, 300 x 1408^2 6.8 / 7.3, column-major A 640 x 1024 x 4096 27.6 / 27.8; int8 145 x
+// 1664 x 8192 row/row 25.0 / 25.6; unaligned 291^3 4.0 / 4.0, 330 x 1047 x 833 9.9 / 7.6).  fp32: by products, 0.145 us a slab and tile (0.20 through registers), the compute unit
+// with the most tiles decides (256^3 4.1 / 3.9, 512^3 5.2 / 5.6, 1024^3 21.5 / 22.3, 1536^3 65.5 / 66.6).
+inline double mfma_32_us(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
+  const double slabs = (double)(((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES);
+  const long long tiles = (long long)((M + 31) / 32) * ((N + 31) / 32);
+  const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
+  if (types == GZ_F32F32F32) return 2.9 + slabs * (pieces ? 0.145 : 0.20) * (double)((tiles + num_cus - 1) / num_cus);
+  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR, wide = mfma_in_size(types) == 2;
+  const double slab_us = !pieces ? (wide ? 0.28 : 0.36) : a_kc && b_kc ? 0.095 : a_kc != b_kc ? (wide ? 0.125 : 0.175) : (wide ? 0.13 : 0.235);
+  const double walk = slabs * slab_us * (double)((tiles + num_cus - 1) / num_cus);
+  const double stream = ((double)M + (double)N) * (double)K * mfma_in_size(types) / 5.0e6;
+  return 2.6 + (walk > stream ? walk : stream);
+}
+
 // The launcher's own choice for one launch over the whole problem; returns the estimate it was chosen by.
-inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, MfmaCfg* out) {
+// (staged_64: every 64 x 64 tile on the register-staged kernel, no smaller one - what the lines of stream-K were drawn
+// against, see mfma_plan_streamk)
+inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, MfmaCfg* out, bool staged_64 = false) {
   if (num_cus <= 0) num_cus = 256;
   const int in_size = mfma_in_size(types);
   const bool a_rows = layoutA == GZ_ROW_MAJOR, b_cols = layoutB == GZ_COL_MAJOR;
@@ -139,11 +214,24 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // tiles leave mostly empty.  8-bit elements on two waves.
       double cost64 = -1.0;
       if (types == GZ_F32F32F32) {
-        // A 128 x 128 tile is 55 us of fp32 products per 1024 of K on one compute unit, whatever the grid.  A
-        // sixteenth of a round of 256 x 256 per tile at 0.75 of the larger tiles' rate (us, 64 x 64 / 128 x 128 tiles,
-        // cubes, row/row: 256 8.1 / 21.0, 512 13.7 / 37.3, 1024 25.4 / 70.2, 1536 86.0 / 103.4, 2048 149.5 / 136.7).
-        const double share = (double)tiles / (16.0 * num_cus);
-        cost64 = (0.05 + 1.35 * (share > 1.0 / 16 ? share : 1.0 / 16)) * 2.2;
+        // A 128 x 128 tile is 55 us of fp32 products per 1024 of K on one compute unit, whatever the grid (us, 32 x 32 /
+        // 64 x 64 / 128 x 128 tiles, cubes, row/row: 256 3.9 / 7.5 / 19, 512 5.6 / 12.4 / 33, 1024 22.3 / 22.7 / 62, 1088
+        // 27.5 / 39.7 / 64, 1280 42.7 / 45.4 / 75, 1536 66.6 / 79.5 / 89, 2048 - / 141 / 119).
+        // (0.77: what the estimate of the larger tiles is short of their times up to 2048^3)
+        // Past four tiles per compute unit a sixteenth of a round of 256 x 256 per tile at 0.75 of the larger tiles' rate.
+        const double round_us = 16.0 + 1.45 * ((double)K * in_size / MFMA_SLAB_BYTES);
+        if (tiles > 4LL * num_cus) cost64 = (0.05 + 1.35 * (double)tiles / (16.0 * num_cus)) * 2.2;
+        else cost64 = 0.77 * mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) / round_us;
+        const double cost32 = 0.77 * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus) / round_us;
+        if (tiles <= 4LL * num_cus && cost32 < cost64 && cost32 < best) {
+          best = cost32;
+          pick = MFMA_CFG_32;
+        }
+      } else if (!staged_64 && mfma_64_own_slabs(types, M, N, K, layoutA, layoutB)) {
+        // slabs of the waves' own: up to two tiles per compute unit (bf16 row/row 1280^3, 1.56, 12.9 against 14.8 on 128 x
+        // 128, 1536^3, 2.25, 19.5 / 16.8; int8 9.8 / 10.1, 15.1 / 11.1; column-major A, 736 x 1792 x 2227 18.9 / 22.3)
+        if (tiles <= 2LL * num_cus)
+          cost64 = mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) / (16.0 + 1.45 * ((double)K * in_size / MFMA_SLAB_BYTES));
       } else if (tiles * 5 <= (b_cols || f8_types ? 10LL : 6LL) * num_cus) {
         // 8- and 16-bit types, up to two tiles per compute unit (int8 and 16-bit, 1.2 with a row-major B: 1280^2 x 2048 22.1 / 20.5, with a
         // K-contiguous B 18.5 / 20.0; 1024 x 2048 x 4096, two per compute unit, 30.1 / 33.5; 1536^2 x 2048, 2.25,
@@ -157,6 +245,19 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       if (cost64 >= 0 && cost64 < best) {
         best = cost64;
         pick = cand[i];
+      }
+      // 32 x 32 tiles of the 8- and 16-bit types, up to two per compute unit: there a 64 x 64 tile's compute unit has one
+      // to itself or none (us, 32 x 32 / 64 x 64: bf16 row/row 256^3 3.0 / 4.6, 512^3 3.7 / 5.9, 768^3, 2.25 per compute
+      // unit, 8.0 / 7.4; 512^2 x 2048 5.9 / 10.3, 256 x 1024 x 4096 8.6 / 15.8; int8 512^3 3.5 / 4.6, 768^3 7.0 / 6.2)
+      const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
+      // (whole 64 x 64 tiles of row-major operands with a K of four slabs at most and half the rows keep that tile)
+      const bool flat = a_rows && !b_cols && M % 64 == 0 && N % 64 == 0 && 2LL * K <= M && (long long)K * in_size <= 4 * MFMA_SLAB_BYTES;
+      if (!staged_64 && !flat && types != GZ_F32F32F32 && pick == MFMA_CFG_64 && tiles32 <= 2LL * num_cus) {
+        const double by = mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus) / mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus);
+        if (by < 1.0) {
+          best *= by;
+          pick = MFMA_CFG_32;
+        }
       }
       continue;
     }
@@ -209,7 +310,9 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // 137 32.7 / 26.5, 300 36.9 / 34.2, 450 44.4 / 42.2; fp16 24.8 / 22.1, 30.4 / 26.9, 37.0 / 34.1; int8 30.7 / 24.7,
       // 32.1 / 26.2, 34.4 / 30.2; 4096 x 4096, one whole round, level or worse).
       const long long big = (long long)((M + 255) / 256) * ((N + 255) / 256), nslab = ((long long)K * in_size + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
-      if (big > num_cus && big % num_cus && nslab < 10) shape_cost *= 0.70 + 0.03 * (double)nslab;
+      // (not a few rows or columns past a multiple of 256: those are cut off)
+      const bool few_past = (M % 256 >= 1 && M % 256 <= 64) || (N % 256 >= 1 && N % 256 <= 64);
+      if (big > num_cus && big % num_cus && nslab < 10 && !few_past) shape_cost *= 0.70 + 0.03 * (double)nslab;
     }
     // 128 x 128 tiles on the register-staged kernel (ragged M / N, K-contiguous B), up to three rounds: measured in
     // rounds of 256 x 256, bf16 K = 4096 - 324 tiles 0.70, 504 0.81, 512 0.80, 576 1.09, 640 1.11, 768 1.19 (the line
@@ -275,8 +378,7 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       pick = cand[i];
     }
   }
-  *out = kMfmaCfgs[pick];
-  if (pick == MFMA_CFG_64 && in_size == 1) *out = kMfmaCfg64Int8;
+  *out = pick == MFMA_CFG_64 ? mfma_64_cfg(types, M, N, K, layoutA, layoutB) : kMfmaCfgs[pick];
   // (The register-staged kernel of the 128 x 128 tile was kept for a K-contiguous B on grids of up to 5/8 of the compute
   // units.  Interleaved runs of the two, int8 / fp16 / bf16 -> bf16 squares 512 ... 1536 at K = 1024 ... 8192: the ring
   // kernel level or 1 - 4 % ahead on all of them but 1536^2 x 8192, 16-bit, 81 against 74 us; the rule is gone.)
@@ -352,9 +454,7 @@ inline bool mfma_resolve(int types, int M, int N, int K, int layoutA, int layout
                          MfmaCfg* out) {
   if (variant < 0 || variant > kNumMfmaCfgs) return false;
   if (variant > 0) {
-    *out = kMfmaCfgs[variant - 1];
-    // (8-bit elements: on two waves)
-    if (out->bm == 64 && mfma_in_size(types) == 1) *out = kMfmaCfg64Int8;
+    *out = variant - 1 == MFMA_CFG_64 ? mfma_64_cfg(types, M, N, K, layoutA, layoutB) : kMfmaCfgs[variant - 1];
     return true;
   }
   (void)mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, out);
@@ -388,7 +488,7 @@ struct MfmaSplit {
   MfmaCfg main, tail;
 };
 inline bool mfma_resolve_split(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, MfmaSplit* out,
-                               double* estimate = nullptr) {
+                               double* estimate = nullptr, bool staged_64 = false) {
   out->rows_main = 0;
   if (num_cus <= 0) num_cus = 256;
   if (layoutA != GZ_ROW_MAJOR || M < 512 || N <= 0 || K <= 0) return false;
@@ -397,7 +497,7 @@ inline bool mfma_resolve_split(int types, int M, int N, int K, int layoutA, int 
   // bf16 4608^2 40.8 / 38.3, 57.2 / 56.9, 159.1 / 170.3; int8 40.3 / 38.2 at K = 1024, 92.6 / 94.1 at 4096)
   if ((long long)K * mfma_in_size(types) < 24 * MFMA_SLAB_BYTES) return false;
   MfmaCfg single;
-  const double cost_single = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &single);
+  const double cost_single = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &single, staged_64);
   const long long tiles_n = (N + 255) / 256, tiles_m = (M + 255) / 256;
   const long long full = tiles_m * tiles_n / num_cus * num_cus;   // tiles in whole rounds
   if (full == 0 || full == tiles_m * tiles_n) return false;
@@ -409,13 +509,13 @@ inline bool mfma_resolve_split(int types, int M, int N, int K, int layoutA, int 
   if (tile_rows <= 0 || tile_rows * 256 >= M) return false;
   const int rows_main = (int)(tile_rows * 256);
   MfmaCfg main_cfg, tail_cfg;
-  double cost_main = mfma_choose(types, rows_main, N, K, layoutA, layoutB, num_cus, &main_cfg);
+  double cost_main = mfma_choose(types, rows_main, N, K, layoutA, layoutB, num_cus, &main_cfg, staged_64);
   if (main_cfg.bm != 256 || main_cfg.bn != 256) return false;
   // only where the first launch runs a direct-to-LDS kernel, whose speed the estimate knows well
   if (mfma_shape_class(main_cfg, mfma_in_size(types), rows_main, N, K, layoutA, layoutB) == MFMA_SHAPE_GENERAL) return false;
   // (fp32 with a K that is not whole slabs: 128 x 128 tiles of the ring kernel spread it as evenly in one launch)
   if (types == GZ_F32F32F32 && K % (MFMA_SLAB_BYTES / 4)) return false;
-  const double cost_tail = mfma_choose(types, M - rows_main, N, K, layoutA, layoutB, num_cus, &tail_cfg);
+  const double cost_tail = mfma_choose(types, M - rows_main, N, K, layoutA, layoutB, num_cus, &tail_cfg, staged_64);
   if (cost_main + cost_tail > 0.97 * cost_single) return false;
   if (estimate) *estimate = cost_main + cost_tail;
   out->rows_main = rows_main;
@@ -442,20 +542,20 @@ struct MfmaColSplit {
 inline bool mfma_transposed_ring(int types, int M, int N, int K, int layoutA, int layoutB, int variant, int num_cus,
                                  MfmaCfg* out, MfmaSplit* split);
 inline bool mfma_resolve_colsplit(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, MfmaColSplit* out,
-                                  double* estimate = nullptr) {
+                                  double* estimate = nullptr, bool staged_64 = false) {
   out->cols_main = 0;
   if (num_cus <= 0) num_cus = 256;
   const int r = N % 256;
   if (N < 512 || r == 0 || r > 64 || M <= 0 || K <= 0) return false;
   MfmaCfg single;
-  double cost_single = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &single);
+  double cost_single = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &single, staged_64);
   const int cols_main = N - r;
   MfmaCfg main_cfg, tail_cfg;
-  double cost_main = mfma_choose(types, M, cols_main, K, layoutA, layoutB, num_cus, &main_cfg);
+  double cost_main = mfma_choose(types, M, cols_main, K, layoutA, layoutB, num_cus, &main_cfg, staged_64);
   // (64 x 64 tiles for the first launch: the columns past a multiple of 256 are half a tile there, not a column of large
   // ones, and a second launch of a few tiles through all of K takes as long as the first: e4m3 562 x 3616 x 2509 row/row
   // 42.4 us in two launches, 23.1 in one; int8 500 x 3090 x 3000 row/col 25.1 / 18.9)
-  if (main_cfg.bm == 64) return false;
+  if (main_cfg.bm <= 64) return false;
   // (column-major A and B: what the ring kernel on the transposed problem costs, where it takes the whole problem
   // and where it takes the first launch)
   if (MfmaCfg t; mfma_transposed_ring(types, M, N, K, layoutA, layoutB, 0, num_cus, &t, nullptr))
@@ -530,7 +630,9 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   const int in_size = mfma_in_size(types);
   if (!(types == GZ_S8S8S32 || in_size == 2) || layoutA != GZ_ROW_MAJOR) return false;
   MfmaCfg cfg;
-  double single_rounds = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &cfg);
+  // (The alternatives below are estimated as they were when these lines were drawn, 64 x 64 tiles on the register-staged
+  // kernel; those of the waves' own slabs have come nearer since: bf16 1024^2 x 8192 stream-K 41 - 44 us.)
+  double single_rounds = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &cfg, true);
   if (forced) cfg = kMfmaCfgs[forced_cfg->waves_n == 4 ? MFMA_CFG_RING_W8 : MFMA_CFG_RING_W4];
   else if (cfg.id != MFMA_VARIANT_RING_W4 && cfg.id != MFMA_VARIANT_RING_W8) {
     // a smaller tile was preferred for the whole problem (few tiles): stream-K still competes, on the 256 x 256 tile
@@ -580,6 +682,10 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   const double overhead_us = 14.0 + 0.058 * out->slots + 0.25 * R;
   out->estimate_us = (double)(full / num_cus) * round_us + (out->q + 1) * slab_us + overhead_us;
   if (forced) return true;
+  // (a grid of no more 32 x 32 tiles than two to a compute unit: those, cut along K or not, us, stream-K / 32 x 32: bf16
+  // 512^2 x 8192 23.8 / 13.9, row/row 24.7 / 19.3, 256^2 x 8192 22.3 / 12.6, int8 300 x 1024 x 12288 24.5 / 19.3)
+  if (full == 0 && (long long)((M + 31) / 32) * ((N + 31) / 32) <= 2LL * num_cus &&
+      mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus) < out->estimate_us) return false;
   // No whole round (a grid smaller than the device): every work-group streams its own K range of its own tile, so
   // nothing is shared through the L2s and the operands come from memory once per tile; against 128 x 128 tiles,
   // one or two per compute unit, that pays only for a long K and few tiles.  Measured, us, stream-K / 128 x 128
@@ -603,8 +709,8 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   MfmaSplit sp;
   MfmaColSplit cs;
   double est_rows = 0, est_cols = 0, best = single_rounds;
-  if (mfma_resolve_split(types, M, N, K, layoutA, layoutB, num_cus, &sp, &est_rows) && est_rows < best) best = est_rows;
-  if (mfma_resolve_colsplit(types, M, N, K, layoutA, layoutB, num_cus, &cs, &est_cols) && est_cols < best) best = est_cols;
+  if (mfma_resolve_split(types, M, N, K, layoutA, layoutB, num_cus, &sp, &est_rows, true) && est_rows < best) best = est_rows;
+  if (mfma_resolve_colsplit(types, M, N, K, layoutA, layoutB, num_cus, &cs, &est_cols, true) && est_cols < best) best = est_cols;
   return out->estimate_us < 0.99 * best * round_us;
 }
 

@@ -227,7 +227,7 @@ inline int skinny_tiles_max_stages(int cols, bool one_round) {
   if (!one_round) return 16 + cols / 4;
   return cols <= 32 ? 8 : 4;
 }
-enum { SKINNY_STREAM = 0, SKINNY_TILES_SPLITK = 1, SKINNY_TILES_64 = 2, SKINNY_TILES = 3 };   // (TILES: the MFMA rung's own choice)
+enum { SKINNY_STREAM = 0, SKINNY_TILES_SPLITK = 1, SKINNY_TILES_64 = 2, SKINNY_TILES = 3, SKINNY_TILES_32 = 4 };   // (TILES: the MFMA rung's own choice)
 inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned long long ws_limit, SplitKPlan* split) {
   if (M <= SKINNY_REG_MAX_M) return SKINNY_STREAM;
   const SkinnyCfg c = skinny_resolve(types, M, N, K, num_cus, ws_limit);
@@ -237,10 +237,22 @@ inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned l
   if (num_cus <= 0) num_cus = 256;
   if (M > 64 && stages <= skinny_tiles_max_stages(c.cols_per_wg, c.grid_n <= num_cus))
     return 2LL * ((N + 63) / 64) <= 3LL * num_cus ? SKINNY_TILES_64 : SKINNY_TILES;
-  if (mfma_best_splitk(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus, split) &&
-      (unsigned long long)split->workspace_bytes <= ws_limit &&
-      split->estimate_us < 0.9 * skinny_tile_estimate_us(stages, c.mb, c.cols_per_wg))
-    return SKINNY_TILES_SPLITK;
+  const double stream_us = skinny_tile_estimate_us(stages, c.mb, c.cols_per_wg);
+  const bool split_ok = mfma_best_splitk(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus, split) &&
+                        (unsigned long long)split->workspace_bytes <= ws_limit;
+  // Few columns: 32 x 32 tiles whose waves share out K, one launch (us, 32 x 32 / tile kernel or split K, whichever was
+  // taken: int8 75 x 1536 x 5376 6.5 / 10.8, 53 x 1408 x 5632 6.6 / 9.7, 106 x 1280 x 5376 6.5 / 9.9, 26 x 2560 x 7200 9.6 / 10.0,
+  // 46 x 1952 x 11648 10.6 / 12.3; bf16 the same)
+  // (Up to 32 rows and a long K the tile kernel spreads the weights over all compute units, which from memory outweighs its
+  // share of A: 32 x 4096 x 11648 14.2 / 17.2.  65 rows and more whose last stage the end of K cuts stay with the tile
+  // kernel, which zeroes it beside its copies.)
+  const bool cut_stage = M > 64 && (long long)K * es % STREAM_TILE_ROW_BYTES != 0;
+  if (cut_stage && stages < 24) return SKINNY_STREAM;
+  if ((long long)((M + 31) / 32) * ((N + 31) / 32) <= num_cus && !cut_stage && (M > 32 || stages <= 48)) {
+    const double small_us = mfma_32_us(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus);
+    if (small_us < 0.9 * stream_us && (!split_ok || small_us < split->estimate_us)) return SKINNY_TILES_32;
+  }
+  if (split_ok && split->estimate_us < 0.9 * stream_us) return SKINNY_TILES_SPLITK;
   return SKINNY_STREAM;
 }
 

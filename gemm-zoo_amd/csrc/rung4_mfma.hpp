@@ -16,7 +16,8 @@
 //                      makes the fragment reads of 16 consecutive rows hit 16 distinct 4-bank groups);
 //                      operands whose contiguous dimension is not K (row-major B, column-major A) are
 //                      transposed in registers on the way in.  Tiles 256x256, 256x128, 128x128 and, for
-//                      grids that those leave mostly empty, 64x64 (16- and 32-bit elements).
+//                      grids that those leave mostly empty, 64x64 (unaligned lines, and fp32).
+//   mfma_wavek_kernel  (rung4_mfma_wavek.hpp) 64x64 tiles of aligned lines and 32x32 tiles, K dealt to the waves.
 //   mfma_dtl_kernel    compiler-scheduled fast path for whole tiles with 16-byte aligned rows: slabs go
 //                      global -> LDS directly (global_load_lds_dwordx4), unpadded swizzled rows.
 //   mfma_ring16_kernel (rung4_mfma_ring16.hpp) the hand-scheduled kernel with the 16x16 matrix instructions
@@ -470,7 +471,7 @@ template <typename in_t, int ROWS, int NT, bool KC, bool EDGE> struct Stager {
   // bytes apart per column step, spread over the LDS banks through their k offset instead of piling onto a few.
   // 32-bit elements are not transposed at all: a k line of the tile goes to LDS as it lies in memory (NAT_PITCH
   // bytes per k line, lanes along the line), and the fragment reads gather one dword per k value instead.
-  static constexpr int MC_LO = 4;
+  static constexpr int MC_LO = ROWS / EPV < 4 ? ROWS / EPV : 4;
   static constexpr int NAT_PITCH = ROWS * 4 + 32;
   __device__ static inline void unit_of(int id, int& mc, int& ku) {
     constexpr int MC = ROWS / EPV;
@@ -1419,12 +1420,14 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
 #undef GZ_LAUNCH_DIRECT
 #undef GZ_LAUNCH_DIRECT_ON
 #undef GZ_KERN
-  if (edge) {
+  // (64 x 64 tiles of 8 and 16 bits come here with unaligned lines only: mfma_wavek_kernel has the others)
+  constexpr bool EDGE_ONLY = BM == 64 && TYPES != GZ_F32F32F32;
+  if (edge || EDGE_ONLY) {
     if (akc && bkc) GZ_LAUNCH(true, true, true);
     else if (akc && !bkc) GZ_LAUNCH(true, false, true);
     else if (!akc && bkc) GZ_LAUNCH(false, true, true);
     else GZ_LAUNCH(false, false, true);
-  } else {
+  } else if constexpr (!EDGE_ONLY) {
     if (akc && bkc) GZ_LAUNCH(true, true, false);
     else if (akc && !bkc) GZ_LAUNCH(true, false, false);
     else if (!akc && bkc) GZ_LAUNCH(false, true, false);
@@ -1631,6 +1634,15 @@ template <int TYPES> static int launch_strip(const GemmArgs<TYPES>& g, hipStream
   return GZ_OK;
 }
 
+// whether both operands' lines can be copied in whole 16-byte pieces, from offsets of 32 bits
+template <int TYPES> static bool wavek_dma_ok(const GemmArgs<TYPES>& g) {
+  constexpr int ES = (int)sizeof(typename Traits<TYPES>::in_t), EPV = 16 / ES;
+  return ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B)) & 15u) == 0 && g.lda % EPV == 0 && g.ldb % EPV == 0 &&
+         mfma_whole_pieces(ES, g.M, g.N, g.K, g.layoutA, g.layoutB) && g.lda * ES * 256 < (1LL << 32) && g.ldb * ES * 256 < (1LL << 32);
+}
+// ... and a 64 x 64 tile of them runs on mfma_wavek_kernel
+template <int TYPES> static bool wavek_64(const GemmArgs<TYPES>& g) { return TYPES != GZ_F32F32F32 && wavek_dma_ok<TYPES>(g); }
+
 template <int TYPES> static int launch_one(const GemmArgs<TYPES>& g, const MfmaCfg& chosen, hipStream_t s, bool adjust = false,
                                            bool transposed = false) {
   using in_t = typename Traits<TYPES>::in_t;
@@ -1648,7 +1660,9 @@ template <int TYPES> static int launch_one(const GemmArgs<TYPES>& g, const MfmaC
     case 9: return launch_cfg<TYPES, 256, 256, 2, 2>(g, edge, 2, s, transposed);
     case 10: return launch_cfg<TYPES, 256, 256, 2, 4>(g, edge, 2, s, transposed);
     case 11: return launch_cfg<TYPES, 128, 128, 2, 2>(g, edge, 2, s, transposed);
-    case 12:   // (8-bit elements on two waves)
+    case 13: return launch_wavek<TYPES>(g, 32, SplitK{}, s);
+    case 12:   // (on the register-staged kernel: 8-bit elements on two waves)
+      if (wavek_64<TYPES>(g)) return launch_wavek<TYPES>(g, 64, SplitK{}, s);
       if constexpr (sizeof(in_t) >= 2) return launch_cfg<TYPES, 64, 64, 2, 2>(g, edge, 0, s);
       else return launch_cfg<TYPES, 64, 64, 1, 2>(g, edge, 0, s);
     default: break;
@@ -1678,7 +1692,9 @@ template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPla
     hipLaunchKernelGGL(kern, grid, block, lds, s, g, tiles_m, tiles_n, sk);                      \
   } while (0)
     const bool akc = g.layoutA == GZ_ROW_MAJOR, bkc = g.layoutB == GZ_COL_MAJOR;
-    if (akc && bkc) GZ_LAUNCH_SPLIT(true, true);
+    if (wavek_64<TYPES>(g)) {
+      if (const int st = launch_wavek<TYPES>(g, 64, sk, s); st != GZ_OK) return st;
+    } else if (akc && bkc) GZ_LAUNCH_SPLIT(true, true);
     else if (akc) GZ_LAUNCH_SPLIT(true, false);
     else if (bkc) GZ_LAUNCH_SPLIT(false, true);
     else GZ_LAUNCH_SPLIT(false, false);
