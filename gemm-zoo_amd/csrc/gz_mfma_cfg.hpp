@@ -49,11 +49,12 @@ enum { MFMA_CFG_256_W4 = 0, MFMA_CFG_256_W8 = 1, MFMA_CFG_128 = 2, MFMA_CFG_256x
        MFMA_CFG_RING_W8 = 5, MFMA_CFG_RING_128 = 10, MFMA_CFG_64 = 11, MFMA_CFG_32 = 12 };
 enum { MFMA_VARIANT_RING_W4 = 5, MFMA_VARIANT_RING_W8 = 6, MFMA_VARIANT_STREAMK_W4 = 7, MFMA_VARIANT_STREAMK_W8 = 8 };
 
-// the most any kernel of the configuration asks for: the ring kernel keeps five buffers of half a slab each, a wave that has
+// the most any kernel of the configuration asks for: the ring kernel keeps five buffers of half a slab each (nine of
+// 128 x 128 tiles where a work-group has a compute unit to itself), a wave that has
 // K slabs to itself two slabs of a 64 x 64 tile or one (padded) of a 32 x 32 tile
 inline int mfma_lds_bytes(const MfmaCfg& c) {
   if (c.k_waves > 1) return c.k_waves * (c.bm == 64 ? 2 * (c.bm + c.bn) * MFMA_SLAB_BYTES : (c.bm + c.bn) * 160);
-  return c.ring ? 5 * (c.bm + c.bn) * 64 : 2 * (c.bm + c.bn) * MFMA_LDS_PITCH;
+  return c.ring ? (c.bm == 128 ? 9 : 5) * (c.bm + c.bn) * 64 : 2 * (c.bm + c.bn) * MFMA_LDS_PITCH;
 }
 
 // How a problem sits on a tile configuration (16-byte alignment of the pointers is the caller's to check):
@@ -397,7 +398,10 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // 386.5 / 401.4.  (A row-major B: eight waves at every size, see below.)
       // (K that is not whole slabs: four, whose instance has the registers for the clamped offsets - e4m3 4096 x 4096 x
       // 4000 57.6 / 58.0, 2048 x 7824 x 1088 25.7 / 28.9, 5008^3 124 / 138, row/row 4096^2 x 1040 27.2 / 26.6)
-      eight = !(tiles >= 4LL * num_cus && b_cols) && !k_tail;
+      // (A K-contiguous B and operands of 40 MB and more, which come from memory more than from the caches: four - us, four / eight: 1000 x 14336 x 4096 51.2 / 57.4, 2000 x 8192 x 4096 51.9 / 57.4, 2048 x 4096 x 8192 80.9 /
+      // 88.6, 4800 x 4864^2 105 / 109; 33 MB and less 4096^3 52.9 / 50.4, 3840^3 47.3 / 44.7, 1500 x 8192 x 2048 29.7 / 27.4)
+      const bool from_memory = b_cols && ((long long)M + N) * K >= 40000000LL;
+      eight = !(tiles >= 4LL * num_cus && b_cols) && !k_tail && !from_memory;
     } else {
       // int8 and the 16-bit types: an estimate of the launch on four and on eight waves, in us per round of tiles,
       // a fixed part (first copies, epilogue) and a part per K slab.  Eight waves (two per SIMD, 128 x 64 per wave)

@@ -1300,6 +1300,15 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   } while (0)
 #define GZ_LAUNCH_DIRECT(KERN, LDS_BYTES, ...) GZ_LAUNCH_DIRECT_ON(grid, GZ_KERN(KERN), LDS_BYTES, ##__VA_ARGS__)
 #define GZ_KERN(...) __VA_ARGS__   // a template-id with commas as one macro argument
+  // The ring kernel's 128 x 128 tile.  A work-group that has a compute unit to itself takes nine buffers, all of its LDS, and
+  // asks for slabs twice as far ahead.
+#define GZ_LAUNCH_128(WM_, WN_, ...)                                                                        \
+  do {                                                                                                      \
+    if constexpr (TYPES != GZ_F32F32F32) {                                                                  \
+      if (deep_ring) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WM_, WN_, __VA_ARGS__, 9>), deep_lds, StreamK{}); \
+    }                                                                                                       \
+    GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WM_, WN_, __VA_ARGS__>), ring_lds, StreamK{}); \
+  } while (0)
 
   // The direct-to-LDS kernels: 16-byte aligned lines (the shape class says so), whole tiles and K slabs or, on the
   // hand-scheduled ring kernel, any M and N and any K of at least a slab.  ring: 0 the compiler-scheduled
@@ -1308,6 +1317,13 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   constexpr bool TILE_256 = BM == 256 && BN == 256 && WAVES_M == 2 && (WAVES_N == 2 || WAVES_N == 4);
   const size_t ring_lds = 5u * (size_t)(BM + BN) * 64;
   const size_t dtl_lds = 2u * (size_t)(BM + BN) * SLAB_BYTES;
+  // From eight slabs on, and where the grid fills most of the device, which the L2s then hold up as much, from 24.  (us, five /
+  // nine buffers: bf16 1024^3 row/row 12.8 / 11.7, 1408^3 15.7 / 13.6, 1792^3 row/col 18.8 / 16.8, 2048^3 row/row 22.6 / 20.7;
+  // int8 1024^3 9.0 / 8.7, 1792^3 12.1 / 11.3; 256 tiles of 8 and 16 slabs fp16 10.0 / 10.2, 13.8 / 13.9, int8 row/col
+  // 13.5 / 13.8.  Not fp32, which its products bind: 2048^3 121 / 124.)
+  const long long grid_tiles = (long long)tiles_m * tiles_n, cus = device_compute_units();
+  const bool deep_ring = grid_tiles <= cus && (long long)g.K * (int)sizeof(typename Traits<TYPES>::in_t) >= (4 * grid_tiles > 3 * cus ? 24 : 8) * SLAB_BYTES;
+  const size_t deep_lds = 9u * (size_t)(BM + BN) * 64;
   const dim3 pgrid((unsigned)(ring == 1 ? mfma_persistent_grid((long long)tiles_m * tiles_n, device_compute_units())
                                         : (long long)tiles_m * tiles_n));
   // fp32 on the hand-scheduled kernel: the 256 x 256 tile on four waves, a row-major A with either layout of B, and
@@ -1334,19 +1350,19 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   if constexpr (TYPES == GZ_F32F32F32 && BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2) {
     if (transposed) {
       if (ring && shape_class == MFMA_SHAPE_RAGGED)
-        GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, true, false, false, true>), ring_lds, StreamK{});
+        GZ_LAUNCH_128(WAVES_N, WAVES_M, true, false, false, true, true);
       if (ring && !edge)
-        GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, false, false, false, true>), ring_lds, StreamK{});
+        GZ_LAUNCH_128(WAVES_N, WAVES_M, false, false, false, true, true);
       set_error("mfma rung: no kernel for the transposed problem on this tile");
       return GZ_ERR_UNSUPPORTED;
     }
     if (ring && akc && shape_class == MFMA_SHAPE_RAGGED) {
-      if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true>), ring_lds, StreamK{});
-      else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false>), ring_lds, StreamK{});
+      if (bkc) GZ_LAUNCH_128(WAVES_M, WAVES_N, true, false, true, false, true);
+      else GZ_LAUNCH_128(WAVES_M, WAVES_N, true, false, false, false, true);
     }
     if (ring && akc && !edge) {
-      if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N>), ring_lds, StreamK{});
-      else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false>), ring_lds, StreamK{});
+      if (bkc) GZ_LAUNCH_128(WAVES_M, WAVES_N, false, false, true, false, true);
+      else GZ_LAUNCH_128(WAVES_M, WAVES_N, false, false, false, false, true);
     }
   }
   if constexpr (TYPES != GZ_F32F32F32) {
@@ -1362,9 +1378,9 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
       }
       if constexpr (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2 && !is_fp8(TYPES)) {
         if (ring && shape_class == MFMA_SHAPE_RAGGED)
-          GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, true, false, false, true>), ring_lds, StreamK{});
+          GZ_LAUNCH_128(WAVES_N, WAVES_M, true, false, false, true, true);
         if (ring && !edge)
-          GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_N, WAVES_M, false, false, false, true>), ring_lds, StreamK{});
+          GZ_LAUNCH_128(WAVES_N, WAVES_M, false, false, false, true, true);
       }
       set_error("mfma rung: no kernel for the transposed problem on this tile");
       return GZ_ERR_UNSUPPORTED;
@@ -1379,9 +1395,9 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
       }
       if constexpr (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2) {
         if (ring && !akc && !bkc && shape_class == MFMA_SHAPE_RAGGED)
-          GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false, false, false>), ring_lds, StreamK{});
+          GZ_LAUNCH_128(WAVES_M, WAVES_N, true, false, false, false, false);
         if (ring && !akc && !bkc && !edge)
-          GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false, false, false>), ring_lds, StreamK{});
+          GZ_LAUNCH_128(WAVES_M, WAVES_N, false, false, false, false, false);
       }
     }
     if constexpr (TILE_256) {
@@ -1397,12 +1413,12 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
     // the same kernel on 128 x 128 tiles (int8 and the 16-bit types), one work-group per tile, two per compute unit
     if constexpr (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2 && !is_fp8(TYPES)) {
       if (ring && akc && shape_class == MFMA_SHAPE_RAGGED) {
-        if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true>), ring_lds, StreamK{});
-        else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, true, false, false>), ring_lds, StreamK{});
+        if (bkc) GZ_LAUNCH_128(WAVES_M, WAVES_N, true, false, true, false, true);
+        else GZ_LAUNCH_128(WAVES_M, WAVES_N, true, false, false, false, true);
       }
       if (ring && akc && !edge) {
-        if (bkc) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N>), ring_lds, StreamK{});
-        else GZ_LAUNCH_DIRECT(GZ_KERN(mfma_ring16_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false, false, false>), ring_lds, StreamK{});
+        if (bkc) GZ_LAUNCH_128(WAVES_M, WAVES_N, false, false, true, false, true);
+        else GZ_LAUNCH_128(WAVES_M, WAVES_N, false, false, false, false, true);
       }
     }
     if (!edge && akc && bkc) {  // whole tiles, both operands K-contiguous
@@ -1417,6 +1433,7 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
       if constexpr (BM == 128 && BN == 128) GZ_LAUNCH_DIRECT(GZ_KERN(mfma_dtl_kernel<TYPES, BM, BN, WAVES_M, WAVES_N, false>), dtl_lds);
     }
   }
+#undef GZ_LAUNCH_128
 #undef GZ_LAUNCH_DIRECT
 #undef GZ_LAUNCH_DIRECT_ON
 #undef GZ_KERN

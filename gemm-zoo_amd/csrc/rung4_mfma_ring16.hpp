@@ -151,10 +151,10 @@ template <int ES, int ROW_BYTES> __host__ __device__ constexpr int ring16_row_sw
 // A_KC = false: a column-major A (K rows of M contiguous elements) beside a row-major B.  A then takes the route of a
 // row-major B: whole K rows per copy, a K step per copy group, fragments through the transposing LDS reads.
 template <int TYPES, int BM, int BN, int WAVES_M, int WAVES_N, bool RAGGED = false, bool STREAMK = false, bool B_KC = true,
-          bool SWAP = false, bool A_KC = true>
+          bool SWAP = false, bool A_KC = true, int NST = 5>
 // (second launch bound: waves per SIMD the registers must leave room for - the 128 x 128 tile, whose five buffers are
 // half the LDS, runs two work-groups per compute unit)
-__global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128) ? 2 : (WAVES_M * WAVES_N) / 4)
+__global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128 && NST == 5) ? 2 : (WAVES_M * WAVES_N) / 4)
     mfma_ring16_kernel(GemmArgs<TYPES> g, int tiles_m, int tiles_n, StreamK sk) {
   using T = Traits<TYPES>;
   using in_t = typename T::in_t;
@@ -163,7 +163,9 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
   constexpr int ES = (int)sizeof(in_t);
   constexpr int LINE = 128;           // K bytes per row and slab
   constexpr int SK = LINE / ES;       // K elements per slab
-  constexpr int NST = 5;              // LDS buffers, one copy group each
+  // NST LDS buffers, one copy group each: a slab asks for the one AHEAD slabs on.  (An odd number: a slab's first group goes
+  // into the buffer that the slab before left at its barrier, its second into the slab's own first.)
+  constexpr int AHEAD = (NST - 1) / 2;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   constexpr int FM = WM / 16, FN = WN / 16;
   constexpr bool F32 = TYPES == GZ_F32F32F32;
@@ -188,7 +190,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
                 "the 256 x 256 tile, or the 128 x 128 tile on four waves for int8 and the 16-bit types");
   static_assert(BM % (16 * NW) == 0 && BN % (16 * NW) == 0, "tile rows must divide over the waves");
   static_assert(A_PW <= 8 && B_PW <= 8 && A_PW % 2 == 0 && B_PW % 2 == 0, "a copy group must fit the immediate offset range");
-  static_assert(NCP == 8 || NCP == 4, "the vmcnt immediates below are written out for 8 or 4 copies per wave and group");
+  static_assert(NST == 5 || (NST == 9 && NCP == 4 && !STREAMK && !F8), "nine buffers of the 128 x 128 tile fill the LDS");
+  static_assert((2 * AHEAD - 2) * NCP < 64, "vmcnt is a 6-bit counter");
 
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
@@ -673,10 +676,17 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
   // Slab 0 (groups 0 and 1) has landed; what was issued after it may still be on its way.  (Persistent: the last
   // epilogue's stores are counted between the two pairs of groups.  Loads return in order, so with no more than two
   // groups' worth of operations outstanding none of them can be a load of groups 0 and 1.)
-  if (nc > 2) {
-    issue_group(std::integral_constant<int, 2>{}, a_tile - a_back, b_tile - b_back);
-    issue_group(std::integral_constant<int, 3>{}, a_tile - a_back, b_tile - b_back);
-    asm volatile("s_waitcnt vmcnt(%0)" : : "i"(2 * NCP) : "memory");
+  if (nc >= 2 * AHEAD) {
+    static_for<2 * AHEAD - 2>([&](auto c) {
+      issue_group(std::integral_constant<int, 2 + decltype(c)::value>{}, a_tile - a_back, b_tile - b_back);
+    });
+    asm volatile("s_waitcnt vmcnt(%0)" : : "i"((2 * AHEAD - 2) * NCP) : "memory");
+  } else if (AHEAD > 2 && nc > 2) {   // (a short run: whatever there is, and all of it)
+    static_for<2 * AHEAD - 4>([&](auto c) {
+      constexpr int C = 2 + decltype(c)::value;
+      if (C < nc) issue_group(std::integral_constant<int, C>{}, a_tile - a_back, b_tile - b_back);
+    });
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
@@ -697,42 +707,41 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     static_for<NRD>([&](auto r) { read_one(I0{}, r, I0{}); });
   }
 
-  // ---- one slab; JR = j % 5 at compile time.  Slab j fetches slab j + 2 (groups 2j + 4 and 2j + 5) from a_cp / b_cp,
+  // ---- one slab; JR = j % 5 at compile time.  Slab j fetches slab j + AHEAD (groups 2j + 4 and 2j + 5 of five buffers) from a_cp / b_cp,
   // or, where the run has no such slab, its last slab again ----
   const int nslab = nc / 2;
-  const int first_fetch = min(2, nslab - 1);
+  const int first_fetch = min(AHEAD, nslab - 1);
   const char* a_cp = a_group(a_tile, 2 * first_fetch) - a_back;
   const char* b_cp = b_group(b_tile, 2 * first_fetch) - b_back;
   auto slab = [&](auto jr_c, int j) {
     constexpr int JR = decltype(jr_c)::value;
     using NEXT = std::integral_constant<int, (JR + 1) % NST>;
-    using ST4 = std::integral_constant<int, (2 * JR + 4) % NST>;
-    using ST5 = std::integral_constant<int, (2 * JR + 5) % NST>;
+    using ST4 = std::integral_constant<int, (2 * JR + 2 * AHEAD) % NST>;
+    using ST5 = std::integral_constant<int, (2 * JR + 2 * AHEAD + 1) % NST>;
     // a row-major B: a group is a K step's rows, the slab's second group lies a step further
     const char* const b_cp1 = B_KC ? b_cp : b_cp + b_group_step;
     const char* const a_cp1 = A_KC ? a_cp : a_cp + a_group_step;
     if constexpr (F8) half_f8(I0{}, jr_c, ST4{}, a_cp, b_cp);
     else kstep(I0{}, jr_c, I0{}, ST4{}, a_cp, b_cp);
-    if (j + 2 < nslab) {  // the copies of group 2j+4 may stay in flight
-      if constexpr (NCP == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // the copies of group 2j+4 (of nine buffers 2j+4 ... 2j+8) may stay in flight; a run shorter than what the prologue
+    // asks for has been waited for altogether
+    if (j + 2 < nslab) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "i"((2 * AHEAD - 3) * NCP) : "memory");
     } else {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
     if constexpr (F8) half_f8(I1{}, jr_c, ST5{}, a_cp1, b_cp1);
     else kstep(I1{}, NEXT{}, I1{}, ST5{}, a_cp1, b_cp1);
-    const bool more = j + 3 < nslab;   // the next slab fetches one further
+    const bool more = j + AHEAD + 1 < nslab;   // the next slab fetches one further
     a_cp += more ? (A_KC ? (size_t)LINE : 2 * a_group_step) : (size_t)0;
     b_cp += more ? (B_KC ? (size_t)LINE : 2 * b_group_step) : (size_t)0;
   };
 
-  for (int j = 0; j < nslab; j += NST) {
-    slab(std::integral_constant<int, 0>{}, j);
-    if (j + 1 < nslab) slab(std::integral_constant<int, 1>{}, j + 1);
-    if (j + 2 < nslab) slab(std::integral_constant<int, 2>{}, j + 2);
-    if (j + 3 < nslab) slab(std::integral_constant<int, 3>{}, j + 3);
-    if (j + 4 < nslab) slab(std::integral_constant<int, 4>{}, j + 4);
-  }
+  for (int j = 0; j < nslab; j += NST)
+    static_for<NST>([&](auto x_c) {
+      constexpr int X = decltype(x_c)::value;
+      if (X == 0 || j + X < nslab) slab(x_c, j + X);
+    });
 
   // no copy may still be in flight when the work-group ends, and the last MFMAs must have written their
   // accumulators before ordinary code reads them
@@ -742,7 +751,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     asm_touch_acc4<TYPES>(acc[Q / FN][Q % FN]);
   });
 
-  // the epilogue passes the accumulators through the end of the operand buffers: 4 and 3 and a little of 2
+  // the epilogue passes the accumulators through the end of the operand buffers: of five, 4 and 3 and a little of 2
   constexpr int EP_COLS32 = (SWAP ? WM : WN) / 32;   // 32-column blocks of the real D per wave
   static_assert(NW * epilogue_region_bytes<EP_COLS32>() <= 3 * STAGE_BYTES, "the epilogue leaves buffers 0 and 1 alone");
   char* const staging = lds + NST * STAGE_BYTES - (NW - wave) * epilogue_region_bytes<EP_COLS32>();
