@@ -251,7 +251,8 @@ bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
     // two launches, the sums written and read back, the slabs of the longest part (us, measured / this line: bf16
     // 24 x 1280 x 11001 in 12 parts 14.4 / 13.7, 100 x 2560 x 12416 in 6 27.6 / 26.7, fp32 512^3 in 4 10.1 / 9.6)
     const double walk = (double)((slabs + p - 1) / p) * slab_us * mfma_64_share(types, own_slabs, (double)(tiles * p) / num_cus);
-    const double t = 6.5 + 0.22 * (double)bytes / (1 << 20) + (walk > stream_us ? walk : stream_us);
+    // (slabs of the waves' own: their sums meet in LDS first - e5m2 97 x 3456 x 3328 in 2 parts 11.1 / 10.8)
+    const double t = (own_slabs ? 7.2 : 6.5) + 0.22 * (double)bytes / (1 << 20) + (walk > stream_us ? walk : stream_us);
     if (parts == 0 || t < best) {
       best = t;
       parts = p;
@@ -282,11 +283,11 @@ bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
   MfmaColSplit cols;
   double est = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &c) * round_us;
   if (c.bm <= 64) {   // the same tile unsplit, or the smaller one, by the same measure
-    // (32 x 32 tiles on less than a sixth of the compute units and forty slabs or more: either may win by a quarter, and the
-    // parts are kept up to that - int8 192 x 128 x 5120 row/col parts / 32 x 32 8.8 / 6.5, row/row 8.8 / 10.0, 64 x 128 x
+    // (32 x 32 tiles on less than a sixth of the compute units and forty slabs or more: either may win by a third, and the
+    // parts are kept up to what their estimate is over that - int8 192 x 128 x 5120 row/col parts / 32 x 32 8.8 / 6.5, row/row 8.8 / 10.0, 64 x 128 x
     // 16384 9.9 / 11.7, bf16 192 x 128 x 2560 row/row 8.7 / 7.8)
     if (c.bm == 32 && (long long)((M + 31) / 32) * ((N + 31) / 32) * 6 <= num_cus && slabs >= 40)
-      return out->estimate_us < 1.3 * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
+      return out->estimate_us < 1.45 * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
     est = c.bm == 64 ? mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) : mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
     return out->estimate_us < 0.90 * est;
   }

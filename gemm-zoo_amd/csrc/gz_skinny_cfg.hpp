@@ -252,7 +252,8 @@ inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned l
     const double small_us = mfma_32_us(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus);
     if (small_us < 0.9 * stream_us && (!split_ok || small_us < split->estimate_us)) return SKINNY_TILES_32;
   }
-  if (split_ok && split->estimate_us < 0.9 * stream_us) return SKINNY_TILES_SPLITK;
+  // (0.85: e5m2 97 x 3456 x 3328 tile kernel / split K 10.0 / 11.1, estimated 12.3 / 10.8)
+  if (split_ok && split->estimate_us < 0.85 * stream_us) return SKINNY_TILES_SPLITK;
   return SKINNY_STREAM;
 }
 
