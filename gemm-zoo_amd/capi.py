@@ -125,14 +125,16 @@ def _ptr(x) -> int:
     return x.data_ptr()
 
 
+_TYPED = {S8S8S32: lib.gz_gemm_s8s8s32, BF16BF16F32: lib.gz_gemm_bf16bf16f32, BF16BF16BF16: lib.gz_gemm_bf16bf16bf16,
+          F16F16F16: lib.gz_gemm_f16f16f16, F32F32F32: lib.gz_gemm_f32f32f32, E4M3E4M3F16: lib.gz_gemm_e4m3e4m3f16,
+          E5M2E5M2F16: lib.gz_gemm_e5m2e5m2f16, BF16BF16BF16_ACC16: lib.gz_gemm_bf16bf16bf16_acc16,
+          F16F16F16_ACC16: lib.gz_gemm_f16f16f16_acc16}
+
+
 def gemm(types: int, a, b, c, d, m: int, n: int, k: int, layout_a: int = ROW_MAJOR, layout_b: int = ROW_MAJOR,
          alpha=1, beta=0, rung: int = RUNG_AUTO, variant: int = 0, stream: int = 0) -> None:
     """Typed entry point dispatch (raises GzError on a non-zero status)."""
-    fn = {S8S8S32: lib.gz_gemm_s8s8s32, BF16BF16F32: lib.gz_gemm_bf16bf16f32,
-          BF16BF16BF16: lib.gz_gemm_bf16bf16bf16, F16F16F16: lib.gz_gemm_f16f16f16,
-          F32F32F32: lib.gz_gemm_f32f32f32, E4M3E4M3F16: lib.gz_gemm_e4m3e4m3f16,
-          E5M2E5M2F16: lib.gz_gemm_e5m2e5m2f16, BF16BF16BF16_ACC16: lib.gz_gemm_bf16bf16bf16_acc16,
-          F16F16F16_ACC16: lib.gz_gemm_f16f16f16_acc16}.get(types)
+    fn = _TYPED.get(types)
     if fn is None:
         raise GzError(ERR_BAD_ARG, f"unknown type bundle {types}")
     if types == S8S8S32:

@@ -1758,16 +1758,39 @@ static int launch_streamk(const GemmArgs<TYPES>& g, const StreamKPlan& p, bool r
   }
 }
 
+// What the launcher itself would make of a problem (variant 0), whatever the pointers and pitches: a function of the sizes
+// alone.  The smallest problems take 3 - 4 us on the device and the estimates behind their plans took 1 us of the host's
+// time on every call, so each thread keeps the last few sizes' plans, as a program with a functor per size keeps its own.
+struct AutoPlan {
+  int M = -1, N = -1, K = -1, layoutA = -1, layoutB = -1, num_cus = -1;
+  bool splitk = false, streamk = false;
+  SplitKPlan skp;
+  StreamKPlan stk;
+  int cut = 0;
+  MfmaSplit sp;
+  MfmaColSplit cs;
+  MfmaCfg cfg;
+};
+template <int TYPES> static const AutoPlan& auto_plan(int M, int N, int K, int layoutA, int layoutB, int num_cus) {
+  constexpr unsigned SLOTS = 16;
+  static thread_local AutoPlan slots[SLOTS];
+  AutoPlan& p = slots[((unsigned)M * 73856093u ^ (unsigned)N * 19349663u ^ (unsigned)K * 83492791u ^ (unsigned)(2 * layoutA + layoutB)) % SLOTS];
+  if (p.M == M && p.N == N && p.K == K && p.layoutA == layoutA && p.layoutB == layoutB && p.num_cus == num_cus) return p;
+  p.splitk = mfma_plan_splitk(TYPES, M, N, K, layoutA, layoutB, num_cus, &p.skp);
+  p.streamk = K > 0 && mfma_plan_streamk(TYPES, M, N, K, layoutA, layoutB, num_cus, false, nullptr, &p.stk);
+  p.cut = K > 0 ? mfma_resolve_cut(TYPES, M, N, K, layoutA, layoutB, num_cus, &p.sp, &p.cs) : 0;
+  (void)mfma_resolve(TYPES, M, N, K, layoutA, layoutB, 0, num_cus, &p.cfg);
+  p.M = M; p.N = N; p.K = K; p.layoutA = layoutA; p.layoutB = layoutB; p.num_cus = num_cus;
+  return p;
+}
+
 template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, hipStream_t s) {
   GemmArgs<TYPES> g = args;
   const int num_cus = device_compute_units();
   g.store_hint = mfma_store_hint(TYPES, g.M, g.N, g.K, (int)sizeof(typename Traits<TYPES>::out_t), num_cus);
-  if (variant == 0) {
-    SplitKPlan skp;
-    if (mfma_plan_splitk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, &skp) &&
-        (unsigned long long)skp.workspace_bytes <= (unsigned long long)workspace_limit(s))
-      if (const int st = launch_splitk<TYPES>(g, skp, s); st >= 0) return st;
-  }
+  const AutoPlan* const own = variant == 0 ? &auto_plan<TYPES>(g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus) : nullptr;
+  if (own && own->splitk && (unsigned long long)own->skp.workspace_bytes <= (unsigned long long)workspace_limit(s))
+    if (const int st = launch_splitk<TYPES>(g, own->skp, s); st >= 0) return st;
   // Column-major A and B: the transposed problem on the ring kernel - one launch, or where the launcher would cut
   // the rows of the transposed problem (a mostly empty last round) two, over column ranges of the real C and D.
   // Returns -1 where that kernel does not take the problem.
@@ -1829,7 +1852,8 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     // the launcher's own choice stays within the workspace this call may use (the entry point that allocates nothing has a
     // fixed one); an explicit stream-K variant that needs more is refused by the lease instead, and where there is none
     // at all (workspace_limit) it runs the plain launch below, as on unaligned operands
-    if (mfma_plan_streamk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, forced != nullptr, forced, &skp) &&
+    if (own) skp = own->stk;
+    if ((own ? own->streamk : mfma_plan_streamk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, true, forced, &skp)) &&
         (forced ? 1 : (size_t)skp.slots * MFMA_STREAMK_SLOT_BYTES) <= workspace_limit(s)) {
       const int cls = mfma_launch_class(skp.cfg, (int)sizeof(typename Traits<TYPES>::in_t),
                                         (int)sizeof(typename Traits<TYPES>::out_t), g.M, g.N, g.K, g.layoutA, g.layoutB,
@@ -1842,10 +1866,9 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     }
   }
   if (variant == 0 && g.K > 0) {
-    MfmaSplit sp;
-    MfmaColSplit cs;
-    const int cut = mfma_resolve_cut(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, &sp, &cs);
-    if (cut == 1) {
+    const MfmaSplit& sp = own->sp;
+    const MfmaColSplit& cs = own->cs;
+    if (own->cut == 1) {
       // a mostly empty last round of 256x256 tiles: the rows that fill whole rounds first, the rest in a second launch
       GemmArgs<TYPES> top = g, bottom = g;
       top.M = sp.rows_main;
@@ -1857,7 +1880,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
       if (st != GZ_OK) return st;
       return launch_one<TYPES>(bottom, sp.tail, s, true);
     }
-    if (cut == 2) {
+    if (own->cut == 2) {
       // a few columns past a multiple of 256: those columns in a launch of their own
       GemmArgs<TYPES> left = g, right = g;
       left.N = cs.cols_main;
@@ -1871,7 +1894,9 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     }
   }
   MfmaCfg cfg;
-  if (!mfma_resolve(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, variant, num_cus, &cfg)) {
+  if (own) {
+    cfg = own->cfg;
+  } else if (!mfma_resolve(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, variant, num_cus, &cfg)) {
     set_error("mfma rung: unknown variant %d", variant);
     return GZ_ERR_UNSUPPORTED;
   }
