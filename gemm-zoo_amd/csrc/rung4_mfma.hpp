@@ -32,6 +32,7 @@
 
 #include "gz_common.hpp"
 #include "gz_mfma_cfg.hpp"
+#include "gz_plan_cache.hpp"
 
 namespace gz {
 
@@ -1760,37 +1761,57 @@ static int launch_streamk(const GemmArgs<TYPES>& g, const StreamKPlan& p, bool r
 
 // What the launcher itself would make of a problem (variant 0), whatever the pointers and pitches: a function of the sizes
 // alone.  The smallest problems take 3 - 4 us on the device and the estimates behind their plans took 1 us of the host's
-// time on every call, so each thread keeps the last few sizes' plans, as a program with a functor per size keeps its own.
-struct AutoPlan {
-  int M = -1, N = -1, K = -1, layoutA = -1, layoutB = -1, num_cus = -1;
-  bool splitk = false, streamk = false;
-  SplitKPlan skp;
-  StreamKPlan stk;
-  int cut = 0;
-  MfmaSplit sp;
-  MfmaColSplit cs;
-  MfmaCfg cfg;
+// time on every call, so each thread keeps the plans of its last sixteen sizes, as a program with a functor per size keeps
+// its own.  A part of a plan is worked out when a launch first comes to it: most end before the last.
+template <int TYPES> class AutoPlan {
+ public:
+  AutoPlan() = default;
+  explicit AutoPlan(const PlanKey& key) : k_(key) {}
+  // null: no such plan
+  const SplitKPlan* split_k() {
+    if (!split_known_) split_ = mfma_plan_splitk(TYPES, k_.M, k_.N, k_.K, k_.layoutA, k_.layoutB, k_.num_cus, &skp_), split_known_ = true;
+    return split_ ? &skp_ : nullptr;
+  }
+  const StreamKPlan* stream_k() {
+    if (!stream_known_)
+      stream_ = k_.K > 0 && mfma_plan_streamk(TYPES, k_.M, k_.N, k_.K, k_.layoutA, k_.layoutB, k_.num_cus, false, nullptr, &stk_), stream_known_ = true;
+    return stream_ ? &stk_ : nullptr;
+  }
+  // 0: one launch; 1: rows() in two; 2: columns() in two
+  int cut() {
+    if (cut_ < 0) cut_ = k_.K > 0 ? mfma_resolve_cut(TYPES, k_.M, k_.N, k_.K, k_.layoutA, k_.layoutB, k_.num_cus, &rows_, &cols_) : 0;
+    return cut_;
+  }
+  const MfmaSplit& rows() const { return rows_; }
+  const MfmaColSplit& columns() const { return cols_; }
+  const MfmaCfg& tile() {
+    if (!tile_known_) tile_known_ = mfma_resolve(TYPES, k_.M, k_.N, k_.K, k_.layoutA, k_.layoutB, 0, k_.num_cus, &tile_);
+    return tile_;
+  }
+
+ private:
+  PlanKey k_ = {};
+  bool split_known_ = false, split_ = false, stream_known_ = false, stream_ = false, tile_known_ = false;
+  int cut_ = -1;
+  SplitKPlan skp_;
+  StreamKPlan stk_;
+  MfmaSplit rows_;
+  MfmaColSplit cols_;
+  MfmaCfg tile_;
 };
-template <int TYPES> static const AutoPlan& auto_plan(int M, int N, int K, int layoutA, int layoutB, int num_cus) {
-  constexpr unsigned SLOTS = 16;
-  static thread_local AutoPlan slots[SLOTS];
-  AutoPlan& p = slots[((unsigned)M * 73856093u ^ (unsigned)N * 19349663u ^ (unsigned)K * 83492791u ^ (unsigned)(2 * layoutA + layoutB)) % SLOTS];
-  if (p.M == M && p.N == N && p.K == K && p.layoutA == layoutA && p.layoutB == layoutB && p.num_cus == num_cus) return p;
-  p.splitk = mfma_plan_splitk(TYPES, M, N, K, layoutA, layoutB, num_cus, &p.skp);
-  p.streamk = K > 0 && mfma_plan_streamk(TYPES, M, N, K, layoutA, layoutB, num_cus, false, nullptr, &p.stk);
-  p.cut = K > 0 ? mfma_resolve_cut(TYPES, M, N, K, layoutA, layoutB, num_cus, &p.sp, &p.cs) : 0;
-  (void)mfma_resolve(TYPES, M, N, K, layoutA, layoutB, 0, num_cus, &p.cfg);
-  p.M = M; p.N = N; p.K = K; p.layoutA = layoutA; p.layoutB = layoutB; p.num_cus = num_cus;
-  return p;
+template <int TYPES> static AutoPlan<TYPES>& auto_plan(int M, int N, int K, int layoutA, int layoutB, int num_cus) {
+  static thread_local RecentPlans<AutoPlan<TYPES>, 16> plans;
+  return plans.of(PlanKey{M, N, K, layoutA, layoutB, num_cus});
 }
 
 template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, hipStream_t s) {
   GemmArgs<TYPES> g = args;
   const int num_cus = device_compute_units();
   g.store_hint = mfma_store_hint(TYPES, g.M, g.N, g.K, (int)sizeof(typename Traits<TYPES>::out_t), num_cus);
-  const AutoPlan* const own = variant == 0 ? &auto_plan<TYPES>(g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus) : nullptr;
-  if (own && own->splitk && (unsigned long long)own->skp.workspace_bytes <= (unsigned long long)workspace_limit(s))
-    if (const int st = launch_splitk<TYPES>(g, own->skp, s); st >= 0) return st;
+  AutoPlan<TYPES>* const own = variant == 0 ? &auto_plan<TYPES>(g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus) : nullptr;
+  if (const SplitKPlan* const kp = own ? own->split_k() : nullptr;
+      kp && (unsigned long long)kp->workspace_bytes <= (unsigned long long)workspace_limit(s))
+    if (const int st = launch_splitk<TYPES>(g, *kp, s); st >= 0) return st;
   // Column-major A and B: the transposed problem on the ring kernel - one launch, or where the launcher would cut
   // the rows of the transposed problem (a mostly empty last round) two, over column ranges of the real C and D.
   // Returns -1 where that kernel does not take the problem.
@@ -1847,28 +1868,30 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
     return st;
   }
   if ((variant == 0 || variant == MFMA_VARIANT_STREAMK_W4 || variant == MFMA_VARIANT_STREAMK_W8) && g.K > 0) {
-    StreamKPlan skp;
+    StreamKPlan named;
     const MfmaCfg* forced = variant == 0 ? nullptr : &kMfmaCfgs[variant - 1];
+    const StreamKPlan* kp = &named;
+    if (own) kp = own->stream_k();
+    else if (!mfma_plan_streamk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, true, forced, &named)) kp = nullptr;
     // the launcher's own choice stays within the workspace this call may use (the entry point that allocates nothing has a
     // fixed one); an explicit stream-K variant that needs more is refused by the lease instead, and where there is none
     // at all (workspace_limit) it runs the plain launch below, as on unaligned operands
-    if (own) skp = own->stk;
-    if ((own ? own->streamk : mfma_plan_streamk(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, num_cus, true, forced, &skp)) &&
-        (forced ? 1 : (size_t)skp.slots * MFMA_STREAMK_SLOT_BYTES) <= workspace_limit(s)) {
-      const int cls = mfma_launch_class(skp.cfg, (int)sizeof(typename Traits<TYPES>::in_t),
+    if (kp && (forced ? 1 : (size_t)kp->slots * MFMA_STREAMK_SLOT_BYTES) <= workspace_limit(s)) {
+      const int cls = mfma_launch_class(kp->cfg, (int)sizeof(typename Traits<TYPES>::in_t),
                                         (int)sizeof(typename Traits<TYPES>::out_t), g.M, g.N, g.K, g.layoutA, g.layoutB,
                                         g.A, g.B, g.C, g.D, g.lda, g.ldb, g.ldc, g.ldd);
       if (cls != MFMA_SHAPE_GENERAL) {   // (unaligned operands: the plain launch below, on the register-staged kernel)
         g.store_hint = 0;   // one round at most ends in each launch: plain stores
-        return skp.cfg.waves_n == 4 ? launch_streamk<TYPES, 4>(g, skp, cls == MFMA_SHAPE_RAGGED, s)
-                                    : launch_streamk<TYPES, 2>(g, skp, cls == MFMA_SHAPE_RAGGED, s);
+        return kp->cfg.waves_n == 4 ? launch_streamk<TYPES, 4>(g, *kp, cls == MFMA_SHAPE_RAGGED, s)
+                                    : launch_streamk<TYPES, 2>(g, *kp, cls == MFMA_SHAPE_RAGGED, s);
       }
     }
   }
-  if (variant == 0 && g.K > 0) {
-    const MfmaSplit& sp = own->sp;
-    const MfmaColSplit& cs = own->cs;
-    if (own->cut == 1) {
+  if (own) {
+    const int cut = own->cut();
+    const MfmaSplit& sp = own->rows();
+    const MfmaColSplit& cs = own->columns();
+    if (cut == 1) {
       // a mostly empty last round of 256x256 tiles: the rows that fill whole rounds first, the rest in a second launch
       GemmArgs<TYPES> top = g, bottom = g;
       top.M = sp.rows_main;
@@ -1880,7 +1903,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
       if (st != GZ_OK) return st;
       return launch_one<TYPES>(bottom, sp.tail, s, true);
     }
-    if (own->cut == 2) {
+    if (cut == 2) {
       // a few columns past a multiple of 256: those columns in a launch of their own
       GemmArgs<TYPES> left = g, right = g;
       left.N = cs.cols_main;
@@ -1895,7 +1918,7 @@ template <int TYPES> int launch_mfma(const GemmArgs<TYPES>& args, int variant, h
   }
   MfmaCfg cfg;
   if (own) {
-    cfg = own->cfg;
+    cfg = own->tile();
   } else if (!mfma_resolve(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, variant, num_cus, &cfg)) {
     set_error("mfma rung: unknown variant %d", variant);
     return GZ_ERR_UNSUPPORTED;
