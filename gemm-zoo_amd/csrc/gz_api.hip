@@ -578,17 +578,33 @@ int gz_variant_count(int types, int rung) {
   }
 }
 
-static void plan_splitk(const SplitKPlan& kp, int types, int m, int n, int k, int layoutA, int layoutB, gz_plan_t* plan) {
-  const int es = in_size(types);
-  const MfmaCfg c = mfma_64_cfg(types, m, n, k, layoutA, layoutB);
+// What gz_plan says of a tile configuration; `grid` is the caller's.  Fails where the device has too little LDS.  (64 x 64
+// tiles with slabs of the waves' own, on a device that has no room for them: the register-staged ones.  The launchers know
+// only gfx950, which has.)
+static int plan_tile(MfmaCfg& c, int types, int shape_class, int m, int n, int k, int layoutA, int layoutB, bool transposed, int parts,
+                     int num_cus, int lds_per_cu, gz_plan_t* plan) {
+  auto lds = [&] { return mfma_lds_bytes(c, types, shape_class, m, n, k, layoutA, layoutB, transposed, parts, num_cus, lds_per_cu); };
+  if (c.k_waves > 1 && c.bm == 64 && lds() > lds_per_cu) c = mfma_in_size(types) == 1 ? kMfmaCfg64StagedInt8 : kMfmaCfg64Staged;
   plan->variant = c.id;
-  plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
-  plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
+  plan->tile_m = transposed ? c.bn : c.bm;   // (the configuration's rows run along N there)
+  plan->tile_n = transposed ? c.bm : c.bn;
+  plan->tile_k = MFMA_SLAB_BYTES / in_size(types);
+  plan->wave_m = transposed ? c.bn / c.waves_m : c.bm / c.waves_m;
+  plan->wave_n = transposed ? c.bm / c.waves_n : c.bn / c.waves_n;
   plan->threads = mfma_threads(c);
-  plan->lds_bytes = mfma_lds_bytes(c);
+  plan->lds_bytes = lds();
+  if (plan->lds_bytes <= lds_per_cu) return GZ_OK;
+  set_error("mfma variant %d needs %d bytes of LDS, device has %d", c.id, plan->lds_bytes, lds_per_cu);
+  return GZ_ERR_UNSUPPORTED;
+}
+
+static int plan_splitk(const SplitKPlan& kp, int types, int m, int n, int k, int layoutA, int layoutB, int num_cus, int lds_per_cu,
+                       gz_plan_t* plan) {
+  MfmaCfg c = mfma_64_cfg(types, m, n, k, layoutA, layoutB);
   plan->split_k = kp.parts;
   plan->grid = (int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * kp.parts;
   plan->workspace_bytes = kp.workspace_bytes;
+  return plan_tile(c, types, MFMA_SHAPE_GENERAL, m, n, k, layoutA, layoutB, false, kp.parts, num_cus, lds_per_cu, plan);
 }
 
 // ws_limit: the most device memory beyond the matrices that the launch may use (what workspace_limit(s) will say
@@ -647,14 +663,8 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
         return GZ_OK;
       }
       if (SplitKPlan kp; variant == 0 && mfma_plan_splitk(types, m, n, k, layoutA, layoutB, num_cus, &kp) &&
-                         (unsigned long long)kp.workspace_bytes <= (unsigned long long)ws_limit) {
-        plan_splitk(kp, types, m, n, k, layoutA, layoutB, plan);
-        if (plan->lds_bytes > lds_per_cu) {
-          set_error("mfma variant %d needs %d bytes of LDS, device has %d", plan->variant, plan->lds_bytes, lds_per_cu);
-          return GZ_ERR_UNSUPPORTED;
-        }
-        return GZ_OK;
-      }
+                         (unsigned long long)kp.workspace_bytes <= (unsigned long long)ws_limit)
+        return plan_splitk(kp, types, m, n, k, layoutA, layoutB, num_cus, lds_per_cu, plan);
       MfmaSplit tsp;
       // (column-major A and B: a few columns past a multiple of 256 are cut off first, as launch_mfma does)
       MfmaColSplit ccs;
@@ -663,13 +673,7 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
       const int n_ring = cc_cut ? ccs.cols_main : n;   // columns that the transposed problem covers
       if (MfmaCfg ct; mfma_transposed_ring(types, m, n_ring, k, layoutA, layoutB, variant, num_cus, &ct, cc_cut ? nullptr : &tsp)) {
         if (cc_cut) tsp.rows_main = 0;
-        // column-major A and B: the ring kernel on the transposed problem (as launch_mfma, aligned operands assumed);
-        // the configuration's rows run along N there
-        plan->variant = ct.id;
-        plan->tile_m = ct.bn; plan->tile_n = ct.bm; plan->tile_k = MFMA_SLAB_BYTES / es;
-        plan->wave_m = ct.bn / ct.waves_m; plan->wave_n = ct.bm / ct.waves_n;
-        plan->threads = mfma_threads(ct);
-        plan->lds_bytes = mfma_lds_bytes(ct);
+        // column-major A and B: the ring kernel on the transposed problem (as launch_mfma, aligned operands assumed)
         const int n_first = tsp.rows_main > 0 ? tsp.rows_main : n_ring;   // columns of the first launch
         plan->grid = (int64_t)ceil_div(n_first, ct.bm) * ceil_div(m, ct.bn);
         const int cls_t = mfma_shape_class(ct, es, n_first, m, k, GZ_ROW_MAJOR, GZ_ROW_MAJOR);
@@ -687,32 +691,20 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
           plan->tail_tile_n = ccs.strip ? plan->tail_cols : ccs.tail.bn;
           plan->tail_grid = ccs.strip ? ceil_div(m, 16) : (int64_t)ceil_div(m, ccs.tail.bm) * ceil_div(n - ccs.cols_main, ccs.tail.bn);
         }
-        if (plan->lds_bytes > lds_per_cu) {
-          set_error("mfma variant %d needs %d bytes of LDS, device has %d", ct.id, plan->lds_bytes, lds_per_cu);
-          return GZ_ERR_UNSUPPORTED;
-        }
-        return GZ_OK;
+        return plan_tile(ct, types, cls_t, n_first, m, k, GZ_ROW_MAJOR, GZ_ROW_MAJOR, true, 1, num_cus, lds_per_cu, plan);
       }
       if ((variant == 0 || variant == MFMA_VARIANT_STREAMK_W4 || variant == MFMA_VARIANT_STREAMK_W8) && k > 0) {   // as launch_mfma, aligned operands assumed
         StreamKPlan skp;
         const MfmaCfg* forced = variant == 0 ? nullptr : &kMfmaCfgs[variant - 1];
         if (mfma_plan_streamk(types, m, n, k, layoutA, layoutB, num_cus, forced != nullptr, forced, &skp) &&
             (forced || (size_t)skp.slots * MFMA_STREAMK_SLOT_BYTES <= ws_limit)) {
-          const MfmaCfg& c = skp.cfg;
-          plan->variant = c.waves_n == 4 ? MFMA_VARIANT_STREAMK_W8 : MFMA_VARIANT_STREAMK_W4;
-          plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
-          plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
-          plan->threads = mfma_threads(c);
-          plan->lds_bytes = mfma_lds_bytes(c);
+          MfmaCfg c = kMfmaCfgs[(skp.cfg.waves_n == 4 ? MFMA_VARIANT_STREAMK_W8 : MFMA_VARIANT_STREAMK_W4) - 1];
           plan->grid = (int64_t)skp.dp_tiles + skp.blocks;
           plan->streamk_tiles = skp.sk_tiles;
           plan->streamk_blocks = skp.blocks;
           plan->workspace_bytes = (int64_t)skp.slots * MFMA_STREAMK_SLOT_BYTES;
-          if (plan->lds_bytes > lds_per_cu) {
-            set_error("mfma variant %d needs %d bytes of LDS, device has %d", plan->variant, plan->lds_bytes, lds_per_cu);
-            return GZ_ERR_UNSUPPORTED;
-          }
-          return GZ_OK;
+          return plan_tile(c, types, mfma_shape_class(c, es, m, n, k, layoutA, layoutB), m, n, k, layoutA, layoutB, false, 1,
+                           num_cus, lds_per_cu, plan);
         }
       }
       MfmaCfg c;
@@ -750,40 +742,38 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
         if (plan->tail_cols && layoutB == GZ_ROW_MAJOR && ((int64_t)n * es) % 16 != 0) cls = MFMA_SHAPE_GENERAL;
         mfma_adjust_general(types, cls, layoutA, layoutB, &c);
       }
-      plan->variant = c.id;
-      plan->tile_m = c.bm; plan->tile_n = c.bn; plan->tile_k = MFMA_SLAB_BYTES / es;
-      plan->wave_m = c.bm / c.waves_m; plan->wave_n = c.bn / c.waves_n;
-      plan->threads = mfma_threads(c);
-      plan->lds_bytes = mfma_lds_bytes(c);
-      plan->grid = (int64_t)ceil_div(m_first, c.bm) * ceil_div(n_first, c.bn);
-      // the ring kernel with the 16x16 instructions (whole tiles, or ragged M and N on its 256 x 256 tile): one
-      // work-group per compute unit walks the tiles
       int cls_g = mfma_shape_class(c, es, m_first, n_first, k, layoutA, layoutB);
       if (plan->tail_cols && layoutB == GZ_ROW_MAJOR && ((int64_t)n * es) % 16 != 0) cls_g = MFMA_SHAPE_GENERAL;
-      if (c.ring == 1 && (layoutA == GZ_ROW_MAJOR || (layoutB == GZ_ROW_MAJOR && !is_fp8(types) && types != GZ_F32F32F32)) &&
-          !(types == GZ_F32F32F32 && c.waves_n != 2) &&
-          cls_g != MFMA_SHAPE_GENERAL)
-        plan->grid = mfma_persistent_grid(plan->grid, num_cus);
-      if (plan->lds_bytes > lds_per_cu) {
-        set_error("mfma variant %d needs %d bytes of LDS, device has %d", c.id, plan->lds_bytes, lds_per_cu);
-        return GZ_ERR_UNSUPPORTED;
-      }
-      return GZ_OK;
+      st = plan_tile(c, types, cls_g, m_first, n_first, k, layoutA, layoutB, false, 1, num_cus, lds_per_cu, plan);
+      plan->grid = (int64_t)ceil_div(m_first, c.bm) * ceil_div(n_first, c.bn);
+      // the ring kernel's 256 x 256 tile: one work-group per compute unit walks the tiles
+      if (c.ring == 1 && mfma_ring_takes(c, types, cls_g, layoutA, layoutB, false)) plan->grid = mfma_persistent_grid(plan->grid, num_cus);
+      return st;
     }
     case GZ_RUNG_SKINNY: {
       if (rung == GZ_RUNG_SKINNY && (st = check_named_skinny(types, m, n, k, layoutA, layoutB)) != GZ_OK) return st;
       if (variant > 1) { set_error("skinny rung has a single variant"); return GZ_ERR_UNSUPPORTED; }
       SplitKPlan kp;
       const int how = rung == GZ_RUNG_AUTO && variant == 0 ? skinny_choose(types, m, n, k, num_cus, ws_limit, &kp) : SKINNY_STREAM;
-      if (how != SKINNY_STREAM) {   // the MFMA rung's 64 x 64 tiles, split along K or not
+      if (how != SKINNY_STREAM) {   // the MFMA rung's tiles, split along K or not
         if (how == SKINNY_TILES_SPLITK) {
-          plan_splitk(kp, types, m, n, k, layoutA, layoutB, plan);
+          st = plan_splitk(kp, types, m, n, k, layoutA, layoutB, num_cus, lds_per_cu, plan);
         } else {
-          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, how == SKINNY_TILES_64 ? kMfmaCfgs[MFMA_CFG_64].id : how == SKINNY_TILES_32 ? kMfmaCfgs[MFMA_CFG_32].id : 0, num_cus, lds_per_cu, ws_limit, plan);
-          if (st != GZ_OK) return st;
+          const int id = how == SKINNY_TILES_64 ? kMfmaCfgs[MFMA_CFG_64].id : how == SKINNY_TILES_32 ? kMfmaCfgs[MFMA_CFG_32].id : 0;
+          st = plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, id, num_cus, lds_per_cu, ws_limit, plan);
         }
+        if (st == GZ_OK) {
+          plan->rung = GZ_RUNG_SKINNY;
+          return GZ_OK;
+        }
+        if (lds_per_cu >= MFMA_LDS_PER_CU) return st;
+        // (a device with less LDS than those tiles take: the streaming kernel)
+        const int va = plan->vector_bytes_a, vb = plan->vector_bytes_b;
+        memset(plan, 0, sizeof(*plan));
         plan->rung = GZ_RUNG_SKINNY;
-        return GZ_OK;
+        plan->split_k = 1;
+        plan->vector_bytes_a = va;
+        plan->vector_bytes_b = vb;
       }
       SkinnyCfg c = skinny_resolve(types, m, n, k, num_cus, (unsigned long long)ws_limit);
       plan->variant = 1;
@@ -807,15 +797,23 @@ static int plan_impl(int types, int64_t M, int64_t N, int64_t K, int layoutA, in
   return GZ_ERR_BAD_ARG;
 }
 
+// The launcher's own choice on a device with less LDS than gfx950's: where that does not fit, the smallest tile there is.
+static int plan_that_fits(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung, int variant, int num_cus,
+                          int lds_per_cu, size_t ws_limit, gz_plan_t* plan) {
+  const int st = plan_impl(types, M, N, K, layoutA, layoutB, rung, variant, num_cus, lds_per_cu, ws_limit, plan);
+  if (st != GZ_ERR_UNSUPPORTED || variant != 0 || lds_per_cu <= 0 || lds_per_cu >= MFMA_LDS_PER_CU || is_acc16(types)) return st;
+  if (rung != GZ_RUNG_MFMA && !(rung == GZ_RUNG_AUTO && plan->rung == GZ_RUNG_MFMA)) return st;
+  return plan_impl(types, M, N, K, layoutA, layoutB, GZ_RUNG_MFMA, kMfmaCfgs[MFMA_CFG_64].id, num_cus, lds_per_cu, ws_limit, plan);
+}
+
 int gz_plan(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung, int variant, int num_cus,
             int lds_per_cu, gz_plan_t* plan) {
-  return plan_impl(types, M, N, K, layoutA, layoutB, rung, variant, num_cus, lds_per_cu, ~(size_t)0, plan);
+  return plan_that_fits(types, M, N, K, layoutA, layoutB, rung, variant, num_cus, lds_per_cu, ~(size_t)0, plan);
 }
 
 int gz_plan_static_scratch(int types, int64_t M, int64_t N, int64_t K, int layoutA, int layoutB, int rung, int variant,
                            int num_cus, int lds_per_cu, gz_plan_t* plan) {
-  return plan_impl(types, M, N, K, layoutA, layoutB, rung, variant, num_cus, lds_per_cu,
-                   (size_t)GZ_STATIC_SCRATCH_BYTES, plan);
+  return plan_that_fits(types, M, N, K, layoutA, layoutB, rung, variant, num_cus, lds_per_cu, (size_t)GZ_STATIC_SCRATCH_BYTES, plan);
 }
 
 const char* gz_rung_name(int rung) { return (rung >= 0 && rung < GZ_NUM_RUNGS) ? kRungNames[rung] : "auto"; }

@@ -49,12 +49,8 @@ enum { MFMA_CFG_256_W4 = 0, MFMA_CFG_256_W8 = 1, MFMA_CFG_128 = 2, MFMA_CFG_256x
        MFMA_CFG_RING_W8 = 5, MFMA_CFG_RING_128 = 10, MFMA_CFG_64 = 11, MFMA_CFG_32 = 12 };
 enum { MFMA_VARIANT_RING_W4 = 5, MFMA_VARIANT_RING_W8 = 6, MFMA_VARIANT_STREAMK_W4 = 7, MFMA_VARIANT_STREAMK_W8 = 8 };
 
-// the most any kernel of the configuration asks for: the ring kernel keeps five buffers of half a slab each (nine of
-// 128 x 128 tiles where a work-group has a compute unit to itself), a wave that has
-// K slabs to itself two slabs of a 64 x 64 tile or one (padded) of a 32 x 32 tile
-inline int mfma_lds_bytes(const MfmaCfg& c) {
-  if (c.k_waves > 1) return c.k_waves * (c.bm == 64 ? 2 * (c.bm + c.bn) * MFMA_SLAB_BYTES : (c.bm + c.bn) * 160);
-  return c.ring ? (c.bm == 128 ? 9 : 5) * (c.bm + c.bn) * 64 : 2 * (c.bm + c.bn) * MFMA_LDS_PITCH;
+inline int mfma_in_size(int types) {
+  return (types == GZ_S8S8S32 || types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16) ? 1 : types == GZ_F32F32F32 ? 4 : 2;
 }
 
 // How a problem sits on a tile configuration (16-byte alignment of the pointers is the caller's to check):
@@ -81,6 +77,50 @@ inline bool mfma_whole_pieces(int in_size, int M, int N, int K, int layoutA, int
   const int epv = 16 / in_size;
   return (layoutA == GZ_ROW_MAJOR ? K : M) % epv == 0 && (layoutB == GZ_COL_MAJOR ? K : N) % epv == 0;
 }
+// LDS of a compute unit, which is what one work-group may have of it
+constexpr int MFMA_LDS_PER_CU = 160 * 1024;
+// What the launches of 128 x 128 tiles on the ring kernel take: nine buffers of half a slab each where a work-group has a
+// compute unit to itself - from eight slabs on, and where the grid fills most of the device, which the L2s then hold up as
+// much, from 24 - and five otherwise.  (us, five / nine buffers: bf16 1024^3 row/row 12.8 / 11.7, 1408^3 15.7 / 13.6, 1792^3
+// row/col 18.8 / 16.8, 2048^3 row/row 22.6 / 20.7; int8 1024^3 9.0 / 8.7, 1792^3 12.1 / 11.3; 256 tiles of 8 and 16 slabs
+// fp16 10.0 / 10.2, 13.8 / 13.9, int8 row/col 13.5 / 13.8.  Not fp32, which its products bind: 2048^3 121 / 124.)
+inline int mfma_ring128_buffers(int types, long long tiles, long long k_bytes, int num_cus, int lds_per_cu) {
+  const bool deep = types != GZ_F32F32F32 && tiles <= num_cus && k_bytes >= (4 * tiles > 3LL * num_cus ? 24 : 8) * MFMA_SLAB_BYTES;
+  return deep && 9 * (128 + 128) * 64 <= lds_per_cu ? 9 : 5;
+}
+// Slabs on their way to each wave of a 64 x 64 tile whose waves have slabs of their own: two, or where there are more
+// work-groups than compute units one, so that two work-groups fit on one.
+inline int mfma_wavek_stages(long long groups, int num_cus, int lds_per_cu) {
+  return groups <= num_cus && 4 * 2 * (64 + 64) * MFMA_SLAB_BYTES <= lds_per_cu ? 2 : 1;
+}
+// whether a launch of a configuration of the ring kernel runs it; `transposed`: two column-major operands as the transposed
+// problem, which the other arguments then describe
+inline bool mfma_ring_takes(const MfmaCfg& c, int types, int shape_class, int layoutA, int layoutB, bool transposed) {
+  if (!c.ring || shape_class == MFMA_SHAPE_GENERAL) return false;
+  const bool f8 = types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16, f32 = types == GZ_F32F32F32;
+  const bool eight = c.waves_m * c.waves_n == 8;
+  if (f32 ? eight : f8 && (c.bm == 128 || (transposed && eight))) return false;
+  return transposed || layoutA == GZ_ROW_MAJOR || (layoutB == GZ_ROW_MAJOR && !f8 && !f32);
+}
+// LDS per work-group of the kernel that a launch runs (16-byte aligned operands; parts: K parts of a split K)
+inline int mfma_lds_bytes(const MfmaCfg& c, int types, int shape_class, int M, int N, int K, int layoutA, int layoutB, bool transposed,
+                          int parts, int num_cus, int lds_per_cu) {
+  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR, f32 = types == GZ_F32F32F32;
+  const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+  const int rows = c.bm + c.bn;
+  if (c.k_waves > 1) {
+    if (c.bm == 64) return c.k_waves * mfma_wavek_stages(tiles * parts, num_cus, lds_per_cu) * rows * MFMA_SLAB_BYTES;
+    if (mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB)) return c.k_waves * rows * MFMA_SLAB_BYTES;
+    // (through registers: padded rows, fp32 lines along M or N whole with a pad of 32 bytes)
+    const int padded = 32 * MFMA_LDS_PITCH, line = (MFMA_SLAB_BYTES / 4) * (32 * 4 + 32);
+    return c.k_waves * ((f32 && !a_kc ? line : padded) + (f32 && !b_kc ? line : padded));
+  }
+  if (mfma_ring_takes(c, types, shape_class, layoutA, layoutB, transposed))
+    return (c.bm == 128 ? mfma_ring128_buffers(types, tiles, (long long)K * mfma_in_size(types), num_cus, lds_per_cu) : 5) * rows * 64;
+  // whole tiles of a row-major A on the compiler-scheduled direct-to-LDS kernel
+  const bool dtl = shape_class == MFMA_SHAPE_WHOLE && !f32 && a_kc && (b_kc ? c.waves_m * c.waves_n == 8 : c.bm == 128 && c.bn == 128);
+  return 2 * rows * (dtl ? MFMA_SLAB_BYTES : MFMA_LDS_PITCH);
+}
 inline bool mfma_whole_tiles(const MfmaCfg& c, int in_size, int M, int N, int K) {
   return mfma_shape_class(c, in_size, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR) == MFMA_SHAPE_WHOLE;
 }
@@ -106,9 +146,6 @@ inline bool mfma_whole_tiles(const MfmaCfg& c, int in_size, int M, int N, int K)
 // row-major B: four waves), the smaller tiles the register-staged kernel without predication (128x128 with a
 // row-major B: a compiler-scheduled direct-to-LDS kernel with transposing LDS reads); on any other problem the same
 // tile runs the predicated kernel, so choosing them is always safe.
-inline int mfma_in_size(int types) {
-  return (types == GZ_S8S8S32 || types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16) ? 1 : types == GZ_F32F32F32 ? 4 : 2;
-}
 
 // Whether the stores of D carry the non-temporal hint.  Measured in interleaved runs, plain / non-temporal (us):
 // outputs of 64 MiB: bf16 4096 x 4096 x {64, 1024, 4096} 17.9 / 17.5, 43.5 / 42.0, 120.2 / 119.1; several rounds of

@@ -1301,8 +1301,7 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   } while (0)
 #define GZ_LAUNCH_DIRECT(KERN, LDS_BYTES, ...) GZ_LAUNCH_DIRECT_ON(grid, GZ_KERN(KERN), LDS_BYTES, ##__VA_ARGS__)
 #define GZ_KERN(...) __VA_ARGS__   // a template-id with commas as one macro argument
-  // The ring kernel's 128 x 128 tile.  A work-group that has a compute unit to itself takes nine buffers, all of its LDS, and
-  // asks for slabs twice as far ahead.
+  // The ring kernel's 128 x 128 tile (mfma_ring128_buffers: nine buffers ask for slabs twice as far ahead).
 #define GZ_LAUNCH_128(WM_, WN_, ...)                                                                        \
   do {                                                                                                      \
     if constexpr (TYPES != GZ_F32F32F32) {                                                                  \
@@ -1318,12 +1317,9 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
   constexpr bool TILE_256 = BM == 256 && BN == 256 && WAVES_M == 2 && (WAVES_N == 2 || WAVES_N == 4);
   const size_t ring_lds = 5u * (size_t)(BM + BN) * 64;
   const size_t dtl_lds = 2u * (size_t)(BM + BN) * SLAB_BYTES;
-  // From eight slabs on, and where the grid fills most of the device, which the L2s then hold up as much, from 24.  (us, five /
-  // nine buffers: bf16 1024^3 row/row 12.8 / 11.7, 1408^3 15.7 / 13.6, 1792^3 row/col 18.8 / 16.8, 2048^3 row/row 22.6 / 20.7;
-  // int8 1024^3 9.0 / 8.7, 1792^3 12.1 / 11.3; 256 tiles of 8 and 16 slabs fp16 10.0 / 10.2, 13.8 / 13.9, int8 row/col
-  // 13.5 / 13.8.  Not fp32, which its products bind: 2048^3 121 / 124.)
-  const long long grid_tiles = (long long)tiles_m * tiles_n, cus = device_compute_units();
-  const bool deep_ring = grid_tiles <= cus && (long long)g.K * (int)sizeof(typename Traits<TYPES>::in_t) >= (4 * grid_tiles > 3 * cus ? 24 : 8) * SLAB_BYTES;
+  const bool deep_ring = BM == 128 && BN == 128 &&
+                         mfma_ring128_buffers(TYPES, (long long)tiles_m * tiles_n, (long long)g.K * (int)sizeof(typename Traits<TYPES>::in_t),
+                                              device_compute_units(), MFMA_LDS_PER_CU) == 9;
   const size_t deep_lds = 9u * (size_t)(BM + BN) * 64;
   const dim3 pgrid((unsigned)(ring == 1 ? mfma_persistent_grid((long long)tiles_m * tiles_n, device_compute_units())
                                         : (long long)tiles_m * tiles_n));

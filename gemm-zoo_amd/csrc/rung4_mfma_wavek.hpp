@@ -496,16 +496,15 @@ static int launch_wavek_as(const GemmArgs<TYPES>& g, const SplitK& sk, hipStream
   return GZ_OK;
 }
 
-// Tiles of 64 x 64 (four waves, aligned lines) or 32 x 32 (eight).  More 64 x 64 work-groups than compute units: an instance
-// of which two fit on one, with a slab per wave on its way instead of two.
+// Tiles of 64 x 64 (four waves, aligned lines; mfma_wavek_stages) or 32 x 32 (eight).
 template <int TYPES> int launch_wavek(const GemmArgs<TYPES>& g, int tile, const SplitK& sk, hipStream_t s) {
   if (tile == 32)
     return wavek_dma_ok<TYPES>(g) ? launch_wavek_as<TYPES, 32, 32, 8, 1, 2, FEED_DMA>(g, sk, s)
                                   : launch_wavek_as<TYPES, 32, 32, 8, 1, 2, FEED_REG>(g, sk, s);
   if constexpr (TYPES != GZ_F32F32F32) {
     const long long groups = (long long)ceil_div(g.M, 64) * ceil_div(g.N, 64) * sk.parts;
-    return groups > device_compute_units() ? launch_wavek_as<TYPES, 64, 64, 4, 1, 2, FEED_DMA>(g, sk, s)
-                                           : launch_wavek_as<TYPES, 64, 64, 4, 2, 1, FEED_DMA>(g, sk, s);
+    return mfma_wavek_stages(groups, device_compute_units(), MFMA_LDS_PER_CU) == 1 ? launch_wavek_as<TYPES, 64, 64, 4, 1, 2, FEED_DMA>(g, sk, s)
+                                                                                   : launch_wavek_as<TYPES, 64, 64, 4, 2, 1, FEED_DMA>(g, sk, s);
   }
   set_error("mfma rung: no 64 x 64 tile with its K dealt to the waves for this type bundle");
   return GZ_ERR_UNSUPPORTED;

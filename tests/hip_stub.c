@@ -75,8 +75,9 @@ int __hipPushCallConfiguration(dim grid, dim block, size_t lds, void* s) { retur
 int __hipPopCallConfiguration(dim* grid, dim* block, size_t* lds, void** s) { return *grid = grid_, *block = block_, *lds = lds_, *s = stream_, OK; }
 int hipLaunchKernel(const void* f, dim grid, dim block, void** args, size_t lds, void* s) {
   Dl_info info;
-  (void)block; (void)args; (void)lds;
+  (void)args;
   note("launch", (uintptr_t)s, grid.x, dladdr(f, &info) && info.dli_sname ? info.dli_sname : "?");
+  note("group", (uintptr_t)block.x * block.y * block.z, lds, "-");   /* threads and LDS bytes of its work-groups */
   return OK;
 }
 
