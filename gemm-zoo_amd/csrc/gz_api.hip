@@ -239,8 +239,7 @@ bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
   const long long slabs = ((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
   const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
   if (slabs < 4 || tiles > 4LL * num_cus) return false;
-  const double slab_us = mfma_64_slab_us(types, M, N, K, layoutA, layoutB);
-  const bool own_slabs = mfma_64_own_slabs(types, M, N, K, layoutA, layoutB);
+  const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
   // (a large operand that is read once: bf16 50 x 9600 x 8192 in 3 parts 39 us, of which 8 are the two launches)
   const double stream_us = ((double)M + (double)N) * (double)K * mfma_in_size(types) / 5.5e6;
   double best = 0;
@@ -250,9 +249,18 @@ bool mfma_best_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
     if (bytes > MFMA_SPLITK_MAX_BYTES || tiles * p > 8LL * num_cus) break;
     // two launches, the sums written and read back, the slabs of the longest part (us, measured / this line: bf16
     // 24 x 1280 x 11001 in 12 parts 14.4 / 13.7, 100 x 2560 x 12416 in 6 27.6 / 26.7, fp32 512^3 in 4 10.1 / 9.6)
+    const bool own_slabs = mfma_64_own_slabs(types, M, N, K, layoutA, layoutB, p);
+    // (those keep the L2's path to a compute unit busy: e5m2 1192 x 2176 x 7680 in two parts, five to a compute unit, 44.8,
+    // one launch of 128 x 128 tiles 32.4)
+    if (own_slabs && tiles * p > 4LL * num_cus) continue;
+    const double slab_us = mfma_64_slab_us(types, layoutA, layoutB, own_slabs, pieces);
     const double walk = (double)((slabs + p - 1) / p) * slab_us * mfma_64_share(types, own_slabs, (double)(tiles * p) / num_cus);
-    // (slabs of the waves' own: their sums meet in LDS first - e5m2 97 x 3456 x 3328 in 2 parts 11.1 / 10.8)
-    const double t = (own_slabs ? 7.2 : 6.5) + 0.22 * (double)bytes / (1 << 20) + (walk > stream_us ? walk : stream_us);
+    // (slabs of the waves' own: their sums meet in LDS first - e5m2 97 x 3456 x 3328 in 2 parts 11.1 / 10.8; more than eight
+    // parts: the second launch adds them one after the other - measured less this line without that term, 4 - 11 parts -0.6,
+    // 12 - 19 -0.2, 24 - 31 +0.9, 32 +1.8; e4m3 122 x 576 x 14296 in 28 13.9, in 14 10.2, e5m2 546 x 37 x 3104 in 25 9.1, in 13
+    // 7.9)
+    const double fixed = (own_slabs ? 7.2 : 6.5) + (p > 8 ? 0.05 * (p - 8) : 0.0);
+    const double t = fixed + 0.22 * (double)bytes / (1 << 20) + (walk > stream_us ? walk : stream_us);
     if (parts == 0 || t < best) {
       best = t;
       parts = p;
@@ -600,7 +608,7 @@ static int plan_tile(MfmaCfg& c, int types, int shape_class, int m, int n, int k
 
 static int plan_splitk(const SplitKPlan& kp, int types, int m, int n, int k, int layoutA, int layoutB, int num_cus, int lds_per_cu,
                        gz_plan_t* plan) {
-  MfmaCfg c = mfma_64_cfg(types, m, n, k, layoutA, layoutB);
+  MfmaCfg c = mfma_64_cfg(types, m, n, k, layoutA, layoutB, kp.parts);
   plan->split_k = kp.parts;
   plan->grid = (int64_t)ceil_div(m, c.bm) * ceil_div(n, c.bn) * kp.parts;
   plan->workspace_bytes = kp.workspace_bytes;

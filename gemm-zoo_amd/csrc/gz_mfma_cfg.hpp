@@ -37,7 +37,7 @@ static const MfmaCfg kMfmaCfgs[] = {
     {10, 256, 256, 2, 4, 2, false},  // variant 6, the same
     {11, 128, 128, 2, 2, 2, false},  // tile of variant 3 on the ring kernel, two work-groups per compute unit
     {12, 64, 64, 1, 1, 0, false, 4},   // grids that 128x128 tiles leave mostly empty: four waves, each the whole tile over its own slabs
-                                       // (unaligned lines and fp32: kMfmaCfg64Staged)
+                                       // (unaligned lines, a short K and fp32: kMfmaCfg64Staged)
     {13, 32, 32, 1, 1, 0, false, 8},   // grids that 64x64 tiles leave mostly empty: eight waves, the same
 };
 constexpr int kNumMfmaCfgs = (int)(sizeof(kMfmaCfgs) / sizeof(kMfmaCfgs[0]));
@@ -164,24 +164,37 @@ inline int mfma_store_hint(int types, long long M, long long N, long long K, int
 }
 
 // ---- the small tiles ----
-// whether a 64 x 64 tile runs on the kernel whose waves have slabs of their own (mfma_wavek_kernel) or on the register-staged one
-inline bool mfma_64_own_slabs(int types, int M, int N, int K, int layoutA, int layoutB) {
-  return types != GZ_F32F32F32 && mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
+// Whether a 64 x 64 tile runs on the kernel whose waves have slabs of their own (mfma_wavek_kernel) or on the register-staged
+// one.  The four waves' sums meet in LDS at the end, 1 us that the slabs have to earn back, the sooner the more transposing
+// stores the staged kernel has: own slabs / staged, both states of the caches, geometric means over 1600 problems of up to
+// 512 tiles. 16 bits: row/col, up to 8 slabs 1.05 - 1.22, 9 - 14 1.02 - 1.08, 15 - 24 0.91 - 1.01, more 0.72 - 1.0; row/row
+// up to 6 0.99 - 1.12, 7 - 10 0.94 - 1.0, more 0.62 - 0.93; column-major A, row-major B up to 6 0.91 - 1.06, more 0.52 -
+// 0.93; both column-major up to 8 1.01 - 1.19, more 0.62 - 0.99.  8 bits: row/col up to 10 0.97 - 1.17, 11 - 14 0.98 -
+// 1.05, 15 - 24 0.87 - 0.98, more 0.72 - 0.99; the others one slab 0.98 - 1.09, more 0.5 - 0.98.  The parts of a split K,
+// whose sums go to the workspace either way: row/col 1 - 7 slabs 1.0 - 1.09, more 0.93 - 1.0; the others one slab 1.01 -
+// 1.09, two 0.97 - 1.03, more 0.77 - 0.99.
+inline bool mfma_64_own_slabs(int types, int M, int N, int K, int layoutA, int layoutB, int parts = 1) {
+  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR, wide = mfma_in_size(types) == 2;
+  const long long slabs = ((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES / parts;
+  const int from = parts > 1 ? (a_kc && b_kc ? 8 : wide ? 3 : 2) : a_kc && b_kc ? 15 : !wide ? 2 : !a_kc && b_kc ? 9 : 7;
+  return types != GZ_F32F32F32 && slabs >= from && mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
 }
-inline MfmaCfg mfma_64_cfg(int types, int M, int N, int K, int layoutA, int layoutB) {
-  if (mfma_64_own_slabs(types, M, N, K, layoutA, layoutB)) return kMfmaCfgs[MFMA_CFG_64];
+inline MfmaCfg mfma_64_cfg(int types, int M, int N, int K, int layoutA, int layoutB, int parts = 1) {
+  if (mfma_64_own_slabs(types, M, N, K, layoutA, layoutB, parts)) return kMfmaCfgs[MFMA_CFG_64];
   return mfma_in_size(types) == 1 ? kMfmaCfg64StagedInt8 : kMfmaCfg64Staged;
 }
 // us per 128-byte slab of a 64 x 64 tile whose work-group has a compute unit to itself.  Register-staged (measured over
 // 20 ... 880 tiles and 7 ... 194 slabs): what a layout costs is its transposing stores (row-major B, column-major A), and
 // 8-bit rows that are not whole 16-byte pieces are loaded from unaligned addresses.  Slabs of the waves' own (64 ... 256
 // tiles, 16 ... 64 slabs): what comes in through the L2, lines of 64 bytes where 8-bit elements lie along M or N.
-inline double mfma_64_slab_us(int types, int M, int N, int K, int layoutA, int layoutB) {
+inline double mfma_64_slab_us(int types, int layoutA, int layoutB, bool own_slabs, bool pieces) {
   const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR;
   if (types == GZ_F32F32F32) return 0.54;
-  const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
-  if (pieces) return mfma_in_size(types) == 2 ? 0.235 : a_kc && b_kc ? 0.22 : a_kc != b_kc ? 0.27 : 0.31;
-  if (mfma_in_size(types) == 1) return a_kc && b_kc ? 0.50 : a_kc != b_kc ? 0.70 : 0.74;
+  if (own_slabs) return mfma_in_size(types) == 2 ? 0.235 : a_kc && b_kc ? 0.22 : a_kc != b_kc ? 0.27 : 0.31;
+  if (mfma_in_size(types) == 1) {
+    if (a_kc && b_kc) return pieces ? 0.40 : 0.50;
+    return a_kc != b_kc ? (pieces ? 0.56 : 0.70) : 0.74;
+  }
   return a_kc && b_kc ? 0.42 : a_kc ? 0.48 : b_kc ? 0.40 : 0.60;
 }
 // How much longer a slab takes with w work-groups per compute unit.  fp32 is bound by its matrix rate: the compute unit
@@ -204,8 +217,9 @@ inline double mfma_64_us(int types, int M, int N, int K, int layoutA, int layout
   const double slabs = (double)(((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES);
   const bool own_slabs = mfma_64_own_slabs(types, M, N, K, layoutA, layoutB);
   const double w = (double)((M + 63) / 64) * (double)((N + 63) / 64) / num_cus;
-  const double fixed = own_slabs ? (slabs < 8 ? 3.3 + 0.2 * slabs : 4.9) : types == GZ_F32F32F32 ? 3.0 : 2.6;
-  return fixed + slabs * mfma_64_slab_us(types, M, N, K, layoutA, layoutB) * mfma_64_share(types, own_slabs, w);
+  const double fixed = own_slabs ? 4.9 : types == GZ_F32F32F32 ? 3.0 : 2.6;
+  const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
+  return fixed + slabs * mfma_64_slab_us(types, layoutA, layoutB, own_slabs, pieces) * mfma_64_share(types, own_slabs, w);
 }
 // ... and of 32 x 32 tiles.  8- and 16-bit types: a slab of every tile of a compute unit in turn, 0.095 us through copies
 // (lines of 64 and of 32 bytes, elements along M or N: more), 0.28 (0.36 for 8 bits) through registers, and the operands
@@ -265,9 +279,12 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
           best = cost32;
           pick = MFMA_CFG_32;
         }
-      } else if (!staged_64 && mfma_64_own_slabs(types, M, N, K, layoutA, layoutB)) {
-        // slabs of the waves' own: up to two tiles per compute unit (bf16 row/row 1280^3, 1.56, 12.9 against 14.8 on 128 x
-        // 128, 1536^3, 2.25, 19.5 / 16.8; int8 9.8 / 10.1, 15.1 / 11.1; column-major A, 736 x 1792 x 2227 18.9 / 22.3)
+      } else if (!staged_64 && (mfma_64_own_slabs(types, M, N, K, layoutA, layoutB) ||
+                                (!(a_rows && b_cols) && mfma_whole_pieces(in_size, M, N, K, layoutA, layoutB)))) {
+        // slabs of the waves' own, or so short a K that the staged kernel's are as cheap (mfma_64_own_slabs; int8 row/row
+        // 1152 x 1280 x 128 staged / 128 x 128 4.7 / 5.9, bf16 880 x 1904 x 128 5.4 / 7.2): up to two tiles per compute
+        // unit (bf16 row/row 1280^3, 1.56, 12.9 against 14.8 on 128 x 128, 1536^3, 2.25, 19.5 / 16.8; int8 9.8 / 10.1, 15.1
+        // / 11.1; column-major A, 736 x 1792 x 2227 18.9 / 22.3)
         if (tiles <= 2LL * num_cus)
           cost64 = mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) / (16.0 + 1.45 * ((double)K * in_size / MFMA_SLAB_BYTES));
       } else if (tiles * 5 <= (b_cols || f8_types ? 10LL : 6LL) * num_cus) {
@@ -757,7 +774,7 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
 
 // Split K on 64 x 64 tiles: a grid that leaves most of the device empty, or waiting for a single long column of slabs per
 // compute unit, is cut along K as well; the parts' 32-bit sums meet in a workspace and a second launch adds them in
-// their order.  Any shape, layout and alignment (the register-staged kernel).
+// their order.  Any shape, layout and alignment, each part on the kernel that mfma_64_own_slabs says.
 struct SplitKPlan {
   int parts, q, rem;           // K parts; slabs per part, the first rem parts one more
   long long workspace_bytes;   // parts x tiles x 16 KiB of 32-bit sums

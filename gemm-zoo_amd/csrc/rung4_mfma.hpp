@@ -16,8 +16,8 @@
 //                      makes the fragment reads of 16 consecutive rows hit 16 distinct 4-bank groups);
 //                      operands whose contiguous dimension is not K (row-major B, column-major A) are
 //                      transposed in registers on the way in.  Tiles 256x256, 256x128, 128x128 and, for
-//                      grids that those leave mostly empty, 64x64 (unaligned lines, and fp32).
-//   mfma_wavek_kernel  (rung4_mfma_wavek.hpp) 64x64 tiles of aligned lines and 32x32 tiles, K dealt to the waves.
+//                      grids that those leave mostly empty, 64x64 (unaligned lines, a short K, and fp32).
+//   mfma_wavek_kernel  (rung4_mfma_wavek.hpp) 64x64 tiles of aligned lines and a longer K and 32x32 tiles, K dealt to the waves.
 //   mfma_dtl_kernel    compiler-scheduled fast path for whole tiles with 16-byte aligned rows: slabs go
 //                      global -> LDS directly (global_load_lds_dwordx4), unpadded swizzled rows.
 //   mfma_ring16_kernel (rung4_mfma_ring16.hpp) the hand-scheduled kernel with the 16x16 matrix instructions
@@ -1434,14 +1434,12 @@ static int launch_cfg(const GemmArgs<TYPES>& g, int shape_class, int ring, hipSt
 #undef GZ_LAUNCH_DIRECT
 #undef GZ_LAUNCH_DIRECT_ON
 #undef GZ_KERN
-  // (64 x 64 tiles of 8 and 16 bits come here with unaligned lines only: mfma_wavek_kernel has the others)
-  constexpr bool EDGE_ONLY = BM == 64 && TYPES != GZ_F32F32F32;
-  if (edge || EDGE_ONLY) {
+  if (edge) {
     if (akc && bkc) GZ_LAUNCH(true, true, true);
     else if (akc && !bkc) GZ_LAUNCH(true, false, true);
     else if (!akc && bkc) GZ_LAUNCH(false, true, true);
     else GZ_LAUNCH(false, false, true);
-  } else if constexpr (!EDGE_ONLY) {
+  } else {
     if (akc && bkc) GZ_LAUNCH(true, true, false);
     else if (akc && !bkc) GZ_LAUNCH(true, false, false);
     else if (!akc && bkc) GZ_LAUNCH(false, true, false);
@@ -1655,7 +1653,9 @@ template <int TYPES> static bool wavek_dma_ok(const GemmArgs<TYPES>& g) {
          mfma_whole_pieces(ES, g.M, g.N, g.K, g.layoutA, g.layoutB) && g.lda * ES * 256 < (1LL << 32) && g.ldb * ES * 256 < (1LL << 32);
 }
 // ... and a 64 x 64 tile of them runs on mfma_wavek_kernel
-template <int TYPES> static bool wavek_64(const GemmArgs<TYPES>& g) { return TYPES != GZ_F32F32F32 && wavek_dma_ok<TYPES>(g); }
+template <int TYPES> static bool wavek_64(const GemmArgs<TYPES>& g, int parts = 1) {
+  return mfma_64_own_slabs(TYPES, g.M, g.N, g.K, g.layoutA, g.layoutB, parts) && wavek_dma_ok<TYPES>(g);
+}
 
 template <int TYPES> static int launch_one(const GemmArgs<TYPES>& g, const MfmaCfg& chosen, hipStream_t s, bool adjust = false,
                                            bool transposed = false) {
@@ -1706,7 +1706,7 @@ template <int TYPES> int launch_splitk(const GemmArgs<TYPES>& g, const SplitKPla
     hipLaunchKernelGGL(kern, grid, block, lds, s, g, tiles_m, tiles_n, sk);                      \
   } while (0)
     const bool akc = g.layoutA == GZ_ROW_MAJOR, bkc = g.layoutB == GZ_COL_MAJOR;
-    if (wavek_64<TYPES>(g)) {
+    if (wavek_64<TYPES>(g, p.parts)) {
       if (const int st = launch_wavek<TYPES>(g, 64, sk, s); st != GZ_OK) return st;
     } else if (akc && bkc) GZ_LAUNCH_SPLIT(true, true);
     else if (akc) GZ_LAUNCH_SPLIT(true, false);

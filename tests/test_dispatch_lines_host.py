@@ -1,0 +1,32 @@
+"""Where the launcher's lines between the small tiles, the larger ones, split K, stream-K and the streaming kernels lie: problems
+timed on both sides (us beside them), which a line drawn elsewhere had made slower."""
+import pytest
+
+S8, BF16F32, BF16, F16, F32, E4M3, E5M2 = range(7)
+
+
+def kind(p, capi):
+    if p.streamk_tiles:
+        return "stream-K"
+    if p.split_k > 1 and p.tile_m == 64:
+        return "split K"
+    if p.rung == capi.RUNG_SKINNY and p.variant == 1:
+        return "stream"
+    if (p.tile_m, p.tile_n) == (64, 64):   # four waves of the whole tile each, or the register-staged kernel
+        return "64 own slabs" if (p.wave_m, p.wave_n, p.threads) == (64, 64, 256) else "64 staged"
+    return p.tile_m
+
+
+@pytest.mark.parametrize("types,m,n,k,la,lb,want", [
+    # 64 x 64 tiles: slabs of the waves' own from as many as earn the sums in LDS back (own slabs / staged)
+    (BF16F32, 896, 1408, 128, 0, 1, "64 staged"),        # 5.3 / 4.3
+    (BF16F32, 816, 1296, 64, 0, 1, "64 staged"),         # 6.0 / 4.5
+    (BF16, 1152, 1280, 128, 0, 1, "64 staged"),          # 5.3 / 4.3
+    (E4M3, 960, 960, 960, 0, 1, "64 staged"),            # 6.9 / 5.9
+    (S8, 1024, 1024, 1024, 0, 0, "64 own slabs"),        # 6.3 / 7.2
+    (BF16F32, 1024, 1024, 1024, 0, 0, "64 own slabs"),
+    (S8, 1024, 1024, 2048, 0, 1, "64 own slabs"),
+])
+def test_line(capi, types, m, n, k, la, lb, want):
+    p = capi.plan(types, m, n, k, la, lb)
+    assert p.tile_m <= 64 if want == "small" else kind(p, capi) == want, (kind(p, capi), p.as_dict())

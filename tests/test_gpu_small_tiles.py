@@ -1,6 +1,7 @@
-"""The small tiles whose waves share out K (variants 12 and 13): every number of slabs around a full set of stages, slabs that
-the end of K cuts, rows and columns around the edges of a tile and of a 16-byte piece, aligned and unaligned lines (two
-ways into LDS).  Exact inputs, so a slab or a piece lost, counted twice or not zeroed shows."""
+"""The small tiles (variants 12 and 13): 32 x 32 and, from a longer K on, 64 x 64 tiles whose waves share out K, and the
+register-staged 64 x 64 ones.  Every number of slabs around a full set of stages, slabs that the end of K cuts, rows and columns
+around the edges of a tile and of a 16-byte piece, aligned and unaligned lines (two ways into LDS).  Exact inputs, so a slab or
+a piece lost, counted twice or not zeroed shows."""
 import itertools
 
 import numpy as np
@@ -38,12 +39,36 @@ def test_slabs_edges_and_alignment(G, types, la, lb):
         assert np.array_equal(got, O.gemm(types, a, b, c, m, n, k, la, lb, 1, beta)), (types, la, lb, variant, m, n, k, beta, misalign)
 
 
+@pytest.mark.parametrize("la,lb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("types", (O.S8S8S32, O.BF16BF16F32, O.F16F16F16, O.E5M2E5M2F16))
+def test_64x64_tiles_with_slabs_of_the_waves_own(G, types, la, lb):
+    """A K long enough for the kernel whose four waves have slabs of their own: every number of slabs around full sets of its
+    stages, cut last slabs, rows and columns past the edges, rows of D that are no whole vectors; one work-group per compute
+    unit (two slabs on their way to each wave) and more (one)."""
+    es = np.dtype(O.IN_DTYPE[types]).itemsize
+    slab, piece = 128 // es, 16 // es
+    kind = O.FILL_INT8_UNIFORM if types == O.S8S8S32 else O.FILL_SMALL_INT
+    cases = [(64, 128, (17 + i) * slab) for i in range(9)] + [(96, 64 + piece, 17 * slab + piece), (128, 80, 25 * slab - piece)]
+    # (lines along M and N in whole pieces; otherwise any)
+    cases += [(64 + (1 if la == 0 else piece), 64 + (5 if lb == 1 else piece), 20 * slab + piece), (1088, 1024, 25 * slab)]
+    for (m, n, k), beta in itertools.product(cases, (0, 1)):
+        p = G.capi.plan(types, m, n, k, la, lb, MFMA, 12)
+        assert (p.wave_m, p.wave_n, p.threads) == (64, 64, 256), "slabs of the waves' own"
+        if m > 1000 and beta:
+            continue
+        a, b, c = O.make_inputs(types, m, n, k, kind=kind, seed=k + m)
+        print("case", types, la, lb, m, n, k, beta, p.lds_bytes, flush=True)
+        got = G.run_gemm(types, a, b, c, m, n, k, la, lb, 1, beta, MFMA, 12)
+        assert np.array_equal(got, O.gemm(types, a, b, c, m, n, k, la, lb, 1, beta)), (types, la, lb, m, n, k, beta)
+
+
 @pytest.mark.parametrize("variant", (12, 13))
 @pytest.mark.parametrize("la,lb", [(0, 1), (1, 0)])
 def test_an_infinity_beside_the_end_of_k(G, variant, la, lb):
     """A slab that the end of K cuts holds repeated elements there until they are zeroed, on both operands."""
-    types, m, n, k = O.BF16BF16F32, 64, 64, 2 * 64 + 8
-    a, b, _ = O.make_inputs(types, m, n, k, kind=O.FILL_UNIFORM_PM1, seed=4)
-    a.reshape(-1)[5 * k + k - 1 if la == 0 else (k - 1) * m + 5] = 0x7F80
-    got = G.run_gemm(types, a, b, None, m, n, k, la, lb, 1, 0, MFMA, variant).astype(np.float64)
-    assert np.isinf(got[5]).all() and np.isfinite(np.delete(got, 5, axis=0)).all()
+    types, m, n = O.BF16BF16F32, 64, 64
+    for k in (2 * 64 + 8, 20 * 64 + 8):
+        a, b, _ = O.make_inputs(types, m, n, k, kind=O.FILL_UNIFORM_PM1, seed=4)
+        a.reshape(-1)[5 * k + k - 1 if la == 0 else (k - 1) * m + 5] = 0x7F80
+        got = G.run_gemm(types, a, b, None, m, n, k, la, lb, 1, 0, MFMA, variant).astype(np.float64)
+        assert np.isinf(got[5]).all() and np.isfinite(np.delete(got, 5, axis=0)).all()
