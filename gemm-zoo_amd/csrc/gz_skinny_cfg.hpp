@@ -235,25 +235,31 @@ inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned l
   const int es = skinny_rung_types(types) ? 2 : 1;
   const int stages = (int)(((long long)K * es + STREAM_TILE_ROW_BYTES - 1) / STREAM_TILE_ROW_BYTES);
   if (num_cus <= 0) num_cus = 256;
-  if (M > 64 && stages <= skinny_tiles_max_stages(c.cols_per_wg, c.grid_n <= num_cus))
-    return 2LL * ((N + 63) / 64) <= 3LL * num_cus ? SKINNY_TILES_64 : SKINNY_TILES;
+  // 32 x 32 tiles whose waves share out K, one launch.  Up to one tile per compute unit, and up to 1.75, or 32 rows, while K is
+  // not so long that the tile kernel's spreading of the weights over all compute units, or a split K, outweighs its share of A
+  // from memory (us, 32 x 32 / tile kernel / split K, operands just used; from memory: bf16 78 x 1024 x 2048 4.7 / 12.3 / 8.5;
+  // 5.7 / 13.4 / 8.9, 100 x 2100 x 1136 6.3 / 9.0 / 9.7; 7.0 / 10.0 / 10.2, 36 x 7296 x 7168 24.8 / 29.3 / 21.5; 30.6 / 29.5 /
+  // 26.2, int8 46 x 5632 x 10944 18.9 / 27.8 / 18.2; 29.1 / 28.6 / 24.3, e4m3 32 x 4096 x 11648 14.2 / 17.2 / -).
+  const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
+  const double small_us = mfma_32_us(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus);
   const double stream_us = skinny_tile_estimate_us(stages, c.mb, c.cols_per_wg);
+  // (the rows of a short K below: 64 x 64 tiles that leave compute units idle are the slower ones - int8 65 x 1024 x 512
+  // 3.4 / 2.8, bf16 70 x 2762 x 192 4.5 / 3.3)
+  if (M > 64 && stages <= skinny_tiles_max_stages(c.cols_per_wg, c.grid_n <= num_cus)) {
+    if (4 * tiles32 <= 3LL * num_cus && small_us < mfma_64_us(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus)) return SKINNY_TILES_32;
+    return 2LL * ((N + 63) / 64) <= 3LL * num_cus ? SKINNY_TILES_64 : SKINNY_TILES;
+  }
+  // (65 rows and more, rows of D that are not whole 16-byte pieces and a last stage that the end of K cuts: the tile kernel
+  // up to 24 stages.  The figures are against it (bf16 70 x 1029 x 1136 8.3 / 4.5 on 32 x 32 tiles, 128 x 2100 x 1176 10.2
+  // / 6.4): a test alone holds it, which takes this kernel's cut stages for such problems.)
+  if (M > 64 && stages < 24 && N % 8 != 0 && (long long)K * es % STREAM_TILE_ROW_BYTES != 0) return SKINNY_STREAM;
   const bool split_ok = mfma_best_splitk(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus, split) &&
                         (unsigned long long)split->workspace_bytes <= ws_limit;
-  // Few columns: 32 x 32 tiles whose waves share out K, one launch (us, 32 x 32 / tile kernel or split K, whichever was
-  // taken: int8 75 x 1536 x 5376 6.5 / 10.8, 53 x 1408 x 5632 6.6 / 9.7, 106 x 1280 x 5376 6.5 / 9.9, 26 x 2560 x 7200 9.6 / 10.0,
-  // 46 x 1952 x 11648 10.6 / 12.3; bf16 the same)
-  // (Up to 32 rows and a long K the tile kernel spreads the weights over all compute units, which from memory outweighs its
-  // share of A: 32 x 4096 x 11648 14.2 / 17.2.  65 rows and more whose last stage the end of K cuts stay with the tile
-  // kernel, which zeroes it beside its copies.)
-  const bool cut_stage = M > 64 && (long long)K * es % STREAM_TILE_ROW_BYTES != 0;
-  if (cut_stage && stages < 24) return SKINNY_STREAM;
-  if ((long long)((M + 31) / 32) * ((N + 31) / 32) <= num_cus && !cut_stage && (M > 32 || stages <= 48)) {
-    const double small_us = mfma_32_us(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus);
-    if (small_us < 0.9 * stream_us && (!split_ok || small_us < split->estimate_us)) return SKINNY_TILES_32;
-  }
-  // (0.85: e5m2 97 x 3456 x 3328 tile kernel / split K 10.0 / 11.1, estimated 12.3 / 10.8)
-  if (split_ok && split->estimate_us < 0.85 * stream_us) return SKINNY_TILES_SPLITK;
+  if (((M > 32 && tiles32 <= num_cus) || (4 * tiles32 <= 7LL * num_cus && stages <= 48)) && small_us < stream_us &&
+      (!split_ok || small_us < split->estimate_us))
+    return SKINNY_TILES_32;
+  // (0.9: bf16 30 x 1280 x 4224 tile kernel / split K 10.9 / 8.4, 36 x 7296 x 7168 above; e5m2 97 x 3456 x 3328 10.0 / 11.1)
+  if (split_ok && split->estimate_us < 0.9 * stream_us) return SKINNY_TILES_SPLITK;
   return SKINNY_STREAM;
 }
 

@@ -26,7 +26,24 @@ def kind(p, capi):
     (S8, 1024, 1024, 1024, 0, 0, "64 own slabs"),        # 6.3 / 7.2
     (BF16F32, 1024, 1024, 1024, 0, 0, "64 own slabs"),
     (S8, 1024, 1024, 2048, 0, 1, "64 own slabs"),
+    # decode, 65 rows and more with a short K: 32 x 32 tiles instead of 64 x 64 that leave compute units idle
+    (E4M3, 113, 857, 640, 0, 1, 32),                     # 7.8 on 64 x 64 own slabs, 5.6 staged, 3.3
+    (BF16, 69, 314, 384, 0, 1, 32),                      # 8.0, 5.2, 3.4
+    (BF16F32, 96, 1024, 128, 0, 1, 32),                  # 4.1, 3.3, 2.8
+    # ... with a last stage that the end of K cuts
+    (BF16, 124, 768, 1424, 0, 1, 32),                    # 13.0 on the tile kernel
+    (E4M3, 112, 128, 2784, 0, 1, 32),                    # 8.8
+    # few rows and a long K: in parts, or 32 x 32 tiles, not the tile kernel
+    (BF16F32, 30, 1280, 4224, 0, 1, "split K"),          # 10.9 on the tile kernel, 8.4
+    (BF16F32, 36, 7296, 7168, 0, 1, "split K"),          # 29.3 on the tile kernel, 21.5
+    (F16, 56, 7168, 8472, 0, 1, "split K"),              # 41.7 on the tile kernel, 27.8
 ])
 def test_line(capi, types, m, n, k, la, lb, want):
     p = capi.plan(types, m, n, k, la, lb)
     assert p.tile_m <= 64 if want == "small" else kind(p, capi) == want, (kind(p, capi), p.as_dict())
+
+
+def test_short_parts_of_a_split_k_run_on_the_staged_kernel(capi):
+    short, long = capi.plan(BF16F32, 62, 256, 8320, 0, 1), capi.plan(BF16F32, 36, 7296, 7168, 0, 1)
+    assert short.split_k > 1 and short.wave_m == 32      # 9.2 us staged, 10.2 on slabs of the waves' own
+    assert long.split_k > 1 and long.wave_m == 64
