@@ -212,12 +212,14 @@ inline double mfma_64_share(int types, bool own_slabs, double w) {
   // slab and not 0.5)
   return 0.5 * (line(w) + line(whole));
 }
-// us of an unsplit launch of 64 x 64 tiles (bf16 row/row cubes 256, 512, 1024, 1280: 4.6, 5.9, 8.7, 12.9)
+// us of an unsplit launch of 64 x 64 tiles (bf16 row/row cubes 256, 512, 1024, 1280: 4.6, 5.9, 8.7, 12.9; fp32, measured / this
+// line: 1472^3 76 / 80, 1984^3 147 / 140, 2176^3 200 / 190, 2837 x 1834 x 540 65.6 / 61)
 inline double mfma_64_us(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
   const double slabs = (double)(((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES);
   const bool own_slabs = mfma_64_own_slabs(types, M, N, K, layoutA, layoutB);
   const double w = (double)((M + 63) / 64) * (double)((N + 63) / 64) / num_cus;
-  const double fixed = own_slabs ? 4.9 : types == GZ_F32F32F32 ? 3.0 : 2.6;
+  if (types == GZ_F32F32F32) return 2.6 + (0.5 + 0.545 * slabs) * mfma_64_share(types, false, w < 1.0 ? 1.0 : w);
+  const double fixed = own_slabs ? 4.9 : 2.6;
   const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
   return fixed + slabs * mfma_64_slab_us(types, layoutA, layoutB, own_slabs, pieces) * mfma_64_share(types, own_slabs, w);
 }
@@ -225,18 +227,31 @@ inline double mfma_64_us(int types, int M, int N, int K, int layoutA, int layout
 // (lines of 64 and of 32 bytes, elements along M or N: more), 0.28 (0.36 for 8 bits) through registers, and the operands
 // from memory once (us, this line / measured: bf16 row/row 512^3 3.6 / 3.7, 512^2 x 8192 19.2 / 19.3, row/col 512^2 x 2048
 // 5.6 / 5.9, 256 x 1024 x 4096 8.7 / 8.6, 300 x 1408^2 6.8 / 7.3, column-major A 640 x 1024 x 4096 27.6 / 27.8; int8 145 x
-// 1664 x 8192 row/row 25.0 / 25.6; unaligned 291^3 4.0 / 4.0, 330 x 1047 x 833 9.9 / 7.6).  fp32: by products, 0.145 us a slab and tile (0.20 through registers), the compute unit
-// with the most tiles decides (256^3 4.1 / 3.9, 512^3 5.2 / 5.6, 1024^3 21.5 / 22.3, 1536^3 65.5 / 66.6).
+// 1664 x 8192 row/row 25.0 / 25.6; unaligned 291^3 4.0 / 4.0, 330 x 1047 x 833 9.9 / 7.6).
+// fp32: by products, 0.145 us a slab of the first tile and 1.1 + 0.122 of the next (0.20 and 1.1 + 0.165 through
+// registers), the compute unit with the most tiles decides (256^3 4.1 / 3.9, 512^3 5.2 / 5.6, 1024^3 22.6 / 21.9, 1984^3
+// 142 / 138, 2352^3 222 / 232).
 inline double mfma_32_us(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
   const double slabs = (double)(((long long)K * mfma_in_size(types) + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES);
   const long long tiles = (long long)((M + 31) / 32) * ((N + 31) / 32);
   const bool pieces = mfma_whole_pieces(mfma_in_size(types), M, N, K, layoutA, layoutB);
-  if (types == GZ_F32F32F32) return 2.9 + slabs * (pieces ? 0.145 : 0.20) * (double)((tiles + num_cus - 1) / num_cus);
+  if (types == GZ_F32F32F32)
+    return 2.9 + slabs * (pieces ? 0.145 : 0.20) + (1.1 + slabs * (pieces ? 0.122 : 0.165)) * (double)((tiles - 1) / num_cus);
   const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR, wide = mfma_in_size(types) == 2;
   const double slab_us = !pieces ? (wide ? 0.28 : 0.36) : a_kc && b_kc ? 0.095 : a_kc != b_kc ? (wide ? 0.125 : 0.175) : (wide ? 0.13 : 0.235);
   const double walk = slabs * slab_us * (double)((tiles + num_cus - 1) / num_cus);
   const double stream = ((double)M + (double)N) * (double)K * mfma_in_size(types) / 5.0e6;
   return 2.6 + (walk > stream ? walk : stream);
+}
+
+// ... and fp32 on the larger tiles (candidate 0: 256 x 256, 1: 256 x 128, 2: 128 x 128; direct: the ring kernel), `rounds` of
+// them on the compute unit that has the most (us, measured / this line: 128 x 128 446^3 34.7 / 35.1, 1984^3 116 / 118,
+// 2160^3, 289 tiles, 245 / 245, 2352^3, 361, 267 / 266; staged 1963^3 136 / 135, 1600 x 2457 x 1024, 260, 137 / 139; 256 x
+// 128 1984^3 233 / 232; 256 x 256 440 / 439)
+inline double mfma_f32_large_tile_us(int candidate, bool direct, long long k_bytes, long long rounds) {
+  const double slabs = (double)((k_bytes + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES);
+  if (candidate == 2) return (direct ? 11.0 : 8.5) + slabs * (direct ? 1.72 : 2.04) * (double)rounds;
+  return 11.0 + slabs * (candidate == 0 ? 6.9 : 3.56) * (double)rounds;
 }
 
 // The launcher's own choice for one launch over the whole problem; returns the estimate it was chosen by.
@@ -258,6 +273,11 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
                        ring128_ok ? MFMA_CFG_RING_128 : MFMA_CFG_128, MFMA_CFG_64};
   double best = 0;
   int pick = cand[0];
+  // fp32 on up to one and a half 128 x 128 tiles per compute unit: every tile by its time in us, which the products of the
+  // compute unit with the most tiles decide (0.77: the larger grids' estimates, which the row and column cuts weigh these
+  // against, are that much short of their times)
+  constexpr double F32_SMALL_GRID_UNIT = 0.77;
+  const bool f32_small_grid = types == GZ_F32F32F32 && 2LL * ((M + 127) / 128) * ((N + 127) / 128) <= 3LL * num_cus;
   for (int i = 0; i < 4; i++) {
     const MfmaCfg& c = kMfmaCfgs[cand[i]];
     const long long tiles = (long long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
@@ -266,16 +286,12 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // tiles leave mostly empty.  8-bit elements on two waves.
       double cost64 = -1.0;
       if (types == GZ_F32F32F32) {
-        // A 128 x 128 tile is 55 us of fp32 products per 1024 of K on one compute unit, whatever the grid (us, 32 x 32 /
-        // 64 x 64 / 128 x 128 tiles, cubes, row/row: 256 3.9 / 7.5 / 19, 512 5.6 / 12.4 / 33, 1024 22.3 / 22.7 / 62, 1088
-        // 27.5 / 39.7 / 64, 1280 42.7 / 45.4 / 75, 1536 66.6 / 79.5 / 89, 2048 - / 141 / 119).
-        // (0.77: what the estimate of the larger tiles is short of their times up to 2048^3)
-        // Past four tiles per compute unit a sixteenth of a round of 256 x 256 per tile at 0.75 of the larger tiles' rate.
+        // Past what f32_small_grid takes, a sixteenth of a round of 256 x 256 per tile at 0.75 of the larger tiles' rate.
         const double round_us = 16.0 + 1.45 * ((double)K * in_size / MFMA_SLAB_BYTES);
-        if (tiles > 4LL * num_cus) cost64 = (0.05 + 1.35 * (double)tiles / (16.0 * num_cus)) * 2.2;
-        else cost64 = 0.77 * mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) / round_us;
-        const double cost32 = 0.77 * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus) / round_us;
-        if (tiles <= 4LL * num_cus && cost32 < cost64 && cost32 < best) {
+        if (!f32_small_grid) cost64 = (0.05 + 1.35 * (double)tiles / (16.0 * num_cus)) * 2.2;
+        else cost64 = F32_SMALL_GRID_UNIT * mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) / round_us;
+        const double cost32 = F32_SMALL_GRID_UNIT * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus) / round_us;
+        if (f32_small_grid && cost32 < cost64 && cost32 < best) {
           best = cost32;
           pick = MFMA_CFG_32;
         }
@@ -426,8 +442,10 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
     const bool f8 = types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16;
     const double staged = f32 ? 2.2 : i == 2 ? 1.05 + 0.05 * (rounds > 4 ? rounds - 4 : 0)
                                     : f8 ? 1.3 + 1000.0 / (double)(K > 0 ? K : 1) : 1.2;
-    const double cost = f32 ? shape_cost * (direct ? 0.95 * 2.2 : 2.2)
-                            : shape_cost * rowb * (direct || fitted128 ? 1.0 : staged);
+    double cost = f32 ? shape_cost * (direct ? 0.95 * 2.2 : 2.2)
+                      : shape_cost * rowb * (direct || fitted128 ? 1.0 : staged);
+    if (f32_small_grid)
+      cost = F32_SMALL_GRID_UNIT * mfma_f32_large_tile_us(i, direct, (long long)K * in_size, rounds) / (16.0 + 1.45 * ((double)K * in_size / MFMA_SLAB_BYTES));
     if (i == 0 || cost < best) {
       best = cost;
       pick = cand[i];

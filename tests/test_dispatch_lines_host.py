@@ -37,6 +37,12 @@ def kind(p, capi):
     (BF16F32, 30, 1280, 4224, 0, 1, "split K"),          # 10.9 on the tile kernel, 8.4
     (BF16F32, 36, 7296, 7168, 0, 1, "split K"),          # 29.3 on the tile kernel, 21.5
     (F16, 56, 7168, 8472, 0, 1, "split K"),              # 41.7 on the tile kernel, 27.8
+    # fp32: a 128 x 128 tile's products take the compute unit that has two of them twice as long
+    (F32, 2112, 2112, 2112, 0, 0, "small"),              # 238 on 128 x 128, 186 on 64 x 64
+    (F32, 2240, 2240, 2240, 0, 1, "small"),              # 250, 207, 196 on 32 x 32
+    (F32, 1600, 2457, 1024, 0, 0, "small"),              # 137 on 128 x 128 staged, 78 on 64 x 64
+    (F32, 1938, 2092, 1999, 0, 0, "small"),              # 262, 152
+    (F32, 2048, 2048, 2048, 0, 0, 128),                  # 120, 138 on 64 x 64
 ])
 def test_line(capi, types, m, n, k, la, lb, want):
     p = capi.plan(types, m, n, k, la, lb)
