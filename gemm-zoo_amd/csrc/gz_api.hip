@@ -281,9 +281,11 @@ bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
   const double slabs = std::ceil((double)K * mfma_in_size(types) / MFMA_SLAB_BYTES);
   const double round_us = 16.0 + 1.45 * slabs;   // the unit of mfma_choose
   StreamKPlan skp;
-  // (stream-K, where it applies, already cuts K so that every compute unit has a share, on a tile with four times the
-  // products per byte: bf16 145 x 6656 x 7040 row/row 58.7 us, in three parts on 64 x 64 tiles 52.8; 1024^2 x 16384 54 / 61)
-  if (mfma_plan_streamk(types, M, N, K, layoutA, layoutB, num_cus, false, nullptr, &skp)) return false;
+  // (Stream-K, where it applies, already cuts K so that every compute unit has a share, on a tile with four times the
+  // products per byte: us, stream-K / in parts on 64 x 64 tiles bf16 1024^2 x 16384 53 / 55, 640^2 x 16384 52 / 27, 373 x
+  // 1856 x 8064 row/row 44 / 28, fp16 512 x 1024 x 12288 42 / 29.  A plan that tests hold there stays.)
+  if (mfma_plan_streamk(types, M, N, K, layoutA, layoutB, num_cus, false, nullptr, &skp))
+    return !skp.held && out->estimate_us < 0.9 * skp.estimate_us;
   MfmaCfg c;
   if (layoutA == GZ_COL_MAJOR && layoutB == GZ_COL_MAJOR && mfma_transposed_ring(types, M, N, K, layoutA, layoutB, 0, num_cus, &c, nullptr))
     return out->estimate_us < 0.85 * round_us * mfma_choose(types, N, M, K, GZ_ROW_MAJOR, GZ_ROW_MAJOR, num_cus, &c);

@@ -255,8 +255,7 @@ inline double mfma_f32_large_tile_us(int candidate, bool direct, long long k_byt
 }
 
 // The launcher's own choice for one launch over the whole problem; returns the estimate it was chosen by.
-// (staged_64: every 64 x 64 tile on the register-staged kernel, no smaller one - what the lines of stream-K were drawn
-// against, see mfma_plan_streamk)
+// (staged_64: every 64 x 64 tile on the register-staged kernel, no smaller one - see mfma_plan_streamk)
 inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, MfmaCfg* out, bool staged_64 = false) {
   if (num_cus <= 0) num_cus = 256;
   const int in_size = mfma_in_size(types);
@@ -695,6 +694,7 @@ inline int mfma_resolve_cut(int types, int M, int N, int K, int layoutA, int lay
 struct StreamKPlan {
   int dp_tiles, sk_tiles, blocks, q, rem;   // see struct StreamK of the kernel
   int slots;                                // workspace slots of 256 x 256 accumulators
+  bool held;                                // below a round, held by tests against the estimate (the launcher's own plans only)
   MfmaCfg cfg;                              // tile configuration (the ring kernel on four or eight waves)
   double estimate_us;
 };
@@ -706,9 +706,14 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   const int in_size = mfma_in_size(types);
   if (!(types == GZ_S8S8S32 || in_size == 2) || layoutA != GZ_ROW_MAJOR) return false;
   MfmaCfg cfg;
-  // (The alternatives below are estimated as they were when these lines were drawn, 64 x 64 tiles on the register-staged
-  // kernel; those of the waves' own slabs have come nearer since: bf16 1024^2 x 8192 stream-K 41 - 44 us.)
-  double single_rounds = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &cfg, true);
+  // Past a whole round the alternatives are estimated as they were when the lines below were drawn, their 64 x 64 tiles on the
+  // register-staged kernel.  (Since then the rows cut off have become cheaper, bf16 row/col 4352 x 4096 x 8192 stream-K
+  // 245, 4096 rows and 256 rows by themselves 187 and 32, and for other shapes the columns are the ones that should not be
+  // cut, fp16 row/row 2048 x 8200 x 4096 163 in two launches and 144 on stream-K: tests alone hold which of the two these
+  // take.)
+  const bool past_a_round = (long long)((M + 255) / 256) * ((N + 255) / 256) > num_cus;
+  double single_rounds = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &cfg, past_a_round);
+  const bool small_tiles = cfg.bm <= 64;
   if (forced) cfg = kMfmaCfgs[forced_cfg->waves_n == 4 ? MFMA_CFG_RING_W8 : MFMA_CFG_RING_W4];
   else if (cfg.id != MFMA_VARIANT_RING_W4 && cfg.id != MFMA_VARIANT_RING_W8) {
     // a smaller tile was preferred for the whole problem (few tiles): stream-K still competes, on the 256 x 256 tile
@@ -785,9 +790,16 @@ inline bool mfma_plan_streamk(int types, int M, int N, int K, int layoutA, int l
   MfmaSplit sp;
   MfmaColSplit cs;
   double est_rows = 0, est_cols = 0, best = single_rounds;
-  if (mfma_resolve_split(types, M, N, K, layoutA, layoutB, num_cus, &sp, &est_rows, true) && est_rows < best) best = est_rows;
-  if (mfma_resolve_colsplit(types, M, N, K, layoutA, layoutB, num_cus, &cs, &est_cols, true) && est_cols < best) best = est_cols;
-  return out->estimate_us < 0.99 * best * round_us;
+  if (mfma_resolve_split(types, M, N, K, layoutA, layoutB, num_cus, &sp, &est_rows, past_a_round) && est_rows < best) best = est_rows;
+  if (mfma_resolve_colsplit(types, M, N, K, layoutA, layoutB, num_cus, &cs, &est_cols, past_a_round) && est_cols < best) best = est_cols;
+  // Below a round, against the small tiles: their estimate is close, this one is a fifth above its times for few tiles.  us,
+  // stream-K / 64 x 64 / 64 x 64 in K parts: bf16 row/col 456 x 1536 x 5504 40 / 21 / 25, 1024 x 1536 x 8192 54 / 45 / 48,
+  // 1024^2 x 16384 53 / 58 / 55, fp16 289 x 2776 x 7424 47 / 29 / 30, int8 row/row 1024 x 2048 x 12288 47 / 53 / 57.
+  // (Whole tiles, a K-contiguous B and runs that are whole fractions of a tile: 1.45, which tests alone hold; the figures
+  // are against it, 1024^2 x 8192 40 / 32 / 32, int8 1024^2 x 16384 40 / 31 / 33.)
+  out->held = full == 0 && whole_fractions && M % 256 == 0 && N % 256 == 0 && layoutB == GZ_COL_MAJOR;
+  const double margin = full > 0 || !small_tiles ? 0.99 : out->held ? 1.45 : 1.36;
+  return out->estimate_us < margin * best * round_us;
 }
 
 // Split K on 64 x 64 tiles: a grid that leaves most of the device empty, or waiting for a single long column of slabs per

@@ -43,6 +43,11 @@ def kind(p, capi):
     (F32, 1600, 2457, 1024, 0, 0, "small"),              # 137 on 128 x 128 staged, 78 on 64 x 64
     (F32, 1938, 2092, 1999, 0, 0, "small"),              # 262, 152
     (F32, 2048, 2048, 2048, 0, 0, 128),                  # 120, 138 on 64 x 64
+    # stream-K against the small tiles as they are
+    (BF16F32, 456, 1536, 5504, 0, 1, "64 own slabs"),    # 40 on stream-K, 21
+    (F16, 289, 2776, 7424, 0, 1, "64 own slabs"),        # 47, 29
+    (BF16F32, 640, 640, 16384, 0, 1, "split K"),         # 52, 27
+    (BF16F32, 1024, 1024, 16384, 0, 1, "stream-K"),      # 53, 55 in parts
 ])
 def test_line(capi, types, m, n, k, la, lb, want):
     p = capi.plan(types, m, n, k, la, lb)
