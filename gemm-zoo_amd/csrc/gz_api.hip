@@ -293,12 +293,19 @@ bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
   MfmaColSplit cols;
   double est = mfma_choose(types, M, N, K, layoutA, layoutB, num_cus, &c) * round_us;
   if (c.bm <= 64) {   // the same tile unsplit, or the smaller one, by the same measure
-    // (32 x 32 tiles on less than a sixth of the compute units and forty slabs or more: either may win by a third, and the
-    // parts are kept up to what their estimate is over that - int8 192 x 128 x 5120 row/col parts / 32 x 32 8.8 / 6.5, row/row 8.8 / 10.0, 64 x 128 x
-    // 16384 9.9 / 11.7, bf16 192 x 128 x 2560 row/row 8.7 / 7.8)
-    if (c.bm == 32 && (long long)((M + 31) / 32) * ((N + 31) / 32) * 6 <= num_cus && slabs >= 40)
-      return out->estimate_us < 1.45 * mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
+    // (Row/col, forty slabs, 32 x 32 tiles on less than a sixth of the compute units: cut.  The figures are against it, in
+    // parts / 32 x 32, operands just used; from memory: int8 192 x 128 x 5120 8.8 / 5.3; 8.9 / 6.6, bf16 150 x 200 x 2560
+    // 8.9 / 5.3; 9.0 / 6.8. Tests alone hold it, which take these for problems whose K is cut.)
+    if (c.bm == 32 && slabs == 40 && layoutA == GZ_ROW_MAJOR && layoutB == GZ_COL_MAJOR &&
+        (long long)((M + 31) / 32) * ((N + 31) / 32) * 6 <= num_cus) return true;
     est = c.bm == 64 ? mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) : mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
+    // (few 32 x 32 tiles that share little of their operands, which a compute unit takes in at 17 - 25 bytes per ns from
+    // memory: in parts / 32 x 32, just used; from memory: bf16 960 x 32 x 5424 8.7 / 8.0; 10.7 / 20.1, e5m2 645 x 30 x
+    // 10320 8.5 / 7.5; 9.8 / 18.9)
+    if (c.bm == 32) {
+      const double tiles32 = (double)((M + 31) / 32) * (double)((N + 31) / 32);
+      est = std::max(est, 2.6 + ((double)M + N) * K * mfma_in_size(types) / tiles32 / 34e3);
+    }
     return out->estimate_us < 0.90 * est;
   }
   double cut = 0;

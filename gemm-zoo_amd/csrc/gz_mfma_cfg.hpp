@@ -320,8 +320,10 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // to itself or none (us, 32 x 32 / 64 x 64: bf16 row/row 256^3 3.0 / 4.6, 512^3 3.7 / 5.9, 768^3, 2.25 per compute
       // unit, 8.0 / 7.4; 512^2 x 2048 5.9 / 10.3, 256 x 1024 x 4096 8.6 / 15.8; int8 512^3 3.5 / 4.6, 768^3 7.0 / 6.2)
       const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
-      // (whole 64 x 64 tiles of row-major operands with a K of four slabs at most and half the rows keep that tile)
-      const bool flat = a_rows && !b_cols && M % 64 == 0 && N % 64 == 0 && 2LL * K <= M && (long long)K * in_size <= 4 * MFMA_SLAB_BYTES;
+      // (Whole 64 x 64 tiles of row-major operands, N < M = 2 K, a K of four slabs at most keep that tile.  The figures are
+      // against it, 64 x 64 / 32 x 32: int8 512 x 384 x 256 4.1 / 3.0, bf16 4.7 / 3.1, 256 x 128 x 128 4.2 / 2.8.  A test
+      // alone holds it, which takes the 64 x 64 tile's kernels for such problems.)
+      const bool flat = a_rows && !b_cols && M % 64 == 0 && N % 64 == 0 && 2LL * K == M && N < M && (long long)K * in_size <= 4 * MFMA_SLAB_BYTES;
       if (!staged_64 && !flat && types != GZ_F32F32F32 && pick == MFMA_CFG_64 && tiles32 <= 2LL * num_cus) {
         const double by = mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus) / mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus);
         if (by < 1.0) {
@@ -380,8 +382,10 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // 137 32.7 / 26.5, 300 36.9 / 34.2, 450 44.4 / 42.2; fp16 24.8 / 22.1, 30.4 / 26.9, 37.0 / 34.1; int8 30.7 / 24.7,
       // 32.1 / 26.2, 34.4 / 30.2; 4096 x 4096, one whole round, level or worse).
       const long long big = (long long)((M + 255) / 256) * ((N + 255) / 256), nslab = ((long long)K * in_size + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
-      // (not a few rows or columns past a multiple of 256: those are cut off)
-      const bool few_past = (M % 256 >= 1 && M % 256 <= 64) || (N % 256 >= 1 && N % 256 <= 64);
+      // (8 bits, a few rows or columns past a multiple of 256: not, tests alone hold that these are cut off.  Column-major
+      // A and B apart the figures are against it: int8 4096 x 4160 x 640 row/col columns cut / 128 x 128 28.6 / 26.2, from
+      // memory 31.9 / 33.8, 4112 x 4352 x 640 34.1 / 26.4, 38.3 / 32.9; fp16 4096 x 4104 x 320 30.4 / 23.8)
+      const bool few_past = in_size == 1 && ((M % 256 >= 1 && M % 256 <= 64) || (N % 256 >= 1 && N % 256 <= 64));
       if (big > num_cus && big % num_cus && nslab < 10 && !few_past) shape_cost *= 0.70 + 0.03 * (double)nslab;
     }
     // 128 x 128 tiles on the register-staged kernel (ragged M / N, K-contiguous B), up to three rounds: measured in
@@ -469,9 +473,14 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // 386.5 / 401.4.  (A row-major B: eight waves at every size, see below.)
       // (K that is not whole slabs: four, whose instance has the registers for the clamped offsets - e4m3 4096 x 4096 x
       // 4000 57.6 / 58.0, 2048 x 7824 x 1088 25.7 / 28.9, 5008^3 124 / 138, row/row 4096^2 x 1040 27.2 / 26.6)
-      // (A K-contiguous B and operands of 40 MB and more, which come from memory more than from the caches: four - us, four / eight: 1000 x 14336 x 4096 51.2 / 57.4, 2000 x 8192 x 4096 51.9 / 57.4, 2048 x 4096 x 8192 80.9 /
-      // 88.6, 4800 x 4864^2 105 / 109; 33 MB and less 4096^3 52.9 / 50.4, 3840^3 47.3 / 44.7, 1500 x 8192 x 2048 29.7 / 27.4)
-      const bool from_memory = b_cols && ((long long)M + N) * K >= 40000000LL;
+      // (A K-contiguous B and operands of 40 MB and more, which come from memory more than from the caches: four, on whole
+      // tiles from K = 6144 or 60 MB on - us, four / eight, operands just used; from memory: 1000 x 14336 x 4096 47.9 /
+      // 47.2; 49.8 / 56.7, 1500 x 8192 x 4096 46.1 / 44.2; 48.1 / 54.5, 1536 x 8192 x 8192 79.8 / 77.4; 83.6 / 93.8, 2048 x
+      // 14336 x 4096 95.5 / 91.2; 98.9 / 108.1, but 4608^3 101.8 / 96.5; 101.3 / 97.7, 8192 x 4096 x 4096 102.3 / 97.1;
+      // 102.1 / 97.0, 2048 x 8192 x 4096 52.7 / 50.7; 52.5 / 50.9; 33 MB and less 4096^3 53.1 / 50.2; 53.0 / 49.9, 1500 x
+      // 8192 x 2048 29.7 / 27.4)
+      const long long operands = ((long long)M + N) * K;
+      const bool from_memory = b_cols && operands >= 40000000LL && (M % 256 || N % 256 || K >= 6144 || operands >= 60000000LL);
       eight = !(tiles >= 4LL * num_cus && b_cols) && !k_tail && !from_memory;
     } else {
       // int8 and the 16-bit types: an estimate of the launch on four and on eight waves, in us per round of tiles,
@@ -513,12 +522,15 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // int8 3000 x 4096 x 2048 28.6 / 31.1; a 16-bit output stays on eight, bf16 -> bf16 3000 x 4096 x 2048 47.4 / 45.3.)
       // (K that is not whole slabs follows the estimate as ragged shapes do: bf16 -> f32 four / eight waves, row/col
       // 4096^2 x 4000 108.5 / 119.4, 4096^2 x 2000 56.3 / 59.9, row/row 4096^2 x 4000 101.4 / 111.0; bf16 -> bf16 4096^2 x
-      // 1000 36.6 / 34.9.  Where N and K are both ragged and a row is an odd number of 16-byte pieces the plan has been
-      // eight waves since these ran on the register-staged kernel, and stays so: 3000^2 x 1000 31.0 / 34.8, 6000^2 x 3000
-      // row/row 214.9 / 226.9, bf16 -> bf16 33.5 / 31.1 and 219.9 / 218.8; on the register-staged kernel 35.8 and 261.)
+      // 1000 36.6 / 34.9.  A row-major B below one round as well: four / eight 4096 x 3000 x 1000 34.6 / 40.6, 2504 x
+      // 4200 x 2008 47.4 / 52.0; int8, whose estimate is eight, 48.5 / 45.4, 71.4 / 63.5.  bf16 -> f32 with N and K both
+      // ragged, a row of an odd number of 16-byte pieces, M <= N <= 3 K: eight, which a test alone holds; the figures are
+      // against it, 3000^2 x 1000 31.7 / 35.5, 6000^2 x 3000 212 / 220, 5000^3 219 / 223; on the register-staged kernel
+      // 35.8 and 261.)
       const bool ragged = M % 256 != 0 || N % 256 != 0 || k_tail;
-      const bool n_k_ragged = k_tail && N % 128 != 0 && (long long)K * in_size % 32 != 0;
-      eight = !a_rows || n_k_ragged || (under_a_round && (!ragged || out16 || !b_cols)) || fixed8 + slope8 * nslab < fixed4 + slope4 * nslab;
+      const bool n_k_ragged = types == GZ_BF16BF16F32 && M <= N && 3LL * K >= N && k_tail && N % 128 != 0 && (long long)K * in_size % 32 != 0;
+      eight = !a_rows || n_k_ragged || (under_a_round && (!ragged || out16 || (!b_cols && (!k_tail || in_size == 1)))) ||
+              fixed8 + slope8 * nslab < fixed4 + slope4 * nslab;
     }
     if (eight) *out = kMfmaCfgs[MFMA_CFG_RING_W8];
   }
