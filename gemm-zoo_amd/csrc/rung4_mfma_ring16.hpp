@@ -1,8 +1,8 @@
-// MFMA rung, whole-line ring of five LDS buffers with the 16x16 matrix instructions.
+// MFMA rung, whole-line ring of five LDS buffers (nine of a lone 128 x 128 tile) with the 16x16 matrix instructions.
 //
 // Data movement: every copy asks the L2 for whole 128-byte lines (8 rows x 128 bytes of K per instruction), so a K
 // slab (128 bytes of K per row) is cut by ROWS into two copy groups; a group fills one of five 32 KiB buffers (all of
-// the LDS), one barrier per slab.  Arithmetic:
+// the LDS; of 128 x 128 tiles one of five or nine of 16 KiB), one barrier per slab.  Arithmetic:
 //     v_mfma_f32_16x16x32_{bf16,f16}   v_mfma_i32_16x16x64_i8   v_mfma_f32_16x16x128_f8f6f4
 // rather than the 32x32 forms.  A 16x16 instruction sums 64 bytes of K per row inside the matrix pipe before it
 // touches the accumulators, a 32x32 one 32 bytes, so the same product costs half the accumulator reads and writes -
@@ -153,7 +153,7 @@ template <int ES, int ROW_BYTES> __host__ __device__ constexpr int ring16_row_sw
 template <int TYPES, int BM, int BN, int WAVES_M, int WAVES_N, bool RAGGED = false, bool STREAMK = false, bool B_KC = true,
           bool SWAP = false, bool A_KC = true, int NST = 5>
 // (second launch bound: waves per SIMD the registers must leave room for - the 128 x 128 tile, whose five buffers are
-// half the LDS, runs two work-groups per compute unit)
+// half the LDS, runs two work-groups per compute unit; with nine, one)
 __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128 && NST == 5) ? 2 : (WAVES_M * WAVES_N) / 4)
     mfma_ring16_kernel(GemmArgs<TYPES> g, int tiles_m, int tiles_n, StreamK sk) {
   using T = Traits<TYPES>;
@@ -681,13 +681,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
       issue_group(std::integral_constant<int, 2 + decltype(c)::value>{}, a_tile - a_back, b_tile - b_back);
     });
     asm volatile("s_waitcnt vmcnt(%0)" : : "i"((2 * AHEAD - 2) * NCP) : "memory");
-  } else if (AHEAD > 2 && nc > 2) {   // (a short run: whatever there is, and all of it)
-    static_for<2 * AHEAD - 4>([&](auto c) {
-      constexpr int C = 2 + decltype(c)::value;
-      if (C < nc) issue_group(std::integral_constant<int, C>{}, a_tile - a_back, b_tile - b_back);
-    });
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
+  } else {   // (a run of one slab; nine buffers are launched from eight slabs on)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   if constexpr (RAGGED && !STREAMK) {
@@ -707,8 +701,8 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     static_for<NRD>([&](auto r) { read_one(I0{}, r, I0{}); });
   }
 
-  // ---- one slab; JR = j % 5 at compile time.  Slab j fetches slab j + AHEAD (groups 2j + 4 and 2j + 5 of five buffers) from a_cp / b_cp,
-  // or, where the run has no such slab, its last slab again ----
+  // ---- one slab; JR = j % NST at compile time.  Slab j fetches slab j + AHEAD (with five buffers groups 2j + 4 and 2j + 5)
+  // from a_cp / b_cp, or, where the run has no such slab, its last slab again ----
   const int nslab = nc / 2;
   const int first_fetch = min(AHEAD, nslab - 1);
   const char* a_cp = a_group(a_tile, 2 * first_fetch) - a_back;
@@ -723,8 +717,7 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     const char* const a_cp1 = A_KC ? a_cp : a_cp + a_group_step;
     if constexpr (F8) half_f8(I0{}, jr_c, ST4{}, a_cp, b_cp);
     else kstep(I0{}, jr_c, I0{}, ST4{}, a_cp, b_cp);
-    // the copies of group 2j+4 (of nine buffers 2j+4 ... 2j+8) may stay in flight; a run shorter than what the prologue
-    // asks for has been waited for altogether
+    // the copies of group 2j+4 (of nine buffers 2j+4 ... 2j+8) may stay in flight
     if (j + 2 < nslab) {
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "i"((2 * AHEAD - 3) * NCP) : "memory");
     } else {

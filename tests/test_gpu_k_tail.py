@@ -40,6 +40,42 @@ def test_every_tail_is_counted_once(G, types, la, lb):
         assert np.array_equal(got, O.gemm(types, a, b, c, m, n, k, la, lb, 1, 1)), (types, la, lb, variant, m, n, k)
 
 
+@pytest.mark.parametrize("la,lb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("types", (O.S8S8S32, O.BF16BF16F32, O.F16F16F16))
+def test_nine_buffers_and_a_tail(G, types, la, lb):
+    """128 x 128 tiles that have a compute unit to themselves, from eight whole slabs on: the ring of nine buffers, one turn of
+    it and two, whole and ragged M and N."""
+    es = np.dtype(O.IN_DTYPE[types]).itemsize
+    slab, piece = 128 // es, 16 // es
+    tails = [0, piece, slab - piece] + ([] if la == 0 or lb == 1 else [1, slab // 2 + 1])
+    for whole, tail, (m, n) in itertools.product((8, 9, 10, 17, 18), tails, ((256, 128), (144, 272))):
+        k = whole * slab + tail
+        p = G.capi.plan(types, m, n, k, la, lb, MFMA, 11)
+        assert p.lds_bytes == 9 * 256 * 64, "nine buffers"
+        a, b, c = O.make_inputs(types, m, n, k, kind=exact_kind(types), seed=k)
+        print("case", types, la, lb, m, n, k, flush=True)
+        got = G.run_gemm(types, a, b, c, m, n, k, la, lb, 1, 1, MFMA, 11)
+        assert np.array_equal(got, O.gemm(types, a, b, c, m, n, k, la, lb, 1, 1)), (types, la, lb, m, n, k)
+
+
+@pytest.mark.parametrize("variant", (5, 6))
+@pytest.mark.parametrize("types", TYPES)
+def test_a_tail_where_work_groups_walk_several_tiles(G, types, variant):
+    """288 tiles of 256 x 256: the first slab of the next tile is asked for before the current one is stored, and is cut when it
+    has landed.  First rows, rows of second tiles and the last rows."""
+    es = np.dtype(O.IN_DTYPE[types]).itemsize
+    m, n = 4360, 4096
+    for k, lb in ((128 // es + 16 // es, 1), (3 * (128 // es) - 16 // es, 0)):
+        a, b, c = O.make_inputs(types, m, n, k, kind=exact_kind(types), seed=k)
+        print("case", types, variant, m, n, k, lb, flush=True)
+        got = G.run_gemm(types, a, b, c, m, n, k, 0, lb, 2, 1, MFMA, variant)
+        for rows in ((0, 8), (2040, 2056), (4096 - 4, 4096 + 4), (m - 8, m)):
+            ref = O.gemm(types, a, b, c, m, n, k, 0, lb, 2, 1, rows=rows)
+            assert np.array_equal(got[rows[0]:rows[1]], ref[rows[0]:rows[1]]), (types, variant, k, lb, rows)
+        one = G.run_gemm(types, a, b, c, m, n, k, 0, lb, 2, 1, MFMA, variant + 4)
+        assert np.array_equal(got, one)
+
+
 @pytest.mark.parametrize("types,inf", [(O.BF16BF16F32, 0x7F80), (O.F32F32F32, np.inf)])
 @pytest.mark.parametrize("la,lb", [(0, 1), (1, 0)])
 def test_an_infinity_in_the_overlap_stays_one(G, types, inf, la, lb):
