@@ -647,13 +647,13 @@ __global__ void __launch_bounds__(WAVES_M* WAVES_N * 64, (BM == 128 && BN == 128
     const int head = SK - tail_back;
     int l = 0;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "+v"(l));
-    const uint32_t at = lds_base + (uint32_t)(wave * A_PW * 1024) + (uint32_t)(l * 16);
-    auto clear = [](uint32_t at, auto offset) {
-      constexpr int OFFSET = decltype(offset)::value;
+    // (a lane's 16 bytes word by word, eight lanes further in another order: 16 bytes apart they would meet in 8 banks)
+    uint32_t at = lds_base + (uint32_t)(wave * A_PW * 1024) + (uint32_t)(l * 16 + ((l >> 1) & 12));
+    auto clear = [](uint32_t& at, auto offset) {
       asm volatile(
-          "ds_write_b32 %0, %1 offset:%2\n\tds_write_b32 %0, %1 offset:%3\n\t"
-          "ds_write_b32 %0, %1 offset:%4\n\tds_write_b32 %0, %1 offset:%5"
-          : : "v"(at), "v"(0), "i"(OFFSET), "i"(OFFSET + 4), "i"(OFFSET + 8), "i"(OFFSET + 12) : "memory");
+          "ds_write_b32 %0, %1 offset:%2\n\tv_xor_b32 %0, 4, %0\n\tds_write_b32 %0, %1 offset:%2\n\tv_xor_b32 %0, 8, %0\n\t"
+          "ds_write_b32 %0, %1 offset:%2\n\tv_xor_b32 %0, 4, %0\n\tds_write_b32 %0, %1 offset:%2\n\tv_xor_b32 %0, 8, %0"
+          : "+v"(at) : "v"(0), "i"(decltype(offset)::value) : "memory");
     };
     auto operand = [&](auto kc_c, auto base_c, int row) {
       static_for<2 * A_PW>([&](auto i_c) {
