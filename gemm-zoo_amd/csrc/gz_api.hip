@@ -298,14 +298,8 @@ bool mfma_plan_splitk(int types, int M, int N, int K, int layoutA, int layoutB, 
     // 8.9 / 5.3; 9.0 / 6.8. Tests alone hold it, which take these for problems whose K is cut.)
     if (c.bm == 32 && slabs == 40 && layoutA == GZ_ROW_MAJOR && layoutB == GZ_COL_MAJOR &&
         (long long)((M + 31) / 32) * ((N + 31) / 32) * 6 <= num_cus) return true;
-    est = c.bm == 64 ? mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) : mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
-    // (few 32 x 32 tiles that share little of their operands, which a compute unit takes in at 17 - 25 bytes per ns from
-    // memory: in parts / 32 x 32, just used; from memory: bf16 960 x 32 x 5424 8.7 / 8.0; 10.7 / 20.1, e5m2 645 x 30 x
-    // 10320 8.5 / 7.5; 9.8 / 18.9)
-    if (c.bm == 32) {
-      const double tiles32 = (double)((M + 31) / 32) * (double)((N + 31) / 32);
-      est = std::max(est, 2.6 + ((double)M + N) * K * mfma_in_size(types) / tiles32 / 34e3);
-    }
+    est = c.bm == 64 ? mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus)
+                     : mfma_32_not_in_parts_us(types, M, N, K, layoutA, layoutB, num_cus);
     return out->estimate_us < 0.90 * est;
   }
   double cut = 0;

@@ -244,6 +244,23 @@ inline double mfma_32_us(int types, int M, int N, int K, int layoutA, int layout
   return 2.6 + (walk > stream ? walk : stream);
 }
 
+// ... and of those where the alternative is K in parts on fewer, larger tiles.  Rows that do not begin on whole 64 bytes (lines of
+// a column-major A: 128) ask the L2 for more lines than they hold.  A round that is more than half full waits for that
+// (measured / mfma_32_us, geometric means of operands just used and from memory, row/col: 1.03 on whole lines, 1.34 on
+// others; bf16 in parts / 32 x 32 89 x 1856 x 7632 15.7 / 17.5; 18.5 / 23.9, but 37 x 2248 x 5088, rows of 79.5 lines, 11.0 / 7.9;
+// 13.6 / 13.1), and so do a few that share little, 17 - 25 bytes per ns to a compute unit from memory (bf16 960 x 32 x 5424
+// 8.7 / 8.0; 10.7 / 20.1, e5m2 645 x 30 x 10320 8.5 / 7.5; 9.8 / 18.9).
+inline double mfma_32_not_in_parts_us(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
+  const long long es = mfma_in_size(types), tiles = (long long)((M + 31) / 32) * ((N + 31) / 32);
+  const bool a_kc = layoutA == GZ_ROW_MAJOR, b_kc = layoutB == GZ_COL_MAJOR;
+  const double us = mfma_32_us(types, M, N, K, layoutA, layoutB, num_cus);
+  const bool cut_lines = ((a_kc || b_kc) && K * es % 64) || (!a_kc && M * es % MFMA_SLAB_BYTES);
+  if (types == GZ_F32F32F32 || !cut_lines || !mfma_whole_pieces((int)es, M, N, K, layoutA, layoutB)) return us;
+  const double busy = 2 * ((tiles - 1) % num_cus + 1) > num_cus ? 2.6 + 1.25 * (us - 2.6) : us;
+  const double alone = 2.6 + ((double)M + N) * (double)K * (double)es / (double)tiles / 34e3;
+  return busy > alone ? busy : alone;
+}
+
 // ... and fp32 on the larger tiles (candidate 0: 256 x 256, 1: 256 x 128, 2: 128 x 128; direct: the ring kernel), `rounds` of
 // them on the compute unit that has the most (us, measured / this line: 128 x 128 446^3 34.7 / 35.1, 1984^3 116 / 118,
 // 2160^3, 289 tiles, 245 / 245, 2352^3, 361, 267 / 266; staged 1963^3 136 / 135, 1600 x 2457 x 1024, 260, 137 / 139; 256 x

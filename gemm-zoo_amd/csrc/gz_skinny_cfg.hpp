@@ -255,12 +255,12 @@ inline int skinny_choose(int types, int M, int N, int K, int num_cus, unsigned l
   if (M > 64 && stages < 24 && N % 8 != 0 && (long long)K * es % STREAM_TILE_ROW_BYTES != 0) return SKINNY_STREAM;
   const bool split_ok = mfma_best_splitk(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus, split) &&
                         (unsigned long long)split->workspace_bytes <= ws_limit;
-  if (((M > 32 && tiles32 <= num_cus) || (4 * tiles32 <= 7LL * num_cus && stages <= 48)) && small_us < stream_us &&
-      (!split_ok || small_us < split->estimate_us))
+  const bool small = ((M > 32 && tiles32 <= num_cus) || (4 * tiles32 <= 7LL * num_cus && stages <= 48)) && small_us < stream_us;
+  if (small && (!split_ok || mfma_32_not_in_parts_us(types, M, N, K, GZ_ROW_MAJOR, GZ_COL_MAJOR, num_cus) < split->estimate_us))
     return SKINNY_TILES_32;
   // (0.9: bf16 30 x 1280 x 4224 tile kernel / split K 10.9 / 8.4, 36 x 7296 x 7168 above; e5m2 97 x 3456 x 3328 10.0 / 11.1)
   if (split_ok && split->estimate_us < 0.9 * stream_us) return SKINNY_TILES_SPLITK;
-  return SKINNY_STREAM;
+  return small ? SKINNY_TILES_32 : SKINNY_STREAM;
 }
 
 }  // namespace gz

@@ -37,6 +37,10 @@ def kind(p, capi):
     (BF16F32, 30, 1280, 4224, 0, 1, "split K"),          # 10.9 on the tile kernel, 8.4
     (BF16F32, 36, 7296, 7168, 0, 1, "split K"),          # 29.3 on the tile kernel, 21.5
     (F16, 56, 7168, 8472, 0, 1, "split K"),              # 41.7 on the tile kernel, 27.8
+    # 32 x 32 tiles of rows that begin inside a line (from memory: rows of whole and half lines)
+    (BF16F32, 89, 1856, 7632, 0, 1, "split K"),          # 23.9 on 32 x 32 tiles, 18.5
+    (BF16F32, 37, 2248, 5088, 0, 1, 32),                 # 13.1, 13.6 in parts
+    (BF16, 960, 32, 5424, 0, 1, "split K"),              # 20.1 on 32 x 32 tiles, 10.7
     # fp32: a 128 x 128 tile's products take the compute unit that has two of them twice as long
     (F32, 2112, 2112, 2112, 0, 0, "small"),              # 238 on 128 x 128, 186 on 64 x 64
     (F32, 2240, 2240, 2240, 0, 1, "small"),              # 250, 207, 196 on 32 x 32
