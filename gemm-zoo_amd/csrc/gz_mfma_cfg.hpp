@@ -271,6 +271,22 @@ inline double mfma_f32_large_tile_us(int candidate, bool direct, long long k_byt
   return 11.0 + slabs * (candidate == 0 ? 6.9 : 3.56) * (double)rounds;
 }
 
+// A K that is not whole slabs and so short that the ring kernel, whose first two slabs overlap, does not earn its start: the
+// register-staged kernel (ring / staged, geometric means of operands just used and from memory, each on the better number of
+// waves).  Up to two slabs: the same tile bf16 row/col 256 x 256 1.12, row/row 1.10, 128 x 128 0.98, 1.05, int8 row/col 1.08 and
+// 1.14, row/row 0.99 and 1.04; column-major A, row-major B 0.93 - 1.01, these stay.  8-bit floats, 256 x 256 on the ring against
+// 128 x 128: up to two slabs 1.08 - 1.40; past a round with a last one less than half full 3 slabs 1.02 - 1.28, 4 1.02 - 1.25, 6
+// 1.03 - 1.07 (e5m2 6736 x 6944 x 160 44 / 37 us).
+inline bool mfma_short_k_tail(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus) {
+  const long long k_bytes = (long long)K * mfma_in_size(types), slabs = (k_bytes + MFMA_SLAB_BYTES - 1) / MFMA_SLAB_BYTES;
+  if (k_bytes % MFMA_SLAB_BYTES == 0) return false;
+  if (types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16) {
+    const long long tiles = (long long)((M + 255) / 256) * ((N + 255) / 256), last = tiles % num_cus;
+    return slabs <= 2 || (slabs <= 6 && tiles > num_cus && last > 0 && 2 * last < num_cus);
+  }
+  return slabs <= 2 && !(layoutA == GZ_COL_MAJOR && layoutB == GZ_ROW_MAJOR);
+}
+
 // The launcher's own choice for one launch over the whole problem; returns the estimate it was chosen by.
 // (staged_64: every 64 x 64 tile on the register-staged kernel, no smaller one - see mfma_plan_streamk)
 inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layoutB, int num_cus, MfmaCfg* out, bool staged_64 = false) {
@@ -281,9 +297,10 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
   // (a column-major A beside a row-major B goes through the transposing reads like B, not for the 8-bit floats; beside
   // a column-major B the launcher runs the transposed problem where it can, see mfma_transposed_ring)
   const bool f8_types = types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16;
-  const bool a_direct = a_rows || (!b_cols && !f8_types);
+  const bool short_tail = mfma_short_k_tail(types, M, N, K, layoutA, layoutB, num_cus);
+  const bool a_direct = (a_rows || (!b_cols && !f8_types)) && !short_tail;
   // (fp32: four waves with a row-major A)
-  const bool ring_ok = types == GZ_F32F32F32 ? a_rows : a_direct;
+  const bool ring_ok = types == GZ_F32F32F32 ? a_rows && !short_tail : a_direct;
   const bool ring128_ok = ring_ok && !f8_types;
   const int cand[4] = {ring_ok ? MFMA_CFG_RING_W4 : MFMA_CFG_256_W4, MFMA_CFG_256x128,
                        ring128_ok ? MFMA_CFG_RING_128 : MFMA_CFG_128, MFMA_CFG_64};
@@ -352,7 +369,7 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
     }
     const long long rounds = (tiles + num_cus - 1) / num_cus;
     // whole tiles: every candidate has a direct-to-LDS kernel; ragged M, N or K: the ring kernel
-    const int cls = mfma_shape_class(c, in_size, M, N, K, layoutA, layoutB);
+    const int cls = short_tail ? (int)MFMA_SHAPE_GENERAL : mfma_shape_class(c, in_size, M, N, K, layoutA, layoutB);
     const bool direct = (types == GZ_F32F32F32 ? a_rows && (i == 0 || i == 2) : a_direct) &&
                         (cls == MFMA_SHAPE_WHOLE || (cls == MFMA_SHAPE_RAGGED && (i == 0 || (i == 2 && ring128_ok))));
     // (128 x 128 beyond four rounds: each further round costs a little more, 6144^2 x 6144 = 9 rounds measured
@@ -574,7 +591,7 @@ inline void mfma_adjust_general(int types, int cls, int layoutA, int layoutB, Mf
   // 4096^3, int8 84 / 77, bf16 135 / 124 and 144 / 128 with a row-major B)
   const bool f8 = types == GZ_E4M3E4M3F16 || types == GZ_E5M2E5M2F16;
   const bool a_staged = layoutA != GZ_ROW_MAJOR && (layoutB != GZ_ROW_MAJOR || f8 || types == GZ_F32F32F32);
-  const bool staged = cls == MFMA_SHAPE_GENERAL || a_staged;
+  const bool staged = cls == MFMA_SHAPE_GENERAL || (cls == MFMA_SHAPE_RAGGED && c->ring == 0) || a_staged;
   if (!staged || c->bm != 256 || c->bn != 256) return;
   if (f8) *c = kMfmaCfgs[MFMA_CFG_256_W4];
   else if (types != GZ_F32F32F32) *c = kMfmaCfgs[MFMA_CFG_256_W8];
@@ -616,7 +633,8 @@ inline bool mfma_resolve_split(int types, int M, int N, int K, int layoutA, int 
   double cost_main = mfma_choose(types, rows_main, N, K, layoutA, layoutB, num_cus, &main_cfg, staged_64);
   if (main_cfg.bm != 256 || main_cfg.bn != 256) return false;
   // only where the first launch runs a direct-to-LDS kernel, whose speed the estimate knows well
-  if (mfma_shape_class(main_cfg, mfma_in_size(types), rows_main, N, K, layoutA, layoutB) == MFMA_SHAPE_GENERAL) return false;
+  const int cls = mfma_shape_class(main_cfg, mfma_in_size(types), rows_main, N, K, layoutA, layoutB);
+  if (cls == MFMA_SHAPE_GENERAL || (cls == MFMA_SHAPE_RAGGED && main_cfg.ring == 0)) return false;
   // (fp32 with a K that is not whole slabs: 128 x 128 tiles of the ring kernel spread it as evenly in one launch)
   if (types == GZ_F32F32F32 && K % (MFMA_SLAB_BYTES / 4)) return false;
   const double cost_tail = mfma_choose(types, M - rows_main, N, K, layoutA, layoutB, num_cus, &tail_cfg, staged_64);

@@ -72,3 +72,17 @@ def test_short_parts_of_a_split_k_run_on_the_staged_kernel(capi):
     short, long = capi.plan(BF16F32, 62, 256, 8320, 0, 1), capi.plan(BF16F32, 36, 7296, 7168, 0, 1)
     assert short.split_k > 1 and short.wave_m == 32      # 9.2 us staged, 10.2 on slabs of the waves' own
     assert long.split_k > 1 and long.wave_m == 64
+
+
+@pytest.mark.parametrize("types,m,n,k,la,lb,tile,ring", [
+    (E5M2, 6736, 6944, 160, 0, 1, 128, False),     # 44 on the ring kernel's 256 x 256, 37
+    (E4M3, 4160, 4928, 368, 0, 0, 128, False),     # past a round, the last one less than half full
+    (E4M3, 3520, 3520, 368, 0, 0, 256, True),      # one round
+    (S8, 3328, 2944, 240, 0, 1, 256, False),       # 1.08 of the staged kernel's time on the ring kernel
+    (BF16F32, 4096, 2240, 120, 1, 1, 256, False),  # 14.4 on the ring kernel, 13.1
+    (BF16F32, 4096, 2240, 120, 1, 0, 256, True),
+    (BF16F32, 4096, 2240, 248, 0, 0, 256, True),   # four slabs
+])
+def test_a_short_k_tail(capi, types, m, n, k, la, lb, tile, ring):
+    p = capi.plan(types, m, n, k, la, lb)
+    assert p.tile_m == tile and (p.variant in (5, 6, 11)) == ring, p.as_dict()

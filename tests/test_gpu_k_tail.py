@@ -76,6 +76,24 @@ def test_a_tail_where_work_groups_walk_several_tiles(G, types, variant):
         assert np.array_equal(got, one)
 
 
+@pytest.mark.parametrize("la,lb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("types", TYPES)
+def test_a_tail_of_two_slabs_on_the_launchers_choice(G, types, la, lb):
+    """One slab and a piece, two slabs less a piece: the launcher's own tile, which the ring kernel's start would hold up, and
+    the ring kernel itself."""
+    es = np.dtype(O.IN_DTYPE[types]).itemsize
+    slab, piece = 128 // es, 16 // es
+    m, n = 2560 + 48, 3072 + 16
+    for k in (slab + piece, 2 * slab - piece):
+        a, b, c = O.make_inputs(types, m, n, k, kind=exact_kind(types), seed=k)
+        print("case", types, m, n, k, la, lb, flush=True)
+        got = G.run_gemm(types, a, b, c, m, n, k, la, lb, 1, 1, MFMA, 0)
+        for rows in ((0, 8), (1276, 1284), (m - 8, m)):
+            ref = O.gemm(types, a, b, c, m, n, k, la, lb, 1, 1, rows=rows)
+            assert np.array_equal(got[rows[0]:rows[1]], ref[rows[0]:rows[1]]), (types, k, la, lb, rows)
+        assert np.array_equal(got, G.run_gemm(types, a, b, c, m, n, k, la, lb, 1, 1, MFMA, 5))
+
+
 @pytest.mark.parametrize("types,inf", [(O.BF16BF16F32, 0x7F80), (O.F32F32F32, np.inf)])
 @pytest.mark.parametrize("la,lb", [(0, 1), (1, 0)])
 def test_an_infinity_in_the_overlap_stays_one(G, types, inf, la, lb):
