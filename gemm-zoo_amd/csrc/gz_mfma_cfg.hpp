@@ -505,8 +505,9 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // four beyond.  e4m3, us, four / eight waves, row/row: 4096^3 56.2 / 53.3, 5120^3 122.8 / 115.7, 6144^3
       // 221.5 / 213.0, 4096^2 x 8192 99.6 / 99.0, 8192^3 404.9 / 419.4; row/col 4096^3 53.8 / 50.9, 8192^3
       // 386.5 / 401.4.  (A row-major B: eight waves at every size, see below.)
-      // (K that is not whole slabs: four, whose instance has the registers for the clamped offsets - e4m3 4096 x 4096 x
-      // 4000 57.6 / 58.0, 2048 x 7824 x 1088 25.7 / 28.9, 5008^3 124 / 138, row/row 4096^2 x 1040 27.2 / 26.6)
+      // (K that is not whole slabs: four past 24 slabs with a K-contiguous B, eight / four 16 slabs 0.92 - 0.97, 24
+      // 0.97 - 1.00, 32 0.97 - 1.05, 48 1.02 - 1.07, from memory more (6976 x 2384 x 3472 80.8 / 71.5); a row-major B
+      // eight, 0.77 - 0.95 up to 16 slabs, 0.96 - 1.01 at 64.)
       // (A K-contiguous B and operands of 40 MB and more, which come from memory more than from the caches: four, on whole
       // tiles from K = 6144 or 60 MB on - us, four / eight, operands just used; from memory: 1000 x 14336 x 4096 47.9 /
       // 47.2; 49.8 / 56.7, 1500 x 8192 x 4096 46.1 / 44.2; 48.1 / 54.5, 1536 x 8192 x 8192 79.8 / 77.4; 83.6 / 93.8, 2048 x
@@ -515,7 +516,7 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
       // 8192 x 2048 29.7 / 27.4)
       const long long operands = ((long long)M + N) * K;
       const bool from_memory = b_cols && operands >= 40000000LL && (M % 256 || N % 256 || K >= 6144 || operands >= 60000000LL);
-      eight = !(tiles >= 4LL * num_cus && b_cols) && !k_tail && !from_memory;
+      eight = !(b_cols && (tiles >= 4LL * num_cus || (k_tail && K > 24 * MFMA_SLAB_BYTES))) && !from_memory;
     } else {
       // int8 and the 16-bit types: an estimate of the launch on four and on eight waves, in us per round of tiles,
       // a fixed part (first copies, epilogue) and a part per K slab.  Eight waves (two per SIMD, 128 x 64 per wave)

@@ -86,3 +86,13 @@ def test_short_parts_of_a_split_k_run_on_the_staged_kernel(capi):
 def test_a_short_k_tail(capi, types, m, n, k, la, lb, tile, ring):
     p = capi.plan(types, m, n, k, la, lb)
     assert p.tile_m == tile and (p.variant in (5, 6, 11)) == ring, p.as_dict()
+
+
+def test_waves_of_the_8_bit_floats_with_a_k_tail(capi):
+    """Eight, but for a K-contiguous B past 24 slabs (eight / four 0.92 - 1.00 up to 24 slabs, 0.97 - 1.05 at 32; a row-major
+    B 0.77 - 1.01)."""
+    for types in (E4M3, E5M2):
+        assert capi.plan(types, 3520, 3520, 1040, 0, 0).threads == 512
+        assert capi.plan(types, 3520, 3520, 4000, 0, 0).threads == 512
+        assert capi.plan(types, 3520, 3520, 1040, 0, 1).threads == 512
+        assert capi.plan(types, 3520, 3520, 4000, 0, 1).threads == 256
