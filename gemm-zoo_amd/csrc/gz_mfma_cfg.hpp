@@ -130,11 +130,12 @@ inline bool mfma_whole_tiles(const MfmaCfg& c, int in_size, int M, int N, int K)
 //     256x256   rounds                      one work-group per compute unit
 //     256x128   0.75 rounds                 one work-group per compute unit, more operand bytes per flop
 //     128x128   0.40 + 0.27 rounds          two work-groups share a compute unit; a lone one cannot fill it
-// (rounds = tiles of that size / compute units, rounded up), times the register-staged kernel's factor (see `staged` below) where the
-// problem cannot use a direct-to-LDS kernel, times 1.12 / 1.15 for the two smaller tiles on a row-major B (4096^3 row/row: 152 / 150 / 119).  A 256x256 tile needs the fewest bytes per flop and runs the hand-scheduled kernels, but a grid that does
-// not fill the device, or that leaves a nearly empty last round (N = 4097: 17 tile columns for one column of data),
-// is better served by smaller tiles.  Fitted to bf16 row/col squares, K = M = N (us, variants 3 / 4 / 6 =
-// 128x128 / 256x128 / 256x256):
+// (rounds = tiles of that size / compute units, rounded up), times the register-staged kernel's factor (see `staged` below)
+// where the problem cannot use a direct-to-LDS kernel, times 1.12 / 1.15 for the two smaller tiles on a row-major B (4096^3
+// row/row: 152 / 150 / 119).  A 256x256 tile needs the fewest bytes per flop and runs the hand-scheduled kernels, but a
+// grid that does not fill the device, or that leaves a nearly empty last round (N = 4097: 17 tile columns for one column of
+// data), is better served by smaller tiles.  Fitted to bf16 row/col squares, K = M = N (us, variants 3 / 4 / 6 = 128x128 /
+// 256x128 / 256x256):
 //     2048: 32 / 41 / 54     2560: 49 / 49 / 65     2816: 57 / 54 / 69     3072: 85 / 106 / 75
 //     3328: 92 / 112 / 82    3584: 117 / 119 / 96   3840: 131 / 130 / 110  6144 (K 4096): 312 / 332 / 318
 // and fp16 4095 x 4097 x 1023 on the predicated kernel: 112 / 143 / 153.
@@ -337,12 +338,11 @@ inline double mfma_choose(int types, int M, int N, int K, int layoutA, int layou
         if (tiles <= 2LL * num_cus)
           cost64 = mfma_64_us(types, M, N, K, layoutA, layoutB, num_cus) / (16.0 + 1.45 * ((double)K * in_size / MFMA_SLAB_BYTES));
       } else if (tiles * 5 <= (b_cols || f8_types ? 10LL : 6LL) * num_cus) {
-        // 8- and 16-bit types, up to two tiles per compute unit (int8 and 16-bit, 1.2 with a row-major B: 1280^2 x 2048 22.1 / 20.5, with a
-        // K-contiguous B 18.5 / 20.0; 1024 x 2048 x 4096, two per compute unit, 30.1 / 33.5; 1536^2 x 2048, 2.25,
-        // 22.1 / 19.9): a tile costs 1.3 + 0.49 us per slab against the
-        // 16 + 1.45 of a round of 256 x 256 (us, 64 x 64 / 128 x 128 ring, bf16 -> f32 cubes, row/col: 256 4.7 / 6.3,
-        // 512 5.2 / 7.6, 768 7.5 / 10.6, 1024 9.1 / 12.4, 1280 12.5 / 14.5, 1536 18.8 / 16.6; row/row 1024
-        // 10.5 / 12.8, 1280 14.8 / 14.9; fp16 the same).
+        // 8- and 16-bit types, up to two tiles per compute unit (int8 and 16-bit, 1.2 with a row-major B: 1280^2 x 2048
+        // 22.1 / 20.5, with a K-contiguous B 18.5 / 20.0; 1024 x 2048 x 4096, two per compute unit, 30.1 / 33.5; 1536^2 x
+        // 2048, 2.25, 22.1 / 19.9): a tile costs 1.3 + 0.49 us per slab against the 16 + 1.45 of a round of 256 x 256 (us,
+        // 64 x 64 / 128 x 128 ring, bf16 -> f32 cubes, row/col: 256 4.7 / 6.3, 512 5.2 / 7.6, 768 7.5 / 10.6, 1024 9.1 /
+        // 12.4, 1280 12.5 / 14.5, 1536 18.8 / 16.6; row/row 1024 10.5 / 12.8, 1280 14.8 / 14.9; fp16 the same).
         const double nslab = (double)K * in_size / MFMA_SLAB_BYTES, t = (double)tiles / num_cus;
         cost64 = (1.3 + 0.49 * nslab) / (16.0 + 1.45 * nslab) * (t <= 1.0 ? 0.8 + 0.2 * t : 1.0 + 0.35 * (t - 1.0));
       }
